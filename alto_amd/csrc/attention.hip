@@ -6,8 +6,10 @@
 // that land in lanes): S tiles and O tiles keep the query row in the lane (lane % 32) and spread keys / value columns
 // over the 16 accumulator registers, so the per-row softmax state (running max, rescale factor) is one scalar per lane
 // and the only cross-lane traffic is between the two lanes (l, l ^ 32) that share a row.
+#include <algorithm>
 #include <type_traits>
 #include <utility>
+#include <vector>
 
 #include "common.h"
 
@@ -17,14 +19,32 @@ struct AttnArgs {
   const uint8_t* q;  const uint8_t* qs;    // [B, Hq, Sq, D/2],  [B, Hq, Sq/32, D/32]
   const uint8_t* k;  const uint8_t* ks;    // [B, Hk, Sk, D/2],  [B, Hk, Sk/32, D/32]
   const uint8_t* vt; const uint8_t* vs;    // [B, Hk, Dv, Sk/2] packed along keys, [B, Hk, Sk/32, Dv/32]
-  void* out; float* lse;                   // [B, Hq, Sq, Dv] bf16, [B, Hq, Sq] fp32
-  int Hq, Hk, Sq, Sk, Sk_used;             // Sk keys are allocated (a multiple of 64), the first Sk_used exist
+  void* out; float* lse;                   // bf16 and fp32, element (b, h, row, column) at the strides below
+  int64_t o_sb, o_sh, o_ss, l_sb, l_sh, l_ss;
+  int Hq, Hk, Sq, Sk, Sk_used;             // Sk keys are allocated, the first Sk_used exist (packed sequences: Sq and Sk are token counts)
+  int64_t k_bytes, v_bytes;                // extent of the code buffers
   float sm_scale;
   int causal;
   // optional additive terms on the scaled scores (triton_flash_attention_mxfp4.py:288-299), fp32:
   const float* bias;  int64_t bias_sb, bias_sh, bias_sm, bias_bytes;   // element (b, h, m, n) at b sb + h sh + m sm + n; NULL: none
   const float* alibi; int64_t alibi_sb, alibi_sh;                      // slope of (b, h) at b sb + h sh; NULL: none
 };
+
+// Sequences packed along the tokens (B = 1): sequence i owns query rows q0[i] .. + qn[i] and keys k0[i] .. + kn[i] (all
+// multiples of 32) and the row blocks z0[i] .. z0[i+1] of the grid.  By value, in the kernel arguments: no copy to the
+// device, nothing to keep alive.
+constexpr int ATTN_MAX_SEQS = 64;
+struct AttnSeqs {
+  int n;
+  int z0[ATTN_MAX_SEQS + 1], q0[ATTN_MAX_SEQS], qn[ATTN_MAX_SEQS], k0[ATTN_MAX_SEQS], kn[ATTN_MAX_SEQS];
+};
+struct AttnNoSeqs {};
+
+// Uniform 4-byte aligned data through the scalar cache: as vector loads these sat in the same counter as the direct-to-LDS
+// prefetch, and the wait for a block's scale bytes drained the prefetched block with them (three workgroups per CU hide
+// that: 205 us either way at 4 x 2048 x 64 heads x 128, causal).
+typedef const __attribute__((address_space(4))) uint32_t* scalar_u32;
+__device__ __forceinline__ scalar_u32 scalar_ptr(const uint8_t* p) { return (scalar_u32)(uintptr_t)p; }
 
 #ifndef ATTN_WG_PER_CU
 #define ATTN_WG_PER_CU 3
@@ -69,8 +89,10 @@ struct AttnTile {
 // in flight across the LDS reads that follow (unmarked, it puts an `s_waitcnt vmcnt(0)` before the next LDS read).
 // BIASED: the scores get a.bias and / or the ALiBi term -slope |row + Sk - Sq - key| added after the scaling and the mask,
 // before the running maximum (:288-308); a separate instantiation, the plain one carries none of it.
-template <int NK, int ND, bool BIASED>
-__device__ __forceinline__ void attn_fwd_body(const AttnArgs& a, __bf16* __restrict__ out, float* __restrict__ lse_out, uint8_t* ring) {
+// SEQS: AttnSeqs, or AttnNoSeqs for B sequences of one length.
+template <int NK, int ND, bool BIASED, typename SEQS>
+__device__ __forceinline__ void attn_fwd_body(const AttnArgs& a, const SEQS& seqs, __bf16* __restrict__ out, float* __restrict__ lse_out, uint8_t* ring) {
+  constexpr bool PACKED = std::is_same<SEQS, AttnSeqs>::value;
   constexpr int D = NK * 64, DV = ND * 32;
   constexpr int K_BYTES = AttnTile<NK, ND>::K_BYTES, V_BYTES = AttnTile<NK, ND>::V_BYTES, SLOT = AttnTile<NK, ND>::SLOT;
   constexpr int K_PIECES = K_BYTES / 16, V_PIECES = V_BYTES / 16;
@@ -81,23 +103,35 @@ __device__ __forceinline__ void attn_fwd_body(const AttnArgs& a, __bf16* __restr
   const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int r = lane & 31, h = lane >> 5;
   // grid (heads, batch, row blocks): with a causal mask every head's longest rows are dispatched before anybody's shorter
-  // ones, so the launch ends with the cheapest workgroups
-  const int qblk = a.causal ? (int)(gridDim.z - 1 - blockIdx.z) : (int)blockIdx.z;
+  // ones, so the launch ends with the cheapest workgroups (packed sequences: the host passes them longest first)
+  int qn = a.Sq, kn = a.Sk_used, q_first = 0, k_first = 0, z = (int)blockIdx.z, nz = (int)gridDim.z;
+  if constexpr (PACKED) {
+    int lo = 0, hi = seqs.n - 1;   // the sequence this row block belongs to: the last one with z0[i] <= z
+    while (lo < hi) {
+      const int mid = (lo + hi + 1) >> 1;
+      if (seqs.z0[mid] <= z) lo = mid; else hi = mid - 1;
+    }
+    qn = seqs.qn[lo]; kn = seqs.kn[lo]; q_first = seqs.q0[lo]; k_first = seqs.k0[lo];
+    nz = seqs.z0[lo + 1] - seqs.z0[lo];
+    z -= seqs.z0[lo];
+  }
+  const int qblk = a.causal ? nz - 1 - z : z;
   const int q0 = (qblk * 4 + wave) * 32;
-  const bool live = q0 < a.Sq;                    // a wave past the last row still helps with loads and barriers
+  const bool live = q0 < qn;                      // a wave past the last row still helps with loads and barriers
   const int hq = blockIdx.x, b = blockIdx.y;
   const int hk = hq / (a.Hq / a.Hk);
-  const int64_t bhq = (int64_t)b * a.Hq + hq, bhk = (int64_t)b * a.Hk + hk;
+  // rows of the operand buffers where this (sequence, head) starts
+  const int64_t q_base = ((int64_t)b * a.Hq + hq) * a.Sq + q_first, bhk = (int64_t)b * a.Hk + hk, k_base = bhk * a.Sk + k_first;
   const int qrow = live ? q0 + r : 0;
-  const int shift = a.Sk_used - a.Sq;                  // causal mask is aligned to the bottom-right corner
+  const int shift = kn - qn;                           // causal mask is aligned to the bottom-right corner
 
   // ---- Q pieces: row qrow, K step ks, half h -> 16 bytes; one scale byte per (32-row block, 32-column block)
   v8i_t qf[NK];
   int qsc[NK];
 #pragma unroll
   for (int s = 0; s < NK; ++s) {
-    qf[s] = frag16(a.q + (bhq * a.Sq + qrow) * (D / 2) + s * 32 + h * 16);
-    qsc[s] = a.qs[(bhq * (a.Sq / 32) + qrow / 32) * (D / 32) + 2 * s + h];
+    qf[s] = frag16(a.q + (q_base + qrow) * (D / 2) + s * 32 + h * 16);
+    qsc[s] = a.qs[(q_base / 32 + qrow / 32) * (D / 32) + 2 * s + h];
   }
 
   v16f_t acc_o[ND], acc_l;
@@ -119,13 +153,13 @@ __device__ __forceinline__ void attn_fwd_body(const AttnArgs& a, __bf16* __restr
   const v8i_t ones = v8i_t{0x22222222, 0x22222222, 0x22222222, 0x22222222, 0, 0, 0, 0};   // E2M1 code 2 = 1.0
 
   // blocks this wave needs, and the most any wave of the workgroup needs (the last wave's rows reach furthest)
-  const int all_blk = (a.Sk_used + 63) / 64;
+  const int all_blk = (kn + 63) / 64;
   int nblk = all_blk, wg_blk = all_blk;
   if (a.causal) {
     const int lim = (q0 + 32 + shift + 63) / 64;
     nblk = lim < all_blk ? lim : all_blk;
     int q_end = qblk * 128 + 128;
-    q_end = q_end < a.Sq ? q_end : a.Sq;
+    q_end = q_end < qn ? q_end : qn;
     const int wlim = (q_end + shift + 63) / 64;
     wg_blk = wlim < all_blk ? wlim : all_blk;
   }
@@ -133,10 +167,13 @@ __device__ __forceinline__ void attn_fwd_body(const AttnArgs& a, __bf16* __restr
 
   // ---- cooperative fetch of one block: wave instruction j moves pieces [256 j + 64 wave, + 64) of the block, K pieces
   // first (contiguous in memory), then V pieces (piece p = 16 bytes of row p / 2, half p % 2); the piece index is also the
-  // position in the slot.  Blocks beyond the keys are out of the descriptors' range and arrive as zeros.
+  // position in the slot.  A last block that reaches past its sequence holds whatever codes follow in the buffer (zeros
+  // beyond its end): those keys are masked, so their probabilities are exact zeros.
   typedef __attribute__((address_space(3))) uint8_t lds_u8;
-  const __amdgpu_buffer_rsrc_t rsrc_k = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(a.k + bhk * a.Sk * (D / 2)), 0, a.Sk * (D / 2), 0x00020000);
-  const __amdgpu_buffer_rsrc_t rsrc_v = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(a.vt + bhk * DV * (int64_t)(a.Sk / 2)), 0, DV * (a.Sk / 2), 0x00020000);
+  auto extent = [](int64_t want, int64_t left) { return (int)(want < left ? want : left); };   // (want < 2^31: checked on the host)
+  const int64_t k_off = k_base * (D / 2), v_off = bhk * DV * (int64_t)(a.Sk / 2) + k_first / 2;
+  const __amdgpu_buffer_rsrc_t rsrc_k = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(a.k + k_off), 0, extent((int64_t)all_blk * 64 * (D / 2), a.k_bytes - k_off), 0x00020000);
+  const __amdgpu_buffer_rsrc_t rsrc_v = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(a.vt + v_off), 0, extent((int64_t)DV * (a.Sk / 2) + 32, a.v_bytes - v_off), 0x00020000);
   // Where a piece sits inside its row of the slot: the LDS serves a 16-byte read of 16 lanes per pass from 64 banks
   // (256 bytes), and the 16 lanes of a fragment read ask for the same piece of 16 consecutive rows.  With PR pieces per
   // row, 16 / PR rows share a 256-byte line; piece c of row `row` goes to position c ^ ((row / (16 / PR)) % PR), which
@@ -170,17 +207,34 @@ __device__ __forceinline__ void attn_fwd_body(const AttnArgs& a, __bf16* __restr
     else __builtin_amdgcn_s_waitcnt(0x0070 | 0x0F00 | ((DMA_MAX - 1) & 15));
   };
   // Scale bytes of a block: 2 D/32 bytes of K (key tile t, 32-column block j at byte t D/32 + j) and 2 Dv/32 bytes of V
-  // (key tile t, column block d at byte t Dv/32 + d) sit at wave-uniform, 4-byte aligned addresses: whole dwords, one
-  // block ahead; the MFMA picks a byte of a dword with op_sel, the lane half h shifts its byte into place.
+  // (key tile t, column block d at byte t Dv/32 + d) sit at wave-uniform addresses: whole dwords by scalar loads, one block
+  // ahead; the MFMA picks a byte of a dword with op_sel, the lane half h shifts its byte into place.  The address is a
+  // multiple of 4 except for head dims of 64 and 192, whose 32-row bands have 2 or 6 bytes: a sequence or head that starts
+  // at an odd band is then read from the dword below and shifted down by two bytes.
   constexpr int KS_DW = 2 * (D / 32) / 4, VS_DW = (2 * (DV / 32) + 3) / 4;
+  constexpr bool K_ODD = (D / 32) % 4 != 0, V_ODD = (DV / 32) % 4 != 0;
   uint32_t ksw[KS_DW], vsw[VS_DW], ksw_next[KS_DW], vsw_next[VS_DW];
+  auto fetch = [](const uint8_t* p, auto oddc, auto& w) {
+    constexpr int N = sizeof(w) / 4;
+    if constexpr (decltype(oddc)::value) {
+      const uint32_t odd = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)p & 2u);
+      const scalar_u32 q = scalar_ptr(p - odd);
+      uint32_t t[N + 1];
+#pragma unroll
+      for (int i = 0; i < N; ++i) t[i] = q[i];
+      t[N] = q[odd ? N : 0];   // (never past the dword that holds the last byte)
+#pragma unroll
+      for (int i = 0; i < N; ++i) w[i] = (uint32_t)((((uint64_t)t[i + 1] << 32) | t[i]) >> (8 * odd));
+    } else {
+      const scalar_u32 q = scalar_ptr(p);
+#pragma unroll
+      for (int i = 0; i < N; ++i) w[i] = q[i];
+    }
+  };
   auto fetch_scales = [&](int kb, uint32_t (&kw)[KS_DW], uint32_t (&vw)[VS_DW]) {
-    const uint32_t* kp = reinterpret_cast<const uint32_t*>(a.ks + (bhk * (a.Sk / 32) + kb * 2) * (D / 32));
-    const uint32_t* vp = reinterpret_cast<const uint32_t*>(a.vs + (bhk * (a.Sk / 32) + kb * 2) * (DV / 32));
-#pragma unroll
-    for (int i = 0; i < KS_DW; ++i) kw[i] = kp[i];
-#pragma unroll
-    for (int i = 0; i < VS_DW; ++i) vw[i] = vp[i];
+    const int64_t band = k_base / 32 + kb * 2;
+    fetch(a.ks + band * (D / 32), std::bool_constant<K_ODD>{}, kw);
+    fetch(a.vs + band * (DV / 32), std::bool_constant<V_ODD>{}, vw);
   };
   if (wg_blk > 0) {
     fetch_scales(0, ksw_next, vsw_next);
@@ -243,14 +297,14 @@ __device__ __forceinline__ void attn_fwd_body(const AttnArgs& a, __bf16* __restr
           }
       }
       // ---- mask (only blocks the diagonal crosses or that reach past the last key), running max kept in the base-2 domain: m = max(S) * sm_scale * log2(e)
-      if ((a.causal && key0 + 63 > q0 + shift) || key0 + 64 > a.Sk_used) {
+      if ((a.causal && key0 + 63 > q0 + shift) || key0 + 64 > kn) {
         asm volatile("" ::: "memory");   // keep this a branch: most blocks skip it
 #pragma unroll
         for (int t = 0; t < 2; ++t)
 #pragma unroll
           for (int v = 0; v < 16; ++v) {
             const int key = key0 + 32 * t + 8 * (v >> 2) + 4 * h + (v & 3);
-            if ((a.causal && key > qrow + shift) || key >= a.Sk_used) S[t][v] = -__builtin_inff();
+            if ((a.causal && key > qrow + shift) || key >= kn) S[t][v] = -__builtin_inff();
           }
       }
       float tmx[2];   // row maximum of each 32-key tile (exp2 is monotonic: its largest probability comes from this score)
@@ -328,7 +382,7 @@ __device__ __forceinline__ void attn_fwd_body(const AttnArgs& a, __bf16* __restr
   // ---- O = acc / l, bf16; log-sum-exp
   const float l = acc_l[0];
   const float rl = 1.0f / l;
-  __bf16* orow = out + (bhq * a.Sq + qrow) * DV;
+  __bf16* orow = out + b * a.o_sb + hq * a.o_sh + (q_first + qrow) * a.o_ss;
 #pragma unroll
   for (int d = 0; d < ND; ++d)
 #pragma unroll
@@ -343,28 +397,34 @@ __device__ __forceinline__ void attn_fwd_body(const AttnArgs& a, __bf16* __restr
       w.y = __builtin_bit_cast(uint32_t, hi);
       *reinterpret_cast<uint2*>(orow + 32 * d + 8 * g + 4 * h) = w;
     }
-  if (h == 0) lse_out[bhq * a.Sq + qrow] = (m_i + log2f(l)) * ATTN_LN2;
+  if (h == 0) lse_out[b * a.l_sb + hq * a.l_sh + (q_first + qrow) * a.l_ss] = (m_i + log2f(l)) * ATTN_LN2;
 }
 
-template <int NK, int ND, bool BIASED>
-__global__ __launch_bounds__(256, BIASED ? 2 : ATTN_WG_PER_CU) void attn_fwd_kernel(AttnArgs a) {
+template <int NK, int ND, bool BIASED, typename SEQS>
+__global__ __launch_bounds__(256, BIASED ? 2 : ATTN_WG_PER_CU) void attn_fwd_kernel(AttnArgs a, SEQS seqs) {
   __shared__ __attribute__((aligned(16))) uint8_t ring[ATTN_RING * AttnTile<NK, ND>::SLOT];
-  attn_fwd_body<NK, ND, BIASED>(a, reinterpret_cast<__bf16*>(a.out), a.lse, ring);
+  attn_fwd_body<NK, ND, BIASED>(a, seqs, reinterpret_cast<__bf16*>(a.out), a.lse, ring);
 }
 
-template <int NK, int ND>
-static int launch_attn(const AttnArgs& a, int B, hipStream_t st) {
-  dim3 grid((unsigned)a.Hq, (unsigned)B, (unsigned)((a.Sq + 127) / 128));
-  if (a.bias || a.alibi) hipLaunchKernelGGL((attn_fwd_kernel<NK, ND, true>), grid, dim3(256), 0, st, a);
-  else hipLaunchKernelGGL((attn_fwd_kernel<NK, ND, false>), grid, dim3(256), 0, st, a);
+template <int NK, int ND, typename SEQS>
+static int launch_attn(const AttnArgs& a, const SEQS& seqs, int B, int row_blocks, hipStream_t st) {
+  dim3 grid((unsigned)a.Hq, (unsigned)B, (unsigned)row_blocks);
+  if (a.bias || a.alibi) hipLaunchKernelGGL((attn_fwd_kernel<NK, ND, true, SEQS>), grid, dim3(256), 0, st, a, seqs);
+  else hipLaunchKernelGGL((attn_fwd_kernel<NK, ND, false, SEQS>), grid, dim3(256), 0, st, a, seqs);
   return check_launch("attention_fwd");
 }
 
-template <int NK>
-static int launch_attn_nd(const AttnArgs& a, int B, int Dv, hipStream_t st) {
-  switch (Dv) {
-    case 64: return launch_attn<NK, 2>(a, B, st);
-    case 128: return launch_attn<NK, 4>(a, B, st);
+template <typename SEQS>
+static int launch_attn_dims(const AttnArgs& a, const SEQS& seqs, int B, int row_blocks, int64_t D, int64_t Dv, hipStream_t st) {
+  switch (D + (Dv == 128 ? 1 : 0)) {
+    case 64: return launch_attn<1, 2>(a, seqs, B, row_blocks, st);
+    case 65: return launch_attn<1, 4>(a, seqs, B, row_blocks, st);
+    case 128: return launch_attn<2, 2>(a, seqs, B, row_blocks, st);
+    case 129: return launch_attn<2, 4>(a, seqs, B, row_blocks, st);
+    case 192: return launch_attn<3, 2>(a, seqs, B, row_blocks, st);
+    case 193: return launch_attn<3, 4>(a, seqs, B, row_blocks, st);
+    case 256: return launch_attn<4, 2>(a, seqs, B, row_blocks, st);
+    case 257: return launch_attn<4, 4>(a, seqs, B, row_blocks, st);
   }
   return ALTO_MXFP4_EINVAL;
 }
@@ -403,16 +463,71 @@ extern "C" int alto_mxfp4_attention_fwd_ex(const void* q_codes, const void* q_sc
   ALTO_REQUIRE(((uintptr_t)k_scales | (uintptr_t)v_scales | (uintptr_t)lse | (uintptr_t)alibi_slopes) % 4 == 0,
                "attention_fwd: K and V scale pointers, lse and the alibi slopes must be 4-byte aligned");
   AttnArgs a{(const uint8_t*)q_codes, (const uint8_t*)q_scales, (const uint8_t*)k_codes, (const uint8_t*)k_scales,
-             (const uint8_t*)vt_codes, (const uint8_t*)v_scales, out, lse, (int)Hq, (int)Hk, (int)Sq, (int)Sk, (int)Sk_used, sm_scale, causal ? 1 : 0,
+             (const uint8_t*)vt_codes, (const uint8_t*)v_scales, out, lse, Hq * Sq * Dv, Sq * Dv, Dv, Hq * Sq, Sq, 1, (int)Hq, (int)Hk, (int)Sq, (int)Sk,
+             (int)Sk_used, B * Hk * Sk * (D / 2), B * Hk * Dv * (Sk / 2), sm_scale, causal ? 1 : 0,
              bias, bias_sb, bias_sh, bias_sm, bias_bytes, alibi_slopes, alibi_sb, alibi_sh};
+  return launch_attn_dims(a, AttnNoSeqs{}, (int)B, (int)((Sq + 127) / 128), D, Dv, (hipStream_t)stream);
+}
+
+extern "C" int alto_mxfp4_attention_fwd_strided(const void* q_codes, const void* q_scales, const void* k_codes, const void* k_scales,
+                                                const void* vt_codes, const void* v_scales, void* out, float* lse, int64_t B, int64_t Hq,
+                                                int64_t Hk, int64_t Sq, int64_t Sk, int64_t D, int64_t Dv, int64_t o_sb, int64_t o_sh, int64_t o_ss,
+                                                int64_t l_sb, int64_t l_sh, int64_t l_ss, int n_seqs, const int32_t* cu_q, const int32_t* cu_k,
+                                                float sm_scale, int causal, const float* alibi_slopes, int64_t alibi_sb, int64_t alibi_sh, void* stream) {
+  using namespace alto;
+  ALTO_REQUIRE(q_codes && q_scales && k_codes && k_scales && vt_codes && v_scales && out && lse, "attention_fwd: null pointer");
+  ALTO_REQUIRE(!alibi_slopes || (alibi_sb >= 0 && alibi_sh >= 0), "attention_fwd: negative alibi strides");
+  ALTO_REQUIRE(B > 0 && Hq > 0 && Hk > 0 && Hq % Hk == 0, "attention_fwd: Hq=%lld must be a positive multiple of Hk=%lld", (long long)Hq, (long long)Hk);
+  ALTO_REQUIRE(Sq > 0 && Sq % 32 == 0 && Sk > 0 && Sk % 32 == 0, "attention_fwd: Sq=%lld and Sk=%lld must be positive multiples of 32", (long long)Sq, (long long)Sk);
+  ALTO_REQUIRE(D == 64 || D == 128 || D == 192 || D == 256, "attention_fwd: head dim D=%lld must be 64, 128, 192 or 256", (long long)D);
+  ALTO_REQUIRE(Dv == 64 || Dv == 128, "attention_fwd: value dim Dv=%lld must be 64 or 128", (long long)Dv);
+  ALTO_REQUIRE(B <= 65535 && Sq < (1ll << 31) && Sk < (1ll << 31) && Hq < (1ll << 31), "attention_fwd: size out of range");
+  ALTO_REQUIRE(product_below(1ll << 40, B * Sq, Hq, D > Dv ? D : Dv) && product_below(1ll << 40, B * Sk, Hk, D > Dv ? D : Dv) && product_below(1ll << 31, Sk, D) &&
+                   product_below(1ll << 31, Sk, Dv), "attention_fwd: tensor too large");
+  ALTO_REQUIRE(o_sb >= 0 && o_sh >= 0 && o_ss >= 0 && l_sb >= 0 && l_sh >= 0 && l_ss >= 0 && (o_sb | o_sh | o_ss) % 4 == 0,
+               "attention_fwd: output strides must be non-negative, those of out multiples of 4 elements");
+  ALTO_REQUIRE((o_sb | o_sh | o_ss | l_sb | l_sh | l_ss) < (1ll << 40), "attention_fwd: output stride out of range");
+  ALTO_REQUIRE(((uintptr_t)q_codes | (uintptr_t)k_codes | (uintptr_t)vt_codes) % 16 == 0 && (uintptr_t)out % 8 == 0,
+               "attention_fwd: code pointers must be 16-byte aligned, out 8-byte aligned");
+  ALTO_REQUIRE(((uintptr_t)k_scales | (uintptr_t)v_scales | (uintptr_t)lse | (uintptr_t)alibi_slopes) % 4 == 0,
+               "attention_fwd: K and V scale pointers, lse and the alibi slopes must be 4-byte aligned");
+  AttnArgs a{(const uint8_t*)q_codes, (const uint8_t*)q_scales, (const uint8_t*)k_codes, (const uint8_t*)k_scales,
+             (const uint8_t*)vt_codes, (const uint8_t*)v_scales, out, lse, o_sb, o_sh, o_ss, l_sb, l_sh, l_ss, (int)Hq, (int)Hk, (int)Sq, (int)Sk,
+             (int)Sk, B * Hk * Sk * (D / 2), B * Hk * Dv * (Sk / 2), sm_scale, causal ? 1 : 0, nullptr, 0, 0, 0, 0, alibi_slopes, alibi_sb, alibi_sh};
   hipStream_t st = (hipStream_t)stream;
-  switch (D) {
-    case 64: return launch_attn_nd<1>(a, (int)B, (int)Dv, st);
-    case 128: return launch_attn_nd<2>(a, (int)B, (int)Dv, st);
-    case 192: return launch_attn_nd<3>(a, (int)B, (int)Dv, st);
-    case 256: return launch_attn_nd<4>(a, (int)B, (int)Dv, st);
+  if (n_seqs == 0) {
+    ALTO_REQUIRE(!causal || Sq <= Sk, "attention_fwd: causal attention needs Sq <= Sk (got %lld > %lld)", (long long)Sq, (long long)Sk);
+    ALTO_REQUIRE((Sq + 127) / 128 <= 65535, "attention_fwd: Sq / 128 must fit a grid dimension");
+    return launch_attn_dims(a, AttnNoSeqs{}, (int)B, (int)((Sq + 127) / 128), D, Dv, st);
   }
-  return ALTO_MXFP4_EINVAL;
+  ALTO_REQUIRE(n_seqs > 0 && cu_q && cu_k && B == 1, "attention_fwd: packed sequences need their boundaries and B = 1");
+  ALTO_REQUIRE(cu_q[0] == 0 && cu_k[0] == 0 && cu_q[n_seqs] == Sq && cu_k[n_seqs] == Sk, "attention_fwd: the sequence boundaries must run from 0 to the token counts");
+  for (int i = 0; i < n_seqs; ++i) {
+    ALTO_REQUIRE(cu_q[i + 1] > cu_q[i] && cu_k[i + 1] > cu_k[i] && cu_q[i + 1] % 32 == 0 && cu_k[i + 1] % 32 == 0,
+                 "attention_fwd: sequence boundaries must be increasing multiples of 32 tokens");
+    ALTO_REQUIRE(!causal || cu_q[i + 1] - cu_q[i] <= cu_k[i + 1] - cu_k[i], "attention_fwd: causal attention needs Sq <= Sk (got %d > %d)", cu_q[i + 1] - cu_q[i],
+                 cu_k[i + 1] - cu_k[i]);
+  }
+  // longest sequences first, up to ATTN_MAX_SEQS of them and 65535 row blocks per launch
+  std::vector<int> order((size_t)n_seqs);
+  for (int i = 0; i < n_seqs; ++i) order[(size_t)i] = i;
+  std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return cu_k[x + 1] - cu_k[x] > cu_k[y + 1] - cu_k[y]; });
+  for (int at = 0; at < n_seqs;) {
+    AttnSeqs t;
+    t.n = 0;
+    t.z0[0] = 0;
+    for (; at < n_seqs && t.n < ATTN_MAX_SEQS; ++at) {
+      const int s = order[(size_t)at], qn = cu_q[s + 1] - cu_q[s], blocks = (qn + 127) / 128;
+      ALTO_REQUIRE(blocks <= 65535, "attention_fwd: Sq / 128 must fit a grid dimension");
+      if (t.z0[t.n] + blocks > 65535) break;
+      t.q0[t.n] = cu_q[s]; t.qn[t.n] = qn; t.k0[t.n] = cu_k[s]; t.kn[t.n] = cu_k[s + 1] - cu_k[s];
+      t.z0[t.n + 1] = t.z0[t.n] + blocks;
+      ++t.n;
+    }
+    const int rc = launch_attn_dims(a, t, 1, t.z0[t.n], D, Dv, st);
+    if (rc != ALTO_MXFP4_OK) return rc;
+  }
+  return ALTO_MXFP4_OK;
 }
 
 extern "C" int alto_mxfp4_attention_fwd(const void* q_codes, const void* q_scales, const void* k_codes, const void* k_scales,

@@ -427,6 +427,34 @@ int alto_mxfp4_attention_fwd_ex(const void* q_codes, const void* q_scales, const
                                 const float* alibi_slopes, int64_t alibi_sb, int64_t alibi_sh, void* stream);
 
 /*
+ * Quantizes Q, K and V for the attention forward in one launch (the three 2D-block quantisations of
+ * triton_flash_attention_mxfp4.py:1105-1107, round to nearest even), reading the operands where they lie: q [B][Hq][Sq][D],
+ * k [B][Hk][Sk][D], v [B][Hk][Sk][Dv], bf16 or f32, element strides *_sb / *_sh / *_ss of the batch, head and row dims
+ * (multiples of 16 bytes), unit stride along the head dim.  Outputs dense, as alto_mxfp4_attention_fwd takes them:
+ * q_codes [B][Hq][Sq][D/2], k_codes [B][Hk][Sk][D/2], vt_codes [B][Hk][Dv][Sk/2] packed along the keys, scales
+ * [B][H][S/32][D/32].  Sq % 32 == 0, Sk % 32 == 0, D and Dv multiples of 64.
+ */
+int alto_mxfp4_attention_quantize(const void* q, const void* k, const void* v, int dtype, int64_t B, int64_t Hq, int64_t Hk, int64_t Sq,
+                                  int64_t Sk, int64_t D, int64_t Dv, int64_t q_sb, int64_t q_sh, int64_t q_ss, int64_t k_sb, int64_t k_sh,
+                                  int64_t k_ss, int64_t v_sb, int64_t v_sh, int64_t v_ss, uint8_t* q_codes, uint8_t* q_scales,
+                                  uint8_t* k_codes, uint8_t* k_scales, uint8_t* vt_codes, uint8_t* v_scales, void* stream);
+
+/*
+ * alto_mxfp4_attention_fwd on operands whose key count is any multiple of 32 (nothing is padded; the last block of 64 keys
+ * reads what follows in the buffers and masks it: allocate 16 bytes behind k_scales and v_scales), with the outputs at
+ * element strides o_* / l_* of batch, head and row (unit stride along Dv).
+ * n_seqs > 0: B = 1 and Sq / Sk count the tokens of n_seqs sequences packed along them (layout "thd" of
+ * triton_flash_attention_mxfp4.py:1199-1203): cu_q / cu_k are HOST arrays of n_seqs + 1 boundaries, multiples of 32 from
+ * 0 to Sq / Sk; every sequence attends to itself only, a causal mask sits in the bottom-right corner of its own score
+ * matrix.  alibi_slopes as in alto_mxfp4_attention_fwd_ex (distances inside the sequence), NULL: none.
+ */
+int alto_mxfp4_attention_fwd_strided(const void* q_codes, const void* q_scales, const void* k_codes, const void* k_scales,
+                                     const void* vt_codes, const void* v_scales, void* out, float* lse, int64_t B, int64_t Hq,
+                                     int64_t Hk, int64_t Sq, int64_t Sk, int64_t D, int64_t Dv, int64_t o_sb, int64_t o_sh, int64_t o_ss,
+                                     int64_t l_sb, int64_t l_sh, int64_t l_ss, int n_seqs, const int32_t* cu_q, const int32_t* cu_k,
+                                     float sm_scale, int causal, const float* alibi_slopes, int64_t alibi_sb, int64_t alibi_sh, void* stream);
+
+/*
  * Fills out[0 .. n) with random 32-bit words for stochastic rounding: word 4 c + j is word j of Philox4x32-10 (Salmon et
  * al., SC'11) with the 128-bit counter c + offset and the 64-bit key `seed`.  The reference draws its bits inside its
  * kernel from the same generator family (tl.randint4x, alto/kernels/fp4/fp4_common/triton_fp4_ops.py:15-18) with

@@ -206,8 +206,25 @@ Entry g_entries[] = {
      [](const Args& a) { return alto_mxfp4_random_bits(P(uint32_t, 0), a.s[0], a.u[0], a.u[1], nullptr); }},
     {"probe_mfma", 0, 3, 2, {{}, {1, 16, 256}, {D, D}, 1.0f, {0, 0}, g_signs, g_perm},
      [](const Args& a) { return alto_mxfp4_probe_mfma(a.i[0], a.i[1], a.i[2], P(float, 0), P(uint64_t, 1), nullptr); }},
+    // B, Hq, Hk, Sq, Sk, D, Dv, strides of q, k, v
+    {"attention_quantize", 16, 1, 9, {{2, 8, 2, 256, 96, 128, 64, 256 * 1024, 128, 1024, 96 * 256, 128, 256, 96 * 128, 64, 128}, {0}, {D, D, D, D, D, D, D, D, D}, 1.0f, {0, 0}, g_signs, g_perm},
+     [](const Args& a) {
+       return alto_mxfp4_attention_quantize(a.p[0], a.p[1], a.p[2], a.i[0], a.s[0], a.s[1], a.s[2], a.s[3], a.s[4], a.s[5], a.s[6], a.s[7], a.s[8], a.s[9],
+                                            a.s[10], a.s[11], a.s[12], a.s[13], a.s[14], a.s[15], P(uint8_t, 3), P(uint8_t, 4), P(uint8_t, 5), P(uint8_t, 6),
+                                            P(uint8_t, 7), P(uint8_t, 8), nullptr);
+     }},
+    // B, Hq, Hk, Sq, Sk, D, Dv, strides of out and lse, alibi strides; two sequences
+    {"attention_fwd_strided", 15, 2, 9, {{1, 8, 2, 256, 288, 128, 64, 0, 64, 512, 0, 1, 8, 8, 1}, {2, 1}, {D, D, D, D, D, D, D, D, D}, 0.088388f, {0, 0}, g_signs, g_perm},
+     [](const Args& a) {
+       static const int32_t cu_q[3] = {0, 96, 256}, cu_k[3] = {0, 128, 288};
+       const int n = a.i[0] == 2 ? 2 : 0;   // (the boundary arrays hold two sequences)
+       return alto_mxfp4_attention_fwd_strided(a.p[0], a.p[1], a.p[2], a.p[3], a.p[4], a.p[5], a.p[6], P(float, 7), a.s[0], a.s[1], a.s[2], a.s[3], a.s[4],
+                                               a.s[5], a.s[6], a.s[7], a.s[8], a.s[9], a.s[10], a.s[11], a.s[12], n, cu_q, cu_k, a.f, a.i[1],
+                                               P(const float, 8), a.s[13], a.s[14], nullptr);
+     }},
 };
 constexpr int kEntries = sizeof(g_entries) / sizeof(g_entries[0]);
+constexpr int kFirstTable = 30;   // entries behind these are counted by themselves
 
 void mutate(Args& a, const Entry& e) {
   const int fields = e.ns + e.ni + e.np + 4;   // + float, one of the two u64, signs, perm
@@ -238,7 +255,7 @@ int main(int argc, char** argv) {
   }
   std::printf("version %d\n", alto_mxfp4_version());
   (void)alto_mxfp4_init();   // no device here: must fail cleanly or do nothing
-  long calls = 0;
+  long calls = 0, more = 0;
   for (long it = 0; it < rounds; ++it) {
     for (int n = 0; n < kEntries; ++n) {
       Entry& e = g_entries[n];
@@ -246,7 +263,7 @@ int main(int argc, char** argv) {
       const int changes = (int)(next_u64() % 4);
       for (int c = 0; c < changes; ++c) mutate(a, e);
       const int rc = e.call(a);
-      ++calls;
+      ++(n < kFirstTable ? calls : more);
       ++e.calls;
       if (rc == -100) {
         std::fprintf(stderr, "call %ld (%s): a size query returned a negative number\n", calls, e.name);
@@ -278,6 +295,6 @@ int main(int argc, char** argv) {
     std::fprintf(stderr, "%d entry points never got past their argument checks: their valid argument set is not valid\n", never);
     return 4;
   }
-  std::printf("calls %ld\n", calls);
+  std::printf("calls %ld\nmore %ld\n", calls, more);
   return 0;
 }

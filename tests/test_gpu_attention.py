@@ -268,3 +268,46 @@ def test_reference_attention_configs(m, cfg):
     cos = float(torch.nn.functional.cosine_similarity(ref.float().flatten(), out.float().flatten(), dim=0))
     print(f"  SNR {snr:.2f} dB, cosine {cos:.5f}", flush=True)
     assert snr > 11.0 and cos > 0.96
+
+
+@pytest.mark.parametrize("dims", [(64, 64), (128, 128), (192, 64), (256, 128)], ids=lambda d: f"D{d[0]}_Dv{d[1]}")
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_operand_quantizer_reads_any_layout(m, dims, dtype):
+    """One launch for Q, K and V: codes and scales equal the oracle's for dense [B, H, S, D] tensors, [B, S, H, D] views and
+    slices of wider rows; row counts that leave one to four bands in the last group of 128 rows."""
+    D, Dv = dims
+    g = torch.Generator().manual_seed(D + Dv)
+    for B, Hq, Hk, Sq, Sk in ((1, 2, 1, 32, 96), (2, 3, 3, 160, 64), (1, 4, 2, 128, 288)):
+        for order in ("bhsd", "bshd", "slice"):
+            src = []
+            for H, S, d in ((Hq, Sq, D), (Hk, Sk, D), (Hk, Sk, Dv)):
+                x = torch.randn(B, H, S, d, generator=g) * torch.exp2(torch.randint(-8, 8, (B, H, S, 1), generator=g).float())
+                src.append(x.to(dtype))
+            if order == "bhsd":
+                dev = [x.to(DEV) for x in src]
+            elif order == "bshd":
+                dev = [x.transpose(1, 2).contiguous().to(DEV).transpose(1, 2) for x in src]
+            else:
+                dev = [torch.nn.functional.pad(x, (8, 16)).to(DEV)[..., 8:8 + x.shape[-1]] for x in src]
+            qq, qs, kq, ks, vq, vs = m.quantize_qkv(*dev)
+            for got, got_s, x in ((qq, qs, src[0]), (kq, ks, src[1])):
+                c, s = O.quantize(x, axis=-1, is_2d_block=True)
+                assert torch.equal(got.cpu(), c) and torch.equal(got_s.cpu(), s), (order, Sq, Sk)
+            c, s = O.quantize(src[2].transpose(-1, -2).contiguous(), axis=-1, is_2d_block=True)
+            assert torch.equal(vq.cpu(), c) and torch.equal(vs.cpu(), s.transpose(-1, -2)), (order, Sq, Sk)
+
+
+@pytest.mark.parametrize("D,Dv", [(64, 64), (192, 64), (128, 128)])
+def test_packed_sequences_that_start_at_odd_bands(m, D, Dv):
+    """Sequences of 32 to 416 tokens, 70 of them (more than one launch takes): key blocks that start at odd multiples of 32
+    tokens and reach into the next sequence; each sequence equals its own 'bhsd' attention bit for bit."""
+    lens = [32, 96, 32, 64, 416, 160] + [32] * 64
+    cu = [0] + torch.tensor(lens).cumsum(0).tolist()
+    g = torch.Generator().manual_seed(5)
+    q, k, v = (torch.randn(cu[-1], h, d, generator=g).to(torch.bfloat16).to(DEV) for h, d in ((4, D), (2, D), (2, Dv)))
+    for causal in (True, False):
+        out, lse, _ = m.triton_attention_mxfp4(q, k, v, cu_seqlens_q=cu, cu_seqlens_k=cu, causal=causal, layout="thd")
+        for i in list(range(8)) + [len(lens) - 1]:
+            qi, ki, vi = (t[cu[i]:cu[i + 1]].transpose(0, 1).unsqueeze(0).contiguous() for t in (q, k, v))
+            o1, l1, _ = m.triton_attention_mxfp4(qi, ki, vi, causal=causal)
+            assert torch.equal(out[cu[i]:cu[i + 1]].transpose(0, 1), o1[0]) and torch.equal(lse[cu[i]:cu[i + 1]].transpose(0, 1), l1[0]), (i, causal)
