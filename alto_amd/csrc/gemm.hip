@@ -41,7 +41,18 @@ extern "C" int alto_mxfp4_gemm(const uint8_t* a, int64_t lda, const uint8_t* a_s
   OperandView A{a, lda, a_scales, a_ss_r, a_ss_k, a_is_2d};
   OperandView B{b, ldb, b_scales, b_ss_r, b_ss_k, b_is_2d};
 
-  if (gemm_tiled_supported(A, B, M, N, K, c, c_dtype, ldc)) {
+  if (gemm_skinny_supported(A, B, M, N, K)) {
+    gemm_skinny_launch(A, B, M, N, K, c, c_dtype, ldc, out_scale, st);
+    return check_launch("gemm(skinny)");
+  }
+  const bool tiled = gemm_tiled_supported(A, B, M, N, K, c, c_dtype, ldc);
+  int tile = gemm_mid_tile_size(M, N, c_dtype);
+  if (tile == 256 && !tiled) tile = 128;   // (a long, narrow result or a short reduction)
+  if (tile != 256 && gemm_mid_supported(A, B, M, N, K, c, ldc)) {
+    gemm_mid_launch(tile, A, B, M, N, K, c, c_dtype, ldc, out_scale, false, st);
+    return check_launch("gemm(mid)");
+  }
+  if (tiled) {
     gemm_tiled_launch(A, B, M, N, K, c, c_dtype, ldc, out_scale, st);
     return check_launch("gemm(tiled)");
   }
@@ -92,6 +103,8 @@ extern "C" int alto_mxfp4_gemm_ps(const uint8_t* a, int64_t lda, const uint8_t* 
     set_error("gemm_ps: shape (%lld, %lld, %lld) is not served by the tile kernel; use alto_mxfp4_gemm with plain scales", (long long)M, (long long)N, (long long)K);
     return ALTO_MXFP4_ENOTIMPL;
   }
-  gemm_tiled_launch_ps(A, B, M, N, K, c, ldc, out_scale, reinterpret_cast<hipStream_t>(stream));
+  const int tile = gemm_mid_tile_size(M, N, ALTO_DT_BF16);
+  if (tile != 256) gemm_mid_launch(tile, A, B, M, N, K, c, ALTO_DT_BF16, ldc, out_scale, true, reinterpret_cast<hipStream_t>(stream));
+  else gemm_tiled_launch_ps(A, B, M, N, K, c, ldc, out_scale, reinterpret_cast<hipStream_t>(stream));
   return check_launch("gemm_ps");
 }

@@ -34,6 +34,25 @@ constexpr int GT_SCALE_PITCH = 5;                                // dwords per r
 constexpr int GT_SCALE_BUF_DW = (GT_TM + GT_TN) * GT_SCALE_PITCH;  // one buffer, in dwords
 constexpr int GT_LDS_BYTES = GT_NSTAGE * GT_STAGE_BYTES + 2 * GT_SCALE_BUF_DW * 4;  // 131072 + 20480 = 151552
 
+// Workgroups are dealt round-robin to the 8 XCDs (each with its own L2).  Every XCD gets a contiguous range of the
+// tile sequence, and the sequence walks 8 N-tiles per M-tile before moving on, so the ~32 tiles an XCD has in flight
+// share A rows and B rows through its L2.
+__device__ __forceinline__ bool tile_coords(int wg, int tiles_m, int tiles_n, int& tm, int& tn) {
+  const int T = tiles_m * tiles_n;
+  const int per_xcd = (T + 7) / 8;
+  const int u = (wg & 7) * per_xcd + (wg >> 3);
+  if ((wg >> 3) >= per_xcd || u >= T) return false;
+  const int GN = 8;
+  const int in_group = GN * tiles_m;
+  const int group = u / in_group;
+  const int first_n = group * GN;
+  const int gsize = (tiles_n - first_n) < GN ? (tiles_n - first_n) : GN;
+  const int w = u % in_group;
+  tn = first_n + w % gsize;
+  tm = w / gsize;
+  return true;
+}
+
 struct TileArgs {
   OperandView A, B;
   int64_t m0, n0;          // first row of the tile in A / B

@@ -7,25 +7,6 @@
 namespace alto {
 namespace {
 
-// Workgroups are dealt round-robin to the 8 XCDs (each with its own L2).  Every XCD gets a contiguous range of the
-// tile sequence, and the sequence walks 8 N-tiles per M-tile before moving on, so the ~32 tiles an XCD has in flight
-// share A rows and B rows through its L2.
-__device__ __forceinline__ bool tile_coords(int wg, int tiles_m, int tiles_n, int& tm, int& tn) {
-  const int T = tiles_m * tiles_n;
-  const int per_xcd = (T + 7) / 8;
-  const int u = (wg & 7) * per_xcd + (wg >> 3);
-  if ((wg >> 3) >= per_xcd || u >= T) return false;
-  const int GN = 8;
-  const int in_group = GN * tiles_m;
-  const int group = u / in_group;
-  const int first_n = group * GN;
-  const int gsize = (tiles_n - first_n) < GN ? (tiles_n - first_n) : GN;
-  const int w = u % in_group;
-  tn = first_n + w % gsize;
-  tm = w / gsize;
-  return true;
-}
-
 template <typename OutT, bool KTAIL, int LMS, int NST, bool PS>
 __global__ __launch_bounds__(GT_THREADS) void gemm_tiled_kernel(OperandView A, OperandView B, int64_t M, int64_t N, int G,
                                                          OutT* c, int64_t ldc, float out_scale, int tiles_m, int tiles_n) {
