@@ -12,6 +12,7 @@ from . import build as _build
 
 _lock = threading.Lock()
 _lib = None
+_host = None
 
 c_i64 = ctypes.c_int64
 c_int = ctypes.c_int
@@ -108,7 +109,7 @@ def load():
             _lib = lib
             return lib
         path = _build.lib_path()
-        if not os.path.exists(path):
+        if not os.path.exists(path) or not os.path.exists(_build.host_path()):
             _build.build(verbose=False)
         elif _build.is_stale():
             if os.environ.get("ALTO_MXFP4_NO_REBUILD") == "1":
@@ -123,6 +124,27 @@ def load():
             fn.argtypes = args
         _lib = lib
         return lib
+
+
+def host():
+    """The native host side (csrc/host.cpp), bound to the functions of the library that ``load`` gives."""
+    global _host
+    if _host is not None:
+        return _host
+    lib = load()
+    with _lock:
+        if _host is None:
+            import importlib.machinery
+            import importlib.util
+            path = _build.host_path()
+            if not os.path.exists(path):   # (an explicit library was loaded from a tree that has not been built)
+                _build.build(verbose=False)
+            loader = importlib.machinery.ExtensionFileLoader("alto_mxfp4_host", path)
+            mod = importlib.util.module_from_spec(importlib.util.spec_from_file_location("alto_mxfp4_host", path, loader=loader))
+            loader.exec_module(mod)
+            mod.bind({name: ctypes.cast(getattr(lib, name), c_vp).value for name in SIGNATURES}, check)
+            _host = mod
+    return _host
 
 
 def check(rc: int, what: str) -> None:

@@ -1,4 +1,4 @@
-"""Builds libalto_mxfp4.so (hand-written HIP for gfx950) in-tree with hipcc.
+"""Builds libalto_mxfp4.so (hand-written HIP for gfx950, hipcc) and alto_mxfp4_host.so (the native host side, g++) in-tree.
 
 Usage: ``python -m alto_amd.build [--force]``.  The library lands in ``alto_amd/lib/`` next to the
 sources so that it travels with the tree; nothing is installed outside the repository.
@@ -16,6 +16,7 @@ CSRC = os.path.join(HERE, "csrc")
 LIBDIR = os.path.join(HERE, "lib")
 OBJDIR = os.path.join(HERE, "lib", "obj")
 LIBNAME = "libalto_mxfp4.so"
+HOSTNAME = "alto_mxfp4_host.so"   # CPython module of csrc/host.cpp, named as its PYBIND11_MODULE
 
 SOURCES = ["capi.hip", "quantize.hip", "dequantize.hip", "gemm.hip", "gemm_tiled.hip", "gemm_mid.hip", "gemm_skinny.hip", "grouped_gemm.hip", "probe.hip", "qdq.hip", "attention.hip", "attention_quantize.hip", "quantize_dynamic.hip", "random.hip"]
 
@@ -35,6 +36,10 @@ def lib_path() -> str:
     return os.path.join(LIBDIR, LIBNAME)
 
 
+def host_path() -> str:
+    return os.path.join(LIBDIR, HOSTNAME)
+
+
 def stamp_path() -> str:
     return lib_path() + ".srchash"
 
@@ -43,7 +48,7 @@ def source_hash() -> str:
     """Digest of every file the library is built from (kernels, their headers, the C ABI header, the compiler flags)."""
     import hashlib
     h = hashlib.sha256(" ".join(HIPCC_FLAGS).encode())
-    files = sorted(os.path.join(CSRC, f) for f in os.listdir(CSRC) if f.endswith((".hip", ".h")))
+    files = sorted(os.path.join(CSRC, f) for f in os.listdir(CSRC) if f.endswith((".hip", ".h", ".cpp")))
     files.append(os.path.join(HERE, "..", "include", "alto_mxfp4.h"))
     for f in files:
         h.update(os.path.basename(f).encode())
@@ -77,12 +82,30 @@ def _compile(src: str) -> str:
     return obj
 
 
+def _compile_host() -> None:
+    """csrc/host.cpp against the installed torch: host code only, so the host compiler does it."""
+    import sysconfig
+
+    import torch
+    tdir = os.path.dirname(torch.__file__)
+    out = host_path()
+    cmd = [shutil.which("g++") or "g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", f"-I{tdir}/include", f"-I{tdir}/include/torch/csrc/api/include",
+           f"-I{sysconfig.get_paths()['include']}", os.path.join(CSRC, "host.cpp"), "-o", out + ".tmp", f"-L{tdir}/lib", "-lc10", "-ltorch_cpu", "-ltorch_python"]
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    if res.returncode != 0:
+        raise RuntimeError(f"g++ failed for host.cpp:\n{res.stdout}\n{res.stderr}")
+    os.replace(out + ".tmp", out)
+
+
 def build(verbose: bool = True) -> str:
-    """Compile every HIP source and link the shared library; always rebuilds."""
+    """Compile every HIP source, link the shared library and build the host module; always rebuilds."""
     os.makedirs(OBJDIR, exist_ok=True)
     digest = source_hash()   # taken before compiling: an edit made during the build leaves the library marked stale
     with ThreadPoolExecutor(max_workers=min(8, len(SOURCES))) as pool:
+        host = pool.submit(_compile_host)
         objs = list(pool.map(_compile, SOURCES))
+        host.result()
     out = lib_path()
     tmp = out + ".tmp"
     cmd = [_hipcc(), "--offload-arch=gfx950", "-shared", "-fPIC", "-o", tmp, *objs]

@@ -34,11 +34,16 @@ def ptr(t: Optional[torch.Tensor]) -> Optional[int]:
 
 
 def stream_ptr(device: torch.device) -> int:
-    return torch.cuda.current_stream(device).cuda_stream
+    idx = device.index
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if idx is None else idx)
 
 
 def lib():
     return _lib.load()
+
+
+def host():
+    return _lib._host or _lib.host()
 
 
 # ---------------------------------------------------------------------------------------------- random bits

@@ -111,6 +111,8 @@ def _attend(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, sm_scale: float, 
             alibi_slopes: Optional[torch.Tensor] = None, cu_q=None, cu_k=None) -> None:
     """Quantizer and attention kernel on q, k, v [B,H,S,D] views; ``out`` [B,Hq,Sq,Dv] and ``lse`` [B,Hq,Sq] are views of the
     caller's results in whatever layout they have.  ``cu_q`` / ``cu_k``: boundaries (host ints) of sequences packed along S."""
+    if alibi_slopes is None and rt.host().attend(q, k, v, sm_scale, bool(causal), out, lse, cu_q or [], cu_k or [], rt.stream_ptr(q.device)):
+        return
     qq, qs, kq, ks, vq, vs = quantize_qkv(q, k, v)
     (B, Hq, Sq, D), (_, Hk, Sk, Dv) = q.shape, v.shape
     sl = None

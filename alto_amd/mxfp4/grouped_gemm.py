@@ -103,20 +103,15 @@ def pack_expert_scales(w_s: torch.Tensor, N: int, K: int, is_2d_block: bool) -> 
 
 def grouped_forward_packed(a_q, a_ps, w_q, w_ps, groups: Groups, plan=None, return_plan=False):
     """:func:`grouped_forward` on packed scales (bf16 output): ``a_ps`` [ceil(K/512), M, 16], ``w_ps`` [E, ceil(K/512), N, 16]."""
+    res = rt.host().grouped_packed(a_q, a_ps, w_q, w_ps, groups.offs, groups.expert, groups.n, plan, rt.stream_ptr(a_q.device))
+    if res is not None:
+        return res if return_plan else res[0]
     E, N = w_q.shape[0], w_q.shape[1]
     M, K = a_q.shape[0], a_q.shape[1] * 2
     assert w_q.shape[2] * 2 == K and a_q.stride(1) == 1 and w_q.stride(2) == 1
     KB = -(-(K // 32) // 16)
     assert a_ps.shape == (KB, M, 16) and w_ps.shape == (E, KB, N, 16) and a_ps.is_contiguous() and w_ps.is_contiguous()
-    out = torch.empty((M, N), dtype=torch.bfloat16, device=a_q.device)
-    ws_bytes = rt.lib().alto_mxfp4_grouped_gemm_workspace_bytes(M, groups.n)
-    ws = plan if plan is not None else torch.empty(ws_bytes, dtype=torch.uint8, device=a_q.device)
-    rc = rt.lib().alto_mxfp4_grouped_gemm_ps(
-        a_q.data_ptr(), a_q.stride(0), a_ps.data_ptr(), w_q.data_ptr(), w_q.stride(0), w_q.stride(1), w_ps.data_ptr(), w_ps.stride(0),
-        groups.offs.data_ptr(), rt.ptr(groups.expert), groups.n, E, M, N, K, out.data_ptr(), out.stride(0),
-        ws.data_ptr(), ws.numel(), int(plan is not None), rt.stream_ptr(a_q.device))
-    check(rc, "alto_mxfp4_grouped_gemm_ps")
-    return (out, ws) if return_plan else out
+    raise AssertionError("grouped_forward_packed: uint8 GPU tensors expected")
 
 
 def grouped_packed_supported(M: int, N: int, K: int, num_groups: int, lda: Optional[int] = None, ldw: Optional[int] = None) -> bool:
@@ -221,14 +216,9 @@ def grouped_dw_packed(go_qm, go_ps, x_qm, x_ps, groups: Groups, num_experts, tra
         x_qm = x_qm.contiguous()
     KB = -(-M_total // 512)
     assert go_ps.shape == (KB, N, 16) and x_ps.shape == (KB, K, 16) and go_ps.is_contiguous() and x_ps.is_contiguous()
-    shape = (num_experts, N, K) if trans_weights else (num_experts, K, N)
-    dw = torch.empty(shape, dtype=torch.bfloat16, device=go_qm.device)
-    s_e, s_n, s_k = (dw.stride(0), dw.stride(1), dw.stride(2)) if trans_weights else (dw.stride(0), dw.stride(2), dw.stride(1))
-    rc = rt.lib().alto_mxfp4_grouped_gemm_dw_ps(
-        go_qm.data_ptr(), go_qm.stride(0), go_ps.data_ptr(), x_qm.data_ptr(), x_qm.stride(0), x_ps.data_ptr(),
-        groups.offs.data_ptr(), rt.ptr(groups.expert), groups.n, num_experts, M_total, N, K, dw.data_ptr(), s_e, s_n, s_k,
-        float(out_scale), rt.stream_ptr(go_qm.device))
-    check(rc, "alto_mxfp4_grouped_gemm_dw_ps")
+    dw = rt.host().grouped_dw_packed(go_qm, go_ps, x_qm, x_ps, groups.offs, groups.expert, groups.n, num_experts, bool(trans_weights), out_scale,
+                                     rt.stream_ptr(go_qm.device))
+    assert dw is not None, "grouped_dw_packed: uint8 GPU tensors expected"
     return dw
 
 

@@ -70,7 +70,8 @@ class HadamardFactory:
     def create_transform(cls, device=None) -> HadamardTransform:
         if not cls.randomized:
             return HadamardTransform(torch.ones(BLOCK, dtype=torch.int8), None)
-        q = torch.randint(low=0, high=2, size=(BLOCK,), generator=cls.generator, dtype=cls.dtype)
-        q = q * 2 - 1
-        perm = torch.randperm(BLOCK, generator=cls.generator)
-        return HadamardTransform(q.to(torch.int8), perm)
+        # randint(0, 2, (32,)) in cls.dtype, then randperm(32): valid by construction, so the checks of __init__ are not run
+        from .._lib import host
+        h = HadamardTransform.__new__(HadamardTransform)
+        h.signs, h.perm = host().draw_hadamard(cls.generator, cls.dtype)
+        return h

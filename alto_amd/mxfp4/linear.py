@@ -161,14 +161,13 @@ def _k_major(codes: torch.Tensor) -> torch.Tensor:
 
 def gemm_packed(a_q: torch.Tensor, a_ps: torch.Tensor, b_q: torch.Tensor, b_ps: torch.Tensor, out_scale: float = 1.0) -> torch.Tensor:
     """C [M, N] (bf16) = A [M, K] . B [N, K]^T with codes packed along K and scales in the form of :func:`pack_scales`."""
+    out = rt.host().gemm_packed(a_q, a_ps, b_q, b_ps, out_scale, rt.stream_ptr(a_q.device))
+    if out is not None:
+        return out
     M, N, K = a_q.shape[0], b_q.shape[0], a_q.shape[1] * 2
     assert b_q.shape[1] * 2 == K and a_q.stride(1) == 1 and b_q.stride(1) == 1
     assert a_ps.shape == (-(-(K // 32) // 16), M, 16) and b_ps.shape == (-(-(K // 32) // 16), N, 16) and a_ps.is_contiguous() and b_ps.is_contiguous()
-    c = torch.empty((M, N), dtype=torch.bfloat16, device=a_q.device)
-    rc = rt.lib().alto_mxfp4_gemm_ps(a_q.data_ptr(), a_q.stride(0), a_ps.data_ptr(), b_q.data_ptr(), b_q.stride(0), b_ps.data_ptr(), M, N, K,
-                                     c.data_ptr(), c.stride(0), float(out_scale), rt.stream_ptr(a_q.device))
-    check(rc, "alto_mxfp4_gemm_ps")
-    return c
+    raise AssertionError("gemm_packed: uint8 GPU tensors expected")
 
 
 def blockwise_mxfp4_gemm(
@@ -194,6 +193,11 @@ def blockwise_mxfp4_gemm(
     assert a.dim() == 2 and b.dim() == 2
     assert block_size == BLOCK_SIZE_DEFAULT
     rt.require_gpu(a, a_s, b, b_s)
+    if k_pack_a and k_pack_b and (output_dtype is torch.float32 or output_dtype is torch.bfloat16):
+        out = rt.host().gemm(a, a_s, b, b_s, bool(use_2dblock_a), bool(use_2dblock_b), bool(trans_a), bool(trans_b), output_dtype is torch.float32, out_scale,
+                             rt.stream_ptr(a.device))
+        if out is not None:
+            return out
     if trans_a:
         K, M = a.shape
     else:

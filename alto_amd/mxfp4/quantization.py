@@ -33,24 +33,10 @@ def _as_i32(r: torch.Tensor) -> torch.Tensor:
     return r
 
 
-def _signs_perm_ptrs(h: Optional[HadamardTransform]):
-    if h is None:
-        return 0, None, None
-    return 1, h.signs.data_ptr(), (None if h.perm is None else h.perm.data_ptr())
-
-
-def _code_buffer(B: int, R: int, nbytes: int, dev, pad: bool) -> torch.Tensor:
-    """[B, R, nbytes] code tensor; with ``pad`` its rows start on 128-byte boundaries (a view over padded storage)."""
-    pitch = (nbytes + 127) // 128 * 128 if pad else nbytes
-    if pitch == nbytes:
-        return torch.empty((B, R, nbytes), dtype=torch.uint8, device=dev)
-    return torch.empty((B, R, pitch), dtype=torch.uint8, device=dev)[:, :, :nbytes]
-
-
 def _quantize_call(x3: torch.Tensor, want_row: bool, want_col: bool, is_2d: bool, use_sr: bool,
                    rand3: Optional[torch.Tensor], hadamard: Optional[HadamardTransform], clip: int, use_uos: bool,
                    pad_codes: bool = False, philox: Optional[Tuple[int, int]] = None, hw_sr: bool = False,
-                   pack_row_scales: bool = False, pack_col_scales: bool = False):
+                   pack_row_scales: bool = False, pack_col_scales: bool = False, flat: bool = False):
     """x3: [B, M, C] with unit stride along C and uniform row / batch strides. Returns the outputs (or None): dense, or
     with ``pad_codes`` code tensors whose rows are padded to whole 128-byte cache lines (for GEMM operands).
     ``philox = (seed, offset)`` with ``use_sr`` and no ``rand3``: the kernel makes the random words itself, element
@@ -59,82 +45,23 @@ def _quantize_call(x3: torch.Tensor, want_row: bool, want_col: bool, is_2d: bool
     counter moved past the B M C words afterwards (nothing about the draw is a kernel argument: safe under graph capture).
     ``hw_sr``: round with the hardware's stochastic converts (``alto_mxfp4_quantize_sr_hw``; needs ``philox``).
     ``pack_row_scales`` / ``pack_col_scales``: that scale output comes in the packed form of ``linear.pack_scales`` --
-    [B, ceil(C/512), M, 16] resp. [B, ceil(M/512), C, 16] -- written by the kernel itself."""
-    B, M, C = x3.shape
-    dev = x3.device
-    packed = pack_row_scales or pack_col_scales
-    row_codes = row_scales = col_codes = col_scales = None
-    if want_row:
-        row_codes = _code_buffer(B, M, C // 2, dev, pad_codes)
-        if pack_row_scales:
-            row_scales = torch.empty((B, -(-(C // 32) // 16), M, 16), dtype=torch.uint8, device=dev)
-        else:
-            row_scales = torch.empty((B, M // 32, C // 32) if is_2d else (B, M, C // 32), dtype=torch.uint8, device=dev)
-    if want_col:
-        col_codes = _code_buffer(B, C, M // 2, dev, pad_codes)
-        if pack_col_scales:
-            col_scales = torch.empty((B, -(-(M // 32) // 16), C, 16), dtype=torch.uint8, device=dev)
-        else:
-            col_scales = torch.empty((B, C // 32, M // 32) if is_2d else (B, C, M // 32), dtype=torch.uint8, device=dev)
-    had, sp, pp = _signs_perm_ptrs(hadamard)
-    ld_x = x3.stride(1) if M > 1 else C
-    bs_x = x3.stride(0) if B > 1 else M * ld_x
-    ld_r = bs_r = 0
+    [B, ceil(C/512), M, 16] resp. [B, ceil(M/512), C, 16] -- written by the kernel itself.
+    ``flat``: x3 is [M, C] (any strides) and the outputs come as :func:`quantize_rowcol` returns them."""
+    state, seed, offset, sr_mode = None, 0, 0, 0
     if use_sr and rand3 is not None:
-        ld_r = rand3.stride(1) if M > 1 else C
-        bs_r = rand3.stride(0) if B > 1 else M * ld_r
-    if packed:   # the general entry point: every rounding mode plus the layout flags
-        state, seed, offset, sr_mode = None, 0, 0, 0
-        if use_sr and rand3 is not None:
-            sr_mode = 1
-        elif use_sr:
-            assert philox is not None, "stochastic rounding needs rand_bits or a Philox (seed, offset)"
-            state = philox if isinstance(philox, torch.Tensor) else None
-            seed, offset = (0, 0) if state is not None else (philox[0] & (2 ** 64 - 1), philox[1] & (2 ** 64 - 1))
-            sr_mode = 3 if hw_sr else 2
-        rc = rt.lib().alto_mxfp4_quantize_ex(
-            x3.data_ptr(), rt.dtype_code(x3.dtype), B, M, C, ld_x, bs_x,
-            rt.ptr(row_codes), rt.ptr(row_scales), rt.ptr(col_codes), rt.ptr(col_scales),
-            row_codes.stride(1) if want_row else 0, col_codes.stride(1) if want_col else 0,
-            int(is_2d), sr_mode, rt.ptr(rand3) if sr_mode == 1 else None, ld_r, bs_r, seed, offset, rt.ptr(state),
-            had, sp, pp, clip, int(use_uos), int(pack_row_scales) | (int(pack_col_scales) << 1), rt.stream_ptr(dev))
-        check(rc, "alto_mxfp4_quantize_ex")
-        if state is not None:
-            rt.philox_advance(state, rt.lib().alto_mxfp4_quantize_sr_hw_words(rt.dtype_code(x3.dtype), B, M, C) if hw_sr else B * M * C)
-        return row_codes, row_scales, col_codes, col_scales
-    if use_sr and rand3 is None:
+        sr_mode = 1
+    elif use_sr:
         assert philox is not None, "stochastic rounding needs rand_bits or a Philox (seed, offset)"
-        state = philox if isinstance(philox, torch.Tensor) else None
-        seed, offset = (0, 0) if state is not None else (philox[0] & (2 ** 64 - 1), philox[1] & (2 ** 64 - 1))
-        if hw_sr:
-            rc = rt.lib().alto_mxfp4_quantize_sr_hw(
-                x3.data_ptr(), rt.dtype_code(x3.dtype), B, M, C, ld_x, bs_x,
-                rt.ptr(row_codes), rt.ptr(row_scales), rt.ptr(col_codes), rt.ptr(col_scales),
-                row_codes.stride(1) if want_row else 0, col_codes.stride(1) if want_col else 0,
-                int(is_2d), seed, offset, rt.ptr(state),
-                had, sp, pp, clip, int(use_uos), rt.stream_ptr(dev))
-            check(rc, "alto_mxfp4_quantize_sr_hw")
-            if state is not None:
-                rt.philox_advance(state, rt.lib().alto_mxfp4_quantize_sr_hw_words(rt.dtype_code(x3.dtype), B, M, C))
-            return row_codes, row_scales, col_codes, col_scales
-        rc = rt.lib().alto_mxfp4_quantize_sr_philox(
-            x3.data_ptr(), rt.dtype_code(x3.dtype), B, M, C, ld_x, bs_x,
-            rt.ptr(row_codes), rt.ptr(row_scales), rt.ptr(col_codes), rt.ptr(col_scales),
-            row_codes.stride(1) if want_row else 0, col_codes.stride(1) if want_col else 0,
-            int(is_2d), seed, offset, rt.ptr(state),
-            had, sp, pp, clip, int(use_uos), rt.stream_ptr(dev))
-        check(rc, "alto_mxfp4_quantize_sr_philox")
-        if state is not None:
-            rt.philox_advance(state, B * M * C)
-        return row_codes, row_scales, col_codes, col_scales
-    rc = rt.lib().alto_mxfp4_quantize_pitched(
-        x3.data_ptr(), rt.dtype_code(x3.dtype), B, M, C, ld_x, bs_x,
-        rt.ptr(row_codes), rt.ptr(row_scales), rt.ptr(col_codes), rt.ptr(col_scales),
-        row_codes.stride(1) if want_row else 0, col_codes.stride(1) if want_col else 0,
-        int(is_2d), rt.ROUND_SR if use_sr else rt.ROUND_RNE, rt.ptr(rand3), ld_r, bs_r,
-        had, sp, pp, clip, int(use_uos), rt.stream_ptr(dev))
-    check(rc, "alto_mxfp4_quantize_pitched")
-    return row_codes, row_scales, col_codes, col_scales
+        if isinstance(philox, torch.Tensor):
+            state = philox
+        else:
+            seed, offset = philox[0] & (2 ** 64 - 1), philox[1] & (2 ** 64 - 1)
+        sr_mode = 3 if hw_sr else 2
+    out = rt.host().quantize(x3, flat, want_row, want_col, is_2d, sr_mode, rand3 if sr_mode == 1 else None, seed, offset, state,
+                             None if hadamard is None else hadamard.signs, None if hadamard is None else hadamard.perm, clip, use_uos, pad_codes,
+                             pack_row_scales, pack_col_scales, rt.stream_ptr(x3.device))
+    assert out is not None, "the quantizer takes bf16 / fp32 GPU tensors with unit stride along C and 16-byte aligned rows"
+    return out
 
 
 def _batched_view(t: torch.Tensor) -> Optional[torch.Tensor]:
@@ -196,6 +123,14 @@ def convert_to_mxfp4(
     counter start ``philox_seed``/``philox_offset`` if given, else a draw from torch's CPU generator).  ``hadamard`` fuses ``hadamard(x, left_mul=True)`` in front of
     an ``axis=-2`` quantisation of a 2D tensor.
     """
+    if (not use_sr and hadamard is None and block_size == BLOCK_SIZE_DEFAULT and data_hp.dim() == 2 and axis in (-1, 1, -2, 0) and data_hp.is_cuda
+            and clip_mode in ("none", "static") and data_hp.dtype in (torch.bfloat16, torch.float32)):
+        # the everyday call (a matrix, round to nearest): straight to the kernel when the checks below hold
+        M, C = data_hp.shape
+        last = axis in (-1, 1)
+        if M and C and (C % 32 == 0 if last else (M % 32 == 0 and C % 8 == 0)) and not (is_2d_block and (M % 32 or C % 32)):
+            out = _quantize_call(data_hp, last, not last, bool(is_2d_block), False, None, None, rt.CLIP[clip_mode], bool(use_uos), flat=True)
+            return out[:2] if last else out[2:]
     assert block_size == BLOCK_SIZE_DEFAULT, "only block_size=32 is implemented"
     torch._check(data_hp.shape[axis] % block_size == 0)
     assert not is_2d_block or data_hp.size(-2) % block_size == 0
@@ -352,15 +287,13 @@ def quantize_rowcol(
         cc, cs = convert_to_mxfp4(x, axis=0, is_2d_block=is_2d_block, use_sr=use_sr, clip_mode="dynamic", use_uos=use_uos,
                                   rand_bits=rand_bits, hadamard=hadamard)
         return rc, rs, cc, cs
-    x3 = _prep(x)
     r3 = None
     if use_sr and philox is None:
         assert rand_bits.shape == x.shape
         r3 = _as_i32(rand_bits)
         r3 = _batched_view(r3 if r3.stride(-1) == 1 and r3.stride(0) % 4 == 0 and r3.data_ptr() % 16 == 0 else r3.contiguous())
-    rc, rs, cc, cs = _quantize_call(x3, True, True, is_2d_block, use_sr, r3, hadamard, clip, use_uos, pad_codes, philox=philox, hw_sr=hw_sr,
-                                    pack_row_scales=pack_row_scales, pack_col_scales=pack_col_scales)
-    return rc[0], rs[0], cc[0].transpose(0, 1), cs[0] if pack_col_scales else cs[0].transpose(0, 1)
+    return _quantize_call(x, True, True, bool(is_2d_block), use_sr, r3, hadamard, clip, bool(use_uos), pad_codes, philox=philox, hw_sr=hw_sr,
+                          pack_row_scales=pack_row_scales, pack_col_scales=pack_col_scales, flat=True)
 
 
 def hadamard_apply(x: torch.Tensor, h: HadamardTransform, inverse: bool = False, left_mul: bool = False) -> torch.Tensor:
@@ -410,6 +343,10 @@ def convert_from_mxfp4(
     assert block_size == BLOCK_SIZE_DEFAULT
     clip = _clip_code(clip_mode)
     rt.require_gpu(data_lp, scales)
+    if axis in (-1, 1, -2, 0) and data_lp.dim() == 2:
+        out = rt.host().dequantize(data_lp, scales, output_dtype == torch.float32, axis in (-1, 1), bool(is_2d_block), clip, rt.stream_ptr(data_lp.device))
+        if out is not None:
+            return out
     lt = data_lp.transpose(axis, -1)
     st = scales.transpose(axis, -1)
     orig = (*lt.shape[:-1], lt.shape[-1] * 2)
