@@ -129,13 +129,20 @@ __global__ __launch_bounds__(256) void grouped_dw_simple_kernel(OperandView GO, 
 
 // ----------------------------------------------------------------------------- 256x256 tiles (large problems)
 
-// Tile order of the grouped kernels.  As in the dense kernel an XCD (wg % 8) works on 8 neighbouring N-tiles of a few row
-// bands at a time, so its L2 shares the A rows and the expert's weight rows; but the row bands are dealt to the XCDs
-// round-robin (band tm belongs to XCD tm % 8) instead of in contiguous ranges: a band that an expert boundary cuts runs
-// once per segment, such bands cluster where the small experts sit, and contiguous ranges left one XCD with most of them.
-__device__ __forceinline__ bool grouped_tile_coords(int wg, int tiles_m, int tiles_n, int& tm, int& tn) {
+// Tile order of the grouped kernels.  As in the dense kernel an XCD (wg % 8) works on 8 neighbouring N-tiles of a few passes
+// at a time, so its L2 shares the A rows and the expert's weight rows.  The passes are dealt to the XCDs in runs of
+// 2^run_log2 (what is left of the last round one by one, so that no XCD has two passes more than another).  Runs of 4: the 32
+// tiles that an XCD has in flight are then 8 N-tiles x 4 neighbouring passes, mostly of one expert, whose weights come into
+// fewer L2s and once for 4 passes instead of once per pass.  65536 x 5760 x 2880, 32 experts, forward / dX in us, one by one ->
+// runs of 4: equal experts 649 / 588 -> 612 / 552, Zipf 629 / 592 -> 612 / 585; 16384 x 4096 x 2048, 16 experts 91 / 76 -> 83 / 70.
+// One contiguous range per XCD is best for equal experts (589 / 545) and worst for sorted Zipf experts (638 / 596): the XCD
+// with the many small experts, whose weights all come from memory, is then last.  With about one pass per expert there is
+// nothing to share and runs are 3 % slower (8192 x 2048 x 1024, 32 experts): the host asks for them from 4 passes per
+// expert on.
+__device__ __forceinline__ bool grouped_tile_coords(int wg, int n_pass, int tiles_n, int run_log2, int& tm, int& tn) {
   const int k = wg & 7, j = wg >> 3;
-  const int nb = (tiles_m - k + 7) / 8;          // bands of this XCD
+  const int in_runs = (n_pass >> (3 + run_log2)) << run_log2;                         // passes of this XCD that come in runs,
+  const int nb = in_runs + ((n_pass - 8 * in_runs - k + 7) >> 3);                     // and all of them
   if (nb <= 0 || j >= nb * tiles_n) return false;
   const int GN = 8;
   const int group = j / (GN * nb);
@@ -143,7 +150,8 @@ __device__ __forceinline__ bool grouped_tile_coords(int wg, int tiles_m, int til
   const int gsize = (tiles_n - first_n) < GN ? (tiles_n - first_n) : GN;
   const int w = j - group * GN * nb;
   tn = first_n + w % gsize;
-  tm = k + 8 * (w / gsize);
+  const int i = w / gsize;
+  tm = i < in_runs ? ((((i >> run_log2) << 3) + k) << run_log2) + (i & ((1 << run_log2) - 1)) : 8 * i + k;
   return true;
 }
 // workgroups to launch for that order: 8 x the tile count of the XCD with the most bands
@@ -298,11 +306,11 @@ __global__ __launch_bounds__(PLAN_THREADS) void grouped_plan_kernel(PassWalk wk,
 template <typename OutT, bool KTAIL, int LMS, int NST, bool PS>
 __global__ __launch_bounds__(GT_THREADS) void grouped_tiled_kernel(OperandView A, const uint8_t* w, int64_t w_stride_e, int64_t ldw,
                                                                    const uint8_t* w_scales, int64_t ws_stride_e, int64_t ws_r, int w_is_2d,
-                                                                   const int32_t* plan, int64_t M_total, int64_t N, int G, OutT* out, int64_t ldo, int tiles_n) {
+                                                                   const int32_t* plan, int64_t M_total, int64_t N, int G, OutT* out, int64_t ldo, int tiles_n, int run_log2) {
   extern __shared__ __align__(16) uint8_t smem[];
   const int n_pass = __builtin_amdgcn_readfirstlane(plan[0]);
   int pi, tn;
-  if (!grouped_tile_coords(blockIdx.x, n_pass, tiles_n, pi, tn)) return;
+  if (!grouped_tile_coords(blockIdx.x, n_pass, tiles_n, run_log2, pi, tn)) return;
   const int4 d = reinterpret_cast<const int4*>(plan + 4)[pi];
   const int row0 = __builtin_amdgcn_readfirstlane(d.x), m_lo = __builtin_amdgcn_readfirstlane(d.y), m_hi = __builtin_amdgcn_readfirstlane(d.z);
   const int e = __builtin_amdgcn_readfirstlane(d.w);
@@ -478,7 +486,7 @@ int launch_grouped_tiled(const OperandView& A, const uint8_t* w, int64_t w_strid
   PassWalk wk{offs, group_expert, num_groups, num_experts, M_total};
   if (build_plan) hipLaunchKernelGGL(grouped_plan_kernel, dim3(1), dim3(PLAN_THREADS), 0, st, wk, tiles_m, plan, max_pass);
   hipLaunchKernelGGL(kern, dim3((unsigned)grouped_grid_size(max_pass, tiles_n)), dim3(GT_THREADS), GT_LDS_BYTES, st, A, w, w_stride_e, ldw, w_scales, ws_stride_e, ws_r,
-                     w_is_2d, plan, M_total, N, (int)(K / 32), (OutT*)out, ldo, tiles_n);
+                     w_is_2d, plan, M_total, N, (int)(K / 32), (OutT*)out, ldo, tiles_n, M_total >= 4ll * GT_TM * num_experts ? 2 : 0);
   return 0;
 }
 

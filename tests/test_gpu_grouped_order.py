@@ -1,0 +1,41 @@
+"""The order in which the grouped forward / dX kernel deals its passes to the XCDs (one by one, or in runs of four from 1024 rows
+per expert on, the rest of the last round one by one): every row and column of every expert is computed, with the bits of
+the dense product on that expert's rows."""
+import pytest
+import torch
+
+from tests.helpers import randn_outliers
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+@pytest.fixture(scope="module")
+def m():
+    import alto_amd.mxfp4 as mod
+    assert torch.cuda.is_available()
+    return mod
+
+
+# passes: 4 + 0, 32 + 0, 32 + 1, 64 + 7 in runs + one by one; then experts too short for runs, and rows of nobody at the end
+@pytest.mark.parametrize("sizes,tail", [([1024], 0), ([8192], 0), ([4096, 4097], 0), ([2300, 5, 9000, 6690], 0), ([300, 0, 700, 256], 0), ([1100, 2900], 640)])
+@pytest.mark.parametrize("N", [264, 2304])
+@pytest.mark.parametrize("packed", [False, True])
+def test_every_pass_and_column_tile(m, sizes, tail, N, packed):
+    from alto_amd.mxfp4 import grouped_gemm as G
+    from alto_amd.mxfp4.linear import pack_scales
+    K, E, M = 544, len(sizes), sum(sizes) + tail
+    aq, as_ = m.convert_to_mxfp4(randn_outliers((M, K), torch.bfloat16, seed=M).to(DEV))
+    wq, ws = m.convert_to_mxfp4((randn_outliers((E, N, K), torch.bfloat16, seed=N) * 0.02).to(DEV))
+    groups = G.groups_from_offsets(torch.tensor([0] + sizes).cumsum(0).to(torch.int32).to(DEV))
+    if packed:
+        out = G.grouped_forward_packed(aq, pack_scales(as_, M, K), wq, G.pack_expert_scales(ws, N, K, False), groups)
+    else:
+        out = G.grouped_forward(aq, as_, wq, ws, groups, False, False, torch.bfloat16)
+    lo = 0
+    for e, n in enumerate(sizes):
+        if n:
+            ref = m.blockwise_mxfp4_gemm(aq[lo:lo + n], as_[lo:lo + n], wq[e], ws[e], trans_b=True, output_dtype=torch.bfloat16)
+            assert torch.equal(out[lo:lo + n], ref), f"expert {e} of {sizes}"
+        lo += n
+    assert not out[lo:].any()
