@@ -136,5 +136,7 @@ __device__ __forceinline__ uint32_t dpp_u32(uint32_t v) {
 // quad_perm controls: lane ^ 1 and lane ^ 2 inside each group of 4 lanes
 #define ALTO_DPP_QUAD_XOR1 0xB1
 #define ALTO_DPP_QUAD_XOR2 0x4E
+// lane -> 7 - lane inside each group of 8
+#define ALTO_DPP_HALF_MIRROR 0x141
 
 }  // namespace alto
