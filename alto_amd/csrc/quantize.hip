@@ -109,10 +109,12 @@ __device__ __forceinline__ float round_to_T(float v) {
 // BPW: 32-row bands one workgroup walks (1, or 8 for 2D blocks with a column output: the workgroup then holds the eight
 // 16-byte pieces of a 128-byte line of every column's codes and stores whole lines, eight columns per wave instruction,
 // instead of one piece of 64 different lines per instruction).
-template <typename T, bool DO_ROW, bool DO_COL, int SR, bool RHT, bool B2D, bool GEN, int BPW = 1>
+// STREAM: loads of x, row-code stores and (BPW = 8) column-code stores are non-temporal.
+template <typename T, bool DO_ROW, bool DO_COL, int SR, bool RHT, bool B2D, bool GEN, int BPW = 1, bool STREAM = false>
 __global__ __launch_bounds__(256) void quant_kernel(const QuantParams p) {
   static_assert(BPW == 1 || (BPW == 8 && DO_COL && B2D), "bands per workgroup: 1, or 8 for the column output of 2D blocks");
   constexpr bool BF = sizeof(T) == 2;
+  constexpr int NT = STREAM ? 2 : 0;   // cache policy operand of the buffer instructions
   // Both phases consume the same random word per element.  Supplied words (SR == 1): each phase loads them in its own
   // layout, and the column phase's loads go out at the very start, beside the row phase's, so the second request for a
   // line meets the first one in the L2 and memory is read once (measured: fetch = 1.03 x the tensor); staging them in
@@ -231,10 +233,10 @@ __global__ __launch_bounds__(256) void quant_kernel(const QuantParams p) {
       valid[i] = (row0 + r < M) && cok;
       // rows past M are out of the descriptor's range and read as zeros; columns past C get an out-of-range offset
       const int voff = valid[i] ? rsub * ldx_b + c * (int)sizeof(T) : OOB;
-      const v4i_t v0 = __builtin_amdgcn_raw_buffer_load_b128(rsrc_x, voff, 8 * i * ldx_b, 0);
+      const v4i_t v0 = __builtin_amdgcn_raw_buffer_load_b128(rsrc_x, voff, 8 * i * ldx_b, NT);
       w[i][0] = v0[0]; w[i][1] = v0[1]; w[i][2] = v0[2]; w[i][3] = v0[3];
       if constexpr (!BF) {
-        const v4i_t v1 = __builtin_amdgcn_raw_buffer_load_b128(rsrc_x, voff, 8 * i * ldx_b + 16, 0);
+        const v4i_t v1 = __builtin_amdgcn_raw_buffer_load_b128(rsrc_x, voff, 8 * i * ldx_b + 16, NT);
         w[i][4] = v1[0]; w[i][5] = v1[1]; w[i][6] = v1[2]; w[i][7] = v1[3];
       }
       if constexpr (SR == 1 && (DO_ROW || STASH)) {
@@ -379,7 +381,7 @@ __global__ __launch_bounds__(256) void quant_kernel(const QuantParams p) {
   #pragma unroll
           for (int e = 0; e < 8; ++e) out |= e2m1_sr_mag(v[e] * inv, rr[i][e]) << (4 * e);
         }
-        if constexpr (DO_ROW) __builtin_amdgcn_raw_buffer_store_b32(out, rsrc_rc, valid[i] ? rsub * ldrc + (c >> 1) : OOB, 8 * i * ldrc, 0);
+        if constexpr (DO_ROW) __builtin_amdgcn_raw_buffer_store_b32(out, rsrc_rc, valid[i] ? rsub * ldrc + (c >> 1) : OOB, 8 * i * ldrc, NT);
         if constexpr (XCODES) {   // one code per byte, in column order, for the column packing
           const uint32_t ev = out & 0x0F0F0F0Fu, od = (out >> 4) & 0x0F0F0F0Fu;
           uint2 two;
@@ -646,7 +648,7 @@ __global__ __launch_bounds__(256) void quant_kernel(const QuantParams p) {
         const uint4 v = stage[idx];
         const int ccol = col0 + half * 128 + cl;
         __builtin_amdgcn_raw_buffer_store_b128(v4u_t{v.x, v.y, v.z, v.w}, rsrc_cc,
-                                               (ccol < C && q >= first) ? (half * 128 + cl) * (int)p.ld_cc + (q - first) * 16 : OOB, 0, 0);
+                                               (ccol < C && q >= first) ? (half * 128 + cl) * (int)p.ld_cc + (q - first) * 16 : OOB, 0, NT);
       }
     }
   }
@@ -764,8 +766,15 @@ int fill_hadamard(QuantParams& p, const int8_t* signs, const uint8_t* perm, cons
 }
 
 // bpw8: the caller laid the grid out for workgroups of 8 bands (column outputs of large 2D-block tensors, !GEN only)
+// stream: the tensor is larger than every cache (row + column passes of the training step only)
 template <typename T, bool DO_ROW, bool DO_COL, int SR, bool RHT, bool B2D, bool GEN>
-void launch(const QuantParams& p, dim3 grid, hipStream_t st, bool bpw8) {
+void launch(const QuantParams& p, dim3 grid, hipStream_t st, bool bpw8, bool stream) {
+  if constexpr (DO_ROW && DO_COL && !GEN && (B2D ? SR == 0 : (SR == 0 || SR == 3))) {
+    if (stream && bpw8 == B2D) {
+      hipLaunchKernelGGL((quant_kernel<T, DO_ROW, DO_COL, SR, RHT, B2D, GEN, B2D ? 8 : 1, true>), grid, dim3(256), 0, st, p);
+      return;
+    }
+  }
   if constexpr (DO_COL && B2D && !GEN) {
     if (bpw8) {
       hipLaunchKernelGGL((quant_kernel<T, DO_ROW, DO_COL, SR, RHT, B2D, GEN, 8>), grid, dim3(256), 0, st, p);
@@ -776,34 +785,34 @@ void launch(const QuantParams& p, dim3 grid, hipStream_t st, bool bpw8) {
 }
 
 template <typename T, int SR, bool GEN>
-void dispatch_mode(const QuantParams& p, dim3 grid, hipStream_t st, bool do_row, bool do_col, bool rht, bool b2d, bool bpw8) {
+void dispatch_mode(const QuantParams& p, dim3 grid, hipStream_t st, bool do_row, bool do_col, bool rht, bool b2d, bool bpw8, bool stream) {
   if (b2d) {
-    if (do_row && do_col) launch<T, true, true, SR, false, true, GEN>(p, grid, st, bpw8);
-    else if (do_row) launch<T, true, false, SR, false, true, GEN>(p, grid, st, bpw8);
-    else launch<T, false, true, SR, false, true, GEN>(p, grid, st, bpw8);
+    if (do_row && do_col) launch<T, true, true, SR, false, true, GEN>(p, grid, st, bpw8, stream);
+    else if (do_row) launch<T, true, false, SR, false, true, GEN>(p, grid, st, bpw8, stream);
+    else launch<T, false, true, SR, false, true, GEN>(p, grid, st, bpw8, stream);
   } else if (do_row && do_col) {
-    if (rht) launch<T, true, true, SR, true, false, GEN>(p, grid, st, bpw8);
-    else launch<T, true, true, SR, false, false, GEN>(p, grid, st, bpw8);
+    if (rht) launch<T, true, true, SR, true, false, GEN>(p, grid, st, bpw8, stream);
+    else launch<T, true, true, SR, false, false, GEN>(p, grid, st, bpw8, stream);
   } else if (do_row) {
-    launch<T, true, false, SR, false, false, GEN>(p, grid, st, bpw8);
+    launch<T, true, false, SR, false, false, GEN>(p, grid, st, bpw8, stream);
   } else {
-    if (rht) launch<T, false, true, SR, true, false, GEN>(p, grid, st, bpw8);
-    else launch<T, false, true, SR, false, false, GEN>(p, grid, st, bpw8);
+    if (rht) launch<T, false, true, SR, true, false, GEN>(p, grid, st, bpw8, stream);
+    else launch<T, false, true, SR, false, false, GEN>(p, grid, st, bpw8, stream);
   }
 }
 
 template <typename T>
-void dispatch(const QuantParams& p, dim3 grid, hipStream_t st, bool do_row, bool do_col, bool rht, bool b2d, int sr, bool gen, bool bpw8) {
+void dispatch(const QuantParams& p, dim3 grid, hipStream_t st, bool do_row, bool do_col, bool rht, bool b2d, int sr, bool gen, bool bpw8, bool stream) {
   if (gen) {
-    if (sr == 3) dispatch_mode<T, 3, true>(p, grid, st, do_row, do_col, rht, b2d, bpw8);
-    else if (sr == 2) dispatch_mode<T, 2, true>(p, grid, st, do_row, do_col, rht, b2d, bpw8);
-    else if (sr == 1) dispatch_mode<T, 1, true>(p, grid, st, do_row, do_col, rht, b2d, bpw8);
-    else dispatch_mode<T, 0, true>(p, grid, st, do_row, do_col, rht, b2d, bpw8);
+    if (sr == 3) dispatch_mode<T, 3, true>(p, grid, st, do_row, do_col, rht, b2d, bpw8, stream);
+    else if (sr == 2) dispatch_mode<T, 2, true>(p, grid, st, do_row, do_col, rht, b2d, bpw8, stream);
+    else if (sr == 1) dispatch_mode<T, 1, true>(p, grid, st, do_row, do_col, rht, b2d, bpw8, stream);
+    else dispatch_mode<T, 0, true>(p, grid, st, do_row, do_col, rht, b2d, bpw8, stream);
   } else {
-    if (sr == 3) dispatch_mode<T, 3, false>(p, grid, st, do_row, do_col, rht, b2d, bpw8);
-    else if (sr == 2) dispatch_mode<T, 2, false>(p, grid, st, do_row, do_col, rht, b2d, bpw8);
-    else if (sr == 1) dispatch_mode<T, 1, false>(p, grid, st, do_row, do_col, rht, b2d, bpw8);
-    else dispatch_mode<T, 0, false>(p, grid, st, do_row, do_col, rht, b2d, bpw8);
+    if (sr == 3) dispatch_mode<T, 3, false>(p, grid, st, do_row, do_col, rht, b2d, bpw8, stream);
+    else if (sr == 2) dispatch_mode<T, 2, false>(p, grid, st, do_row, do_col, rht, b2d, bpw8, stream);
+    else if (sr == 1) dispatch_mode<T, 1, false>(p, grid, st, do_row, do_col, rht, b2d, bpw8, stream);
+    else dispatch_mode<T, 0, false>(p, grid, st, do_row, do_col, rht, b2d, bpw8, stream);
   }
 }
 
@@ -905,6 +914,11 @@ int quantize_impl(const void* x, int dtype, int64_t batch, int64_t M, int64_t C,
   // all of those keep one band per workgroup.  ALTO_MXFP4_QUANT_BANDS=1|8 overrides the choice (tests, measurements).
   static const int force_bpw = [] { const char* e = getenv("ALTO_MXFP4_QUANT_BANDS"); return e ? atoi(e) : 0; }();
   const bool bpw8 = do_col && is_2d && !gen && (force_bpw == 8 || (force_bpw != 1 && tiles_x * ((bands + 7) / 8) * batch >= 4096));
+  // Tensors above the 256 MB of the last-level cache stream through: loads and whole-line stores then bypass the caches
+  // (us, before -> now: 65536 x 2880 round to nearest 130 -> 123, 65536 x 5760 254 -> 240, stochastic 293 -> 288, the 32 x 5760 x 2880
+  // expert weights 362 -> 302).  Smaller ones may still sit in the cache, or leave their codes there for the GEMM that
+  // follows: 14336 x 4096 (117 MB) weights 30 -> 38 when streamed, 2048 x 4096 with its GEMM 47 -> 51.
+  const bool streaming = batch * M * C * (dtype == ALTO_DT_BF16 ? 2 : 4) >= (256ll << 20);
   const int64_t wrows = bpw8 ? (bands + 7) / 8 : bands;   // workgroup rows
   // With a column output: 2^unit_shift workgroup rows per unit, units padded to a multiple of 8.  The largest unit (up to the
   // 128 bands of a line of plain column scales) whose padding launches at most 5 % more workgroups than there are tiles;
@@ -917,8 +931,8 @@ int quantize_impl(const void* x, int dtype, int64_t batch, int64_t M, int64_t C,
   ALTO_REQUIRE(do_col ? padded(us) < (1ll << 31) : (tiles_x < (1ll << 31) && bands <= 65535), "quantize: %lld x %lld exceeds the grid", (long long)M, (long long)C);
   const dim3 grid = do_col ? dim3((unsigned)padded(us), 1, (unsigned)batch) : dim3((unsigned)tiles_x, (unsigned)bands, (unsigned)batch);
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-  if (dtype == ALTO_DT_BF16) dispatch<__bf16>(p, grid, st, do_row, do_col, hadamard != 0, is_2d != 0, sr_mode, gen, bpw8);
-  else dispatch<float>(p, grid, st, do_row, do_col, hadamard != 0, is_2d != 0, sr_mode, gen, bpw8);
+  if (dtype == ALTO_DT_BF16) dispatch<__bf16>(p, grid, st, do_row, do_col, hadamard != 0, is_2d != 0, sr_mode, gen, bpw8, streaming);
+  else dispatch<float>(p, grid, st, do_row, do_col, hadamard != 0, is_2d != 0, sr_mode, gen, bpw8, streaming);
   return check_launch("quantize");
 }
 

@@ -1,0 +1,49 @@
+"""Tensors from 256 MB on are quantized with non-temporal loads and stores: the same bytes as the same rows in a smaller tensor."""
+import pytest
+import torch
+
+from tests.helpers import hadamard_from_seed
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("rht", [False, True])
+def test_rows_and_columns_of_a_large_matrix(dtype, rht):
+    import alto_amd.mxfp4 as m
+    C = 2080   # a last column tile of 32
+    M = -(-(256 << 20) // (C * dtype.itemsize * 32)) * 32
+    h = m.HadamardTransform(*hadamard_from_seed(3)) if rht else None
+    x = torch.randn((M, C), device=DEV, generator=torch.Generator(DEV).manual_seed(1)).to(dtype)
+    assert x.numel() * x.element_size() >= 256 << 20 > x[:M // 2].numel() * x.element_size()
+    q, s, cq, cs = m.quantize_rowcol(x, False, hadamard=h)
+    for lo in (0, M - 4096):
+        q1, s1, cq1, cs1 = m.quantize_rowcol(x[lo:lo + 4096], False, hadamard=h)
+        assert torch.equal(q[lo:lo + 4096], q1) and torch.equal(s[lo:lo + 4096], s1)
+        assert torch.equal(cq[lo // 2:lo // 2 + 2048], cq1) and torch.equal(cs[lo // 32:lo // 32 + 128], cs1)
+
+
+@pytest.mark.parametrize("M,C", [(4128, 2080), (8192, 2048)])
+def test_experts_larger_than_the_cache(M, C):
+    """2D blocks, workgroups of eight bands; M = 4128 leaves one band to the last workgroup."""
+    from alto_amd.mxfp4.quantization import _quantize_call
+    E = -(-(512 << 20) // (M * C * 2)) + 1
+    w = torch.randn((E, M, C), device=DEV, generator=torch.Generator(DEV).manual_seed(2)).bfloat16()
+    args = (True, True, True, False, None, None, 0, False, True)
+    big = _quantize_call(w, *args)
+    for e in (0, E - 1):
+        one = _quantize_call(w[e:e + 1], *args)
+        assert all(torch.equal(a[e], b[0]) for a, b in zip(big, one))
+
+
+def test_stochastic_words_of_a_large_matrix():
+    """Hardware stochastic rounding: the words belong to (row, column) of the whole matrix, so a device-resident state at the
+    same counter gives the same codes whatever the cache policy; checked against the packed-scale call on the same tensor."""
+    import alto_amd.mxfp4 as m
+    x = torch.randn((65568, 2080), device=DEV, generator=torch.Generator(DEV).manual_seed(4)).bfloat16()
+    outs = []
+    for clip in ("none", "static"):   # (the clipping kernels are not streamed; the row output is not clipped)
+        torch.manual_seed(5)
+        outs.append(m.quantize_rowcol(x, False, use_sr=True, clip_mode=clip, pad_codes=True)[:2])
+    assert torch.equal(outs[0][0], outs[1][0]) and torch.equal(outs[0][1], outs[1][1])
