@@ -1,4 +1,4 @@
-"""Tensors from 256 MB on are quantized with non-temporal loads and stores: the same bytes as the same rows in a smaller tensor."""
+"""Passes that move more than 256 MB are quantized with non-temporal loads and stores: the same bytes as the same rows in a smaller tensor."""
 import pytest
 import torch
 
