@@ -68,7 +68,8 @@ __device__ __forceinline__ uint32_t encode8(const uint32_t* w, float scale) {
   return o;
 }
 
-template <typename T, int COLS>
+// STREAM: non-temporal loads.
+template <typename T, int COLS, bool STREAM>
 __global__ __launch_bounds__(256) void attn_quant_kernel(const AttnQuantArgs a) {
   constexpr int DW = sizeof(T) == 2 ? 4 : 8;       // dwords of 8 elements
   constexpr int LPR = COLS / 8;                    // lanes per row
@@ -101,12 +102,11 @@ __global__ __launch_bounds__(256) void attn_quant_kernel(const AttnQuantArgs a) 
     const T* x = reinterpret_cast<const T*>(p.x) + b * p.sb + head * p.sh + col;
 #pragma unroll
     for (int i = 0; i < NI; ++i) {
-      const uint4* src = reinterpret_cast<const uint4*>(x + (int64_t)(row0 + i * RPI) * p.ss);
-      const uint4 v0 = src[0];
-      w[i][0] = v0.x; w[i][1] = v0.y; w[i][2] = v0.z; w[i][3] = v0.w;
-      if constexpr (DW == 8) {
-        const uint4 v1 = src[1];
-        w[i][4] = v1.x; w[i][5] = v1.y; w[i][6] = v1.z; w[i][7] = v1.w;
+      const v4i_t* src = reinterpret_cast<const v4i_t*>(x + (int64_t)(row0 + i * RPI) * p.ss);
+#pragma unroll
+      for (int e = 0; e < DW / 4; ++e) {
+        const v4i_t v = STREAM ? __builtin_nontemporal_load(src + e) : src[e];
+        w[i][4 * e + 0] = v[0]; w[i][4 * e + 1] = v[1]; w[i][4 * e + 2] = v[2]; w[i][4 * e + 3] = v[3];
       }
     }
     // the block's 32 rows x 32 columns sit in the lanes that agree in (lane % LPR) / 4
@@ -189,12 +189,17 @@ extern "C" int alto_mxfp4_attention_quantize(const void* q, const void* k, const
   ALTO_REQUIRE(nq > 0 && nk > 0 && nv > 0 && nq + nk + nv < (1ll << 31), "attention_quantize: too many workgroups");
   const dim3 grid((unsigned)(nq + nk + nv));
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+  // Operands of 128 MB and more are read past the caches, which then keep the codes for the attention kernel (whole calls, bf16,
+  // causal, changing inputs, without -> with, us: 160 MB 216 -> 213, 192 MB 346 -> 341, 320 MB 432 -> 420).  Smaller ones may be in a
+  // cache already (20 MB 32.2 -> 33.0, 40 MB 65 -> 67; 80 and 96 MB the same).
+  const bool stream_in = (B * Hq * Sq * D + B * Hk * Sk * (D + Dv)) * (dtype == ALTO_DT_BF16 ? 2 : 4) >= (128ll << 20);
+  auto go = [&](auto kern) { hipLaunchKernelGGL(kern, grid, dim3(256), 0, st, a); };
   if (dtype == ALTO_DT_BF16) {
-    if (cols == 128) hipLaunchKernelGGL((attn_quant_kernel<__bf16, 128>), grid, dim3(256), 0, st, a);
-    else hipLaunchKernelGGL((attn_quant_kernel<__bf16, 64>), grid, dim3(256), 0, st, a);
+    if (cols == 128) stream_in ? go(attn_quant_kernel<__bf16, 128, true>) : go(attn_quant_kernel<__bf16, 128, false>);
+    else stream_in ? go(attn_quant_kernel<__bf16, 64, true>) : go(attn_quant_kernel<__bf16, 64, false>);
   } else {
-    if (cols == 128) hipLaunchKernelGGL((attn_quant_kernel<float, 128>), grid, dim3(256), 0, st, a);
-    else hipLaunchKernelGGL((attn_quant_kernel<float, 64>), grid, dim3(256), 0, st, a);
+    if (cols == 128) stream_in ? go(attn_quant_kernel<float, 128, true>) : go(attn_quant_kernel<float, 128, false>);
+    else stream_in ? go(attn_quant_kernel<float, 64, true>) : go(attn_quant_kernel<float, 64, false>);
   }
   return check_launch("attention_quantize");
 }

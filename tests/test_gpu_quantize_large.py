@@ -47,3 +47,18 @@ def test_stochastic_words_of_a_large_matrix():
         torch.manual_seed(5)
         outs.append(m.quantize_rowcol(x, False, use_sr=True, clip_mode=clip, pad_codes=True)[:2])
     assert torch.equal(outs[0][0], outs[1][0]) and torch.equal(outs[0][1], outs[1][1])
+
+
+@pytest.mark.parametrize("dtype,D", [(torch.bfloat16, 128), (torch.bfloat16, 64), (torch.float32, 128), (torch.float32, 64)])
+def test_attention_operands_larger_than_128_mb(dtype, D):
+    """Batch by batch (below the line) and all at once (above it)."""
+    from alto_amd.mxfp4.attention import quantize_qkv
+    S, Hq, Hk = 1056, 24, 4
+    B = -(-(128 << 20) // (S * (Hq + 2 * Hk) * D * dtype.itemsize))
+    assert B >= 2
+    g = torch.Generator(DEV).manual_seed(6)
+    q, k, v = (torch.randn((B, S, h, D), device=DEV, generator=g).to(dtype).transpose(1, 2) for h in (Hq, Hk, Hk))
+    whole = quantize_qkv(q, k, v)
+    for b in (0, B - 1):
+        part = quantize_qkv(q[b:b + 1], k[b:b + 1], v[b:b + 1])
+        assert all(torch.equal(w[b:b + 1], p) for w, p in zip(whole, part))
