@@ -168,7 +168,7 @@ __device__ __forceinline__ void attn_fwd_body(const AttnArgs& a, const SEQS& seq
   // ---- cooperative fetch of one block: wave instruction j moves pieces [256 j + 64 wave, + 64) of the block, K pieces
   // first (contiguous in memory), then V pieces (piece p = 16 bytes of row p / 2, half p % 2); the piece index is also the
   // position in the slot.  A last block that reaches past its sequence holds whatever codes follow in the buffer (zeros
-  // beyond its end): those keys are masked, so their probabilities are exact zeros.
+  // beyond its end): those keys are masked, so their probabilities are exact zeros (and their V scales are replaced below).
   typedef __attribute__((address_space(3))) uint8_t lds_u8;
   auto extent = [](int64_t want, int64_t left) { return (int)(want < left ? want : left); };   // (want < 2^31: checked on the host)
   const int64_t k_off = k_base * (D / 2), v_off = bhk * DV * (int64_t)(a.Sk / 2) + k_first / 2;
@@ -306,6 +306,9 @@ __device__ __forceinline__ void attn_fwd_body(const AttnArgs& a, const SEQS& seq
             const int key = key0 + 32 * t + 8 * (v >> 2) + 4 * h + (v & 3);
             if ((a.causal && key > qrow + shift) || key >= kn) S[t][v] = -__builtin_inff();
           }
+        // A block that ends with its first 32 keys: the V scale bytes of the other 32 belong to what follows in the buffer, or
+        // were never written.  The codes of those probabilities are zeros, but a zero code times the E8M0 NaN (0xFF) is NaN.
+        if (key0 + 32 >= kn) vsw[VS_DW - 1] = DV == 128 ? 0x7F7F7F7Fu : (vsw[0] & 0xFFFFu) | 0x7F7F0000u;
       }
       float tmx[2];   // row maximum of each 32-key tile (exp2 is monotonic: its largest probability comes from this score)
 #pragma unroll

@@ -441,8 +441,8 @@ int alto_mxfp4_attention_quantize(const void* q, const void* k, const void* v, i
 
 /*
  * alto_mxfp4_attention_fwd on operands whose key count is any multiple of 32 (nothing is padded; the last block of 64 keys
- * reads what follows in the buffers and masks it: allocate 16 bytes behind k_scales and v_scales), with the outputs at
- * element strides o_* / l_* of batch, head and row (unit stride along Dv).
+ * reads what follows in the buffers and masks it: allocate 16 bytes behind k_scales and v_scales, whose content does not
+ * matter), with the outputs at element strides o_* / l_* of batch, head and row (unit stride along Dv).
  * n_seqs > 0: B = 1 and Sq / Sk count the tokens of n_seqs sequences packed along them (layout "thd" of
  * triton_flash_attention_mxfp4.py:1199-1203): cu_q / cu_k are HOST arrays of n_seqs + 1 boundaries, multiples of 32 from
  * 0 to Sq / Sk; every sequence attends to itself only, a causal mask sits in the bottom-right corner of its own score

@@ -311,3 +311,40 @@ def test_packed_sequences_that_start_at_odd_bands(m, D, Dv):
             qi, ki, vi = (t[cu[i]:cu[i + 1]].transpose(0, 1).unsqueeze(0).contiguous() for t in (q, k, v))
             o1, l1, _ = m.triton_attention_mxfp4(qi, ki, vi, causal=causal)
             assert torch.equal(out[cu[i]:cu[i + 1]].transpose(0, 1), o1[0]) and torch.equal(lse[cu[i]:cu[i + 1]].transpose(0, 1), l1[0]), (i, causal)
+
+
+def _strided_call(operands, dims, causal, fill, seqs=None):
+    """``alto_mxfp4_attention_fwd_strided`` on copies of ``operands`` whose scale buffers end in 16 bytes of ``fill``."""
+    import ctypes
+
+    from alto_amd import _lib
+    B, Hq, Hk, Sq, Sk, D, Dv = dims
+    bufs = [torch.cat([t.flatten(), torch.full((16,), fill, dtype=torch.uint8, device=DEV)]) for t in operands]
+    out = torch.empty((B, Hq, Sq, Dv), dtype=torch.bfloat16, device=DEV)
+    lse = torch.empty((B, Hq, Sq), dtype=torch.float32, device=DEV)
+    n = 0 if seqs is None else len(seqs[0]) - 1
+    cu = [None, None] if seqs is None else [(ctypes.c_int32 * (n + 1))(*c) for c in seqs]
+    rc = _lib.load().alto_mxfp4_attention_fwd_strided(*(t.data_ptr() for t in bufs), out.data_ptr(), lse.data_ptr(), *dims, *out.stride()[:3], *lse.stride(), n, *cu,
+                                                      D ** -0.5, int(causal), None, 0, 0, torch.cuda.current_stream().cuda_stream)
+    _lib.check(rc, "alto_mxfp4_attention_fwd_strided")
+    return out, lse
+
+
+@pytest.mark.parametrize("D,Dv", [(64, 64), (64, 128), (128, 64), (128, 128), (192, 64), (256, 128)])
+@pytest.mark.parametrize("causal", [True, False])
+def test_scale_bytes_behind_the_keys_are_not_used(m, D, Dv, causal):
+    """An odd number of 32-key bands: the second half of the last 64-key block does not exist, and what its scale bytes hold
+    (0xFF is the E8M0 NaN, which a zero code turns into NaN) must not reach the result."""
+    for B, Hq, Hk, Sq, Sk, seqs in ((1, 2, 1, 32, 32, None), (2, 4, 2, 96, 96, None), (1, 2, 2, 160, 288, None),
+                                    (1, 2, 2, 160, 160, ([0, 64, 160], [0, 64, 160])), (1, 4, 1, 160, 224, ([0, 96, 128, 160], [0, 96, 128, 224]))):
+        q, k, v = _qkv(B, Hq, Hk, Sq, Sk, D, Dv, seed=Sq + Sk + D)
+        qq, qs, kq, ks, vq, vs = m.quantize_qkv(q.to(DEV), k.to(DEV), v.to(DEV))
+        got = [_strided_call((qq, qs, kq, ks, vq, vs), (B, Hq, Hk, Sq, Sk, D, Dv), causal, fill, seqs) for fill in (0x7F, 0xFF, 0xFE, 0)]
+        out, lse = got[0]
+        for o, l in got[1:]:
+            assert torch.equal(o, out) and torch.equal(l, lse), (Sq, Sk, seqs)
+        cq, ck = ([0, Sq], [0, Sk]) if seqs is None else seqs
+        for q0, q1, k0, k1 in zip(cq, cq[1:], ck, ck[1:]):
+            ref, ref_lse = attention_fwd_ref(q[:, :, q0:q1], k[:, :, k0:k1], v[:, :, k0:k1], causal=causal)
+            assert _rel(out[:, :, q0:q1].cpu(), ref) <= REL_L2
+            assert float((lse[:, :, q0:q1].cpu() - ref_lse).abs().max()) <= 1e-4
