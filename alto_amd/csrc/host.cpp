@@ -100,10 +100,10 @@ py::object quantize(const Tensor& x_in, bool flat, bool want_row, bool want_col,
   Tensor x = x_in;
   if (!on_gpu(x) || !is_float(x) || x.dim() != (flat ? 2 : 3)) return py::none();
   const int64_t vec = x.scalar_type() == at::kBFloat16 ? 8 : 4;
-  auto readable = [&](const Tensor& t) {   // unit stride along C, everything else in whole 16-byte units
+  auto readable = [&](const Tensor& t) {   // unit stride along C, everything else in whole 16-byte units (a dim of one has no stride to speak of)
     if (t.stride(-1) != 1 || !aligned16(t)) return false;
     for (int64_t d = 0; d + 1 < t.dim(); ++d)
-      if (t.stride(d) % vec != 0) return false;
+      if (t.size(d) != 1 && t.stride(d) % vec != 0) return false;
     return true;
   };
   if (!readable(x)) {

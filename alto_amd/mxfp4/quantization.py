@@ -79,7 +79,7 @@ def _batched_view(t: torch.Tensor) -> Optional[torch.Tensor]:
 
 def _aligned(t: torch.Tensor) -> bool:
     vec = 8 if t.dtype == torch.bfloat16 else 4
-    return t.data_ptr() % 16 == 0 and all(s % vec == 0 for s in t.stride()[:-1])
+    return t.data_ptr() % 16 == 0 and all(n == 1 or s % vec == 0 for n, s in zip(t.shape[:-1], t.stride()))
 
 
 def _prep(t: torch.Tensor) -> torch.Tensor:

@@ -45,6 +45,35 @@ def test_convert_of_a_matrix_equals_the_batched_call(m, dtype, axis, is_2d, clip
                 assert torch.equal(back, back3[0]) and back.stride() == back3[0].stride(), (name, M, C)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_strides_of_dimensions_of_size_one_do_not_matter(m, dtype):
+    """One row cut from an odd pitch or a transposed column, a batch of one with an odd batch stride, one row per batch entry
+    with an odd row stride: ``contiguous()`` returns these as they are."""
+    C = 96
+    big = randn_outliers((4, 64 * C + 3), dtype, seed=11).to(DEV)   # rows off 16 bytes
+    rows = {"odd pitch": big[:1, :C], "column": big[0, :C].unsqueeze(1).t()}
+    for name, x in rows.items():
+        assert x.shape == (1, C) and x.stride(0) in (1, big.stride(0)) and x.is_contiguous()
+        for t, i in ((x, 0), (x[None], (0, 0)), (x[:, None], (0, 0))):
+            for kw in ({}, dict(clip_mode="static"), dict(use_uos=True)):
+                ref = m.convert_to_mxfp4(big[0, :C].clone()[None].repeat(2, 1), **kw)
+                q, s = m.convert_to_mxfp4(t, **kw)
+                assert torch.equal(q[i], ref[0][0]) and torch.equal(s[i], ref[1][0]), (name, t.shape, kw)
+            q, s = m.convert_to_mxfp4(t, use_sr=True, philox_seed=5)
+            ref = m.convert_to_mxfp4(torch.empty(t.shape, dtype=dtype, device=DEV).copy_(t), use_sr=True, philox_seed=5)
+            assert torch.equal(q, ref[0]) and torch.equal(s, ref[1]), (name, t.shape)
+    x = big[:1, :64 * C].unflatten(1, (64, C))          # [1, 64, C], batch stride off 16 bytes
+    for axis in (-1, -2):
+        for is_2d in (False, True):
+            q, s = m.convert_to_mxfp4(x, axis=axis, is_2d_block=is_2d)
+            ref = m.convert_to_mxfp4(x[0].clone(), axis=axis, is_2d_block=is_2d)
+            assert torch.equal(q[0], ref[0]) and torch.equal(s[0], ref[1]), (axis, is_2d)
+    z = big[0, :8 * C].as_strided((8, 1, C), (C, 3, 1))   # [8, 1, C], row stride 3
+    q, s = m.convert_to_mxfp4(z)
+    ref = m.convert_to_mxfp4(z.reshape(8, C).clone())
+    assert torch.equal(q[:, 0], ref[0]) and torch.equal(s[:, 0], ref[1])
+
+
 @pytest.mark.parametrize("sr", [False, True])
 @pytest.mark.parametrize("pack", [False, True])
 def test_quantize_rowcol_reads_every_stride(m, sr, pack):
