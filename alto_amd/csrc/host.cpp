@@ -77,6 +77,7 @@ bool is_float(const Tensor& t) { return t.scalar_type() == at::kBFloat16 || t.sc
 bool on_gpu(const Tensor& t) { return t.is_cuda() && t.layout() == at::kStrided; }
 uint8_t* bytes(const Tensor& t) { return t.defined() ? static_cast<uint8_t*>(t.data_ptr()) : nullptr; }
 bool aligned16(const Tensor& t) { return (reinterpret_cast<uintptr_t>(t.data_ptr()) & 15) == 0; }
+int64_t stride_of(const Tensor& t, int64_t d) { return t.size(d) == 1 ? 0 : t.stride(d); }   // a dim of one is never stepped over: its stride may be anything
 int64_t div_up(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
 struct Alloc {
@@ -100,10 +101,10 @@ py::object quantize(const Tensor& x_in, bool flat, bool want_row, bool want_col,
   Tensor x = x_in;
   if (!on_gpu(x) || !is_float(x) || x.dim() != (flat ? 2 : 3)) return py::none();
   const int64_t vec = x.scalar_type() == at::kBFloat16 ? 8 : 4;
-  auto readable = [&](const Tensor& t) {   // unit stride along C, everything else in whole 16-byte units (a dim of one has no stride to speak of)
+  auto readable = [&](const Tensor& t) {   // unit stride along C, everything else in whole 16-byte units
     if (t.stride(-1) != 1 || !aligned16(t)) return false;
     for (int64_t d = 0; d + 1 < t.dim(); ++d)
-      if (t.size(d) != 1 && t.stride(d) % vec != 0) return false;
+      if (stride_of(t, d) % vec != 0) return false;
     return true;
   };
   if (!readable(x)) {
@@ -237,7 +238,7 @@ bool attend(const Tensor& q_in, const Tensor& k_in, const Tensor& v_in, double s
   for (Tensor* t : {&q, &k, &v}) {
     if (!on_gpu(*t) || !is_float(*t) || t->dim() != 4 || t->scalar_type() != q_in.scalar_type()) return false;
     const int64_t vec = t->scalar_type() == at::kBFloat16 ? 8 : 4;
-    if (t->stride(3) != 1 || !aligned16(*t) || t->stride(0) % vec != 0 || t->stride(1) % vec != 0 || t->stride(2) % vec != 0) *t = t->contiguous();
+    if (t->stride(3) != 1 || !aligned16(*t) || stride_of(*t, 0) % vec != 0 || stride_of(*t, 1) % vec != 0 || stride_of(*t, 2) % vec != 0) *t = t->contiguous();
   }
   const int64_t B = q.size(0), Hq = q.size(1), Sq = q.size(2), D = q.size(3), Hk = v.size(1), Sk = v.size(2), Dv = v.size(3);
   if (k.size(0) != v.size(0) || k.size(1) != Hk || k.size(2) != Sk || B != k.size(0) || k.size(3) != D) return false;
@@ -252,8 +253,8 @@ bool attend(const Tensor& q_in, const Tensor& k_in, const Tensor& v_in, double s
   uint8_t* p = bytes(buf);
   uint8_t *qq = p + start[0], *kq = p + start[1], *vq = p + start[2], *qs = p + start[3], *ks = p + start[4], *vs = p + start[5];
   void* s = reinterpret_cast<void*>(stream);
-  call("alto_mxfp4_attention_quantize", api.attention_quantize, q.data_ptr(), k.data_ptr(), v.data_ptr(), dtype_code(q.scalar_type()), B, Hq, Hk, Sq, Sk, D, Dv, q.stride(0),
-       q.stride(1), q.stride(2), k.stride(0), k.stride(1), k.stride(2), v.stride(0), v.stride(1), v.stride(2), qq, qs, kq, ks, vq, vs, s);
+  call("alto_mxfp4_attention_quantize", api.attention_quantize, q.data_ptr(), k.data_ptr(), v.data_ptr(), dtype_code(q.scalar_type()), B, Hq, Hk, Sq, Sk, D, Dv, stride_of(q, 0),
+       stride_of(q, 1), stride_of(q, 2), stride_of(k, 0), stride_of(k, 1), stride_of(k, 2), stride_of(v, 0), stride_of(v, 1), stride_of(v, 2), qq, qs, kq, ks, vq, vs, s);
   const int n = cu_q.empty() ? 0 : (int)cu_q.size() - 1;
   call("alto_mxfp4_attention_fwd_strided", api.attention_fwd_strided, qq, qs, kq, ks, vq, vs, out.data_ptr(), static_cast<float*>(lse.data_ptr()), B, Hq, Hk, Sq, Sk, D, Dv,
        out.stride(0), out.stride(1), out.stride(2), lse.stride(0), lse.stride(1), lse.stride(2), n, n ? cu_q.data() : nullptr, n ? cu_k.data() : nullptr, (float)sm_scale,

@@ -74,11 +74,16 @@ def attention_mxfp4_forward(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, q
     return out, lse
 
 
+def _strides(t: torch.Tensor) -> list:
+    """Element strides of batch, head and row; 0 for a dim of one, which is never stepped over and may have any."""
+    return [0 if n == 1 else s for n, s in zip(t.shape[:3], t.stride())]
+
+
 def _readable(t: torch.Tensor) -> torch.Tensor:
     """``t`` [B, H, S, D] as the operand quantizer reads it: any strides of the first three dims in whole 16-byte units, unit
     stride along D.  Anything else is copied."""
     vec = 8 if t.dtype == torch.bfloat16 else 4
-    ok = t.stride(3) == 1 and t.data_ptr() % 16 == 0 and all(s % vec == 0 for s in t.stride()[:3])
+    ok = t.stride(3) == 1 and t.data_ptr() % 16 == 0 and all(s % vec == 0 for s in _strides(t))
     return t if ok else t.contiguous()
 
 
@@ -101,7 +106,7 @@ def quantize_qkv(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor):
     buf = torch.empty(total, dtype=torch.uint8, device=q.device)
     qq, kq, vq, qs, ks, vs = (buf[o:o + n] for o, n in zip(starts, sizes))
     check(rt.lib().alto_mxfp4_attention_quantize(
-        q.data_ptr(), k.data_ptr(), v.data_ptr(), rt.dtype_code(q.dtype), B, Hq, Hk, Sq, Sk, D, Dv, *q.stride()[:3], *k.stride()[:3], *v.stride()[:3],
+        q.data_ptr(), k.data_ptr(), v.data_ptr(), rt.dtype_code(q.dtype), B, Hq, Hk, Sq, Sk, D, Dv, *_strides(q), *_strides(k), *_strides(v),
         qq.data_ptr(), qs.data_ptr(), kq.data_ptr(), ks.data_ptr(), vq.data_ptr(), vs.data_ptr(), rt.stream_ptr(q.device)), "alto_mxfp4_attention_quantize")
     return (qq.view(B, Hq, Sq, D // 2), qs.view(B, Hq, Sq // 32, D // 32), kq.view(B, Hk, Sk, D // 2), ks.view(B, Hk, Sk // 32, D // 32),
             vq.view(B, Hk, Dv, Sk // 2), vs.view(B, Hk, Sk // 32, Dv // 32))

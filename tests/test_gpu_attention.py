@@ -348,3 +348,19 @@ def test_scale_bytes_behind_the_keys_are_not_used(m, D, Dv, causal):
             ref, ref_lse = attention_fwd_ref(q[:, :, q0:q1], k[:, :, k0:k1], v[:, :, k0:k1], causal=causal)
             assert _rel(out[:, :, q0:q1].cpu(), ref) <= REL_L2
             assert float((lse[:, :, q0:q1].cpu() - ref_lse).abs().max()) <= 1e-4
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("slopes", [False, True])
+def test_strides_of_dimensions_of_size_one_do_not_matter(m, dtype, slopes):
+    """One key / value head whose head stride is 1, and a batch of one cut from an odd pitch."""
+    S, Hq, D = 64, 4, 64
+    g = torch.Generator().manual_seed(8)
+    q, k, v = (torch.randn(1, S, h, D, generator=g).to(dtype).to(DEV) for h in (Hq, 1, 1))
+    al = torch.full((Hq,), 0.25, device=DEV) if slopes else None
+    ref, ref_lse, _ = m.triton_attention_mxfp4(q, k, v, al, causal=True, layout="bshd")
+    k1, v1 = (t[:, :, 0].unsqueeze(-1).transpose(-1, -2) for t in (k, v))                 # [1, S, 1, D], head stride 1
+    q1 = q.as_strided(q.shape, (S * Hq * D + 3, Hq * D, D, 1))                          # batch stride off 16 bytes
+    assert k1.stride(2) == 1 and k1.is_contiguous() and q1.is_contiguous()
+    out, lse, _ = m.triton_attention_mxfp4(q1, k1, v1, al, causal=True, layout="bshd")
+    assert torch.equal(out, ref) and torch.equal(lse, ref_lse)

@@ -62,7 +62,8 @@ def test_strides_of_dimensions_of_size_one_do_not_matter(m, dtype):
             q, s = m.convert_to_mxfp4(t, use_sr=True, philox_seed=5)
             ref = m.convert_to_mxfp4(torch.empty(t.shape, dtype=dtype, device=DEV).copy_(t), use_sr=True, philox_seed=5)
             assert torch.equal(q, ref[0]) and torch.equal(s, ref[1]), (name, t.shape)
-    x = big[:1, :64 * C].unflatten(1, (64, C))          # [1, 64, C], batch stride off 16 bytes
+    x = big[0, :64 * C].as_strided((1, 64, C), (64 * C + 3, C, 1))   # batch stride off 16 bytes
+    assert x.is_contiguous()
     for axis in (-1, -2):
         for is_2d in (False, True):
             q, s = m.convert_to_mxfp4(x, axis=axis, is_2d_block=is_2d)
