@@ -74,7 +74,8 @@ void call(const char* name, F fn, A... args) {
 
 int dtype_code(at::ScalarType t) { return t == at::kBFloat16 ? ALTO_DT_BF16 : ALTO_DT_F32; }
 bool is_float(const Tensor& t) { return t.scalar_type() == at::kBFloat16 || t.scalar_type() == at::kFloat; }
-bool on_gpu(const Tensor& t) { return t.is_cuda() && t.layout() == at::kStrided; }
+// (a wrapper subclass has no storage of its own: the Python route resolves it)
+bool on_gpu(const Tensor& t) { return t.is_cuda() && t.layout() == at::kStrided && !t.unsafeGetTensorImpl()->is_python_dispatch(); }
 uint8_t* bytes(const Tensor& t) { return t.defined() ? static_cast<uint8_t*>(t.data_ptr()) : nullptr; }
 bool aligned16(const Tensor& t) { return (reinterpret_cast<uintptr_t>(t.data_ptr()) & 15) == 0; }
 int64_t stride_of(const Tensor& t, int64_t d) { return t.size(d) == 1 ? 0 : t.stride(d); }   // a dim of one is never stepped over: its stride may be anything

@@ -60,6 +60,12 @@ def _quantize_call(x3: torch.Tensor, want_row: bool, want_col: bool, is_2d: bool
     out = rt.host().quantize(x3, flat, want_row, want_col, is_2d, sr_mode, rand3 if sr_mode == 1 else None, seed, offset, state,
                              None if hadamard is None else hadamard.signs, None if hadamard is None else hadamard.perm, clip, use_uos, pad_codes,
                              pack_row_scales, pack_col_scales, rt.stream_ptr(x3.device))
+    if out is None and flat:   # not a plain matrix (a wrapped weight, say): its view as a batch of one is
+        rc, rs, cc, cs = _quantize_call(_prep(x3), want_row, want_col, is_2d, use_sr, rand3, hadamard, clip, use_uos, pad_codes, philox, hw_sr,
+                                        pack_row_scales, pack_col_scales)
+        row = (rc[0], rs[0]) if want_row else (None, None)
+        col = (cc[0].transpose(0, 1), cs[0] if pack_col_scales else cs[0].transpose(0, 1)) if want_col else (None, None)
+        return row + col
     assert out is not None, "the quantizer takes bf16 / fp32 GPU tensors with unit stride along C and 16-byte aligned rows"
     return out
 

@@ -75,6 +75,22 @@ def test_strides_of_dimensions_of_size_one_do_not_matter(m, dtype):
     assert torch.equal(q[:, 0], ref[0]) and torch.equal(s[:, 0], ref[1])
 
 
+def test_wrapped_weight_is_quantized_like_its_payload(m):
+    """A weight that ``swap_params`` has wrapped has no storage of its own: the calls see the tensor inside."""
+    w = randn_outliers((64, 96), torch.bfloat16, seed=12).to(DEV)
+    lin = torch.nn.Linear(96, 64, bias=False, device="meta")
+    lin.weight = torch.nn.Parameter(w.clone())
+    wrapped = m.swap_params(lin, config=m.TrainingOpConfig()).weight
+    assert type(wrapped.data) is not torch.Tensor
+    for axis in (-1, 0):
+        for is_2d in (False, True):
+            got, ref = (m.convert_to_mxfp4(t, axis=axis, is_2d_block=is_2d) for t in (wrapped, w))
+            assert all(type(a) is torch.Tensor and torch.equal(a, b) and a.stride() == b.stride() for a, b in zip(got, ref)), (axis, is_2d)
+    for pack in (False, True):
+        got, ref = (m.quantize_rowcol(t, True, pad_codes=True, pack_row_scales=pack, pack_col_scales=pack) for t in (wrapped, w))
+        assert all(type(a) is torch.Tensor and torch.equal(a, b) and a.stride() == b.stride() for a, b in zip(got, ref)), pack
+
+
 @pytest.mark.parametrize("sr", [False, True])
 @pytest.mark.parametrize("pack", [False, True])
 def test_quantize_rowcol_reads_every_stride(m, sr, pack):
