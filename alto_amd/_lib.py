@@ -109,7 +109,7 @@ def load():
             _lib = lib
             return lib
         path = _build.lib_path()
-        if not os.path.exists(path) or not os.path.exists(_build.host_path()):
+        if not os.path.exists(path):
             _build.build(verbose=False)
         elif _build.is_stale():
             if os.environ.get("ALTO_MXFP4_NO_REBUILD") == "1":
@@ -127,7 +127,9 @@ def load():
 
 
 def host():
-    """The native host side (csrc/host.cpp), bound to the functions of the library that ``load`` gives."""
+    """The native host side (csrc/host.cpp), bound to the functions of the library that ``load`` gives.  Built first when it does
+    not exist or was made for other sources, another torch or another interpreter than these (also beside an explicit
+    library); ``ALTO_MXFP4_NO_REBUILD=1`` turns a stale one into an error instead."""
     global _host
     if _host is not None:
         return _host
@@ -137,8 +139,13 @@ def host():
             import importlib.machinery
             import importlib.util
             path = _build.host_path()
-            if not os.path.exists(path):   # (an explicit library was loaded from a tree that has not been built)
-                _build.build(verbose=False)
+            if _build.host_is_stale():
+                if os.path.exists(path):
+                    if os.environ.get("ALTO_MXFP4_NO_REBUILD") == "1":
+                        raise AltoMxfp4Error(f"{path} was not built from the sources in this tree for this torch: run `python -m alto_amd.build`")
+                    import sys
+                    print(f"alto_amd: {path} was built from other sources or for another torch, rebuilding", file=sys.stderr, flush=True)
+                _build.build_host()
             loader = importlib.machinery.ExtensionFileLoader("alto_mxfp4_host", path)
             mod = importlib.util.module_from_spec(importlib.util.spec_from_file_location("alto_mxfp4_host", path, loader=loader))
             loader.exec_module(mod)

@@ -17,6 +17,8 @@ LIBDIR = os.path.join(HERE, "lib")
 OBJDIR = os.path.join(HERE, "lib", "obj")
 LIBNAME = "libalto_mxfp4.so"
 HOSTNAME = "alto_mxfp4_host.so"   # CPython module of csrc/host.cpp, named as its PYBIND11_MODULE
+HOSTSRC = os.path.join(CSRC, "host.cpp")
+HEADER = os.path.join(HERE, "..", "include", "alto_mxfp4.h")
 
 SOURCES = ["capi.hip", "quantize.hip", "dequantize.hip", "gemm.hip", "gemm_tiled.hip", "gemm_mid.hip", "gemm_skinny.hip", "grouped_gemm.hip", "probe.hip", "qdq.hip", "attention.hip", "attention_quantize.hip", "quantize_dynamic.hip", "random.hip"]
 
@@ -31,6 +33,8 @@ HIPCC_FLAGS = [
     "-Wno-unused-command-line-argument",
 ]
 
+HOST_FLAGS = ["-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1"]
+
 
 def lib_path() -> str:
     return os.path.join(LIBDIR, LIBNAME)
@@ -40,16 +44,13 @@ def host_path() -> str:
     return os.path.join(LIBDIR, HOSTNAME)
 
 
-def stamp_path() -> str:
-    return lib_path() + ".srchash"
+def stamp_path(path: str = "") -> str:
+    return (path or lib_path()) + ".srchash"
 
 
-def source_hash() -> str:
-    """Digest of every file the library is built from (kernels, their headers, the C ABI header, the compiler flags)."""
+def _digest(first: str, files) -> str:
     import hashlib
-    h = hashlib.sha256(" ".join(HIPCC_FLAGS).encode())
-    files = sorted(os.path.join(CSRC, f) for f in os.listdir(CSRC) if f.endswith((".hip", ".h", ".cpp")))
-    files.append(os.path.join(HERE, "..", "include", "alto_mxfp4.h"))
+    h = hashlib.sha256(first.encode())
     for f in files:
         h.update(os.path.basename(f).encode())
         with open(f, "rb") as fh:
@@ -57,13 +58,35 @@ def source_hash() -> str:
     return h.hexdigest()
 
 
+def source_hash() -> str:
+    """Digest of every file the library is built from (kernels, their headers, the C ABI header, the compiler flags)."""
+    files = sorted(os.path.join(CSRC, f) for f in os.listdir(CSRC) if f.endswith((".hip", ".h")))
+    return _digest(" ".join(HIPCC_FLAGS), files + [HEADER])
+
+
+def host_hash() -> str:
+    """Digest of what the host module is built from: its source, the C ABI header whose functions it calls, the flags, and the
+    interpreter and torch whose binary interfaces it is compiled against."""
+    import torch
+    return _digest(" ".join([*HOST_FLAGS, sys.implementation.cache_tag, torch.__version__, str(torch._C._GLIBCXX_USE_CXX11_ABI)]), [HOSTSRC, HEADER])
+
+
+def _recorded(path: str) -> str:
+    try:
+        with open(stamp_path(path)) as f:
+            return f.read().strip()
+    except OSError:
+        return ""
+
+
 def is_stale() -> bool:
     """True when the built library does not come from the sources in the tree (or carries no record of its sources)."""
-    try:
-        with open(stamp_path()) as f:
-            return f.read().strip() != source_hash()
-    except OSError:
-        return True
+    return _recorded(lib_path()) != source_hash()
+
+
+def host_is_stale() -> bool:
+    """True when there is no host module, or one of other sources, another interpreter or another torch than these."""
+    return not os.path.exists(host_path()) or _recorded(host_path()) != host_hash()
 
 
 def _hipcc() -> str:
@@ -82,20 +105,26 @@ def _compile(src: str) -> str:
     return obj
 
 
-def _compile_host() -> None:
-    """csrc/host.cpp against the installed torch: host code only, so the host compiler does it."""
+def build_host() -> str:
+    """Compile csrc/host.cpp against the installed torch: host code only, so the host compiler does it."""
     import sysconfig
 
     import torch
+    os.makedirs(LIBDIR, exist_ok=True)
+    digest = host_hash()
     tdir = os.path.dirname(torch.__file__)
     out = host_path()
-    cmd = [shutil.which("g++") or "g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
-           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", f"-I{tdir}/include", f"-I{tdir}/include/torch/csrc/api/include",
-           f"-I{sysconfig.get_paths()['include']}", os.path.join(CSRC, "host.cpp"), "-o", out + ".tmp", f"-L{tdir}/lib", "-lc10", "-ltorch_cpu", "-ltorch_python"]
+    tmp = f"{out}.{os.getpid()}.tmp"
+    cmd = [shutil.which("g++") or "g++", *HOST_FLAGS, f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", f"-I{tdir}/include",
+           f"-I{tdir}/include/torch/csrc/api/include", f"-I{sysconfig.get_paths()['include']}", HOSTSRC, "-o", tmp, f"-L{tdir}/lib", "-lc10", "-ltorch_cpu",
+           "-ltorch_python"]
     res = subprocess.run(cmd, capture_output=True, text=True)
     if res.returncode != 0:
         raise RuntimeError(f"g++ failed for host.cpp:\n{res.stdout}\n{res.stderr}")
-    os.replace(out + ".tmp", out)
+    os.replace(tmp, out)
+    with open(stamp_path(out), "w") as f:
+        f.write(digest + "\n")
+    return out
 
 
 def build(verbose: bool = True) -> str:
@@ -103,7 +132,7 @@ def build(verbose: bool = True) -> str:
     os.makedirs(OBJDIR, exist_ok=True)
     digest = source_hash()   # taken before compiling: an edit made during the build leaves the library marked stale
     with ThreadPoolExecutor(max_workers=min(8, len(SOURCES))) as pool:
-        host = pool.submit(_compile_host)
+        host = pool.submit(build_host)
         objs = list(pool.map(_compile, SOURCES))
         host.result()
     out = lib_path()

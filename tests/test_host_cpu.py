@@ -307,3 +307,40 @@ def test_wrapped_weights_and_config_survive_a_weights_only_round_trip(tmp_path):
     assert isinstance(back["weight"], m.MXFP4TrainingWeightWrapperTensor)
     assert back["config"] == cfg and back["weight"].config == cfg
     assert torch.equal(back["weight"]._data, w)
+
+
+def test_host_module_is_stale_for_another_torch_interpreter_or_source(monkeypatch, tmp_path):
+    """The native host module is compiled against one torch and one interpreter: its digest names both, and its source, the C ABI
+    header and the flags; a stale module is an error where rebuilding is switched off, also beside an explicit library."""
+    import shutil
+    import sys
+    from types import SimpleNamespace
+
+    from alto_amd import _lib
+    from alto_amd import build as B
+    _lib.host()
+    assert not B.host_is_stale()
+    with monkeypatch.context() as p:
+        p.setattr(torch, "__version__", "0.0.1")
+        assert B.host_is_stale()
+    with monkeypatch.context() as p:
+        p.setattr(sys, "implementation", SimpleNamespace(**{**vars(sys.implementation), "cache_tag": "other"}))
+        assert B.host_is_stale()
+    with monkeypatch.context() as p:
+        p.setattr(B, "HOST_FLAGS", [*B.HOST_FLAGS, "-g"])
+        assert B.host_is_stale()
+    for name in ("HOSTSRC", "HEADER"):
+        edited = tmp_path / os.path.basename(getattr(B, name))
+        shutil.copy(getattr(B, name), edited)
+        with monkeypatch.context() as p:
+            p.setattr(B, name, str(edited))
+            assert not B.host_is_stale()
+            edited.write_text(edited.read_text() + "\n")
+            assert B.host_is_stale()
+    with monkeypatch.context() as p:   # nothing is imported from a stale file, whichever library was loaded
+        p.setattr(_lib, "_host", None)
+        p.setattr(torch, "__version__", "0.0.1")
+        p.setenv("ALTO_MXFP4_NO_REBUILD", "1")
+        with pytest.raises(_lib.AltoMxfp4Error, match="was not built"):
+            _lib.host()
+    assert not B.host_is_stale()
