@@ -7,9 +7,10 @@
 // over the 16 accumulator registers, so the per-row softmax state (running max, rescale factor) is one scalar per lane
 // and the only cross-lane traffic is between the two lanes (l, l ^ 32) that share a row.
 #include <algorithm>
+#include <memory>
+#include <new>
 #include <type_traits>
 #include <utility>
-#include <vector>
 
 #include "common.h"
 
@@ -512,9 +513,16 @@ extern "C" int alto_mxfp4_attention_fwd_strided(const void* q_codes, const void*
                  cu_k[i + 1] - cu_k[i]);
   }
   // longest sequences first, up to ATTN_MAX_SEQS of them and 65535 row blocks per launch
-  std::vector<int> order((size_t)n_seqs);
+  std::unique_ptr<int[]> order(new (std::nothrow) int[(size_t)n_seqs]);   // (no exception may leave a C entry)
+  if (!order) {
+    set_error("attention_fwd: no host memory for the order of %d sequences", n_seqs);
+    return ALTO_MXFP4_ELAUNCH;
+  }
   for (int i = 0; i < n_seqs; ++i) order[(size_t)i] = i;
-  std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return cu_k[x + 1] - cu_k[x] > cu_k[y + 1] - cu_k[y]; });
+  std::sort(order.get(), order.get() + n_seqs, [&](int x, int y) {
+    const int kx = cu_k[x + 1] - cu_k[x], ky = cu_k[y + 1] - cu_k[y];
+    return kx != ky ? kx > ky : x < y;
+  });
   for (int at = 0; at < n_seqs;) {
     AttnSeqs t;
     t.n = 0;

@@ -13,8 +13,24 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <new>
 
 #include "alto_mxfp4.h"
+
+// Host allocations of the library fail on demand: a C entry must answer that with an error code, not with an exception.
+static bool g_no_memory = false;
+void* operator new(std::size_t n) {
+  void* p = g_no_memory ? nullptr : std::malloc(n ? n : 1);
+  if (p == nullptr) throw std::bad_alloc();
+  return p;
+}
+void* operator new(std::size_t n, const std::nothrow_t&) noexcept { return g_no_memory ? nullptr : std::malloc(n ? n : 1); }
+void* operator new[](std::size_t n) { return operator new(n); }
+void* operator new[](std::size_t n, const std::nothrow_t& t) noexcept { return operator new(n, t); }
+void operator delete(void* p) noexcept { std::free(p); }
+void operator delete(void* p, std::size_t) noexcept { std::free(p); }
+void operator delete[](void* p) noexcept { std::free(p); }
+void operator delete[](void* p, std::size_t) noexcept { std::free(p); }
 
 namespace {
 
@@ -285,6 +301,16 @@ int main(int argc, char** argv) {
       std::fprintf(stderr, "host code wrote through a pointer that stands for device memory (byte %u)\n", k);
       return 3;
     }
+  for (Entry& e : g_entries) {   // the entry that allocates on the host, once without memory (an exception would end the process)
+    if (std::strcmp(e.name, "attention_fwd_strided") != 0) continue;
+    g_no_memory = true;
+    const int rc = e.call(e.valid);
+    g_no_memory = false;
+    if (rc == 0 || std::strstr(alto_mxfp4_last_error(), "memory") == nullptr) {
+      std::fprintf(stderr, "%s without host memory: code %d, %s\n", e.name, rc, alto_mxfp4_last_error());
+      return 5;
+    }
+  }
   int never = 0;
   for (int n = 0; n < kEntries; ++n) {
     const Entry& e = g_entries[n];
