@@ -17,6 +17,25 @@ __global__ __launch_bounds__(256) void gemm_simple_kernel(OperandView A, Operand
   store_tile_32x32<OutT>(acc, c, ldc, m0, n0, 0, M, N, out_scale);
 }
 
+// Reductions shorter than the 512 of the 256x256 tile take the direct kernel, which starts its MFMAs after one trip to memory,
+// until there is enough work to fill the ring of the 64x64 or 128x128 tile and empty it again.  us, direct / tiles:
+//   M x N \ K, bf16          64          192         256         320         416         480
+//   33 x 4096            3.1/4.3     3.3/4.3     3.8/4.3     3.7/4.5     4.1/4.5     4.3/4.5
+//   500 x 4096           3.7/5.8     4.1/5.8     5.6/5.8     4.9/6.2     5.6/6.2     6.0/6.3
+//   1024 x 4096          4.9/7.8     5.9/7.9     8.5/7.8     7.4/8.4     9.0/8.4     9.7/8.6     256 tiles of 128
+//   2048 x 4096          7.9/11.0    8.9/11.1   13.9/11.1   11.8/11.5   14.9/11.6   16.4/12.1    512
+//   8192 x 4096         19.2/31.3   23.9/31.3   43.5/31.6   39.6/34.2   55.3/34.7   62.6/34.8
+//   2048 x 4096, fp32    8.7/14.9    9.8/15.1   15.4/15.1   12.8/15.7   16.2/16.1   17.8/16.4
+//   8192 x 4096, fp32   22.9/43.9   24.8/44.3   45.5/44.3   41.1/47.5   57.5/48.0   64.5/48.7
+// (K = 256: the direct kernel's lanes read rows that are all exactly one 128-byte line apart.)
+bool direct_pays(int64_t M, int64_t N, int64_t K, int c_dtype) {
+  if (K >= 512) return false;
+  const int64_t tiles = ((M + 127) / 128) * ((N + 127) / 128);
+  if (c_dtype == ALTO_DT_F32) return tiles < 432 || K < 416;
+  if (K == 256 || K >= 416) return tiles < 216;
+  return tiles < 432 || K < 256;
+}
+
 }  // namespace
 }  // namespace alto
 
@@ -41,20 +60,22 @@ extern "C" int alto_mxfp4_gemm(const uint8_t* a, int64_t lda, const uint8_t* a_s
   OperandView A{a, lda, a_scales, a_ss_r, a_ss_k, a_is_2d};
   OperandView B{b, ldb, b_scales, b_ss_r, b_ss_k, b_is_2d};
 
-  if (gemm_skinny_supported(A, B, M, N, K)) {
+  if (gemm_skinny_supported(A, B, M, N, K) && gemm_skinny_pays(M, N, K)) {
     gemm_skinny_launch(A, B, M, N, K, c, c_dtype, ldc, out_scale, st);
     return check_launch("gemm(skinny)");
   }
-  const bool tiled = gemm_tiled_supported(A, B, M, N, K, c, c_dtype, ldc);
-  int tile = gemm_mid_tile_size(M, N, c_dtype);
-  if (tile == 256 && !tiled) tile = 128;   // (a long, narrow result or a short reduction)
-  if (tile != 256 && gemm_mid_supported(A, B, M, N, K, c, ldc)) {
-    gemm_mid_launch(tile, A, B, M, N, K, c, c_dtype, ldc, out_scale, false, st);
-    return check_launch("gemm(mid)");
-  }
-  if (tiled) {
-    gemm_tiled_launch(A, B, M, N, K, c, c_dtype, ldc, out_scale, st);
-    return check_launch("gemm(tiled)");
+  if (!(direct_pays(M, N, K, c_dtype) && (M + 63) / 64 <= 65535)) {
+    const bool tiled = gemm_tiled_supported(A, B, M, N, K, c, c_dtype, ldc);
+    int tile = gemm_mid_tile_size(M, N, c_dtype);
+    if (tile == 256 && !tiled) tile = 128;   // (a long, narrow result or a short reduction)
+    if (tile != 256 && gemm_mid_supported(A, B, M, N, K, c, ldc)) {
+      gemm_mid_launch(tile, A, B, M, N, K, c, c_dtype, ldc, out_scale, false, st);
+      return check_launch("gemm(mid)");
+    }
+    if (tiled) {
+      gemm_tiled_launch(A, B, M, N, K, c, c_dtype, ldc, out_scale, st);
+      return check_launch("gemm(tiled)");
+    }
   }
   dim3 grid((unsigned)((N + 63) / 64), (unsigned)((M + 63) / 64));
   ALTO_REQUIRE(grid.y <= 65535u, "gemm: M too large for the fallback kernel");

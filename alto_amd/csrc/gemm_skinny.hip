@@ -160,9 +160,27 @@ void dispatch_rows(const OperandView& A, const OperandView& B, int64_t M, int64_
 
 }  // namespace
 
-// Offsets inside 32 rows of A and of B are 32-bit.
+// Offsets inside 32 rows of A and 64 of B (four strips) are 32-bit.
 bool gemm_skinny_supported(const OperandView& A, const OperandView& B, int64_t M, int64_t N, int64_t K) {
   return M <= 32 && K > 0 && A.ld < (1ll << 25) && B.ld < (1ll << 25);
+}
+
+// Below 1024 K some of the four waves have no piece of the reduction and a partial piece loads its scales byte by byte, so wide
+// results go to the kernels that deal out columns only: the direct kernel below 512, the 64x64 tiles from 512 on.  us,
+// here / there, at 16 and 32 rows:
+//   M x N \ K           320         416         512         544         640         768         992        1024
+//   16 x 4096       3.2/3.4     3.2/3.7     2.7/3.5     2.8/4.1     3.1/4.0     3.3/4.1     3.2/4.4     3.0/4.1
+//   16 x 8192       3.8/3.4     3.8/3.7     2.9/3.4     3.2/4.1     3.7/4.0     4.0/4.0     3.9/4.3     3.4/4.1
+//   16 x 14336      4.9/3.4     4.9/3.8     3.4/3.6     3.9/4.3     4.8/4.2     5.4/4.2     5.1/4.5     4.2/4.2
+//   32 x 4096       3.8/3.6     3.8/4.0     2.9/3.5     3.2/4.2     3.7/4.1     4.0/4.1     3.9/4.4     3.4/4.2
+//   32 x 10240      4.6/3.7     4.6/4.0     3.8/3.6     4.0/4.3     4.7/4.2     5.5/4.2     5.0/4.5     4.9/4.3
+//   32 x 14336      5.7/3.7     5.8/4.1     3.9/3.7     4.6/4.3     5.6/4.2     6.4/4.2     6.3/4.6     4.9/4.3
+bool gemm_skinny_pays(int64_t M, int64_t N, int64_t K) {
+  const int64_t strips = (N + 15) / 16;   // (384 and 640: where a workgroup's columns double)
+  if (K >= 1024) return true;
+  if (K < 512) return strips <= 384 && K >= (M <= 16 ? 320 : 416);
+  if (K <= 544) return K == 512 || M <= 16 || strips <= 640;
+  return strips <= (M <= 16 ? 640 : 384);
 }
 
 void gemm_skinny_launch(const OperandView& A, const OperandView& B, int64_t M, int64_t N, int64_t K, void* c, int c_dtype, int64_t ldc, float out_scale,

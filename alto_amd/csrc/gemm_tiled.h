@@ -12,6 +12,7 @@ void gemm_tiled_launch_ps(const OperandView& A, const OperandView& B, int64_t M,
                           hipStream_t st);
 // Few rows of A (see gemm_skinny.hip).
 bool gemm_skinny_supported(const OperandView& A, const OperandView& B, int64_t M, int64_t N, int64_t K);
+bool gemm_skinny_pays(int64_t M, int64_t N, int64_t K);
 void gemm_skinny_launch(const OperandView& A, const OperandView& B, int64_t M, int64_t N, int64_t K, void* c, int c_dtype, int64_t ldc, float out_scale,
                         hipStream_t st);
 // 128x128 and 64x64 tiles (see gemm_mid.hip): which tile a shape takes (256, 128 or 64), and the launch of the two smaller ones.

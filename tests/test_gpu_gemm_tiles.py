@@ -66,3 +66,26 @@ def test_gemm_tiles_of_every_size_give_the_same_bits(m, K, packed):
     whole = product(2304)
     assert torch.equal(product(1000), whole[:1000])
     assert torch.equal(product(500), whole[:500])
+
+
+# Both sides of the lines where a short reduction goes to the direct kernel, to the kernel for few rows (16, 32 or 64 columns per
+# workgroup) or to the small tiles
+@pytest.mark.parametrize("M,N,K", [(16, 6144, 288), (16, 6144, 320), (17, 6144, 384), (17, 6144, 416), (1, 6160, 480), (1, 6160, 512), (32, 6160, 544),
+                                   (32, 6160, 576), (16, 10256, 512), (17, 10256, 512), (16, 10256, 544), (17, 10256, 544), (16, 10256, 992), (32, 10256, 1056),
+                                   (3328, 1024, 256), (3456, 1024, 256), (3456, 1024, 384), (3328, 1024, 416), (3456, 1024, 416), (3456, 2048, 224),
+                                   (3328, 2048, 288), (3456, 2048, 288), (3456, 2048, 384), (3328, 2048, 416), (3456, 2048, 416)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_gemm_short_reductions(m, M, N, K, dtype):
+    check(m, M, N, K, N % 32 == 0, dtype, strided_scales=(M == 17))
+
+
+def test_gemm_short_reduction_of_many_rows(m):
+    """More rows than a grid dimension of the direct kernel has 64-row groups for."""
+    M, N, K = 65535 * 64 + 96, 8, 32
+    aq = torch.randint(0, 256, (M, K // 2), dtype=torch.uint8, device=DEV, generator=torch.Generator(DEV).manual_seed(1))
+    as_ = torch.full((M, 1), 126, dtype=torch.uint8, device=DEV)
+    bq, bs = m.convert_to_mxfp4(randn_outliers((N, K), torch.bfloat16, seed=7).to(DEV))
+    c = m.blockwise_mxfp4_gemm(aq, as_, bq, bs, trans_b=True)
+    for lo in (0, M - 200):
+        part = m.blockwise_mxfp4_gemm(aq[lo:lo + 200], as_[lo:lo + 200], bq, bs, trans_b=True)
+        assert O.rel_frobenius(c[lo:lo + 200].cpu(), part.cpu()) < TOL[torch.float32]
