@@ -766,10 +766,10 @@ int fill_hadamard(QuantParams& p, const int8_t* signs, const uint8_t* perm, cons
 }
 
 // bpw8: the caller laid the grid out for workgroups of 8 bands (column outputs of large 2D-block tensors, !GEN only)
-// stream: the pass moves more than any cache holds (row + column passes of the training step only)
+// stream: the pass moves more than any cache holds (bf16 row + column passes of the training step only)
 template <typename T, bool DO_ROW, bool DO_COL, int SR, bool RHT, bool B2D, bool GEN>
 void launch(const QuantParams& p, dim3 grid, hipStream_t st, bool bpw8, bool stream) {
-  if constexpr (DO_ROW && DO_COL && !GEN && (B2D ? SR == 0 : (SR == 0 || SR == 3))) {
+  if constexpr (sizeof(T) == 2 && DO_ROW && DO_COL && !GEN && (B2D ? SR == 0 : (SR == 0 || SR == 3))) {
     if (stream && bpw8 == B2D) {
       hipLaunchKernelGGL((quant_kernel<T, DO_ROW, DO_COL, SR, RHT, B2D, GEN, B2D ? 8 : 1, true>), grid, dim3(256), 0, st, p);
       return;
@@ -914,12 +914,14 @@ int quantize_impl(const void* x, int dtype, int64_t batch, int64_t M, int64_t C,
   // all of those keep one band per workgroup.  ALTO_MXFP4_QUANT_BANDS=1|8 overrides the choice (tests, measurements).
   static const int force_bpw = [] { const char* e = getenv("ALTO_MXFP4_QUANT_BANDS"); return e ? atoi(e) : 0; }();
   const bool bpw8 = do_col && is_2d && !gen && (force_bpw == 8 || (force_bpw != 1 && tiles_x * ((bands + 7) / 8) * batch >= 4096));
-  // A pass that reads and writes more than the 256 MB of the last-level cache streams through: loads and whole-line stores
-  // bypass the caches (us, before -> now: 8192 x 14336 round to nearest 83 -> 80, the whole training step around it on changing inputs
-  // 810 -> 806; 65536 x 2880 130 -> 123, 65536 x 5760 254 -> 240, stochastic 293 -> 288, the 32 x 5760 x 2880 expert weights 362 -> 302).
-  // Smaller tensors may still sit in the cache, or leave their codes there for the GEMM that follows: 14336 x 4096 (117 MB)
-  // weights 30 -> 38 when streamed, 2048 x 4096 with its GEMM 47 -> 51.
-  const bool streaming = batch * M * C * (dtype == ALTO_DT_BF16 ? 3 : 5) >= (256ll << 20);
+  // A bf16 pass that reads and writes more than the 256 MB of the last-level cache streams through: loads and whole-line stores
+  // bypass the caches.  us, ordinary -> streamed, the pass by itself: round to nearest 14048 x 8000 83 -> 78, 33728 x 5952
+  // 146 -> 136, with the Hadamard transform 82 -> 79 and 142 -> 136, stochastic 96 -> 95 and 163 -> 162, the 32 x 5760 x 2880
+  // expert weights 346 -> 309.  Smaller tensors may still sit in the cache, or leave their codes there for the GEMM that
+  // follows: 14336 x 4096 (117 MB) weights 30 -> 38 when streamed, 2048 x 4096 with its GEMM 47 -> 51.  fp32 passes lose: each
+  // row is read by two load instructions that use half of its lines each, and the second finds them in no cache (6400 x 9504
+  // 68 -> 77, with the transform 67 -> 79; 33728 x 5952 250 -> 256 and 229 -> 254; expert weights 547 -> 556).
+  const bool streaming = dtype == ALTO_DT_BF16 && batch * M * C * 3 >= (256ll << 20);
   const int64_t wrows = bpw8 ? (bands + 7) / 8 : bands;   // workgroup rows
   // With a column output: 2^unit_shift workgroup rows per unit, units padded to a multiple of 8.  The largest unit (up to the
   // 128 bands of a line of plain column scales) whose padding launches at most 5 % more workgroups than there are tiles;
