@@ -1,4 +1,6 @@
 // MXFP4 dequantizer and nibble transpose (gfx950).
+#include <type_traits>
+
 #include "common.h"
 
 namespace alto {
@@ -21,12 +23,17 @@ __device__ __forceinline__ void decode8(uint32_t w, float sf, int static_clip, f
 // Dense output (unit column stride, rows of C elements, 16-byte aligned): codes, scales (1D) and output are then all linear
 // in the index of the lane's chunk, so nothing is divided per thread except for 2D scales.  A lane stores one 16-byte chunk
 // (8 bf16 or 4 fp32 elements), so that a wave instruction writes a whole kilobyte, and takes DEQ_CHUNKS of them a workgroup
-// apart, with all their loads in flight.  Bound by memory;
-// the results go out as non-temporal stores.  4096 x 4096 to bf16 (42 MB moved) took 25.4 us with the general kernel below (two
-// 64-bit divisions per thread, eight 2-byte stores), 7.9 with this one and ordinary stores, 6.4 now; to fp32 15.9 with two half
-// kilobytes per wave instruction, 12.3 with whole ones, 11.1 with non-temporal stores (8192 x 8192: 58 / 48 / 42.6).
+// apart, with all their loads in flight.  Bound by memory.  4096 x 4096 to bf16 (42 MB moved) took 25.4 us with the general
+// kernel below (two 64-bit divisions per thread, eight 2-byte stores), 7.9 with this one and ordinary stores, 6.4 with
+// non-temporal ones; to fp32 15.9 with two half kilobytes per wave instruction, 12.3 with whole ones, 11.1 with
+// non-temporal stores (8192 x 8192: 58 / 48 / 42.6).
+// STREAM: non-temporal stores, for results of 8 MB and more.  A smaller one gains nothing by them (2 MB: 2.4 us either way) and
+// its reader finds it in no cache: dequantize and multiply by [C, 64], us ordinary / non-temporal: 160 x 2880 17.8 / 20.1,
+// 352 x 2912 17.9 / 20.7, 1024 x 2048 13.5 / 15.2, 2048 x 2048 (8 MB) 15.6 / 16.9 and 3.5 / 3.1 by itself, 2048 x 4096
+// 26.0 / 24.9 and 5.2 / 3.9.
 constexpr int DEQ_CHUNKS = 4;
-template <typename OutT, bool B2D>
+constexpr int64_t DEQ_STREAM_BYTES = 8ll << 20;
+template <typename OutT, bool B2D, bool STREAM>
 __global__ __launch_bounds__(256) void dequant_dense_kernel(const uint8_t* __restrict__ codes, const uint8_t* __restrict__ scales, int64_t n,
                                                             uint32_t chunks_per_row, OutT* __restrict__ out, int static_clip) {
   constexpr bool BF = sizeof(OutT) == 2;
@@ -57,7 +64,9 @@ __global__ __launch_bounds__(256) void dequant_dense_kernel(const uint8_t* __res
     v4i_t o;
     if constexpr (BF) o = v4i_t{(int)pack_bf16x2(v[0], v[1]), (int)pack_bf16x2(v[2], v[3]), (int)pack_bf16x2(v[4], v[5]), (int)pack_bf16x2(v[6], v[7])};
     else o = v4i_t{(int)f2u(v[0]), (int)f2u(v[1]), (int)f2u(v[2]), (int)f2u(v[3])};
-    __builtin_nontemporal_store(o, reinterpret_cast<v4i_t*>(out + k * VEC));
+    v4i_t* dst = reinterpret_cast<v4i_t*>(out + k * VEC);
+    if constexpr (STREAM) __builtin_nontemporal_store(o, dst);
+    else *dst = o;
   }
 }
 
@@ -133,13 +142,15 @@ extern "C" int alto_mxfp4_dequantize(const uint8_t* codes, const uint8_t* scales
     const int64_t nc = out_dtype == ALTO_DT_BF16 ? n : 2 * n;   // chunks of 16 bytes
     const uint32_t cpr = (uint32_t)(C / (out_dtype == ALTO_DT_BF16 ? 8 : 4));
     const dim3 grid((unsigned)((nc + 256 * DEQ_CHUNKS - 1) / (256 * DEQ_CHUNKS)));
-    if (out_dtype == ALTO_DT_BF16) {
-      if (is_2d) hipLaunchKernelGGL((dequant_dense_kernel<__bf16, true>), grid, dim3(256), 0, st, codes, scales, nc, cpr, (__bf16*)out, sc);
-      else hipLaunchKernelGGL((dequant_dense_kernel<__bf16, false>), grid, dim3(256), 0, st, codes, scales, nc, cpr, (__bf16*)out, sc);
-    } else {
-      if (is_2d) hipLaunchKernelGGL((dequant_dense_kernel<float, true>), grid, dim3(256), 0, st, codes, scales, nc, cpr, (float*)out, sc);
-      else hipLaunchKernelGGL((dequant_dense_kernel<float, false>), grid, dim3(256), 0, st, codes, scales, nc, cpr, (float*)out, sc);
-    }
+    const bool stream_out = 16 * nc >= DEQ_STREAM_BYTES;
+    auto go = [&](auto kern, auto* dst) { hipLaunchKernelGGL(kern, grid, dim3(256), 0, st, codes, scales, nc, cpr, dst, sc); };
+    auto pick = [&](auto* dst) {
+      using T = std::remove_pointer_t<decltype(dst)>;
+      if (is_2d) stream_out ? go(dequant_dense_kernel<T, true, true>, dst) : go(dequant_dense_kernel<T, true, false>, dst);
+      else stream_out ? go(dequant_dense_kernel<T, false, true>, dst) : go(dequant_dense_kernel<T, false, false>, dst);
+    };
+    if (out_dtype == ALTO_DT_BF16) pick((__bf16*)out);
+    else pick((float*)out);
     return check_launch("dequantize");
   }
   const dim3 grid((unsigned)((n + 255) / 256));

@@ -16,7 +16,9 @@ def m():
     return mod
 
 
-@pytest.mark.parametrize("rows,C,is_2d", [(256, 512, False), (256, 512, True), (33, 96, False), (32, 32, True), (1, 32, False), (3, 8224, False)])
+@pytest.mark.parametrize("rows,C,is_2d", [(256, 512, False), (256, 512, True), (33, 96, False), (32, 32, True), (1, 32, False), (3, 8224, False),
+                                           # results just below and from 8 MB on (bf16, then fp32): ordinary and non-temporal stores
+                                           (8191, 512, False), (8192, 512, False), (8160, 512, True), (4095, 512, False), (4096, 512, True)])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("clip_mode", ["none", "static"])
 def test_dequantize_every_code_and_scale(m, rows, C, is_2d, dtype, clip_mode):
