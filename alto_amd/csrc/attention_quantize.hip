@@ -189,17 +189,17 @@ extern "C" int alto_mxfp4_attention_quantize(const void* q, const void* k, const
   ALTO_REQUIRE(nq > 0 && nk > 0 && nv > 0 && nq + nk + nv < (1ll << 31), "attention_quantize: too many workgroups");
   const dim3 grid((unsigned)(nq + nk + nv));
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-  // Operands of 128 MB and more are read past the caches, which then keep the codes for the attention kernel (whole calls, bf16,
-  // causal, changing inputs, without -> with, us: 160 MB 216 -> 213, 192 MB 346 -> 341, 320 MB 432 -> 420).  Smaller ones may be in a
-  // cache already (20 MB 32.2 -> 33.0, 40 MB 65 -> 67; 80 and 96 MB the same).
-  const bool stream_in = (B * Hq * Sq * D + B * Hk * Sk * (D + Dv)) * (dtype == ALTO_DT_BF16 ? 2 : 4) >= (128ll << 20);
+  // bf16 operands of 128 MB and more are read past the caches, which then keep the codes for the attention kernel (whole calls,
+  // causal, changing inputs, without -> with, us: 160 MB 222 -> 216, 320 MB 443 -> 430).  Smaller ones may be in a cache already
+  // (96 MB the same).  fp32 operands lose: two load instructions use half of each line, and the second finds it in no cache
+  // (this kernel at 192 MB 45 -> 51, at 640 MB 141 -> 157; whole calls 131 -> 137 and 490 -> 502).
+  const bool stream_in = dtype == ALTO_DT_BF16 && (B * Hq * Sq * D + B * Hk * Sk * (D + Dv)) * 2 >= (128ll << 20);
   auto go = [&](auto kern) { hipLaunchKernelGGL(kern, grid, dim3(256), 0, st, a); };
   if (dtype == ALTO_DT_BF16) {
     if (cols == 128) stream_in ? go(attn_quant_kernel<__bf16, 128, true>) : go(attn_quant_kernel<__bf16, 128, false>);
     else stream_in ? go(attn_quant_kernel<__bf16, 64, true>) : go(attn_quant_kernel<__bf16, 64, false>);
   } else {
-    if (cols == 128) stream_in ? go(attn_quant_kernel<float, 128, true>) : go(attn_quant_kernel<float, 128, false>);
-    else stream_in ? go(attn_quant_kernel<float, 64, true>) : go(attn_quant_kernel<float, 64, false>);
+    cols == 128 ? go(attn_quant_kernel<float, 128, false>) : go(attn_quant_kernel<float, 64, false>);
   }
   return check_launch("attention_quantize");
 }
