@@ -82,7 +82,37 @@ struct Entry {
 };
 
 void* const D = g_mem + 256;   // a well-aligned "device" pointer
+
+// Host arrays of sequence boundaries for the packed attention entry.  The first three are valid for 256 query tokens and 288
+// keys, the last one for 4160 of either (more sequences than one launch takes); the others break one rule each.
+struct Boundaries {
+  int n;
+  int32_t q[132], k[132];
+};
+Boundaries g_bounds[] = {
+    {2, {0, 96, 256}, {0, 128, 288}},
+    {1, {0, 256}, {0, 288}},
+    {8, {0, 32, 64, 96, 128, 160, 192, 224, 256}, {0, 32, 64, 96, 128, 160, 192, 224, 288}},
+    {2, {0, 128, 256}, {0, 96, 288}},              // more queries than keys (refused with a causal mask)
+    {2, {32, 96, 256}, {0, 128, 288}},             // does not start at 0
+    {2, {0, 96, 224}, {0, 128, 288}},              // does not end at the token count
+    {3, {0, 160, 96, 256}, {0, 128, 160, 288}},    // not increasing
+    {3, {0, 96, 96, 256}, {0, 128, 160, 288}},     // an empty sequence
+    {2, {0, 100, 256}, {0, 128, 288}},             // not a multiple of 32
+    {2, {0, INT32_MIN, 256}, {0, 128, 288}},
+    {2, {0, 96, 256}, {0, INT32_MAX, 288}},
+    {-1, {0, 256}, {0, 288}},
+    {130, {}, {}},
+};
+constexpr int kManySequences = sizeof(g_bounds) / sizeof(g_bounds[0]) - 1;
 #define P(T, k) static_cast<T*>(a.p[k])
+
+int call_packed_attention(const Args& a) {
+  const Boundaries& b = g_bounds[(unsigned)a.i[0] % (kManySequences + 1)];
+  return alto_mxfp4_attention_fwd_strided(a.p[0], a.p[1], a.p[2], a.p[3], a.p[4], a.p[5], a.p[6], P(float, 7), a.s[0], a.s[1], a.s[2], a.s[3], a.s[4], a.s[5],
+                                          a.s[6], a.s[7], a.s[8], a.s[9], a.s[10], a.s[11], a.s[12], b.n, b.q, b.k, a.f, a.i[1], P(const float, 8), a.s[13],
+                                          a.s[14], nullptr);
+}
 
 Entry g_entries[] = {
     // x, dtype, batch, M, C, ld_x, bs_x, row_codes, row_scales, col_codes, col_scales, is_2d, rounding, rand, ld_rand, bs_rand, hadamard, ...
@@ -229,18 +259,20 @@ Entry g_entries[] = {
                                             a.s[10], a.s[11], a.s[12], a.s[13], a.s[14], a.s[15], P(uint8_t, 3), P(uint8_t, 4), P(uint8_t, 5), P(uint8_t, 6),
                                             P(uint8_t, 7), P(uint8_t, 8), nullptr);
      }},
-    // B, Hq, Hk, Sq, Sk, D, Dv, strides of out and lse, alibi strides; two sequences
-    {"attention_fwd_strided", 15, 2, 9, {{1, 8, 2, 256, 288, 128, 64, 0, 64, 512, 0, 1, 8, 8, 1}, {2, 1}, {D, D, D, D, D, D, D, D, D}, 0.088388f, {0, 0}, g_signs, g_perm},
+    // B, Hq, Hk, Sq, Sk, D, Dv, strides of out and lse, alibi strides
+    {"attention_fwd_strided", 15, 2, 9, {{2, 8, 2, 256, 288, 128, 64, 131072, 64, 512, 2048, 1, 8, 8, 1}, {0, 1}, {D, D, D, D, D, D, D, D, D}, 0.088388f, {0, 0}, g_signs, g_perm},
      [](const Args& a) {
-       static const int32_t cu_q[3] = {0, 96, 256}, cu_k[3] = {0, 128, 288};
-       const int n = a.i[0] == 2 ? 2 : 0;   // (the boundary arrays hold two sequences)
        return alto_mxfp4_attention_fwd_strided(a.p[0], a.p[1], a.p[2], a.p[3], a.p[4], a.p[5], a.p[6], P(float, 7), a.s[0], a.s[1], a.s[2], a.s[3], a.s[4],
-                                               a.s[5], a.s[6], a.s[7], a.s[8], a.s[9], a.s[10], a.s[11], a.s[12], n, cu_q, cu_k, a.f, a.i[1],
+                                               a.s[5], a.s[6], a.s[7], a.s[8], a.s[9], a.s[10], a.s[11], a.s[12], 0, nullptr, nullptr, a.f, a.i[1],
                                                P(const float, 8), a.s[13], a.s[14], nullptr);
      }},
+    // the same, sequences packed along the tokens: i[0] picks the boundaries
+    {"attention_fwd_packed", 15, 2, 9, {{1, 8, 2, 256, 288, 128, 64, 0, 64, 512, 0, 1, 8, 8, 1}, {0, 1}, {D, D, D, D, D, D, D, D, D}, 0.088388f, {0, 0}, g_signs, g_perm},
+     call_packed_attention},
+    {"attention_fwd_packed_many", 15, 2, 9, {{1, 8, 2, 4160, 4160, 64, 128, 0, 128, 1024, 0, 1, 8, 8, 1}, {kManySequences, 1}, {D, D, D, D, D, D, D, D, D}, 0.125f, {0, 0}, g_signs, g_perm},
+     call_packed_attention},
 };
 constexpr int kEntries = sizeof(g_entries) / sizeof(g_entries[0]);
-constexpr int kFirstTable = 30;   // entries behind these are counted by themselves
 
 void mutate(Args& a, const Entry& e) {
   const int fields = e.ns + e.ni + e.np + 4;   // + float, one of the two u64, signs, perm
@@ -269,9 +301,10 @@ int main(int argc, char** argv) {
     g_signs[k] = (k * 7 % 3 == 0) ? -1 : 1;
     g_perm[k] = (uint8_t)((k * 5 + 3) % 32);
   }
+  for (int k = 0; k <= 130; ++k) g_bounds[kManySequences].q[k] = g_bounds[kManySequences].k[k] = 32 * k;
   std::printf("version %d\n", alto_mxfp4_version());
   (void)alto_mxfp4_init();   // no device here: must fail cleanly or do nothing
-  long calls = 0, more = 0;
+  long calls = 0;
   for (long it = 0; it < rounds; ++it) {
     for (int n = 0; n < kEntries; ++n) {
       Entry& e = g_entries[n];
@@ -279,7 +312,7 @@ int main(int argc, char** argv) {
       const int changes = (int)(next_u64() % 4);
       for (int c = 0; c < changes; ++c) mutate(a, e);
       const int rc = e.call(a);
-      ++(n < kFirstTable ? calls : more);
+      ++calls;
       ++e.calls;
       if (rc == -100) {
         std::fprintf(stderr, "call %ld (%s): a size query returned a negative number\n", calls, e.name);
@@ -302,7 +335,7 @@ int main(int argc, char** argv) {
       return 3;
     }
   for (Entry& e : g_entries) {   // the entry that allocates on the host, once without memory (an exception would end the process)
-    if (std::strcmp(e.name, "attention_fwd_strided") != 0) continue;
+    if (std::strcmp(e.name, "attention_fwd_packed") != 0) continue;
     g_no_memory = true;
     const int rc = e.call(e.valid);
     g_no_memory = false;
@@ -321,6 +354,6 @@ int main(int argc, char** argv) {
     std::fprintf(stderr, "%d entry points never got past their argument checks: their valid argument set is not valid\n", never);
     return 4;
   }
-  std::printf("calls %ld\nmore %ld\n", calls, more);
+  std::printf("entries %d\ncalls %ld\n", kEntries, calls);
   return 0;
 }

@@ -37,16 +37,29 @@ def test_experts_larger_than_the_cache(M, C):
         assert all(torch.equal(a[e], b[0]) for a, b in zip(big, one))
 
 
-def test_stochastic_words_of_a_large_matrix():
-    """Hardware stochastic rounding: the words belong to (row, column) of the whole matrix, so a device-resident state at the
-    same counter gives the same codes whatever the cache policy; checked against the packed-scale call on the same tensor."""
+@pytest.mark.parametrize("rht", [False, True])
+def test_stochastic_words_of_a_large_matrix(rht):
+    """Hardware stochastic rounding, streamed: which random word an element gets is a function of its row and column, so the first and
+    the last rows by themselves, with the counter moved to where their words start, give the same codes and scales in both
+    directions.  (bf16: a band of 32 rows takes C blocks of words for the row copy, and as many behind all of those for the
+    column copy.)"""
     import alto_amd.mxfp4 as m
-    x = torch.randn((65568, 2080), device=DEV, generator=torch.Generator(DEV).manual_seed(4)).bfloat16()
-    outs = []
-    for clip in ("none", "static"):   # (the clipping kernels are not streamed; the row output is not clipped)
-        torch.manual_seed(5)
-        outs.append(m.quantize_rowcol(x, False, use_sr=True, clip_mode=clip, pad_codes=True)[:2])
-    assert torch.equal(outs[0][0], outs[1][0]) and torch.equal(outs[0][1], outs[1][1])
+    M, C, n = 65568, 2080, 4096
+    assert M * C * 3 >= 256 << 20 > n * C * 3
+    h = m.HadamardTransform(*hadamard_from_seed(3)) if rht else None
+    x = torch.randn((M, C), device=DEV, generator=torch.Generator(DEV).manual_seed(4)).bfloat16()
+    torch.manual_seed(5)
+    seed = int(torch.randint(0, 2 ** 63 - 1, (1,), dtype=torch.int64).item())   # the key that the next call draws
+    torch.manual_seed(5)
+    q, s, cq, cs = m.quantize_rowcol(x, False, use_sr=True, hadamard=h, pad_codes=True)
+    for lo in (0, M - n):
+        at = lo // 32 * C
+        q1, s1 = m.convert_to_mxfp4(x[lo:lo + n], axis=-1, use_sr=True, use_asm=True, philox_seed=seed, philox_offset=at)
+        assert torch.equal(q[lo:lo + n], q1) and torch.equal(s[lo:lo + n], s1), lo
+        cq1, cs1 = m.convert_to_mxfp4(x[lo:lo + n], axis=0, use_sr=True, use_asm=True, philox_seed=seed, philox_offset=(M - n) // 32 * C + at, hadamard=h)
+        assert torch.equal(cq[lo // 2:(lo + n) // 2], cq1) and torch.equal(cs[lo // 32:(lo + n) // 32], cs1), lo
+        other = m.convert_to_mxfp4(x[lo:lo + n], axis=0, use_sr=True, use_asm=True, philox_seed=seed, philox_offset=at + 1, hadamard=h)
+        assert not torch.equal(cq1, other[0]) and torch.equal(cs1, other[1])   # (the words do matter)
 
 
 @pytest.mark.parametrize("dtype,D", [(torch.bfloat16, 128), (torch.bfloat16, 64), (torch.float32, 128), (torch.float32, 64)])

@@ -59,4 +59,4 @@ def test_c_abi_host_code_under_asan_and_ubsan():
     assert r.returncode == 0, tail
     assert "runtime error" not in r.stderr and "AddressSanitizer" not in r.stderr, tail
     # every entry point got past its argument checks with its valid set (the driver exits 4 otherwise) and the run is complete
-    assert f"calls {2000 * 30}" in r.stdout, tail
+    assert f"calls {2000 * 34}" in r.stdout, tail
