@@ -7,7 +7,7 @@ namespace alto {
 namespace {
 
 // 8 codes (one dword) of a block with scale sf, decoded to fp32.  The convert decodes with scale 1 (exact) and the scale is
-// a multiplication of its own, so that the scale bytes 0 (0.0) and 255 (inf) mean the same as in e2m1_decode(code) * sf.
+// a multiplication of its own, so that the scale bytes 0 and 255 mean 0.0 and inf, as in value(code) * 2^(byte - 127) made from the bits.
 __device__ __forceinline__ void decode8(uint32_t w, float sf, int static_clip, float (&v)[8]) {
   typedef float f2_t __attribute__((ext_vector_type(2)));
   const f2_t p0 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(w, 1.0f, 0), p1 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(w, 1.0f, 1);

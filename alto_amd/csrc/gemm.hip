@@ -118,10 +118,11 @@ extern "C" int alto_mxfp4_gemm_ps(const uint8_t* a, int64_t lda, const uint8_t* 
   const int64_t KB = (K / 32 + 15) / 16;
   OperandView A{a, lda, a_packed, 16, M * 16, 0};
   OperandView B{b, ldb, b_packed, 16, N * 16, 0};
-  // the packed form exists for the 256x256 tile kernel only: same shape conditions as alto_mxfp4_gemm's choice of it
+  // All three tile sizes read packed scales; the shapes are those that the 256x256 tile can serve (which of the three runs is a matter
+  // of speed: same bits).  Fewer than 128 rows or 512 K take plain scales.
   OperandView Ap{a, lda, a_packed, 1, 1, 0}, Bp{b, ldb, b_packed, 1, 1, 0};
   if (!(gemm_tiled_supported(Ap, Bp, M, N, K, c, ALTO_DT_BF16, ldc) && product_below(1ll << 31, KB, M, 16) && product_below(1ll << 31, KB, N, 16))) {
-    set_error("gemm_ps: shape (%lld, %lld, %lld) is not served by the tile kernel; use alto_mxfp4_gemm with plain scales", (long long)M, (long long)N, (long long)K);
+    set_error("gemm_ps: shape (%lld, %lld, %lld) is not served by the tile kernels; use alto_mxfp4_gemm with plain scales", (long long)M, (long long)N, (long long)K);
     return ALTO_MXFP4_ENOTIMPL;
   }
   const int tile = gemm_mid_tile_size(M, N, ALTO_DT_BF16);

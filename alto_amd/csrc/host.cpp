@@ -168,8 +168,6 @@ py::object dequantize(const Tensor& codes, const Tensor& scales, bool f32, bool 
   return py::cast(last_axis ? out : out.t());
 }
 
-bool k_major(const Tensor& t) { return t.stride(1) == 1 && t.stride(0) % 16 == 0 && aligned16(t); }
-
 // linear.py:blockwise_mxfp4_gemm with both operands packed along K
 py::object gemm(const Tensor& a_in, const Tensor& as_in, const Tensor& b_in, const Tensor& bs_in, bool a_2d, bool b_2d, bool trans_a, bool trans_b, bool f32,
                 double out_scale, uintptr_t stream) {

@@ -130,12 +130,6 @@ def philox_device_state(device: torch.device) -> Optional[torch.Tensor]:
     return st
 
 
-def philox_advance(state: torch.Tensor, words: int) -> None:
-    """Enqueue the counter update of ``state`` past ``words`` random words on the current stream."""
-    from .._lib import check
-    check(lib().alto_mxfp4_philox_advance(state.data_ptr(), int(words), stream_ptr(state.device)), "alto_mxfp4_philox_advance")
-
-
 def draw_rand_bits(shape, device, seed: Optional[int] = None, offset: Optional[int] = None) -> torch.Tensor:
     """32 random bits per element for stochastic rounding (int32 tensor of ``shape`` on ``device``).
 

@@ -134,7 +134,8 @@ def pack_scales(scales: torch.Tensor, rows: int, K: int, is_2d_block: bool = Fal
 
 
 def packed_gemm_supported(M: int, N: int, K: int) -> bool:
-    """Shapes the packed-scale kernel serves (the 256x256 tile kernel's conditions; anything else takes plain scales)."""
+    """Shapes the packed-scale product serves (the 256x256 tile's conditions, whichever tile size then runs; anything else takes
+    plain scales)."""
     return M >= 128 and N >= 128 and K >= 512 and N % 8 == 0 and M * (K // 2) < 2 ** 31 and N * (K // 2) < 2 ** 31
 
 

@@ -243,7 +243,8 @@ int alto_mxfp4_gemm(const uint8_t* a, int64_t lda, const uint8_t* a_scales, int6
 
 /*
  * Packed scales: an internal layout of the scale bytes of one GEMM operand that the 256x256 tile kernels move into LDS
- * with one load per wave and 512-K block, without registers, fix-ups or LDS writes (2 to 5 % of a GEMM).  No counterpart
+ * with one load per wave and 512-K block, without registers, fix-ups or LDS writes (2 to 5 % of a GEMM); the smaller tiles
+ * load a lane's bytes of a 512-K block with one instruction.  No counterpart
  * in the reference.  For an operand of `rows` rows and K / 32 groups:
  *   packed[(kb * rows + row) * 16 + 4 * (2 h + ms) + j] = scale of group 16 kb + 8 ms + 2 j + h of that row
  *   (kb < ceil(K / 512); h, ms in {0, 1}; j < 4), and 127 where that group lies beyond K.
@@ -256,7 +257,7 @@ int alto_mxfp4_pack_scales(const uint8_t* scales, int64_t ss_r, int64_t ss_k, in
 
 /*
  * alto_mxfp4_gemm on operands with packed scales, bf16 output: c[M][N] = a[M][K] . b[N][K]^T * out_scale.  Same results as
- * alto_mxfp4_gemm, bit for bit.  Serves the shapes of the tile kernel only (M, N >= 128, K >= 512, N % 8 == 0, ldc % 8 ==
+ * alto_mxfp4_gemm, bit for bit.  Serves the shapes of the tile kernels only (M, N >= 128, K >= 512, N % 8 == 0, ldc % 8 ==
  * 0, 16-byte aligned c): ALTO_MXFP4_ENOTIMPL otherwise, and the caller keeps plain scales for those.
  */
 int alto_mxfp4_gemm_ps(const uint8_t* a, int64_t lda, const uint8_t* a_packed, const uint8_t* b, int64_t ldb, const uint8_t* b_packed,
