@@ -1,0 +1,134 @@
+// What the attention kernels (attention.hip) and their operand quantizer (attention_quantize.hip) share.
+#pragma once
+#include <type_traits>
+#include <utility>
+
+#include "common.h"
+
+namespace alto {
+
+struct AttnArgs {
+  const uint8_t* q;  const uint8_t* qs;    // [B, Hq, Sq, D/2],  [B, Hq, Sq/32, D/32]; or NULL and, as bf16 values in the caller's layout,
+  const __bf16* qx;  int64_t qx_sb, qx_sh, qx_ss;   // element (b, h, row, column) at these strides, unit stride along D
+  const uint8_t* k;  const uint8_t* ks;    // [B, Hk, Sk, D/2],  [B, Hk, Sk/32, D/32]
+  const uint8_t* vt; const uint8_t* vs;    // [B, Hk, Dv, Sk/2] packed along keys, [B, Hk, Sk/32, Dv/32]
+  void* out; float* lse;                   // bf16 and fp32, element (b, h, row, column) at the strides below
+  int64_t o_sb, o_sh, o_ss, l_sb, l_sh, l_ss;
+  int Hq, Hk, Sq, Sk, Sk_used;             // Sk keys are allocated, the first Sk_used exist (packed sequences: Sq and Sk are token counts)
+  int64_t k_bytes, v_bytes;                // extent of the code buffers
+  float sm_scale;
+  int causal;
+  // optional additive terms on the scaled scores (triton_flash_attention_mxfp4.py:288-299), fp32:
+  const float* bias;  int64_t bias_sb, bias_sh, bias_sm, bias_bytes;   // element (b, h, m, n) at b sb + h sh + m sm + n; NULL: none
+  const float* alibi; int64_t alibi_sb, alibi_sh;                      // slope of (b, h) at b sb + h sh; NULL: none
+};
+
+// Sequences packed along the tokens (B = 1): sequence i owns query rows q0[i] .. + qn[i] and keys k0[i] .. + kn[i] (all
+// multiples of 32) and the row blocks z0[i] .. z0[i+1] of the grid.  By value, in the kernel arguments: no copy to the
+// device, nothing to keep alive.
+constexpr int ATTN_MAX_SEQS = 64;
+struct AttnSeqs {
+  int n;
+  int z0[ATTN_MAX_SEQS + 1], q0[ATTN_MAX_SEQS], qn[ATTN_MAX_SEQS], k0[ATTN_MAX_SEQS], kn[ATTN_MAX_SEQS];
+};
+struct AttnNoSeqs {};
+
+// Uniform 4-byte aligned data through the scalar cache: as vector loads these sit in the same counter as the direct-to-LDS
+// prefetch, and the wait for a block's scale bytes drains the prefetched block with them.  Whole causal calls, us, vector ->
+// scalar: 4 x 4096 tokens x 32 heads x 64 258 -> 248, 2 x 3232 x 16 x 64 60.7 -> 59.2, 1 x 4096 x 32 x 128 110.4 -> 109.3,
+// 4 x 2048 x 64 x 128 218 -> 216, packed sequences the same to 1.5 % faster; 4 x 1024 x 32 x 128 loses, 47.6 -> 48.4.
+typedef const __attribute__((address_space(4))) uint32_t* scalar_u32;
+__device__ __forceinline__ scalar_u32 scalar_ptr(const uint8_t* p) { return (scalar_u32)(uintptr_t)p; }
+
+constexpr float ATTN_RCP_LN2 = 1.4426950408889634f;
+constexpr float ATTN_LN2 = 0.6931471824645996f;
+
+__device__ __forceinline__ v8i_t frag16(const uint8_t* p) {
+  const uint4 w = *reinterpret_cast<const uint4*>(p);
+  return v8i_t{(int)w.x, (int)w.y, (int)w.z, (int)w.w, 0, 0, 0, 0};
+}
+template <int N, typename F, int... I>
+__device__ __forceinline__ void static_for_impl(F&& f, std::integer_sequence<int, I...>) { (f(std::integral_constant<int, I>{}), ...); }
+template <int N, typename F>
+__device__ __forceinline__ void static_for(F&& f) { static_for_impl<N>(static_cast<F&&>(f), std::make_integer_sequence<int, N>{}); }
+
+typedef unsigned v2u_t __attribute__((ext_vector_type(2)));
+typedef int v4i_8_t __attribute__((ext_vector_type(4), aligned(8)));   // 16 bytes at an 8-byte boundary
+// v_permlane32_swap(a, b) returns {a of lanes 0..31 | b of lanes 0..31,  a of lanes 32..63 | b of lanes 32..63}
+// (first | second half of the wave): a value and its copy come back as the low half's and the high half's values.
+__device__ __forceinline__ float pair_max(float v) {   // max over the two lanes l and l ^ 32
+  const v2u_t p = __builtin_amdgcn_permlane32_swap(f2u(v), f2u(v), false, false);
+  return fmaxf(u2f(p[0]), u2f(p[1]));
+}
+
+typedef unsigned short us2a_t __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ uint32_t pk_max_u16a(uint32_t a, uint32_t b) {
+  return __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(us2a_t, a), __builtin_bit_cast(us2a_t, b)));
+}
+
+// absmax bits of 8 consecutive elements held in 4 (bf16) or 8 (fp32) dwords
+template <typename T>
+__device__ __forceinline__ uint32_t absmax8(const uint32_t* w) {
+  if constexpr (sizeof(T) == 2) {
+    const uint32_t a = pk_max_u16a(pk_max_u16a(w[0] & 0x7FFF7FFFu, w[1] & 0x7FFF7FFFu), pk_max_u16a(w[2] & 0x7FFF7FFFu, w[3] & 0x7FFF7FFFu));
+    return max(a & 0xFFFFu, a >> 16);
+  } else {
+    uint32_t a = 0;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) a = max(a, w[e] & 0x7FFFFFFFu);
+    return a;
+  }
+}
+template <typename T>
+__device__ __forceinline__ uint32_t encode8(const uint32_t* w, float scale) {
+  uint32_t o = 0;
+  if constexpr (sizeof(T) == 2) {
+    o = __builtin_amdgcn_cvt_scalef32_pk_fp4_bf16(o, __builtin_bit_cast(bf16x2_t, w[0]), scale, 0);
+    o = __builtin_amdgcn_cvt_scalef32_pk_fp4_bf16(o, __builtin_bit_cast(bf16x2_t, w[1]), scale, 1);
+    o = __builtin_amdgcn_cvt_scalef32_pk_fp4_bf16(o, __builtin_bit_cast(bf16x2_t, w[2]), scale, 2);
+    o = __builtin_amdgcn_cvt_scalef32_pk_fp4_bf16(o, __builtin_bit_cast(bf16x2_t, w[3]), scale, 3);
+  } else {
+    o = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(o, u2f(w[0]), u2f(w[1]), scale, 0);
+    o = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(o, u2f(w[2]), u2f(w[3]), scale, 1);
+    o = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(o, u2f(w[4]), u2f(w[5]), scale, 2);
+    o = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(o, u2f(w[6]), u2f(w[7]), scale, 3);
+  }
+  return o;
+}
+
+
+// A wave's 32 rows of Q, straight from bf16, as the score product takes them: lane (r = lane % 32, h = lane / 32) gets the codes of
+// row r, columns 64 s + 32 h .. + 32, and the scale byte of that 32 x 32 block.  The loads are whole 128-byte lines (8 lanes a row,
+// 8 rows an instruction; a lane that fetched its own 64 bytes cost 32 line lookups an instruction instead of 8); the codes change
+// lanes through `scratch`, NK KB of LDS that only this wave uses, at consecutive addresses both ways.  Codes and scales are those
+// of alto_mxfp4_attention_quantize.
+template <int NK>
+__device__ __forceinline__ void quantize_q(const __bf16* x, int64_t row_stride, int lane, uint8_t* scratch, v8i_t (&qf)[NK], int (&qsc)[NK]) {
+  uint32_t w[NK][4][4];
+#pragma unroll
+  for (int s = 0; s < NK; ++s)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const v4i_t v = __builtin_nontemporal_load(reinterpret_cast<const v4i_t*>(x + (int64_t)(8 * i + (lane >> 3)) * row_stride + 64 * s + 8 * (lane & 7)));
+      w[s][i][0] = v[0]; w[s][i][1] = v[1]; w[s][i][2] = v[2]; w[s][i][3] = v[3];
+    }
+#pragma unroll
+  for (int s = 0; s < NK; ++s) {
+    uint32_t m = max(max(absmax8<__bf16>(w[s][0]), absmax8<__bf16>(w[s][1])), max(absmax8<__bf16>(w[s][2]), absmax8<__bf16>(w[s][3])));
+    m = max(m, dpp_u32<ALTO_DPP_QUAD_XOR1>(m));   // the block's rows and columns: the lanes that agree in bit 2
+    m = max(m, dpp_u32<ALTO_DPP_QUAD_XOR2>(m));
+    m = max(m, dpp_u32<ALTO_DPP_ROW_ROR8>(m));
+    const v2u_t p16 = __builtin_amdgcn_permlane16_swap(m, m, false, false);
+    m = max(p16[0], p16[1]);
+    const v2u_t p32 = __builtin_amdgcn_permlane32_swap(m, m, false, false);
+    m = max(p32[0], p32[1]);
+    const uint32_t e = e8m0_from_bf16_bits(m);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) *reinterpret_cast<uint32_t*>(scratch + 1024 * s + 256 * i + 4 * lane) = encode8<__bf16>(w[s][i], u2f(e << 23));
+    qsc[s] = lane < 32 ? __builtin_amdgcn_readlane((int)e, 0) : __builtin_amdgcn_readlane((int)e, 4);
+  }
+#pragma unroll
+  for (int s = 0; s < NK; ++s) qf[s] = frag16(scratch + 1024 * s + (lane & 31) * 32 + (lane >> 5) * 16);
+}
+
+}  // namespace alto

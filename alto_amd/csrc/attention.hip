@@ -9,68 +9,14 @@
 #include <algorithm>
 #include <memory>
 #include <new>
-#include <type_traits>
-#include <utility>
 
-#include "common.h"
+#include "attention.h"
 
 namespace alto {
-
-struct AttnArgs {
-  const uint8_t* q;  const uint8_t* qs;    // [B, Hq, Sq, D/2],  [B, Hq, Sq/32, D/32]
-  const uint8_t* k;  const uint8_t* ks;    // [B, Hk, Sk, D/2],  [B, Hk, Sk/32, D/32]
-  const uint8_t* vt; const uint8_t* vs;    // [B, Hk, Dv, Sk/2] packed along keys, [B, Hk, Sk/32, Dv/32]
-  void* out; float* lse;                   // bf16 and fp32, element (b, h, row, column) at the strides below
-  int64_t o_sb, o_sh, o_ss, l_sb, l_sh, l_ss;
-  int Hq, Hk, Sq, Sk, Sk_used;             // Sk keys are allocated, the first Sk_used exist (packed sequences: Sq and Sk are token counts)
-  int64_t k_bytes, v_bytes;                // extent of the code buffers
-  float sm_scale;
-  int causal;
-  // optional additive terms on the scaled scores (triton_flash_attention_mxfp4.py:288-299), fp32:
-  const float* bias;  int64_t bias_sb, bias_sh, bias_sm, bias_bytes;   // element (b, h, m, n) at b sb + h sh + m sm + n; NULL: none
-  const float* alibi; int64_t alibi_sb, alibi_sh;                      // slope of (b, h) at b sb + h sh; NULL: none
-};
-
-// Sequences packed along the tokens (B = 1): sequence i owns query rows q0[i] .. + qn[i] and keys k0[i] .. + kn[i] (all
-// multiples of 32) and the row blocks z0[i] .. z0[i+1] of the grid.  By value, in the kernel arguments: no copy to the
-// device, nothing to keep alive.
-constexpr int ATTN_MAX_SEQS = 64;
-struct AttnSeqs {
-  int n;
-  int z0[ATTN_MAX_SEQS + 1], q0[ATTN_MAX_SEQS], qn[ATTN_MAX_SEQS], k0[ATTN_MAX_SEQS], kn[ATTN_MAX_SEQS];
-};
-struct AttnNoSeqs {};
-
-// Uniform 4-byte aligned data through the scalar cache: as vector loads these sit in the same counter as the direct-to-LDS
-// prefetch, and the wait for a block's scale bytes drains the prefetched block with them.  Whole causal calls, us, vector ->
-// scalar: 4 x 4096 tokens x 32 heads x 64 258 -> 248, 2 x 3232 x 16 x 64 60.7 -> 59.2, 1 x 4096 x 32 x 128 110.4 -> 109.3,
-// 4 x 2048 x 64 x 128 218 -> 216, packed sequences the same to 1.5 % faster; 4 x 1024 x 32 x 128 loses, 47.6 -> 48.4.
-typedef const __attribute__((address_space(4))) uint32_t* scalar_u32;
-__device__ __forceinline__ scalar_u32 scalar_ptr(const uint8_t* p) { return (scalar_u32)(uintptr_t)p; }
 
 #ifndef ATTN_WG_PER_CU
 #define ATTN_WG_PER_CU 3
 #endif
-constexpr float ATTN_RCP_LN2 = 1.4426950408889634f;
-constexpr float ATTN_LN2 = 0.6931471824645996f;
-
-__device__ __forceinline__ v8i_t frag16(const uint8_t* p) {
-  const uint4 w = *reinterpret_cast<const uint4*>(p);
-  return v8i_t{(int)w.x, (int)w.y, (int)w.z, (int)w.w, 0, 0, 0, 0};
-}
-template <int N, typename F, int... I>
-__device__ __forceinline__ void static_for_impl(F&& f, std::integer_sequence<int, I...>) { (f(std::integral_constant<int, I>{}), ...); }
-template <int N, typename F>
-__device__ __forceinline__ void static_for(F&& f) { static_for_impl<N>(static_cast<F&&>(f), std::make_integer_sequence<int, N>{}); }
-
-typedef unsigned v2u_t __attribute__((ext_vector_type(2)));
-// v_permlane32_swap(a, b) returns {a of lanes 0..31 | b of lanes 0..31,  a of lanes 32..63 | b of lanes 32..63}
-// (first | second half of the wave): a value and its copy come back as the low half's and the high half's values.
-__device__ __forceinline__ float pair_max(float v) {   // max over the two lanes l and l ^ 32
-  const v2u_t p = __builtin_amdgcn_permlane32_swap(f2u(v), f2u(v), false, false);
-  return fmaxf(u2f(p[0]), u2f(p[1]));
-}
-
 // NK = D / 64 (MFMA K steps of Q K^T), ND = Dv / 32 (output tiles).
 // The four waves of a workgroup own 128 consecutive query rows of one head and walk the key blocks together: a block's
 // K codes (64 rows x D/2 bytes) and V codes (Dv rows x 32 bytes) are fetched once per workgroup, two blocks ahead, with
@@ -84,6 +30,7 @@ struct AttnTile {
   static constexpr int D = NK * 64, DV = ND * 32;
   static constexpr int K_BYTES = 64 * (D / 2), V_BYTES = DV * 32;       // one block of K codes, of V codes
   static constexpr int SLOT = K_BYTES + V_BYTES;
+  static constexpr int LDS = ATTN_RING * SLOT > 128 * DV * 2 ? ATTN_RING * SLOT : 128 * DV * 2;         // the ring, then the 128 result rows
 };
 
 // The body of the kernel as a function of its own because of the `__restrict__` on the outputs: inlining then marks the
@@ -91,8 +38,14 @@ struct AttnTile {
 // in flight across the LDS reads that follow (unmarked, it puts an `s_waitcnt vmcnt(0)` before the next LDS read).
 // BIASED: the scores get a.bias and / or the ALiBi term -slope |row + Sk - Sq - key| added after the scaling and the mask,
 // before the running maximum (:288-308); a separate instantiation, the plain one carries none of it.
+// QBF: Q comes as bf16 values and every wave quantizes its own rows (no other wave reads them), which saves writing the codes
+// and reading them back and leaves the operand quantizer K and V only.  4 x 2048 tokens, 64 / 8 heads of 128, causal (134 of the
+// 168 MB are Q), operand quantizer + this kernel, us: on codes 38.9 + 181.5; every lane fetching the 64 bytes it multiplies
+// 10.6 + 201, whole lines (quantize_q) 10.9 + 197, at raised wave priority 10.6 + 195 (the two other workgroups of the compute unit
+// hide the wait, the priority lets the arithmetic behind it through), with the heads dealt as below 10.3 + 187, with the
+// results stored as whole rows 10.7 + 181, Q read non-temporally 8.7 + 179.
 // SEQS: AttnSeqs, or AttnNoSeqs for B sequences of one length.
-template <int NK, int ND, bool BIASED, typename SEQS>
+template <int NK, int ND, bool BIASED, bool QBF, typename SEQS>
 __device__ __forceinline__ void attn_fwd_body(const AttnArgs& a, const SEQS& seqs, __bf16* __restrict__ out, float* __restrict__ lse_out, uint8_t* ring) {
   constexpr bool PACKED = std::is_same<SEQS, AttnSeqs>::value;
   constexpr int D = NK * 64, DV = ND * 32;
@@ -120,7 +73,9 @@ __device__ __forceinline__ void attn_fwd_body(const AttnArgs& a, const SEQS& seq
   const int qblk = a.causal ? nz - 1 - z : z;
   const int q0 = (qblk * 4 + wave) * 32;
   const bool live = q0 < qn;                      // a wave past the last row still helps with loads and barriers
-  const int hq = blockIdx.x, b = blockIdx.y;
+  // eight neighbouring workgroups go to the eight XCDs in turn: each gets a range of consecutive heads, so a key / value head
+  // comes into one L2 (two, where a range starts inside its query heads) and not into all of them: 195 -> 187 us (QBF above)
+  const int hq = a.Hq % 8 == 0 ? (blockIdx.x & 7) * (a.Hq >> 3) + (blockIdx.x >> 3) : blockIdx.x, b = blockIdx.y;
   const int hk = hq / (a.Hq / a.Hk);
   // rows of the operand buffers where this (sequence, head) starts
   const int64_t q_base = ((int64_t)b * a.Hq + hq) * a.Sq + q_first, bhk = (int64_t)b * a.Hk + hk, k_base = bhk * a.Sk + k_first;
@@ -130,10 +85,12 @@ __device__ __forceinline__ void attn_fwd_body(const AttnArgs& a, const SEQS& seq
   // ---- Q pieces: row qrow, K step ks, half h -> 16 bytes; one scale byte per (32-row block, 32-column block)
   v8i_t qf[NK];
   int qsc[NK];
+  if constexpr (!QBF) {
 #pragma unroll
-  for (int s = 0; s < NK; ++s) {
-    qf[s] = frag16(a.q + (q_base + qrow) * (D / 2) + s * 32 + h * 16);
-    qsc[s] = a.qs[(q_base / 32 + qrow / 32) * (D / 32) + 2 * s + h];
+    for (int s = 0; s < NK; ++s) {
+      qf[s] = frag16(a.q + (q_base + qrow) * (D / 2) + s * 32 + h * 16);
+      qsc[s] = a.qs[(q_base / 32 + qrow / 32) * (D / 32) + 2 * s + h];
+    }
   }
 
   v16f_t acc_o[ND], acc_l;
@@ -242,6 +199,11 @@ __device__ __forceinline__ void attn_fwd_body(const AttnArgs& a, const SEQS& seq
     fetch_scales(0, ksw_next, vsw_next);
     dma(0, 0);
     if (wg_blk > 1) dma(1, 1);
+  }
+  if constexpr (QBF) {   // behind the first blocks' loads, which then travel with it
+    __builtin_amdgcn_s_setprio(3);
+    quantize_q<NK>(a.qx + b * a.qx_sb + hq * a.qx_sh + (int64_t)(q_first + (live ? q0 : 0)) * a.qx_ss, a.qx_ss, lane, ring + AttnTile<NK, ND>::LDS + wave * (NK * 1024), qf, qsc);
+    __builtin_amdgcn_s_setprio(0);
   }
   // (the bare barrier instruction: `__syncthreads()` would first wait for every outstanding load, the prefetched block's
   // included; the ring is written by the direct-to-LDS loads only, and wait_dma has waited for this wave's part)
@@ -387,38 +349,44 @@ __device__ __forceinline__ void attn_fwd_body(const AttnArgs& a, const SEQS& seq
   }
   if (!live) return;
 
-  // ---- O = acc / l, bf16; log-sum-exp
+  // ---- O = acc / l, bf16; log-sum-exp.  The rows change lanes through the LDS (the ring is no longer read: every wave has passed
+  // the loop's last barrier; each wave uses a part of its own), so that a store instruction writes whole rows (8-byte pieces of 32 rows an instruction before: 187 -> 181 us, QBF above).  16-byte piece c of
+  // row r goes to position c ^ (r / (16 / PR)) % PR, PR pieces per row: no bank conflicts either way.
   const float l = acc_l[0];
   const float rl = 1.0f / l;
-  __bf16* orow = out + b * a.o_sb + hq * a.o_sh + (q_first + qrow) * a.o_ss;
+  constexpr int PR = DV / 8;
+  uint8_t* rows = ring + wave * (32 * DV * 2);
 #pragma unroll
   for (int d = 0; d < ND; ++d)
 #pragma unroll
     for (int g = 0; g < 4; ++g) {
-      bf16x2_t lo, hi;
-      lo[0] = (__bf16)(acc_o[d][4 * g + 0] * rl);
-      lo[1] = (__bf16)(acc_o[d][4 * g + 1] * rl);
-      hi[0] = (__bf16)(acc_o[d][4 * g + 2] * rl);
-      hi[1] = (__bf16)(acc_o[d][4 * g + 3] * rl);
       uint2 w;
-      w.x = __builtin_bit_cast(uint32_t, lo);
-      w.y = __builtin_bit_cast(uint32_t, hi);
-      *reinterpret_cast<uint2*>(orow + 32 * d + 8 * g + 4 * h) = w;
+      w.x = pack_bf16x2(acc_o[d][4 * g + 0] * rl, acc_o[d][4 * g + 1] * rl);
+      w.y = pack_bf16x2(acc_o[d][4 * g + 2] * rl, acc_o[d][4 * g + 3] * rl);
+      *reinterpret_cast<uint2*>(rows + r * (DV * 2) + (((4 * d + g) ^ ((r / (16 / PR)) % PR)) * 16 + 8 * h)) = w;
     }
+  __bf16* o_first = out + b * a.o_sb + hq * a.o_sh + (int64_t)(q_first + q0) * a.o_ss;
+#pragma unroll
+  for (int i = 0; i < PR / 2; ++i) {
+    const int p = 64 * i + lane, row = p / PR, c = p % PR;
+    const v4i_t w = *reinterpret_cast<const v4i_t*>(rows + row * (DV * 2) + (c ^ ((row / (16 / PR)) % PR)) * 16);
+    *reinterpret_cast<v4i_8_t*>(o_first + row * a.o_ss + 8 * c) = w;
+  }
   if (h == 0) lse_out[b * a.l_sb + hq * a.l_sh + (q_first + qrow) * a.l_ss] = (m_i + log2f(l)) * ATTN_LN2;
 }
 
-template <int NK, int ND, bool BIASED, typename SEQS>
+template <int NK, int ND, bool BIASED, bool QBF, typename SEQS>
 __global__ __launch_bounds__(256, BIASED ? 2 : ATTN_WG_PER_CU) void attn_fwd_kernel(AttnArgs a, SEQS seqs) {
-  __shared__ __attribute__((aligned(16))) uint8_t ring[ATTN_RING * AttnTile<NK, ND>::SLOT];
-  attn_fwd_body<NK, ND, BIASED>(a, seqs, reinterpret_cast<__bf16*>(a.out), a.lse, ring);
+  __shared__ __attribute__((aligned(16))) uint8_t ring[AttnTile<NK, ND>::LDS + (QBF ? 4 * NK * 1024 : 0)];
+  attn_fwd_body<NK, ND, BIASED, QBF>(a, seqs, reinterpret_cast<__bf16*>(a.out), a.lse, ring);
 }
 
 template <int NK, int ND, typename SEQS>
 static int launch_attn(const AttnArgs& a, const SEQS& seqs, int B, int row_blocks, hipStream_t st) {
   dim3 grid((unsigned)a.Hq, (unsigned)B, (unsigned)row_blocks);
-  if (a.bias || a.alibi) hipLaunchKernelGGL((attn_fwd_kernel<NK, ND, true, SEQS>), grid, dim3(256), 0, st, a, seqs);
-  else hipLaunchKernelGGL((attn_fwd_kernel<NK, ND, false, SEQS>), grid, dim3(256), 0, st, a, seqs);
+  if (a.bias || a.alibi) hipLaunchKernelGGL((attn_fwd_kernel<NK, ND, true, false, SEQS>), grid, dim3(256), 0, st, a, seqs);
+  else if (a.qx) hipLaunchKernelGGL((attn_fwd_kernel<NK, ND, false, true, SEQS>), grid, dim3(256), 0, st, a, seqs);
+  else hipLaunchKernelGGL((attn_fwd_kernel<NK, ND, false, false, SEQS>), grid, dim3(256), 0, st, a, seqs);
   return check_launch("attention_fwd");
 }
 
@@ -470,21 +438,26 @@ extern "C" int alto_mxfp4_attention_fwd_ex(const void* q_codes, const void* q_sc
                "attention_fwd: code pointers must be 16-byte aligned, out 8-byte aligned");
   ALTO_REQUIRE(((uintptr_t)k_scales | (uintptr_t)v_scales | (uintptr_t)lse | (uintptr_t)alibi_slopes) % 4 == 0,
                "attention_fwd: K and V scale pointers, lse and the alibi slopes must be 4-byte aligned");
-  AttnArgs a{(const uint8_t*)q_codes, (const uint8_t*)q_scales, (const uint8_t*)k_codes, (const uint8_t*)k_scales,
+  AttnArgs a{(const uint8_t*)q_codes, (const uint8_t*)q_scales, nullptr, 0, 0, 0, (const uint8_t*)k_codes, (const uint8_t*)k_scales,
              (const uint8_t*)vt_codes, (const uint8_t*)v_scales, out, lse, Hq * Sq * Dv, Sq * Dv, Dv, Hq * Sq, Sq, 1, (int)Hq, (int)Hk, (int)Sq, (int)Sk,
              (int)Sk_used, B * Hk * Sk * (D / 2), B * Hk * Dv * (Sk / 2), sm_scale, causal ? 1 : 0,
              bias, bias_sb, bias_sh, bias_sm, bias_bytes, alibi_slopes, alibi_sb, alibi_sh};
   return launch_attn_dims(a, AttnNoSeqs{}, (int)B, (int)((Sq + 127) / 128), D, Dv, (hipStream_t)stream);
 }
 
-extern "C" int alto_mxfp4_attention_fwd_strided(const void* q_codes, const void* q_scales, const void* k_codes, const void* k_scales,
-                                                const void* vt_codes, const void* v_scales, void* out, float* lse, int64_t B, int64_t Hq,
-                                                int64_t Hk, int64_t Sq, int64_t Sk, int64_t D, int64_t Dv, int64_t o_sb, int64_t o_sh, int64_t o_ss,
-                                                int64_t l_sb, int64_t l_sh, int64_t l_ss, int n_seqs, const int32_t* cu_q, const int32_t* cu_k,
-                                                float sm_scale, int causal, const float* alibi_slopes, int64_t alibi_sb, int64_t alibi_sh, void* stream) {
-  using namespace alto;
-  ALTO_REQUIRE(q_codes && q_scales && k_codes && k_scales && vt_codes && v_scales && out && lse, "attention_fwd: null pointer");
-  ALTO_REQUIRE(!alibi_slopes || (alibi_sb >= 0 && alibi_sh >= 0), "attention_fwd: negative alibi strides");
+namespace alto {
+// Q as the strided entries get it: quantized codes and scales, or bf16 values at element strides
+struct QueryOperand {
+  const void* codes;
+  const void* scales;
+  const void* values;
+  int64_t sb, sh, ss;
+};
+
+static int attention_fwd_strided(const QueryOperand& q, const void* k_codes, const void* k_scales, const void* vt_codes, const void* v_scales, void* out,
+                                 float* lse, int64_t B, int64_t Hq, int64_t Hk, int64_t Sq, int64_t Sk, int64_t D, int64_t Dv, int64_t o_sb, int64_t o_sh,
+                                 int64_t o_ss, int64_t l_sb, int64_t l_sh, int64_t l_ss, int n_seqs, const int32_t* cu_q, const int32_t* cu_k, float sm_scale,
+                                 int causal, const float* alibi_slopes, int64_t alibi_sb, int64_t alibi_sh, hipStream_t st) {
   ALTO_REQUIRE(B > 0 && Hq > 0 && Hk > 0 && Hq % Hk == 0, "attention_fwd: Hq=%lld must be a positive multiple of Hk=%lld", (long long)Hq, (long long)Hk);
   ALTO_REQUIRE(Sq > 0 && Sq % 32 == 0 && Sk > 0 && Sk % 32 == 0, "attention_fwd: Sq=%lld and Sk=%lld must be positive multiples of 32", (long long)Sq, (long long)Sk);
   ALTO_REQUIRE(D == 64 || D == 128 || D == 192 || D == 256, "attention_fwd: head dim D=%lld must be 64, 128, 192 or 256", (long long)D);
@@ -495,14 +468,13 @@ extern "C" int alto_mxfp4_attention_fwd_strided(const void* q_codes, const void*
   ALTO_REQUIRE(o_sb >= 0 && o_sh >= 0 && o_ss >= 0 && l_sb >= 0 && l_sh >= 0 && l_ss >= 0 && (o_sb | o_sh | o_ss) % 4 == 0,
                "attention_fwd: output strides must be non-negative, those of out multiples of 4 elements");
   ALTO_REQUIRE((o_sb | o_sh | o_ss | l_sb | l_sh | l_ss) < (1ll << 40), "attention_fwd: output stride out of range");
-  ALTO_REQUIRE(((uintptr_t)q_codes | (uintptr_t)k_codes | (uintptr_t)vt_codes) % 16 == 0 && (uintptr_t)out % 8 == 0,
-               "attention_fwd: code pointers must be 16-byte aligned, out 8-byte aligned");
+  ALTO_REQUIRE(((uintptr_t)q.codes | (uintptr_t)q.values | (uintptr_t)k_codes | (uintptr_t)vt_codes) % 16 == 0 && (uintptr_t)out % 8 == 0,
+               "attention_fwd: operand pointers must be 16-byte aligned, out 8-byte aligned");
   ALTO_REQUIRE(((uintptr_t)k_scales | (uintptr_t)v_scales | (uintptr_t)lse | (uintptr_t)alibi_slopes) % 4 == 0,
                "attention_fwd: K and V scale pointers, lse and the alibi slopes must be 4-byte aligned");
-  AttnArgs a{(const uint8_t*)q_codes, (const uint8_t*)q_scales, (const uint8_t*)k_codes, (const uint8_t*)k_scales,
+  AttnArgs a{(const uint8_t*)q.codes, (const uint8_t*)q.scales, (const __bf16*)q.values, q.sb, q.sh, q.ss, (const uint8_t*)k_codes, (const uint8_t*)k_scales,
              (const uint8_t*)vt_codes, (const uint8_t*)v_scales, out, lse, o_sb, o_sh, o_ss, l_sb, l_sh, l_ss, (int)Hq, (int)Hk, (int)Sq, (int)Sk,
              (int)Sk, B * Hk * Sk * (D / 2), B * Hk * Dv * (Sk / 2), sm_scale, causal ? 1 : 0, nullptr, 0, 0, 0, 0, alibi_slopes, alibi_sb, alibi_sh};
-  hipStream_t st = (hipStream_t)stream;
   if (n_seqs == 0) {
     ALTO_REQUIRE(!causal || Sq <= Sk, "attention_fwd: causal attention needs Sq <= Sk (got %lld > %lld)", (long long)Sq, (long long)Sk);
     ALTO_REQUIRE((Sq + 127) / 128 <= 65535, "attention_fwd: Sq / 128 must fit a grid dimension");
@@ -543,6 +515,30 @@ extern "C" int alto_mxfp4_attention_fwd_strided(const void* q_codes, const void*
     if (rc != ALTO_MXFP4_OK) return rc;
   }
   return ALTO_MXFP4_OK;
+}
+}  // namespace alto
+
+extern "C" int alto_mxfp4_attention_fwd_strided(const void* q_codes, const void* q_scales, const void* k_codes, const void* k_scales,
+                                                const void* vt_codes, const void* v_scales, void* out, float* lse, int64_t B, int64_t Hq,
+                                                int64_t Hk, int64_t Sq, int64_t Sk, int64_t D, int64_t Dv, int64_t o_sb, int64_t o_sh, int64_t o_ss,
+                                                int64_t l_sb, int64_t l_sh, int64_t l_ss, int n_seqs, const int32_t* cu_q, const int32_t* cu_k,
+                                                float sm_scale, int causal, const float* alibi_slopes, int64_t alibi_sb, int64_t alibi_sh, void* stream) {
+  ALTO_REQUIRE(q_codes && q_scales && k_codes && k_scales && vt_codes && v_scales && out && lse, "attention_fwd: null pointer");
+  ALTO_REQUIRE(!alibi_slopes || (alibi_sb >= 0 && alibi_sh >= 0), "attention_fwd: negative alibi strides");
+  return alto::attention_fwd_strided({q_codes, q_scales, nullptr, 0, 0, 0}, k_codes, k_scales, vt_codes, v_scales, out, lse, B, Hq, Hk, Sq, Sk, D, Dv, o_sb, o_sh, o_ss,
+                                     l_sb, l_sh, l_ss, n_seqs, cu_q, cu_k, sm_scale, causal, alibi_slopes, alibi_sb, alibi_sh, (hipStream_t)stream);
+}
+
+extern "C" int alto_mxfp4_attention_fwd_bf16q(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_ss, const void* k_codes, const void* k_scales,
+                                              const void* vt_codes, const void* v_scales, void* out, float* lse, int64_t B, int64_t Hq, int64_t Hk,
+                                              int64_t Sq, int64_t Sk, int64_t D, int64_t Dv, int64_t o_sb, int64_t o_sh, int64_t o_ss, int64_t l_sb,
+                                              int64_t l_sh, int64_t l_ss, int n_seqs, const int32_t* cu_q, const int32_t* cu_k, float sm_scale, int causal,
+                                              void* stream) {
+  ALTO_REQUIRE(q && k_codes && k_scales && vt_codes && v_scales && out && lse, "attention_fwd: null pointer");
+  for (int64_t s : {q_sb, q_sh, q_ss})
+    ALTO_REQUIRE(s >= 0 && s < (1ll << 44) && s % 8 == 0, "attention_fwd: strides of q must be non-negative multiples of 8 elements");
+  return alto::attention_fwd_strided({nullptr, nullptr, q, q_sb, q_sh, q_ss}, k_codes, k_scales, vt_codes, v_scales, out, lse, B, Hq, Hk, Sq, Sk, D, Dv, o_sb, o_sh, o_ss,
+                                     l_sb, l_sh, l_ss, n_seqs, cu_q, cu_k, sm_scale, causal, nullptr, 0, 0, (hipStream_t)stream);
 }
 
 extern "C" int alto_mxfp4_attention_fwd(const void* q_codes, const void* q_scales, const void* k_codes, const void* k_scales,

@@ -14,7 +14,7 @@
 // are contiguous.  The general quantizer this replaces here wants one batch stride, so [B, S, heads, D] inputs were copied
 // first (three copies, 101 us, and 47 us for four more launches), and its 256-column tile leaves half of the lanes idle at
 // D = 128.  That forward went from 315 to 217 us with it.
-#include "common.h"
+#include "attention.h"
 
 namespace alto {
 namespace {
@@ -32,41 +32,6 @@ struct AttnOperand {
 struct AttnQuantArgs {
   AttnOperand q, k, v;
 };
-
-typedef unsigned short us2a_t __attribute__((ext_vector_type(2)));
-__device__ __forceinline__ uint32_t pk_max_u16a(uint32_t a, uint32_t b) {
-  return __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(us2a_t, a), __builtin_bit_cast(us2a_t, b)));
-}
-
-// absmax bits of 8 consecutive elements held in 4 (bf16) or 8 (fp32) dwords
-template <typename T>
-__device__ __forceinline__ uint32_t absmax8(const uint32_t* w) {
-  if constexpr (sizeof(T) == 2) {
-    const uint32_t a = pk_max_u16a(pk_max_u16a(w[0] & 0x7FFF7FFFu, w[1] & 0x7FFF7FFFu), pk_max_u16a(w[2] & 0x7FFF7FFFu, w[3] & 0x7FFF7FFFu));
-    return max(a & 0xFFFFu, a >> 16);
-  } else {
-    uint32_t a = 0;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) a = max(a, w[e] & 0x7FFFFFFFu);
-    return a;
-  }
-}
-template <typename T>
-__device__ __forceinline__ uint32_t encode8(const uint32_t* w, float scale) {
-  uint32_t o = 0;
-  if constexpr (sizeof(T) == 2) {
-    o = __builtin_amdgcn_cvt_scalef32_pk_fp4_bf16(o, __builtin_bit_cast(bf16x2_t, w[0]), scale, 0);
-    o = __builtin_amdgcn_cvt_scalef32_pk_fp4_bf16(o, __builtin_bit_cast(bf16x2_t, w[1]), scale, 1);
-    o = __builtin_amdgcn_cvt_scalef32_pk_fp4_bf16(o, __builtin_bit_cast(bf16x2_t, w[2]), scale, 2);
-    o = __builtin_amdgcn_cvt_scalef32_pk_fp4_bf16(o, __builtin_bit_cast(bf16x2_t, w[3]), scale, 3);
-  } else {
-    o = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(o, u2f(w[0]), u2f(w[1]), scale, 0);
-    o = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(o, u2f(w[2]), u2f(w[3]), scale, 1);
-    o = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(o, u2f(w[4]), u2f(w[5]), scale, 2);
-    o = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(o, u2f(w[6]), u2f(w[7]), scale, 3);
-  }
-  return o;
-}
 
 // STREAM: non-temporal loads.
 template <typename T, int COLS, bool STREAM>
@@ -159,12 +124,12 @@ __global__ __launch_bounds__(256) void attn_quant_kernel(const AttnQuantArgs a) 
 }  // namespace
 }  // namespace alto
 
-extern "C" int alto_mxfp4_attention_quantize(const void* q, const void* k, const void* v, int dtype, int64_t B, int64_t Hq, int64_t Hk, int64_t Sq,
-                                             int64_t Sk, int64_t D, int64_t Dv, int64_t q_sb, int64_t q_sh, int64_t q_ss, int64_t k_sb, int64_t k_sh,
-                                             int64_t k_ss, int64_t v_sb, int64_t v_sh, int64_t v_ss, uint8_t* q_codes, uint8_t* q_scales,
-                                             uint8_t* k_codes, uint8_t* k_scales, uint8_t* vt_codes, uint8_t* v_scales, void* stream) {
-  using namespace alto;
-  ALTO_REQUIRE(q && k && v && q_codes && q_scales && k_codes && k_scales && vt_codes && v_scales, "attention_quantize: null pointer");
+namespace alto {
+// q == NULL: K and V only
+static int quantize_operands(const void* q, const void* k, const void* v, int dtype, int64_t B, int64_t Hq, int64_t Hk, int64_t Sq, int64_t Sk, int64_t D,
+                             int64_t Dv, int64_t q_sb, int64_t q_sh, int64_t q_ss, int64_t k_sb, int64_t k_sh, int64_t k_ss, int64_t v_sb, int64_t v_sh,
+                             int64_t v_ss, uint8_t* q_codes, uint8_t* q_scales, uint8_t* k_codes, uint8_t* k_scales, uint8_t* vt_codes, uint8_t* v_scales,
+                             hipStream_t st) {
   ALTO_REQUIRE(dtype == ALTO_DT_BF16 || dtype == ALTO_DT_F32, "attention_quantize: dtype %d is neither bf16 (0) nor f32 (1)", dtype);
   ALTO_REQUIRE(B > 0 && Hq > 0 && Hk > 0, "attention_quantize: empty batch or no heads");
   ALTO_REQUIRE(Sq > 0 && Sq % 32 == 0 && Sk > 0 && Sk % 32 == 0, "attention_quantize: Sq=%lld and Sk=%lld must be positive multiples of 32", (long long)Sq, (long long)Sk);
@@ -178,22 +143,21 @@ extern "C" int alto_mxfp4_attention_quantize(const void* q, const void* k, const
   ALTO_REQUIRE((((uintptr_t)q | (uintptr_t)k | (uintptr_t)v | (uintptr_t)vt_codes) & 15) == 0 && (((uintptr_t)q_codes | (uintptr_t)k_codes) & 3) == 0,
                "attention_quantize: inputs and vt_codes must be 16-byte aligned, q_codes and k_codes 4-byte aligned");
   const int cols = (D % 128 == 0 && Dv % 128 == 0) ? 128 : 64;
-  AttnQuantArgs a;
+  AttnQuantArgs a{};
   auto fill = [&](AttnOperand& o, const void* x, int64_t sb, int64_t sh, int64_t ss, uint8_t* codes, uint8_t* scales, int64_t H, int64_t S, int64_t d) {
     const int64_t groups = (S + 127) / 128;
     o = AttnOperand{x, sb, sh, ss, codes, scales, (int)H, (int)S, (int)d, (int)groups, sh > ss ? 1 : 0, 0};
     return product_below(1ll << 31, B * H, groups, d / cols) ? (o.wgs = B * H * groups * (d / cols)) : -1;
   };
-  const int64_t nq = fill(a.q, q, q_sb, q_sh, q_ss, q_codes, q_scales, Hq, Sq, D), nk = fill(a.k, k, k_sb, k_sh, k_ss, k_codes, k_scales, Hk, Sk, D),
+  const int64_t nq = q ? fill(a.q, q, q_sb, q_sh, q_ss, q_codes, q_scales, Hq, Sq, D) : (a.q.wgs = 0), nk = fill(a.k, k, k_sb, k_sh, k_ss, k_codes, k_scales, Hk, Sk, D),
                 nv = fill(a.v, v, v_sb, v_sh, v_ss, vt_codes, v_scales, Hk, Sk, Dv);
-  ALTO_REQUIRE(nq > 0 && nk > 0 && nv > 0 && nq + nk + nv < (1ll << 31), "attention_quantize: too many workgroups");
+  ALTO_REQUIRE(nq >= 0 && nk > 0 && nv > 0 && nq + nk + nv < (1ll << 31), "attention_quantize: too many workgroups");
   const dim3 grid((unsigned)(nq + nk + nv));
-  hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   // bf16 operands of 128 MB and more are read past the caches, which then keep the codes for the attention kernel (whole calls,
   // causal, changing inputs, without -> with, us: 160 MB 222 -> 216, 320 MB 443 -> 430).  Smaller ones may be in a cache already
   // (96 MB the same).  fp32 operands lose: two load instructions use half of each line, and the second finds it in no cache
   // (this kernel at 192 MB 45 -> 51, at 640 MB 141 -> 157; whole calls 131 -> 137 and 490 -> 502).
-  const bool stream_in = dtype == ALTO_DT_BF16 && (B * Hq * Sq * D + B * Hk * Sk * (D + Dv)) * 2 >= (128ll << 20);
+  const bool stream_in = dtype == ALTO_DT_BF16 && ((q ? B * Hq * Sq * D : 0) + B * Hk * Sk * (D + Dv)) * 2 >= (128ll << 20);
   auto go = [&](auto kern) { hipLaunchKernelGGL(kern, grid, dim3(256), 0, st, a); };
   if (dtype == ALTO_DT_BF16) {
     if (cols == 128) stream_in ? go(attn_quant_kernel<__bf16, 128, true>) : go(attn_quant_kernel<__bf16, 128, false>);
@@ -202,4 +166,22 @@ extern "C" int alto_mxfp4_attention_quantize(const void* q, const void* k, const
     cols == 128 ? go(attn_quant_kernel<float, 128, false>) : go(attn_quant_kernel<float, 64, false>);
   }
   return check_launch("attention_quantize");
+}
+}  // namespace alto
+
+extern "C" int alto_mxfp4_attention_quantize(const void* q, const void* k, const void* v, int dtype, int64_t B, int64_t Hq, int64_t Hk, int64_t Sq,
+                                             int64_t Sk, int64_t D, int64_t Dv, int64_t q_sb, int64_t q_sh, int64_t q_ss, int64_t k_sb, int64_t k_sh,
+                                             int64_t k_ss, int64_t v_sb, int64_t v_sh, int64_t v_ss, uint8_t* q_codes, uint8_t* q_scales,
+                                             uint8_t* k_codes, uint8_t* k_scales, uint8_t* vt_codes, uint8_t* v_scales, void* stream) {
+  ALTO_REQUIRE(q && k && v && q_codes && q_scales && k_codes && k_scales && vt_codes && v_scales, "attention_quantize: null pointer");
+  return alto::quantize_operands(q, k, v, dtype, B, Hq, Hk, Sq, Sk, D, Dv, q_sb, q_sh, q_ss, k_sb, k_sh, k_ss, v_sb, v_sh, v_ss, q_codes, q_scales, k_codes, k_scales,
+                                 vt_codes, v_scales, (hipStream_t)stream);
+}
+
+extern "C" int alto_mxfp4_attention_quantize_kv(const void* k, const void* v, int dtype, int64_t B, int64_t Hk, int64_t Sk, int64_t D, int64_t Dv,
+                                                int64_t k_sb, int64_t k_sh, int64_t k_ss, int64_t v_sb, int64_t v_sh, int64_t v_ss, uint8_t* k_codes,
+                                                uint8_t* k_scales, uint8_t* vt_codes, uint8_t* v_scales, void* stream) {
+  ALTO_REQUIRE(k && v && k_codes && k_scales && vt_codes && v_scales, "attention_quantize: null pointer");
+  return alto::quantize_operands(nullptr, k, v, dtype, B, Hk, Hk, Sk, Sk, D, Dv, 0, 0, 0, k_sb, k_sh, k_ss, v_sb, v_sh, v_ss, nullptr, nullptr, k_codes, k_scales, vt_codes,
+                                 v_scales, (hipStream_t)stream);
 }

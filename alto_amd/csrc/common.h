@@ -130,5 +130,7 @@ __device__ __forceinline__ uint32_t dpp_u32(uint32_t v) {
 #define ALTO_DPP_QUAD_XOR2 0x4E
 // lane -> 7 - lane inside each group of 8
 #define ALTO_DPP_HALF_MIRROR 0x141
+// lane ^ 8 inside each group of 16
+#define ALTO_DPP_ROW_ROR8 0x128
 
 }  // namespace alto

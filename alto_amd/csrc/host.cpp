@@ -38,6 +38,8 @@ struct Api {
   ALTO_FN(grouped_gemm_dw_ps);
   ALTO_FN(attention_quantize);
   ALTO_FN(attention_fwd_strided);
+  ALTO_FN(attention_quantize_kv);
+  ALTO_FN(attention_fwd_bf16q);
 #undef ALTO_FN
 } api;
 py::object* check_fn = nullptr;   // _lib.check(rc, name): raises for rc != 0 (never freed: the interpreter may be gone by then)
@@ -56,6 +58,8 @@ void bind(const py::dict& address, py::object check) {
   ALTO_FN(grouped_gemm_dw_ps);
   ALTO_FN(attention_quantize);
   ALTO_FN(attention_fwd_strided);
+  ALTO_FN(attention_quantize_kv);
+  ALTO_FN(attention_fwd_bf16q);
 #undef ALTO_FN
   delete check_fn;
   check_fn = new py::object(std::move(check));
@@ -230,7 +234,8 @@ py::object grouped_dw_packed(const Tensor& go, const Tensor& go_ps, const Tensor
   return py::cast(dw);
 }
 
-// attention.py:_attend without ALiBi slopes: operand quantizer and attention kernel on [B, H, S, D] views
+// attention.py:_attend without ALiBi slopes: operand quantizer and attention kernel on [B, H, S, D] views (bf16: the attention
+// kernel quantizes Q itself)
 bool attend(const Tensor& q_in, const Tensor& k_in, const Tensor& v_in, double sm_scale, bool causal, const Tensor& out, const Tensor& lse,
             const std::vector<int32_t>& cu_q, const std::vector<int32_t>& cu_k, uintptr_t stream) {
   Tensor q = q_in, k = k_in, v = v_in;
@@ -242,22 +247,33 @@ bool attend(const Tensor& q_in, const Tensor& k_in, const Tensor& v_in, double s
   const int64_t B = q.size(0), Hq = q.size(1), Sq = q.size(2), D = q.size(3), Hk = v.size(1), Sk = v.size(2), Dv = v.size(3);
   if (k.size(0) != v.size(0) || k.size(1) != Hk || k.size(2) != Sk || B != k.size(0) || k.size(3) != D) return false;
   // 16 bytes of room behind each part: the attention kernel reads K's and V's scale bytes in whole dwords
-  const int64_t sizes[6] = {B * Hq * Sq * D / 2, B * Hk * Sk * D / 2, B * Hk * Sk * Dv / 2, B * Hq * (Sq / 32) * (D / 32), B * Hk * (Sk / 32) * (D / 32), B * Hk * (Sk / 32) * (Dv / 32)};
+  const bool own_q = q.scalar_type() == at::kBFloat16;
+  const int64_t sizes[6] = {B * Hk * Sk * D / 2, B * Hk * Sk * Dv / 2, B * Hk * (Sk / 32) * (D / 32), B * Hk * (Sk / 32) * (Dv / 32),
+                            own_q ? 0 : B * Hq * Sq * D / 2, own_q ? 0 : B * Hq * (Sq / 32) * (D / 32)};
   int64_t start[6], total = 0;
-  for (int i = 0; i < 6; ++i) {
+  for (int i = 0; i < (own_q ? 4 : 6); ++i) {
     start[i] = total;
     total += div_up(sizes[i] + 16, 256) * 256;
   }
   const Tensor buf = Alloc(q).dense({total});
   uint8_t* p = bytes(buf);
-  uint8_t *qq = p + start[0], *kq = p + start[1], *vq = p + start[2], *qs = p + start[3], *ks = p + start[4], *vs = p + start[5];
+  uint8_t *kq = p + start[0], *vq = p + start[1], *ks = p + start[2], *vs = p + start[3];
   void* s = reinterpret_cast<void*>(stream);
-  call("alto_mxfp4_attention_quantize", api.attention_quantize, q.data_ptr(), k.data_ptr(), v.data_ptr(), dtype_code(q.scalar_type()), B, Hq, Hk, Sq, Sk, D, Dv, stride_of(q, 0),
-       stride_of(q, 1), stride_of(q, 2), stride_of(k, 0), stride_of(k, 1), stride_of(k, 2), stride_of(v, 0), stride_of(v, 1), stride_of(v, 2), qq, qs, kq, ks, vq, vs, s);
   const int n = cu_q.empty() ? 0 : (int)cu_q.size() - 1;
-  call("alto_mxfp4_attention_fwd_strided", api.attention_fwd_strided, qq, qs, kq, ks, vq, vs, out.data_ptr(), static_cast<float*>(lse.data_ptr()), B, Hq, Hk, Sq, Sk, D, Dv,
-       out.stride(0), out.stride(1), out.stride(2), lse.stride(0), lse.stride(1), lse.stride(2), n, n ? cu_q.data() : nullptr, n ? cu_k.data() : nullptr, (float)sm_scale,
-       (int)causal, static_cast<const float*>(nullptr), (int64_t)0, (int64_t)0, s);
+  const int32_t *cq = n ? cu_q.data() : nullptr, *ck = n ? cu_k.data() : nullptr;
+  float* lse_p = static_cast<float*>(lse.data_ptr());
+  if (own_q) {
+    call("alto_mxfp4_attention_quantize_kv", api.attention_quantize_kv, k.data_ptr(), v.data_ptr(), (int)ALTO_DT_BF16, B, Hk, Sk, D, Dv, stride_of(k, 0), stride_of(k, 1),
+         stride_of(k, 2), stride_of(v, 0), stride_of(v, 1), stride_of(v, 2), kq, ks, vq, vs, s);
+    call("alto_mxfp4_attention_fwd_bf16q", api.attention_fwd_bf16q, q.data_ptr(), stride_of(q, 0), stride_of(q, 1), stride_of(q, 2), kq, ks, vq, vs, out.data_ptr(), lse_p, B,
+         Hq, Hk, Sq, Sk, D, Dv, out.stride(0), out.stride(1), out.stride(2), lse.stride(0), lse.stride(1), lse.stride(2), n, cq, ck, (float)sm_scale, (int)causal, s);
+    return true;
+  }
+  uint8_t *qq = p + start[4], *qs = p + start[5];
+  call("alto_mxfp4_attention_quantize", api.attention_quantize, q.data_ptr(), k.data_ptr(), v.data_ptr(), (int)ALTO_DT_F32, B, Hq, Hk, Sq, Sk, D, Dv, stride_of(q, 0),
+       stride_of(q, 1), stride_of(q, 2), stride_of(k, 0), stride_of(k, 1), stride_of(k, 2), stride_of(v, 0), stride_of(v, 1), stride_of(v, 2), qq, qs, kq, ks, vq, vs, s);
+  call("alto_mxfp4_attention_fwd_strided", api.attention_fwd_strided, qq, qs, kq, ks, vq, vs, out.data_ptr(), lse_p, B, Hq, Hk, Sq, Sk, D, Dv, out.stride(0), out.stride(1),
+       out.stride(2), lse.stride(0), lse.stride(1), lse.stride(2), n, cq, ck, (float)sm_scale, (int)causal, static_cast<const float*>(nullptr), (int64_t)0, (int64_t)0, s);
   return true;
 }
 

@@ -441,6 +441,13 @@ int alto_mxfp4_attention_quantize(const void* q, const void* k, const void* v, i
                                   uint8_t* k_codes, uint8_t* k_scales, uint8_t* vt_codes, uint8_t* v_scales, void* stream);
 
 /*
+ * The same for K and V alone: what alto_mxfp4_attention_fwd_bf16q takes.
+ */
+int alto_mxfp4_attention_quantize_kv(const void* k, const void* v, int dtype, int64_t B, int64_t Hk, int64_t Sk, int64_t D, int64_t Dv,
+                                     int64_t k_sb, int64_t k_sh, int64_t k_ss, int64_t v_sb, int64_t v_sh, int64_t v_ss, uint8_t* k_codes,
+                                     uint8_t* k_scales, uint8_t* vt_codes, uint8_t* v_scales, void* stream);
+
+/*
  * alto_mxfp4_attention_fwd on operands whose key count is any multiple of 32 (nothing is padded; the last block of 64 keys
  * reads what follows in the buffers and masks it: allocate 16 bytes behind k_scales and v_scales, whose content does not
  * matter), with the outputs at element strides o_* / l_* of batch, head and row (unit stride along Dv).
@@ -454,6 +461,17 @@ int alto_mxfp4_attention_fwd_strided(const void* q_codes, const void* q_scales, 
                                      int64_t Hk, int64_t Sq, int64_t Sk, int64_t D, int64_t Dv, int64_t o_sb, int64_t o_sh, int64_t o_ss,
                                      int64_t l_sb, int64_t l_sh, int64_t l_ss, int n_seqs, const int32_t* cu_q, const int32_t* cu_k,
                                      float sm_scale, int causal, const float* alibi_slopes, int64_t alibi_sb, int64_t alibi_sh, void* stream);
+
+/*
+ * alto_mxfp4_attention_fwd_strided (without ALiBi slopes) on Q as bf16 values, which the attention kernel quantizes itself, to
+ * the codes and scales of alto_mxfp4_attention_quantize: q [B][Hq][Sq][D] at element strides q_sb / q_sh / q_ss of batch, head
+ * and row (multiples of 8), unit stride along the head dim, 16-byte aligned.  The results are the same bit for bit.
+ */
+int alto_mxfp4_attention_fwd_bf16q(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_ss, const void* k_codes, const void* k_scales,
+                                   const void* vt_codes, const void* v_scales, void* out, float* lse, int64_t B, int64_t Hq, int64_t Hk,
+                                   int64_t Sq, int64_t Sk, int64_t D, int64_t Dv, int64_t o_sb, int64_t o_sh, int64_t o_ss, int64_t l_sb,
+                                   int64_t l_sh, int64_t l_ss, int n_seqs, const int32_t* cu_q, const int32_t* cu_k, float sm_scale, int causal,
+                                   void* stream);
 
 /*
  * Fills out[0 .. n) with random 32-bit words for stochastic rounding: word 4 c + j is word j of Philox4x32-10 (Salmon et

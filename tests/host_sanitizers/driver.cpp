@@ -274,6 +274,27 @@ Entry g_entries[] = {
 };
 constexpr int kEntries = sizeof(g_entries) / sizeof(g_entries[0]);
 
+// Entries with their own count of calls.
+int call_bf16q(const Args& a, const Boundaries* b) {
+  return alto_mxfp4_attention_fwd_bf16q(a.p[0], a.s[13], a.s[14], a.s[15], a.p[1], a.p[2], a.p[3], a.p[4], a.p[5], P(float, 6), a.s[0], a.s[1], a.s[2], a.s[3],
+                                        a.s[4], a.s[5], a.s[6], a.s[7], a.s[8], a.s[9], a.s[10], a.s[11], a.s[12], b ? b->n : 0, b ? b->q : nullptr,
+                                        b ? b->k : nullptr, a.f, a.i[1], nullptr);
+}
+Entry g_bf16q_entries[] = {
+    // B, Hk, Sk, D, Dv, strides of k, v
+    {"attention_quantize_kv", 11, 1, 6, {{2, 2, 96, 128, 64, 96 * 256, 128, 256, 96 * 128, 64, 128}, {0}, {D, D, D, D, D, D}, 1.0f, {0, 0}, g_signs, g_perm},
+     [](const Args& a) {
+       return alto_mxfp4_attention_quantize_kv(a.p[0], a.p[1], a.i[0], a.s[0], a.s[1], a.s[2], a.s[3], a.s[4], a.s[5], a.s[6], a.s[7], a.s[8], a.s[9], a.s[10],
+                                               P(uint8_t, 2), P(uint8_t, 3), P(uint8_t, 4), P(uint8_t, 5), nullptr);
+     }},
+    // B, Hq, Hk, Sq, Sk, D, Dv, strides of out, lse and q
+    {"attention_fwd_bf16q", 16, 2, 7, {{2, 8, 2, 256, 288, 128, 64, 131072, 64, 512, 2048, 1, 8, 262144, 128, 1024}, {0, 1}, {D, D, D, D, D, D, D}, 0.088388f, {0, 0}, g_signs, g_perm},
+     [](const Args& a) { return call_bf16q(a, nullptr); }},
+    {"attention_fwd_bf16q_packed", 16, 2, 7, {{1, 8, 2, 256, 288, 128, 64, 0, 64, 512, 0, 1, 8, 0, 128, 1024}, {0, 1}, {D, D, D, D, D, D, D}, 0.088388f, {0, 0}, g_signs, g_perm},
+     [](const Args& a) { return call_bf16q(a, &g_bounds[(unsigned)a.i[0] % (kManySequences + 1)]); }},
+};
+constexpr int kBf16qEntries = sizeof(g_bf16q_entries) / sizeof(g_bf16q_entries[0]);
+
 void mutate(Args& a, const Entry& e) {
   const int fields = e.ns + e.ni + e.np + 4;   // + float, one of the two u64, signs, perm
   int k = (int)(next_u64() % (uint64_t)fields);
@@ -292,22 +313,10 @@ void mutate(Args& a, const Entry& e) {
   }
 }
 
-}  // namespace
-
-int main(int argc, char** argv) {
-  const long rounds = argc > 1 ? std::atol(argv[1]) : 2000;
-  if (argc > 2) g_state ^= std::strtoull(argv[2], nullptr, 0);   // another sequence of calls
-  for (int k = 0; k < 32; ++k) {
-    g_signs[k] = (k * 7 % 3 == 0) ? -1 : 1;
-    g_perm[k] = (uint8_t)((k * 5 + 3) % 32);
-  }
-  for (int k = 0; k <= 130; ++k) g_bounds[kManySequences].q[k] = g_bounds[kManySequences].k[k] = 32 * k;
-  std::printf("version %d\n", alto_mxfp4_version());
-  (void)alto_mxfp4_init();   // no device here: must fail cleanly or do nothing
-  long calls = 0;
+int run(Entry* entries, int n_entries, long rounds, long& calls) {
   for (long it = 0; it < rounds; ++it) {
-    for (int n = 0; n < kEntries; ++n) {
-      Entry& e = g_entries[n];
+    for (int n = 0; n < n_entries; ++n) {
+      Entry& e = entries[n];
       Args a = e.valid;
       const int changes = (int)(next_u64() % 4);
       for (int c = 0; c < changes; ++c) mutate(a, e);
@@ -329,6 +338,34 @@ int main(int argc, char** argv) {
         ++e.launches;
     }
   }
+  return 0;
+}
+
+int report(const Entry* entries, int n_entries) {   // -> entries that never got past their argument checks
+  int never = 0;
+  for (int n = 0; n < n_entries; ++n) {
+    const Entry& e = entries[n];
+    std::printf("%-24s calls %6ld  returned 0 %6ld  reached the launch %6ld\n", e.name, e.calls, e.ok, e.launches);
+    if (e.launches == 0 && e.ok == 0) ++never;
+  }
+  return never;
+}
+
+}  // namespace
+
+int main(int argc, char** argv) {
+  const long rounds = argc > 1 ? std::atol(argv[1]) : 2000;
+  if (argc > 2) g_state ^= std::strtoull(argv[2], nullptr, 0);   // another sequence of calls
+  for (int k = 0; k < 32; ++k) {
+    g_signs[k] = (k * 7 % 3 == 0) ? -1 : 1;
+    g_perm[k] = (uint8_t)((k * 5 + 3) % 32);
+  }
+  for (int k = 0; k <= 130; ++k) g_bounds[kManySequences].q[k] = g_bounds[kManySequences].k[k] = 32 * k;
+  std::printf("version %d\n", alto_mxfp4_version());
+  (void)alto_mxfp4_init();   // no device here: must fail cleanly or do nothing
+  long calls = 0, bf16q_calls = 0;
+  if (int rc = run(g_entries, kEntries, rounds, calls)) return rc;
+  if (int rc = run(g_bf16q_entries, kBf16qEntries, rounds, bf16q_calls)) return rc;
   for (unsigned k = 0; k < sizeof(g_mem); ++k)
     if (g_mem[k] != 0) {
       std::fprintf(stderr, "host code wrote through a pointer that stands for device memory (byte %u)\n", k);
@@ -344,12 +381,7 @@ int main(int argc, char** argv) {
       return 5;
     }
   }
-  int never = 0;
-  for (int n = 0; n < kEntries; ++n) {
-    const Entry& e = g_entries[n];
-    std::printf("%-24s calls %6ld  returned 0 %6ld  reached the launch %6ld\n", e.name, e.calls, e.ok, e.launches);
-    if (e.launches == 0 && e.ok == 0) ++never;
-  }
+  const int never = report(g_entries, kEntries) + report(g_bf16q_entries, kBf16qEntries);
   if (never != 0 && rounds >= 100) {
     std::fprintf(stderr, "%d entry points never got past their argument checks: their valid argument set is not valid\n", never);
     return 4;
