@@ -20,7 +20,7 @@ HOSTNAME = "alto_mxfp4_host.so"   # CPython module of csrc/host.cpp, named as it
 HOSTSRC = os.path.join(CSRC, "host.cpp")
 HEADER = os.path.join(HERE, "..", "include", "alto_mxfp4.h")
 
-SOURCES = ["capi.hip", "quantize.hip", "dequantize.hip", "gemm.hip", "gemm_tiled.hip", "gemm_mid.hip", "gemm_skinny.hip", "grouped_gemm.hip", "probe.hip", "qdq.hip", "attention.hip", "attention_quantize.hip", "quantize_dynamic.hip", "random.hip"]
+SOURCES = ["capi.hip", "quantize.hip", "dequantize.hip", "gemm.hip", "gemm_tiled.hip", "gemm_mid.hip", "gemm_skinny.hip", "grouped_gemm.hip", "probe.hip", "qdq.hip", "attention.hip", "attention_split.hip", "attention_quantize.hip", "quantize_dynamic.hip", "random.hip"]
 
 HIPCC_FLAGS = [
     "--offload-arch=gfx950",

@@ -131,4 +131,87 @@ __device__ __forceinline__ void quantize_q(const __bf16* x, int64_t row_stride, 
   for (int s = 0; s < NK; ++s) qf[s] = frag16(scratch + 1024 * s + (lane & 31) * 32 + (lane >> 5) * 16);
 }
 
+// What workgroup row `z` of `nz` works on: its sequence and its block of rows, the last rows first with a causal mask.
+struct AttnRows {
+  int qn, kn, q_first, k_first, block;
+};
+template <typename SEQS>
+__device__ __forceinline__ AttnRows attn_rows(const AttnArgs& a, const SEQS& seqs, int z, int nz) {
+  AttnRows w{a.Sq, a.Sk_used, 0, 0, 0};
+  if constexpr (std::is_same<SEQS, AttnSeqs>::value) {
+    int lo = 0, hi = seqs.n - 1;   // the sequence this row block belongs to: the last one with z0[i] <= z
+    while (lo < hi) {
+      const int mid = (lo + hi + 1) >> 1;
+      if (seqs.z0[mid] <= z) lo = mid; else hi = mid - 1;
+    }
+    w.qn = seqs.qn[lo]; w.kn = seqs.kn[lo]; w.q_first = seqs.q0[lo]; w.k_first = seqs.k0[lo];
+    nz = seqs.z0[lo + 1] - seqs.z0[lo];
+    z -= seqs.z0[lo];
+  }
+  w.block = a.causal ? nz - 1 - z : z;
+  return w;
+}
+// Eight neighbouring workgroups go to the eight XCDs in turn: each gets a range of consecutive heads, so a key / value head comes
+// into one L2 (two, where a range starts inside its query heads) and not into all of them: 195 -> 187 us for 4 x 2048 tokens,
+// 64 / 8 heads of 128, causal.
+__device__ __forceinline__ int attn_head(const AttnArgs& a) {
+  return a.Hq % 8 == 0 ? (int)((blockIdx.x & 7) * (a.Hq >> 3) + (blockIdx.x >> 3)) : (int)blockIdx.x;
+}
+
+// Hides the scores of keys that a lane's row may not see: `seen` = how many keys from the lane's first one (4 h of the block) on
+// it does.  (The empty assembly keeps each comparison next to its use: taken together, their 32 results spilled scalars that the
+// loop over the blocks needs.  In attention.hip, whose own form spills none, this one is 0 to 5 % faster with a causal mask and 2 to
+// 4 % slower without.)
+__device__ __forceinline__ void mask_scores(v16f_t (&S)[2], int seen) {
+#pragma unroll
+  for (int t = 0; t < 2; ++t)
+#pragma unroll
+    for (int v = 0; v < 16; ++v) {
+      float x = 32 * t + 8 * (v >> 2) + (v & 3) >= seen ? -__builtin_inff() : S[t][v];
+      asm volatile("" : "+v"(x));
+      S[t][v] = x;
+    }
+}
+
+// Probabilities of a wave's 32 rows and 64 keys (S: scores of this lane's row, keys 8 g + 4 h + (0..3) of tiles of 32; tmx: the
+// row's largest score of each tile; cs: factor into the base-2 domain; m_new: running maximum there): one E8M0 scale per (row,
+// 32 keys), E2M1 codes (round to nearest even), as the second operand of the product with V.
+__device__ __forceinline__ void quantize_probabilities(v16f_t (&S)[2], const float (&tmx)[2], float cs, float m_new, int h, v8i_t& pf, int& pscale) {
+  uint32_t c[2][2];
+  int psc[2];
+#pragma unroll
+  for (int t = 0; t < 2; ++t) {
+#pragma unroll
+    for (int v = 0; v < 16; ++v) S[t][v] = __builtin_amdgcn_exp2f(__builtin_fmaf(S[t][v], cs, -m_new));
+    const float am = __builtin_amdgcn_exp2f(__builtin_fmaf(tmx[t], cs, -m_new));   // = max of the 32 values above
+    const uint32_t e = e8m0_from_f32_bits(f2u(am));
+    psc[t] = (int)e;
+    const float scale_f = u2f(e << 23);
+#pragma unroll
+    for (int w = 0; w < 2; ++w) {
+      uint32_t o = 0;
+      o = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(o, S[t][8 * w + 0], S[t][8 * w + 1], scale_f, 0);
+      o = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(o, S[t][8 * w + 2], S[t][8 * w + 3], scale_f, 1);
+      o = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(o, S[t][8 * w + 4], S[t][8 * w + 5], scale_f, 2);
+      o = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(o, S[t][8 * w + 6], S[t][8 * w + 7], scale_f, 3);
+      c[t][w] = o;
+    }
+  }
+  // Lane (r, h) multiplies tile h of this block and needs that tile's 32 codes of row r in key order; it holds the
+  // keys 8 g + 4 h + (0..3) of both tiles.  One half-wave swap per dword hands lane (r, 0) the tile-0 codes of lane
+  // (r, 1) and lane (r, 1) the tile-1 codes of lane (r, 0); in both halves the swapped pair is then {keys 8 g + 0..3,
+  // keys 8 g + 4..7} = {p[0], p[1]}, interleaved 16 bits at a time.
+  const v2u_t p0 = __builtin_amdgcn_permlane32_swap(c[0][0], c[1][0], false, false);
+  const v2u_t p1 = __builtin_amdgcn_permlane32_swap(c[0][1], c[1][1], false, false);
+  pf = v8i_t{(int)__builtin_amdgcn_perm(p0[1], p0[0], 0x05040100u), (int)__builtin_amdgcn_perm(p0[1], p0[0], 0x07060302u),
+                         (int)__builtin_amdgcn_perm(p1[1], p1[0], 0x05040100u), (int)__builtin_amdgcn_perm(p1[1], p1[0], 0x07060302u),
+                         0, 0, 0, 0};
+  pscale = h ? psc[1] : psc[0];
+}
+
+// Launches of the two kernels (attention.hip: four waves walk the keys of 128 rows; attention_split.hip: they deal out the keys of
+// 32 rows); `row_blocks` in units of 128 and of 32 rows.
+template <typename SEQS>
+int launch_attn_split(const AttnArgs& a, const SEQS& seqs, int B, int row_blocks, int64_t D, int64_t Dv, hipStream_t st);
+
 }  // namespace alto

@@ -47,7 +47,6 @@ struct AttnTile {
 // SEQS: AttnSeqs, or AttnNoSeqs for B sequences of one length.
 template <int NK, int ND, bool BIASED, bool QBF, typename SEQS>
 __device__ __forceinline__ void attn_fwd_body(const AttnArgs& a, const SEQS& seqs, __bf16* __restrict__ out, float* __restrict__ lse_out, uint8_t* ring) {
-  constexpr bool PACKED = std::is_same<SEQS, AttnSeqs>::value;
   constexpr int D = NK * 64, DV = ND * 32;
   constexpr int K_BYTES = AttnTile<NK, ND>::K_BYTES, V_BYTES = AttnTile<NK, ND>::V_BYTES, SLOT = AttnTile<NK, ND>::SLOT;
   constexpr int K_PIECES = K_BYTES / 16, V_PIECES = V_BYTES / 16;
@@ -59,23 +58,12 @@ __device__ __forceinline__ void attn_fwd_body(const AttnArgs& a, const SEQS& seq
   const int r = lane & 31, h = lane >> 5;
   // grid (heads, batch, row blocks): with a causal mask every head's longest rows are dispatched before anybody's shorter
   // ones, so the launch ends with the cheapest workgroups (packed sequences: the host passes them longest first)
-  int qn = a.Sq, kn = a.Sk_used, q_first = 0, k_first = 0, z = (int)blockIdx.z, nz = (int)gridDim.z;
-  if constexpr (PACKED) {
-    int lo = 0, hi = seqs.n - 1;   // the sequence this row block belongs to: the last one with z0[i] <= z
-    while (lo < hi) {
-      const int mid = (lo + hi + 1) >> 1;
-      if (seqs.z0[mid] <= z) lo = mid; else hi = mid - 1;
-    }
-    qn = seqs.qn[lo]; kn = seqs.kn[lo]; q_first = seqs.q0[lo]; k_first = seqs.k0[lo];
-    nz = seqs.z0[lo + 1] - seqs.z0[lo];
-    z -= seqs.z0[lo];
-  }
-  const int qblk = a.causal ? nz - 1 - z : z;
+  const AttnRows w = attn_rows(a, seqs, (int)blockIdx.z, (int)gridDim.z);
+  const int qn = w.qn, kn = w.kn, q_first = w.q_first, k_first = w.k_first;
+  const int qblk = w.block;
   const int q0 = (qblk * 4 + wave) * 32;
   const bool live = q0 < qn;                      // a wave past the last row still helps with loads and barriers
-  // eight neighbouring workgroups go to the eight XCDs in turn: each gets a range of consecutive heads, so a key / value head
-  // comes into one L2 (two, where a range starts inside its query heads) and not into all of them: 195 -> 187 us (QBF above)
-  const int hq = a.Hq % 8 == 0 ? (blockIdx.x & 7) * (a.Hq >> 3) + (blockIdx.x >> 3) : blockIdx.x, b = blockIdx.y;
+  const int hq = attn_head(a), b = blockIdx.y;
   const int hk = hq / (a.Hq / a.Hk);
   // rows of the operand buffers where this (sequence, head) starts
   const int64_t q_base = ((int64_t)b * a.Hq + hq) * a.Sq + q_first, bhk = (int64_t)b * a.Hk + hk, k_base = bhk * a.Sk + k_first;
@@ -294,37 +282,9 @@ __device__ __forceinline__ void attn_fwd_body(const AttnArgs& a, const SEQS& seq
       m_i = m_new;
       m_new = m_sub;
 
-      // ---- probabilities, one E8M0 scale per (row, 32 keys), E2M1 codes (round to nearest even)
-      uint32_t c[2][2];
-      int psc[2];
-#pragma unroll
-      for (int t = 0; t < 2; ++t) {
-#pragma unroll
-        for (int v = 0; v < 16; ++v) S[t][v] = __builtin_amdgcn_exp2f(__builtin_fmaf(S[t][v], cs, -m_new));
-        const float am = __builtin_amdgcn_exp2f(__builtin_fmaf(tmx[t], cs, -m_new));   // = max of the 32 values above
-        const uint32_t e = e8m0_from_f32_bits(f2u(am));
-        psc[t] = (int)e;
-        const float scale_f = u2f(e << 23);
-#pragma unroll
-        for (int w = 0; w < 2; ++w) {
-          uint32_t o = 0;
-          o = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(o, S[t][8 * w + 0], S[t][8 * w + 1], scale_f, 0);
-          o = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(o, S[t][8 * w + 2], S[t][8 * w + 3], scale_f, 1);
-          o = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(o, S[t][8 * w + 4], S[t][8 * w + 5], scale_f, 2);
-          o = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(o, S[t][8 * w + 6], S[t][8 * w + 7], scale_f, 3);
-          c[t][w] = o;
-        }
-      }
-      // Lane (r, h) multiplies tile h of this block and needs that tile's 32 codes of row r in key order; it holds the
-      // keys 8 g + 4 h + (0..3) of both tiles.  One half-wave swap per dword hands lane (r, 0) the tile-0 codes of lane
-      // (r, 1) and lane (r, 1) the tile-1 codes of lane (r, 0); in both halves the swapped pair is then {keys 8 g + 0..3,
-      // keys 8 g + 4..7} = {p[0], p[1]}, interleaved 16 bits at a time.
-      const v2u_t p0 = __builtin_amdgcn_permlane32_swap(c[0][0], c[1][0], false, false);
-      const v2u_t p1 = __builtin_amdgcn_permlane32_swap(c[0][1], c[1][1], false, false);
-      const v8i_t pf = v8i_t{(int)__builtin_amdgcn_perm(p0[1], p0[0], 0x05040100u), (int)__builtin_amdgcn_perm(p0[1], p0[0], 0x07060302u),
-                             (int)__builtin_amdgcn_perm(p1[1], p1[0], 0x05040100u), (int)__builtin_amdgcn_perm(p1[1], p1[0], 0x07060302u),
-                             0, 0, 0, 0};
-      const int pscale = h ? psc[1] : psc[0];
+      v8i_t pf;
+      int pscale;
+      quantize_probabilities(S, tmx, cs, m_new, h, pf, pscale);
 
       // ---- row sums of the quantised probabilities (a column of ones) and O += P V
       if (__builtin_amdgcn_ballot_w64(alpha != 1.0f) != 0) {   // the row maxima settle after a few blocks
@@ -390,8 +350,35 @@ static int launch_attn(const AttnArgs& a, const SEQS& seqs, int B, int row_block
   return check_launch("attention_fwd");
 }
 
+// Rows of one workgroup: 32 where its waves deal out the keys (attention_split.hip), 128 where every wave walks them all.
+//
+// The split kernel takes about 1.5 times the instructions per row and key (1.0 against 0.66 us of a SIMD for 32 rows and 64 keys,
+// head dims of 128) and a quarter of the time for one row's keys, so it pays while the launch is as long as its longest rows,
+// i.e. while its workgroups, each counted as its share of the longest one (6 blocks of keys on top for what does not depend on
+// their number), are about as many as are resident at a time: 4 per compute unit with D = 64, 3 with 128, 2 above, and an
+// eighth more.  Device time, us, 128 rows / 32 rows, share of the slots in brackets:
+//   D = 128, causal: 8 heads x 1024 tokens 22.8 / 13.5 (.22), 8 x 4096 69.3 / 41.5 (.73), 12 x 4096 74.4 / 62.9 (1.1), 24 x 2048
+//   43.5 / 39.5 (1.18), 28 x 2048 44.7 / 44.1 (1.38), 32 x 2048 45.2 / 48.0 (1.58), 4 x 32 heads x 2048 108 / 156;
+//   all keys: 16 x 1024 23.2 / 15.7 (.67), 24 x 1024 25.3 / 21.7 (1.0), 28 x 1024 26.0 / 28.0 (1.17), 8 x 4096 68 / 74 (1.33);
+//   short: 32 x 256 11.8 / 9.2 (.14), 4 x 16 x 512 18.4 / 18.2 (1.0), 4 x 32 x 256 15.0 / 16.5 (1.13);
+//   D = 64: 16 x 2048 causal 36.3 / 23.0 (.59), 28 x 2048 36.8 / 33.0 (1.04), 32 x 2048 37.5 / 35.1 (1.18), 56 x 1024 23.0 / 23.7 (1.15);
+//   D = 192: 16 x 1024 causal 30.3 / 18.1 (.66), D = 256: 16 x 1024 all keys 27.6 / 23.4 (1.0), 32 x 1024 causal 30.5 / 30.6 (1.32).
+static int rows_per_workgroup(const AttnArgs& a, int64_t B, int64_t D, int n_seqs, const int32_t* cu_q, const int32_t* cu_k) {
+  if (a.bias || a.alibi || a.Sq / 32 > 65535) return 128;
+  double work = 0.0;
+  int64_t longest = 0;
+  for (int i = 0; i < (n_seqs ? n_seqs : 1); ++i) {
+    const int64_t bands = (n_seqs ? cu_q[i + 1] - cu_q[i] : a.Sq) / 32, n = ((n_seqs ? cu_k[i + 1] - cu_k[i] : a.Sk_used) + 63) / 64;
+    work += (double)bands * (double)(n + 6) - (a.causal ? 0.25 * (double)bands * (double)(bands - 1) : 0.0);   // (a causal band ends half a block before the next)
+    longest = n > longest ? n : longest;
+  }
+  const int per_cu = D == 64 ? 4 : (D == 128 ? 3 : 2);
+  return (double)B * a.Hq * work <= 288.0 * per_cu * (double)(longest + 6) ? 32 : 128;
+}
+
 template <typename SEQS>
-static int launch_attn_dims(const AttnArgs& a, const SEQS& seqs, int B, int row_blocks, int64_t D, int64_t Dv, hipStream_t st) {
+static int launch_attn_dims(const AttnArgs& a, const SEQS& seqs, int B, int row_blocks, int rows, int64_t D, int64_t Dv, hipStream_t st) {
+  if (rows == 32) return launch_attn_split(a, seqs, B, row_blocks, D, Dv, st);
   switch (D + (Dv == 128 ? 1 : 0)) {
     case 64: return launch_attn<1, 2>(a, seqs, B, row_blocks, st);
     case 65: return launch_attn<1, 4>(a, seqs, B, row_blocks, st);
@@ -442,7 +429,8 @@ extern "C" int alto_mxfp4_attention_fwd_ex(const void* q_codes, const void* q_sc
              (const uint8_t*)vt_codes, (const uint8_t*)v_scales, out, lse, Hq * Sq * Dv, Sq * Dv, Dv, Hq * Sq, Sq, 1, (int)Hq, (int)Hk, (int)Sq, (int)Sk,
              (int)Sk_used, B * Hk * Sk * (D / 2), B * Hk * Dv * (Sk / 2), sm_scale, causal ? 1 : 0,
              bias, bias_sb, bias_sh, bias_sm, bias_bytes, alibi_slopes, alibi_sb, alibi_sh};
-  return launch_attn_dims(a, AttnNoSeqs{}, (int)B, (int)((Sq + 127) / 128), D, Dv, (hipStream_t)stream);
+  const int rows = rows_per_workgroup(a, B, D, 0, nullptr, nullptr);
+  return launch_attn_dims(a, AttnNoSeqs{}, (int)B, (int)((Sq + rows - 1) / rows), rows, D, Dv, (hipStream_t)stream);
 }
 
 namespace alto {
@@ -478,7 +466,8 @@ static int attention_fwd_strided(const QueryOperand& q, const void* k_codes, con
   if (n_seqs == 0) {
     ALTO_REQUIRE(!causal || Sq <= Sk, "attention_fwd: causal attention needs Sq <= Sk (got %lld > %lld)", (long long)Sq, (long long)Sk);
     ALTO_REQUIRE((Sq + 127) / 128 <= 65535, "attention_fwd: Sq / 128 must fit a grid dimension");
-    return launch_attn_dims(a, AttnNoSeqs{}, (int)B, (int)((Sq + 127) / 128), D, Dv, st);
+    const int rows = rows_per_workgroup(a, B, D, 0, nullptr, nullptr);
+    return launch_attn_dims(a, AttnNoSeqs{}, (int)B, (int)((Sq + rows - 1) / rows), rows, D, Dv, st);
   }
   ALTO_REQUIRE(n_seqs > 0 && cu_q && cu_k && B == 1, "attention_fwd: packed sequences need their boundaries and B = 1");
   ALTO_REQUIRE(cu_q[0] == 0 && cu_k[0] == 0 && cu_q[n_seqs] == Sq && cu_k[n_seqs] == Sk, "attention_fwd: the sequence boundaries must run from 0 to the token counts");
@@ -499,19 +488,20 @@ static int attention_fwd_strided(const QueryOperand& q, const void* k_codes, con
     const int kx = cu_k[x + 1] - cu_k[x], ky = cu_k[y + 1] - cu_k[y];
     return kx != ky ? kx > ky : x < y;
   });
+  const int rows = rows_per_workgroup(a, 1, D, n_seqs, cu_q, cu_k);
   for (int at = 0; at < n_seqs;) {
     AttnSeqs t;
     t.n = 0;
     t.z0[0] = 0;
     for (; at < n_seqs && t.n < ATTN_MAX_SEQS; ++at) {
-      const int s = order[(size_t)at], qn = cu_q[s + 1] - cu_q[s], blocks = (qn + 127) / 128;
+      const int s = order[(size_t)at], qn = cu_q[s + 1] - cu_q[s], blocks = (qn + rows - 1) / rows;
       ALTO_REQUIRE(blocks <= 65535, "attention_fwd: Sq / 128 must fit a grid dimension");
       if (t.z0[t.n] + blocks > 65535) break;
       t.q0[t.n] = cu_q[s]; t.qn[t.n] = qn; t.k0[t.n] = cu_k[s]; t.kn[t.n] = cu_k[s + 1] - cu_k[s];
       t.z0[t.n + 1] = t.z0[t.n] + blocks;
       ++t.n;
     }
-    const int rc = launch_attn_dims(a, t, 1, t.z0[t.n], D, Dv, st);
+    const int rc = launch_attn_dims(a, t, 1, t.z0[t.n], rows, D, Dv, st);
     if (rc != ALTO_MXFP4_OK) return rc;
   }
   return ALTO_MXFP4_OK;
