@@ -623,6 +623,24 @@ int grouped_gemm_impl(const uint8_t* a, int64_t lda, const uint8_t* a_scales, in
 }  // namespace
 }  // namespace alto
 
+namespace alto {
+namespace {
+__global__ void offsets_kernel(const int32_t* __restrict__ ends, int n, int32_t* __restrict__ offs) {
+  const int i = (int)(blockIdx.x * 256 + threadIdx.x);
+  if (i <= n) offs[i] = i == 0 ? 0 : ends[i - 1];
+}
+}  // namespace
+}  // namespace alto
+
+extern "C" int alto_mxfp4_grouped_gemm_offsets(const int32_t* ends, int num_groups, int32_t* offs, void* stream) {
+  using namespace alto;
+  ALTO_REQUIRE(ends && offs, "grouped_gemm_offsets: NULL pointer");
+  ALTO_REQUIRE(num_groups > 0 && num_groups < (1 << 24), "grouped_gemm_offsets: number of groups (%d) out of range", num_groups);
+  ALTO_REQUIRE(((reinterpret_cast<uintptr_t>(ends) | reinterpret_cast<uintptr_t>(offs)) & 3) == 0, "grouped_gemm_offsets: pointers must be 4-byte aligned");
+  hipLaunchKernelGGL(offsets_kernel, dim3((unsigned)(num_groups / 256 + 1)), dim3(256), 0, reinterpret_cast<hipStream_t>(stream), ends, num_groups, offs);
+  return check_launch("grouped_gemm_offsets");
+}
+
 extern "C" int64_t alto_mxfp4_grouped_gemm_workspace_bytes(int64_t M_total, int num_groups) {
   if (M_total < 0 || M_total >= (1ll << 31) || num_groups < 0) return 0;   // sizes no grouped call accepts
   return alto::grouped_workspace_bytes(M_total, num_groups);

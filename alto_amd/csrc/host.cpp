@@ -13,6 +13,7 @@
 
 #include <ATen/ATen.h>
 
+#include <algorithm>
 #include <optional>
 #include <vector>
 
@@ -40,6 +41,7 @@ struct Api {
   ALTO_FN(attention_fwd_strided);
   ALTO_FN(attention_quantize_kv);
   ALTO_FN(attention_fwd_bf16q);
+  ALTO_FN(grouped_gemm_offsets);
 #undef ALTO_FN
 } api;
 py::object* check_fn = nullptr;   // _lib.check(rc, name): raises for rc != 0 (never freed: the interpreter may be gone by then)
@@ -60,6 +62,7 @@ void bind(const py::dict& address, py::object check) {
   ALTO_FN(attention_fwd_strided);
   ALTO_FN(attention_quantize_kv);
   ALTO_FN(attention_fwd_bf16q);
+  ALTO_FN(grouped_gemm_offsets);
 #undef ALTO_FN
   delete check_fn;
   check_fn = new py::object(std::move(check));
@@ -277,15 +280,317 @@ bool attend(const Tensor& q_in, const Tensor& k_in, const Tensor& v_in, double s
   return true;
 }
 
+// ------------------------------------------------------------------------------------------------- whole training directions
+// One call per direction of a layer's step: outputs, quantizers and products, with the interpreter lock given up once.  What a
+// direction needs only itself shares one buffer, what the backward needs of either operand has one of its own.  Under the
+// engine's own thread every piece of interpreter work costs twice what it does in a loop (the two threads take turns on two cores):
+// linear step of 512 x 1024 x 1024 forward 71 -> 39 us, backward 53 -> 23, the whole step 188 -> 115 (54 of them a function that does nothing).
+struct Failure {
+  int rc = 0;
+  const char* name = "";
+  bool ok(const char* what, int code) {
+    if (code != 0) { rc = code; name = what; }
+    return code == 0;
+  }
+  void raise() const {
+    if (rc != 0) (*check_fn)(rc, name);
+  }
+};
+
+int64_t pitch128(int64_t n) { return div_up(n, 128) * 128; }
+int64_t up256(int64_t n) { return div_up(n, 256) * 256; }
+int64_t packed_bytes(int64_t K, int64_t rows) { return div_up(K / 32, 16) * rows * 16; }
+
+// One of the two copies a quantizer pass makes of `batch` matrices: codes [rows][pitch of K / 2 bytes], then scales, packed or
+// [rows (/ 32)][K / 32].  Bytes of a buffer from `at` on.
+struct Copy {
+  int64_t rows = 0, K = 0, batch = 1, at = 0;
+  bool packed = false, is_2d = false;
+  int64_t ld() const { return pitch128(K / 2); }
+  int64_t scale_ld() const { return K / 32; }
+  int64_t scale_bytes() const { return packed ? packed_bytes(K, rows) : (is_2d ? rows / 32 : rows) * scale_ld(); }
+  int64_t scales_at() const { return at + up256(batch * rows * ld()); }
+  int64_t end() const { return scales_at() + up256(batch * scale_bytes() + 16); }
+  uint8_t* codes(const Tensor& buf) const { return bytes(buf) + at; }
+  uint8_t* scales(const Tensor& buf) const { return bytes(buf) + scales_at(); }
+};
+
+// [batch][M][C] with unit stride along C in whole 16-byte units, as `quantize` reads it
+bool rows_readable(const Tensor& t) {
+  if (!on_gpu(t) || !is_float(t) || t.stride(-1) != 1 || !aligned16(t)) return false;
+  const int64_t vec = t.scalar_type() == at::kBFloat16 ? 8 : 4;
+  for (int64_t d = 0; d + 1 < t.dim(); ++d)
+    if (t.size(d) != 1 && (t.stride(d) % vec != 0 || t.stride(d) < t.size(-1))) return false;
+  return true;
+}
+
+struct Hadamard {
+  int on = 0;
+  const int8_t* signs = nullptr;
+  const uint8_t* perm = nullptr;
+  Hadamard(const OptTensor& s, const OptTensor& p) {
+    on = s.has_value();
+    if (s.has_value()) signs = static_cast<const int8_t*>(s->data_ptr());
+    if (p.has_value()) perm = static_cast<const uint8_t*>(p->data_ptr());
+  }
+};
+
+// both copies of x (rows `row.rows`, columns `col.rows`); sr_mode 0 (nearest) or 3 (the hardware's stochastic converts)
+bool quantize_both(Failure& f, const Tensor& x, const Copy& row, const Tensor& row_buf, const Copy& col, const Tensor& col_buf, bool is_2d, int sr_mode, uint64_t seed,
+                   const Hadamard& h, int clip, bool uos, void* s) {
+  const int64_t B = row.batch, M = row.rows, C = col.rows, ld = M > 1 ? x.stride(-2) : C, bs = B > 1 ? x.stride(0) : M * ld;
+  const int dt = dtype_code(x.scalar_type());
+  if (sr_mode == 3 && !row.packed && !col.packed)
+    return f.ok("alto_mxfp4_quantize_sr_hw", api.quantize_sr_hw(x.data_ptr(), dt, B, M, C, ld, bs, row.codes(row_buf), row.scales(row_buf), col.codes(col_buf),
+                                                                col.scales(col_buf), row.ld(), col.ld(), (int)is_2d, seed, 0, nullptr, h.on, h.signs, h.perm, clip, (int)uos, s));
+  return f.ok("alto_mxfp4_quantize_ex",
+              api.quantize_ex(x.data_ptr(), dt, B, M, C, ld, bs, row.codes(row_buf), row.scales(row_buf), col.codes(col_buf), col.scales(col_buf), row.ld(), col.ld(),
+                              (int)is_2d, sr_mode, nullptr, 0, 0, seed, 0, nullptr, h.on, h.signs, h.perm, clip, (int)uos,
+                              (row.packed ? ALTO_QUANT_PACK_ROW_SCALES : 0) | (col.packed ? ALTO_QUANT_PACK_COL_SCALES : 0), s));
+}
+
+bool product(Failure& f, const Copy& a, const Tensor& a_buf, const Copy& b, const Tensor& b_buf, const Tensor& c, double out_scale, void* s) {
+  const int64_t N = b.rows;
+  if (a.packed)
+    return f.ok("alto_mxfp4_gemm_ps", api.gemm_ps(a.codes(a_buf), a.ld(), a.scales(a_buf), b.codes(b_buf), b.ld(), b.scales(b_buf), a.rows, N, a.K, c.data_ptr(), N,
+                                                  (float)out_scale, s));
+  return f.ok("alto_mxfp4_gemm", api.gemm(a.codes(a_buf), a.ld(), a.scales(a_buf), a.scale_ld(), 1, (int)a.is_2d, b.codes(b_buf), b.ld(), b.scales(b_buf), b.scale_ld(), 1,
+                                          (int)b.is_2d, a.rows, N, a.K, c.data_ptr(), dtype_code(c.scalar_type()), N, (float)out_scale, s));
+}
+
+// linear.py:packed_gemm_supported
+bool packed_gemm_supported(int64_t M, int64_t N, int64_t K) {
+  return M >= 128 && N >= 128 && K >= 512 && N % 8 == 0 && M * (K / 2) < (1ll << 31) && N * (K / 2) < (1ll << 31);
+}
+
+// What a linear layer's step quantizes: x [M, K] (row, col), W [N, K] (row, col), dY [M, N] (row, col)
+struct LinearCopies {
+  Copy x_row, w_row, x_col, w_col, go_row, go_col;
+  // packed: bits 0, 1, 2 = scales of the forward's, the input gradient's and the weight gradient's operands
+  LinearCopies(int64_t M, int64_t N, int64_t K, int packed) {
+    const bool f = packed & 1, d = packed & 2, w = packed & 4;
+    x_row = {M, K, 1, 0, f, false};
+    w_row = {N, K, 1, x_row.end(), f, !f};
+    x_col = {K, M, 1, 0, w, false};
+    w_col = {K, N, 1, 0, d, !d};
+    go_row = {M, N, 1, 0, d, false};
+    go_col = {N, M, 1, go_row.end(), w, false};
+  }
+};
+
+// linear.py:MXFP4LinearStep.forward -> (y, buffer of x's column copy, buffer of W's column copy, packed bits)
+py::object linear_forward(const Tensor& x_in, const Tensor& w, const OptTensor& signs, const OptTensor& perm, int clip, bool uos, bool allow_packed, uintptr_t stream) {
+  if (!on_gpu(x_in) || x_in.dim() < 2 || w.dim() != 2 || !rows_readable(w)) return py::none();
+  const int64_t N = w.size(0), K = w.size(1);
+  if (x_in.size(-1) != K || x_in.numel() == 0 || N == 0 || N % 32 != 0 || K % 32 != 0) return py::none();
+  const Tensor x = x_in.dim() == 2 ? x_in : x_in.reshape({-1, K});
+  const int64_t M = x.size(0);
+  if (M % 32 != 0 || !rows_readable(x)) return py::none();
+  int packed = 0;
+  if (allow_packed && x.scalar_type() == at::kBFloat16 && M * std::max(N, K) < (1ll << 36) && N * K < (1ll << 36))
+    packed = (int)packed_gemm_supported(M, N, K) | (int)packed_gemm_supported(M, K, N) << 1 | (int)packed_gemm_supported(N, K, M) << 2;
+  const LinearCopies c(M, N, K, packed);
+  const Hadamard h(signs, perm), none(std::nullopt, std::nullopt);
+  Tensor xs, ws, y;
+  Failure f;
+  {
+    py::gil_scoped_release nogil;
+    const Alloc a(x);
+    const Tensor tmp = a.dense({c.w_row.end()});
+    xs = a.dense({c.x_col.end()});
+    ws = a.dense({c.w_col.end()});
+    y = at::empty({M, N}, x.options());
+    void* s = reinterpret_cast<void*>(stream);
+    quantize_both(f, x, c.x_row, tmp, c.x_col, xs, false, 0, 0, h, clip, uos, s) &&
+        quantize_both(f, w, c.w_row, tmp, c.w_col, ws, true, 0, 0, none, 0, uos, s) && product(f, c.x_row, tmp, c.w_row, tmp, y, 1.0, s);
+    if (x_in.dim() != 2) {
+      auto shape = x_in.sizes().vec();
+      shape.back() = N;
+      y = y.view(shape);
+    }
+  }
+  f.raise();
+  return py::make_tuple(y, xs, ws, packed);
+}
+
+bool whole_buffer(const Tensor& t, int64_t n) { return on_gpu(t) && t.scalar_type() == at::kByte && t.dim() == 1 && t.numel() == n && t.is_contiguous() && aligned16(t); }
+
+// philox_seed_offset(None, None)[0] of _runtime.py: the same draw
+uint64_t draw_seed() { return (uint64_t)at::randint(0, INT64_MAX, {1}, at::TensorOptions().dtype(at::kLong).device(at::kCPU)).item<int64_t>(); }
+
+// linear.py:MXFP4LinearStep.backward -> (dx, dw); sr: the hardware's stochastic converts, keyed with a draw from torch's CPU generator
+py::object linear_backward(const Tensor& go_in, const Tensor& xs, const Tensor& ws, int64_t N, int64_t K, int packed, bool sr, const OptTensor& signs, const OptTensor& perm,
+                           int clip, bool uos, double out_scale, uintptr_t stream) {
+  if (!on_gpu(go_in) || go_in.dim() < 2 || go_in.size(-1) != N) return py::none();
+  const Tensor go = go_in.dim() == 2 ? go_in : go_in.reshape({-1, N});
+  const int64_t M = go.size(0);
+  const LinearCopies c(M, N, K, packed);
+  if (!rows_readable(go) || !whole_buffer(xs, c.x_col.end()) || !whole_buffer(ws, c.w_col.end())) return py::none();
+  if (packed != 0 && go.scalar_type() != at::kBFloat16) return py::none();
+  const Hadamard h(signs, perm);
+  Tensor dx, dw;
+  Failure f;
+  {
+    py::gil_scoped_release nogil;
+    const uint64_t seed = sr ? draw_seed() : 0;
+    const Tensor tmp = Alloc(go).dense({c.go_col.end()});
+    dx = at::empty({M, K}, go.options());
+    dw = at::empty({N, K}, go.options());
+    void* s = reinterpret_cast<void*>(stream);
+    quantize_both(f, go, c.go_row, tmp, c.go_col, tmp, false, sr ? 3 : 0, seed, h, clip, uos, s) && product(f, c.go_row, tmp, c.w_col, ws, dx, 1.0, s) &&
+        product(f, c.go_col, tmp, c.x_col, xs, dw, out_scale, s);
+    if (go_in.dim() != 2) {
+      auto shape = go_in.sizes().vec();
+      shape.back() = K;
+      dx = dx.view(shape);
+    }
+  }
+  f.raise();
+  return py::make_tuple(dx, dw);
+}
+
+// (a saved-tensor hook may hand a buffer back at any address)
+Tensor whole_aligned(const Tensor& t) { return t.is_contiguous() && aligned16(t) ? t : t.clone(at::MemoryFormat::Contiguous); }
+
+// The saved buffers as the four tensors that MXFP4LinearFunction saves: column codes and scales of x and of W
+py::tuple linear_saved(const Tensor& xs_in, const Tensor& ws_in, int64_t M, int64_t N, int64_t K, int packed) {
+  const LinearCopies c(M, N, K, packed);
+  const Tensor xs = whole_aligned(xs_in), ws = whole_aligned(ws_in);
+  auto codes = [](const Tensor& b, const Copy& k) { return b.as_strided({k.K / 2, k.rows}, {1, k.ld()}, b.storage_offset() + k.at); };
+  auto scales = [](const Tensor& b, const Copy& k) {
+    const int64_t o = b.storage_offset() + k.scales_at();
+    if (k.packed) return b.as_strided({div_up(k.K / 32, 16), k.rows, 16}, {k.rows * 16, 16, 1}, o);
+    return b.as_strided({k.K / 32, k.is_2d ? k.rows / 32 : k.rows}, {1, k.scale_ld()}, o);
+  };
+  return py::make_tuple(codes(xs, c.x_col), scales(xs, c.x_col), codes(ws, c.w_col), scales(ws, c.w_col));
+}
+
+// grouped_gemm.py:grouped_packed_supported and grouped_dw_packed_supported
+bool grouped_packed_supported(int64_t M, int64_t N, int64_t K, int64_t groups) {
+  const int64_t ld = div_up(K / 2, 16) * 16;
+  return M >= 128 && N >= 128 && K >= 512 && N % 8 == 0 && M * ld < (1ll << 31) && N * ld < (1ll << 31) && div_up(K / 32, 16) * std::max(M, N) * 16 < (1ll << 31) &&
+         (div_up(M, 256) + groups + 2) * div_up(N, 256) < (1ll << 28);
+}
+bool grouped_dw_packed_supported(int64_t M, int64_t N, int64_t K, int64_t groups, int64_t experts) {
+  const int64_t ld = div_up(M / 2, 16) * 16;
+  return M >= 512 && M % 32 == 0 && N >= 128 && K >= 128 && N % 8 == 0 && K % 8 == 0 && N * ld < (1ll << 31) && K * ld < (1ll << 31) && groups <= 32768 && experts <= 65535 &&
+         div_up(M, 512) * std::max(N, K) * 16 < (1ll << 31);
+}
+
+// What a grouped layer's step quantizes, all scales packed: x [M, K], dY [M, N] as above; the experts in one pass over their storage
+// ([E, N, K], or [E, K, N]): copies packed along K for the forward and along N for the input gradient
+struct GroupedCopies {
+  Copy x_row, x_col, wf, wd, go_row, go_col;
+  GroupedCopies(int64_t M, int64_t E, int64_t N, int64_t K) {
+    x_row = {M, K, 1, 0, true, false};
+    wf = {N, K, E, x_row.end(), true, true};
+    x_col = {K, M, 1, 0, true, false};
+    wd = {K, N, E, 0, true, true};
+    go_row = {M, N, 1, 0, true, false};
+    go_col = {N, M, 1, go_row.end(), true, false};
+  }
+};
+
+bool grouped_product(Failure& f, const Copy& a, const Tensor& a_buf, const Copy& w, const Tensor& w_buf, const Tensor& offs, const Tensor& plan, bool planned,
+                     const Tensor& out, void* s) {
+  return f.ok("alto_mxfp4_grouped_gemm_ps",
+              api.grouped_gemm_ps(a.codes(a_buf), a.ld(), a.scales(a_buf), w.codes(w_buf), w.rows * w.ld(), w.ld(), w.scales(w_buf), w.scale_bytes(),
+                                  static_cast<const int32_t*>(offs.data_ptr()), nullptr, (int)w.batch, (int)w.batch, a.rows, w.rows, a.K, out.data_ptr(), w.rows,
+                                  plan.data_ptr(), plan.numel(), (int)planned, s));
+}
+
+// grouped_gemm.py:MXFP4GroupedStep.forward: x [M, K] bf16, w [E, N, K] (trans) or [E, K, N], groups as offsets [E + 1] or, with `ends`, as
+// cumulative group ends [E] -> (out, buffer of x's column copy, buffer of the experts' copy along N, offsets, pass list)
+py::object grouped_forward(const Tensor& x, const Tensor& w, const Tensor& offs_in, bool ends, bool trans_weights, const OptTensor& signs, const OptTensor& perm, int clip,
+                           bool uos, uintptr_t stream) {
+  if (x.dim() != 2 || w.dim() != 3 || !rows_readable(x) || !rows_readable(w) || x.scalar_type() != at::kBFloat16 || !x.is_contiguous() || !w.is_contiguous()) return py::none();
+  if (!on_gpu(offs_in) || offs_in.dim() != 1 || offs_in.scalar_type() != at::kInt || !offs_in.is_contiguous()) return py::none();
+  const int64_t M = x.size(0), E = w.size(0), N = w.size(trans_weights ? 1 : 2), K = w.size(trans_weights ? 2 : 1);
+  if (x.size(1) != K || offs_in.numel() != E + !ends || M == 0 || E == 0 || N % 32 != 0 || K % 32 != 0) return py::none();
+  if (M * std::max(N, K) >= (1ll << 36) || N * K >= (1ll << 36) || !grouped_packed_supported(M, N, K, E) || !grouped_packed_supported(M, K, N, E) ||
+      !grouped_dw_packed_supported(M, N, K, E, E))
+    return py::none();
+  const GroupedCopies c(M, E, N, K);
+  const Hadamard h(signs, perm), none(std::nullopt, std::nullopt);
+  Tensor xs, ws, out, offs = offs_in, plan;
+  Failure f;
+  {
+    py::gil_scoped_release nogil;
+    const Alloc a(x);
+    void* s = reinterpret_cast<void*>(stream);
+    const Tensor tmp = a.dense({c.wf.end()});
+    xs = a.dense({c.x_col.end()});
+    ws = a.dense({c.wd.end()});
+    out = at::empty({M, N}, x.options());
+    plan = a.dense({api.grouped_gemm_workspace_bytes(M, (int)E)});
+    bool ok = true;
+    if (ends) {
+      offs = at::empty({E + 1}, offs_in.options());
+      ok = f.ok("alto_mxfp4_grouped_gemm_offsets", api.grouped_gemm_offsets(static_cast<const int32_t*>(offs_in.data_ptr()), (int)E, static_cast<int32_t*>(offs.data_ptr()), s));
+    }
+    ok = ok && quantize_both(f, x, c.x_row, tmp, c.x_col, xs, false, 0, 0, h, clip, uos, s);
+    ok = ok && (trans_weights ? quantize_both(f, w, c.wf, tmp, c.wd, ws, true, 0, 0, none, 0, uos, s) : quantize_both(f, w, c.wd, ws, c.wf, tmp, true, 0, 0, none, 0, uos, s));
+    ok = ok && grouped_product(f, c.x_row, tmp, c.wf, tmp, offs, plan, false, out, s);
+  }
+  f.raise();
+  return py::make_tuple(out, xs, ws, offs, plan);
+}
+
+// grouped_gemm.py:MXFP4GroupedStep.backward -> (dx, dw)
+py::object grouped_backward(const Tensor& go, const Tensor& xs, const Tensor& ws, const Tensor& offs, const Tensor& plan, int64_t E, int64_t N, int64_t K, bool trans_weights,
+                            bool sr, const OptTensor& signs, const OptTensor& perm, int clip, bool uos, double out_scale, uintptr_t stream) {
+  if (go.dim() != 2 || go.size(1) != N || !rows_readable(go) || go.scalar_type() != at::kBFloat16 || !go.is_contiguous()) return py::none();
+  const int64_t M = go.size(0);
+  const GroupedCopies c(M, E, N, K);
+  if (!whole_buffer(xs, c.x_col.end()) || !whole_buffer(ws, c.wd.end()) || !whole_buffer(plan, api.grouped_gemm_workspace_bytes(M, (int)E))) return py::none();
+  if (!on_gpu(offs) || offs.scalar_type() != at::kInt || offs.numel() != E + 1 || !offs.is_contiguous()) return py::none();
+  const Hadamard h(signs, perm);
+  Tensor dx, dw;
+  Failure f;
+  {
+    py::gil_scoped_release nogil;
+    const uint64_t seed = sr ? draw_seed() : 0;
+    void* s = reinterpret_cast<void*>(stream);
+    const Tensor tmp = Alloc(go).dense({c.go_col.end()});
+    dx = at::empty({M, K}, go.options());
+    dw = trans_weights ? at::empty({E, N, K}, go.options()) : at::empty({E, K, N}, go.options());
+    quantize_both(f, go, c.go_row, tmp, c.go_col, tmp, false, sr ? 3 : 0, seed, h, clip, uos, s) &&
+        grouped_product(f, c.go_row, tmp, c.wd, ws, offs, plan, true, dx, s) &&
+        f.ok("alto_mxfp4_grouped_gemm_dw_ps",
+             api.grouped_gemm_dw_ps(c.go_col.codes(tmp), c.go_col.ld(), c.go_col.scales(tmp), c.x_col.codes(xs), c.x_col.ld(), c.x_col.scales(xs),
+                                    static_cast<const int32_t*>(offs.data_ptr()), nullptr, (int)E, (int)E, M, N, K, dw.data_ptr(), dw.stride(0),
+                                    trans_weights ? dw.stride(1) : dw.stride(2), trans_weights ? dw.stride(2) : dw.stride(1), (float)out_scale, s));
+  }
+  f.raise();
+  return py::make_tuple(dx, dw);
+}
+
+// The saved buffers as the four tensors that MXFP4GroupedGEMM saves: token-packed codes and scales of x, codes [E, K, N / 2] and scales of W
+py::tuple grouped_saved(const Tensor& xs_in, const Tensor& ws_in, int64_t M, int64_t E, int64_t N, int64_t K) {
+  const GroupedCopies c(M, E, N, K);
+  const Tensor xs = whole_aligned(xs_in), ws = whole_aligned(ws_in);
+  const Copy &x = c.x_col, &w = c.wd;
+  const int64_t xo = xs.storage_offset(), wo = ws.storage_offset();
+  return py::make_tuple(xs.as_strided({M / 2, K}, {1, x.ld()}, xo + x.at), xs.as_strided({div_up(M / 32, 16), K, 16}, {K * 16, 16, 1}, xo + x.scales_at()),
+                        ws.as_strided({E, K, N / 2}, {K * w.ld(), w.ld(), 1}, wo + w.at),
+                        ws.as_strided({E, div_up(N / 32, 16), K, 16}, {w.scale_bytes(), K * 16, 16, 1}, wo + w.scales_at()));
+}
+
 // hadamard.py:HadamardFactory.create_transform: the same two draws (randint in the factory's dtype, then randperm) as int8
 // signs and uint8 positions
 py::tuple draw_hadamard(const std::optional<at::Generator>& gen, at::ScalarType dtype) {
   const auto cpu = at::TensorOptions().device(at::kCPU);
-  const Tensor q = at::randint(0, 2, {32}, gen, cpu.dtype(dtype)).to(at::kDouble), p = at::randperm(32, gen, cpu.dtype(at::kLong));
+  Tensor q = at::randint(0, 2, {32}, gen, cpu.dtype(dtype));
+  const Tensor p = at::randperm(32, gen, cpu.dtype(at::kLong));
+  if (dtype != at::kFloat) q = q.to(at::kFloat);   // (zeros and ones)
   const Tensor signs = at::empty({32}, cpu.dtype(at::kChar)), perm = at::empty({32}, cpu.dtype(at::kByte));
+  const float* qv = q.data_ptr<float>();
+  const int64_t* pv = p.data_ptr<int64_t>();
+  int8_t* sv = signs.data_ptr<int8_t>();
+  uint8_t* mv = perm.data_ptr<uint8_t>();
   for (int i = 0; i < 32; ++i) {
-    signs.data_ptr<int8_t>()[i] = q.data_ptr<double>()[i] != 0.0 ? 1 : -1;
-    perm.data_ptr<uint8_t>()[i] = (uint8_t)p.data_ptr<int64_t>()[i];
+    sv[i] = qv[i] != 0.0f ? 1 : -1;
+    mv[i] = (uint8_t)pv[i];
   }
   return py::make_tuple(signs, perm);
 }
@@ -301,5 +606,11 @@ PYBIND11_MODULE(alto_mxfp4_host, m) {
   m.def("grouped_packed", &grouped_packed);
   m.def("grouped_dw_packed", &grouped_dw_packed);
   m.def("attend", &attend);
+  m.def("linear_forward", &linear_forward);
+  m.def("linear_backward", &linear_backward);
+  m.def("linear_saved", &linear_saved);
+  m.def("grouped_forward", &grouped_forward);
+  m.def("grouped_backward", &grouped_backward);
+  m.def("grouped_saved", &grouped_saved);
   m.def("draw_hadamard", &draw_hadamard);
 }

@@ -82,6 +82,11 @@ def hardware_stochastic_rounding(use_asm: Optional[bool] = None) -> bool:
     return bool(use_asm)
 
 
+def host_keyed_hardware_rounding() -> bool:
+    """True when a call without options of its own rounds with the hardware converts, keyed with a draw from torch's CPU generator."""
+    return _hw_rounding_default and _rand_source is None and not _device_state_on
+
+
 def philox_in_kernel() -> bool:
     """True when the quantizer may draw its random words itself (no source installed with ``set_rand_bits_source``)."""
     return _rand_source is None

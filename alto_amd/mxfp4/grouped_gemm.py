@@ -19,7 +19,7 @@ import torch
 from . import _runtime as rt
 from .._lib import check
 from .hadamard import HadamardFactory, HadamardTransform
-from .linear import _wgrad_scale, cached_weight_quantisation, packed_scales_enabled, transpose_codes, unwrap_weight_wrapper
+from .linear import _wgrad_scale, cached_weight_quantisation, packed_scales_enabled, transpose_codes, unwrap_weight_wrapper, weight_cache_enabled
 from .quantization import quantize_rowcol
 
 ALIGN_SIZE_M = 128
@@ -312,30 +312,75 @@ class MXFP4GroupedGEMM(torch.autograd.Function):
     @staticmethod
     def backward(ctx, grad_output):
         a_qm, a_sm, wq_kn, ws_kn, g_offs, g_expert, plan = ctx.saved_tensors
-        groups = Groups(g_offs, g_expert, ctx.num_groups)
-        go = grad_output if grad_output.is_contiguous() else grad_output.contiguous()
-        sr = bool(ctx.use_sr_grad)
-        # random words: made inside the quantizer (Philox) unless a source of explicit words is installed
-        rand = rt.draw_rand_bits(go.shape, go.device) if (sr and not rt.philox_in_kernel()) else None
-        pk_d, pk_w = ctx.packed_dx, ctx.packed_dw
-        if ctx.use_2dblock_x:
-            go_q, go_s, go_qm, go_sm = quantize_rowcol(go, True, use_sr=sr, rand_bits=rand, use_uos=ctx.use_uos, pad_codes=True, pack_row_scales=pk_d,
-                                                       pack_col_scales=pk_w)
-        else:
-            go_q, go_s, go_qm, go_sm = quantize_rowcol(go, False, use_sr=sr, rand_bits=rand, hadamard=ctx.hadamard_transform,
-                                                       clip_mode=ctx.clip_mode, use_uos=ctx.use_uos, pad_codes=True, pack_row_scales=pk_d, pack_col_scales=pk_w)
-        if pk_d:
-            grad_inputs = grouped_forward_packed(go_q, go_s, wq_kn, ws_kn, groups, plan=plan)
-        else:
-            grad_inputs = grouped_forward(go_q, go_s, wq_kn, ws_kn, groups, ctx.use_2dblock_x, ctx.use_2dblock_w, ctx.original_dtype, plan=plan)
-        if pk_w:
-            grad_weights = grouped_dw_packed(go_qm.transpose(0, 1), go_sm, a_qm.transpose(0, 1), a_sm, groups, ctx.num_experts, ctx.trans_weights,
-                                             _wgrad_scale(ctx.clip_mode, ctx.use_dge))
-        else:
-            grad_weights = grouped_dw(go_qm.transpose(0, 1), go_sm.transpose(0, 1), a_qm.transpose(0, 1), a_sm.transpose(0, 1),
-                                      groups, ctx.num_experts, ctx.original_dtype, ctx.trans_weights,
-                                      _wgrad_scale(ctx.clip_mode, ctx.use_dge), is_2d=ctx.use_2dblock_x)
-        return (grad_inputs, grad_weights) + (None,) * 11
+        return _grouped_backward(grad_output, (a_qm, a_sm, wq_kn, ws_kn), Groups(g_offs, g_expert, ctx.num_groups), plan, (ctx.packed_dx, ctx.packed_dw), ctx.num_experts,
+                                 ctx.trans_weights, ctx.use_2dblock_x, ctx.use_2dblock_w, ctx.original_dtype, bool(ctx.use_sr_grad), ctx.hadamard_transform,
+                                 ctx.clip_mode, ctx.use_uos, ctx.use_dge) + (None,) * 11
+
+
+def _grouped_backward(grad_output, saved, groups, plan, packed, num_experts, trans_weights, use_2dblock_x, use_2dblock_w, original_dtype, sr,
+                      hadamard_transform, clip_mode, use_uos, use_dge):
+    a_qm, a_sm, wq_kn, ws_kn = saved
+    go = grad_output if grad_output.is_contiguous() else grad_output.contiguous()
+    # random words: made inside the quantizer (Philox) unless a source of explicit words is installed
+    rand = rt.draw_rand_bits(go.shape, go.device) if (sr and not rt.philox_in_kernel()) else None
+    pk_d, pk_w = packed
+    if use_2dblock_x:
+        go_q, go_s, go_qm, go_sm = quantize_rowcol(go, True, use_sr=sr, rand_bits=rand, use_uos=use_uos, pad_codes=True, pack_row_scales=pk_d,
+                                                   pack_col_scales=pk_w)
+    else:
+        go_q, go_s, go_qm, go_sm = quantize_rowcol(go, False, use_sr=sr, rand_bits=rand, hadamard=hadamard_transform,
+                                                   clip_mode=clip_mode, use_uos=use_uos, pad_codes=True, pack_row_scales=pk_d, pack_col_scales=pk_w)
+    if pk_d:
+        grad_inputs = grouped_forward_packed(go_q, go_s, wq_kn, ws_kn, groups, plan=plan)
+    else:
+        grad_inputs = grouped_forward(go_q, go_s, wq_kn, ws_kn, groups, use_2dblock_x, use_2dblock_w, original_dtype, plan=plan)
+    if pk_w:
+        grad_weights = grouped_dw_packed(go_qm.transpose(0, 1), go_sm, a_qm.transpose(0, 1), a_sm, groups, num_experts, trans_weights,
+                                         _wgrad_scale(clip_mode, use_dge))
+    else:
+        grad_weights = grouped_dw(go_qm.transpose(0, 1), go_sm.transpose(0, 1), a_qm.transpose(0, 1), a_sm.transpose(0, 1),
+                                  groups, num_experts, original_dtype, trans_weights,
+                                  _wgrad_scale(clip_mode, use_dge), is_2d=use_2dblock_x)
+    return grad_inputs, grad_weights
+
+
+@torch.compiler.allow_in_graph
+class MXFP4GroupedStep(MXFP4GroupedGEMM):
+    """:class:`MXFP4GroupedGEMM` for the everyday call (groups by offsets, or by their ends with ``ends``; 1D activation blocks, 2D weight
+    blocks, bf16, no dynamic clip, no weight cache): the same launches and results with one native call per direction.  What
+    those decline takes the general function's way."""
+
+    @staticmethod
+    def forward(ctx, inputs, expert_weights, offsets, ends, trans_weights, use_sr_grad, use_dge, clip_mode, hadamard_transform, use_uos):
+        h = hadamard_transform
+        w = unwrap_weight_wrapper(expert_weights)
+        res = rt.host().grouped_forward(inputs, w, offsets, ends, bool(trans_weights), None if h is None else h.signs, None if h is None else h.perm,
+                                        rt.CLIP[clip_mode], bool(use_uos), rt.stream_ptr(inputs.device)) if inputs.is_cuda and packed_scales_enabled() else None
+        ctx.step = None
+        if res is None:
+            return MXFP4GroupedGEMM.forward(ctx, inputs, expert_weights, None, trans_weights, False, True, use_sr_grad, use_dge, clip_mode, False, h, use_uos,
+                                            offsets_from_ends(offsets) if ends else offsets)
+        out, *saved = res
+        ctx.save_for_backward(*saved)
+        ctx.step = (w.shape[0], out.shape[1], inputs.shape[1])
+        ctx.options = (bool(trans_weights), bool(use_sr_grad), h, clip_mode, bool(use_uos), bool(use_dge))
+        return out
+
+    @staticmethod
+    def backward(ctx, grad_output):
+        if ctx.step is None:
+            return MXFP4GroupedGEMM.backward(ctx, grad_output)[:2] + (None,) * 8
+        E, N, K = ctx.step
+        trans_weights, sr, h, clip_mode, uos, dge = ctx.options
+        x_saved, w_saved, offs, plan = ctx.saved_tensors
+        res = None
+        if not sr or rt.host_keyed_hardware_rounding():
+            res = rt.host().grouped_backward(grad_output, x_saved, w_saved, offs, plan, E, N, K, trans_weights, sr, None if h is None else h.signs,
+                                             None if h is None else h.perm, rt.CLIP[clip_mode], uos, _wgrad_scale(clip_mode, dge), rt.stream_ptr(grad_output.device))
+        if res is None:
+            res = _grouped_backward(grad_output, rt.host().grouped_saved(x_saved, w_saved, grad_output.shape[0], E, N, K), Groups(offs, None, E), plan, (True, True), E,
+                                    trans_weights, False, True, torch.bfloat16, sr, h, clip_mode, uos, dge)
+        return (*res, None, None, None, None, None, None, None, None)
 
 
 def _quantize_experts(owner: torch.Tensor, w: torch.Tensor, is_2d: bool, use_uos: bool, pack_rows: bool = False, pack_cols: bool = False):
@@ -351,6 +396,11 @@ def _quantize_experts(owner: torch.Tensor, w: torch.Tensor, is_2d: bool, use_uos
                                                              pack_row_scales=pack_rows, pack_col_scales=pack_cols))
 
 
+def _everyday(use_2dblock_x, use_2dblock_w, clip_mode, use_macro_block_scaling) -> bool:
+    """What :class:`MXFP4GroupedStep` takes."""
+    return bool(use_2dblock_w) and clip_mode in ("none", "static") and not (use_2dblock_x or use_macro_block_scaling or weight_cache_enabled())
+
+
 def mxfp4_grouped_gemm(inputs, expert_weights, expert_indices, *, trans_weights=True, use_2dblock_x=False, use_2dblock_w=True,
                        use_sr_grad=False, use_dge=False, use_hadamard=False, clip_mode="none", use_macro_block_scaling=False,
                        use_uos=False, offsets: Optional[torch.Tensor] = None) -> torch.Tensor:
@@ -363,6 +413,8 @@ def mxfp4_grouped_gemm(inputs, expert_weights, expert_indices, *, trans_weights=
     if expert_indices is not None and expert_indices.dtype != torch.int32:
         expert_indices = expert_indices.to(torch.int32)
     hadamard_transform = HadamardFactory.create_transform(device=expert_weights.device) if use_hadamard else None
+    if offsets is not None and _everyday(use_2dblock_x, use_2dblock_w, clip_mode, use_macro_block_scaling):
+        return MXFP4GroupedStep.apply(inputs, expert_weights, offsets, False, trans_weights, use_sr_grad, use_dge, clip_mode, hadamard_transform, use_uos)
     return MXFP4GroupedGEMM.apply(inputs, expert_weights, expert_indices, trans_weights, use_2dblock_x, use_2dblock_w, use_sr_grad,
                                   use_dge, clip_mode, use_macro_block_scaling, hadamard_transform, use_uos, offsets)
 
@@ -370,6 +422,9 @@ def mxfp4_grouped_gemm(inputs, expert_weights, expert_indices, *, trans_weights=
 def _quantize_then_mxfp_scaled_grouped_mm(A, B, offs, use_2dblock_x, use_2dblock_w, use_sr_grad, use_dge, use_hadamard, clip_mode,
                                           use_macro_block_scaling, use_uos=False) -> torch.Tensor:
     """``torch._grouped_mm(A, B, offs=offs)`` replacement (functional.py:11-38): B is [E, K, N], offs are group ends."""
+    if _everyday(use_2dblock_x, use_2dblock_w, clip_mode, use_macro_block_scaling):
+        h = HadamardFactory.create_transform(device=B.device) if use_hadamard else None
+        return MXFP4GroupedStep.apply(A, B, offs, True, False, use_sr_grad, use_dge, clip_mode, h, use_uos)
     return mxfp4_grouped_gemm(A, B, None, trans_weights=False, use_2dblock_x=use_2dblock_x, use_2dblock_w=use_2dblock_w,
                               use_sr_grad=use_sr_grad, use_dge=use_dge, use_hadamard=use_hadamard, clip_mode=clip_mode,
                               use_macro_block_scaling=use_macro_block_scaling, use_uos=use_uos, offsets=offsets_from_ends(offs))

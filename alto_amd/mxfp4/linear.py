@@ -49,6 +49,10 @@ def enable_weight_cache(enabled: bool = True) -> None:
         clear_weight_cache()
 
 
+def weight_cache_enabled() -> bool:
+    return _WEIGHT_CACHE_ENABLED
+
+
 def clear_weight_cache() -> None:
     _WEIGHT_CACHE.clear()
     _WEIGHT_CACHE_STATS["hits"] = _WEIGHT_CACHE_STATS["misses"] = 0
@@ -319,38 +323,79 @@ class MXFP4LinearFunction(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, grad_output):
-        original_shape = grad_output.shape
-        go = grad_output.reshape(-1, original_shape[-1])
-        x_qm, x_sm, w_bwd, w_bwd_s = ctx.saved_tensors
-        pk_d, pk_w = ctx.packed
-        sr = bool(ctx.use_sr_grad)
-        # random words: made inside the quantizer (Philox) unless a source of explicit words is installed
-        rand = rt.draw_rand_bits(go.shape, go.device) if (sr and not rt.philox_in_kernel()) else None
-        if ctx.use_2dblock_x:
-            go_q, go_s = convert_to_mxfp4(go, axis=-1, is_2d_block=True, use_sr=sr, rand_bits=rand, use_uos=ctx.use_uos)
-            go_qm, go_sm = go_q, go_s
-        else:
-            go_q, go_s, go_qm, go_sm = quantize_rowcol(go, False, use_sr=sr, rand_bits=rand, hadamard=ctx.hadamard_transform,
-                                                       clip_mode=ctx.clip_mode, use_uos=ctx.use_uos, pad_codes=True,
-                                                       pack_row_scales=pk_d, pack_col_scales=pk_w)
-        # dgrad: reduction over N.  The saved weight operand is already packed along N (both layouts of a 2D-block
-        # quantisation hold the same codes), so no k_pack=False repack is needed here.
-        if pk_d:
-            grad_inputs = gemm_packed(_k_major(go_q), go_s, _k_major(w_bwd.transpose(0, 1)), w_bwd_s)
-        else:
-            grad_inputs = blockwise_mxfp4_gemm(go_q, go_s, w_bwd, w_bwd_s, use_2dblock_a=ctx.use_2dblock_x,
-                                               use_2dblock_b=ctx.use_2dblock_w, k_pack_b=True, output_dtype=ctx.original_dtype)
-        # wgrad: reduction over tokens
-        if pk_w:
-            grad_weights = gemm_packed(_k_major(go_qm.transpose(0, 1)), go_sm, _k_major(x_qm.transpose(0, 1)), x_sm,
-                                       out_scale=_wgrad_scale(ctx.clip_mode, ctx.use_dge))
-        else:
-            grad_weights = blockwise_mxfp4_gemm(go_qm, go_sm, x_qm, x_sm, use_2dblock_a=ctx.use_2dblock_x,
-                                                use_2dblock_b=ctx.use_2dblock_x, trans_a=True,
-                                                k_pack_a=not ctx.use_2dblock_x, k_pack_b=not ctx.use_2dblock_x,
-                                                output_dtype=ctx.original_dtype,
-                                                out_scale=_wgrad_scale(ctx.clip_mode, ctx.use_dge))
-        return grad_inputs.view(*original_shape[:-1], -1), grad_weights, None, None, None, None, None, None, None, None
+        return _linear_backward(grad_output, ctx.saved_tensors, ctx.packed, ctx.use_2dblock_x, ctx.use_2dblock_w, ctx.original_dtype, bool(ctx.use_sr_grad),
+                                ctx.hadamard_transform, ctx.clip_mode, ctx.use_uos, ctx.use_dge)
+
+
+def _linear_backward(grad_output, saved, packed, use_2dblock_x, use_2dblock_w, original_dtype, sr, hadamard_transform, clip_mode, use_uos, use_dge):
+    original_shape = grad_output.shape
+    go = grad_output.reshape(-1, original_shape[-1])
+    x_qm, x_sm, w_bwd, w_bwd_s = saved
+    pk_d, pk_w = packed
+    # random words: made inside the quantizer (Philox) unless a source of explicit words is installed
+    rand = rt.draw_rand_bits(go.shape, go.device) if (sr and not rt.philox_in_kernel()) else None
+    if use_2dblock_x:
+        go_q, go_s = convert_to_mxfp4(go, axis=-1, is_2d_block=True, use_sr=sr, rand_bits=rand, use_uos=use_uos)
+        go_qm, go_sm = go_q, go_s
+    else:
+        go_q, go_s, go_qm, go_sm = quantize_rowcol(go, False, use_sr=sr, rand_bits=rand, hadamard=hadamard_transform,
+                                                   clip_mode=clip_mode, use_uos=use_uos, pad_codes=True,
+                                                   pack_row_scales=pk_d, pack_col_scales=pk_w)
+    # dgrad: reduction over N.  The saved weight operand is already packed along N (both layouts of a 2D-block
+    # quantisation hold the same codes), so no k_pack=False repack is needed here.
+    if pk_d:
+        grad_inputs = gemm_packed(_k_major(go_q), go_s, _k_major(w_bwd.transpose(0, 1)), w_bwd_s)
+    else:
+        grad_inputs = blockwise_mxfp4_gemm(go_q, go_s, w_bwd, w_bwd_s, use_2dblock_a=use_2dblock_x,
+                                           use_2dblock_b=use_2dblock_w, k_pack_b=True, output_dtype=original_dtype)
+    # wgrad: reduction over tokens
+    if pk_w:
+        grad_weights = gemm_packed(_k_major(go_qm.transpose(0, 1)), go_sm, _k_major(x_qm.transpose(0, 1)), x_sm,
+                                   out_scale=_wgrad_scale(clip_mode, use_dge))
+    else:
+        grad_weights = blockwise_mxfp4_gemm(go_qm, go_sm, x_qm, x_sm, use_2dblock_a=use_2dblock_x,
+                                            use_2dblock_b=use_2dblock_x, trans_a=True,
+                                            k_pack_a=not use_2dblock_x, k_pack_b=not use_2dblock_x,
+                                            output_dtype=original_dtype,
+                                            out_scale=_wgrad_scale(clip_mode, use_dge))
+    return grad_inputs.view(*original_shape[:-1], -1), grad_weights, None, None, None, None, None, None, None, None
+
+
+@torch.compiler.allow_in_graph
+class MXFP4LinearStep(MXFP4LinearFunction):
+    """:class:`MXFP4LinearFunction` for the everyday call (1D activation blocks, 2D weight blocks, no dynamic clip, no weight cache):
+    the same launches and results with one native call per direction.  What those decline takes the general function's way."""
+
+    @staticmethod
+    def forward(ctx, x, weight, use_2dblock_x, use_2dblock_w, use_sr_grad, use_dge, clip_mode, use_macro_block_scaling,
+                hadamard_transform: Optional[HadamardTransform] = None, use_uos: bool = False):
+        h = hadamard_transform
+        res = rt.host().linear_forward(x, unwrap_weight_wrapper(weight), None if h is None else h.signs, None if h is None else h.perm, rt.CLIP[clip_mode],
+                                       bool(use_uos), _PACKED_SCALES, rt.stream_ptr(x.device)) if x.is_cuda else None
+        ctx.step = None
+        if res is None:
+            return MXFP4LinearFunction.forward(ctx, x, weight, use_2dblock_x, use_2dblock_w, use_sr_grad, use_dge, clip_mode, use_macro_block_scaling, h, use_uos)
+        y, x_saved, w_saved, packed = res
+        ctx.save_for_backward(x_saved, w_saved)
+        ctx.step = (*weight.shape, packed)
+        ctx.original_dtype = x.dtype
+        ctx.options = (bool(use_sr_grad), h, clip_mode, bool(use_uos), bool(use_dge))
+        return y
+
+    @staticmethod
+    def backward(ctx, grad_output):
+        if ctx.step is None:
+            return MXFP4LinearFunction.backward(ctx, grad_output)
+        N, K, packed = ctx.step
+        sr, h, clip_mode, uos, dge = ctx.options
+        x_saved, w_saved = ctx.saved_tensors
+        if grad_output.dtype is ctx.original_dtype and (not sr or rt.host_keyed_hardware_rounding()):
+            res = rt.host().linear_backward(grad_output, x_saved, w_saved, N, K, packed, sr, None if h is None else h.signs, None if h is None else h.perm,
+                                            rt.CLIP[clip_mode], uos, _wgrad_scale(clip_mode, dge), rt.stream_ptr(grad_output.device))
+            if res is not None:
+                return (*res, None, None, None, None, None, None, None, None)
+        return _linear_backward(grad_output, rt.host().linear_saved(x_saved, w_saved, grad_output.numel() // N, N, K, packed), (bool(packed & 2), bool(packed & 4)),
+                                False, True, ctx.original_dtype, sr, h, clip_mode, uos, dge)
 
 
 def _to_mxfp4_then_scaled_mm(
@@ -367,5 +412,6 @@ def _to_mxfp4_then_scaled_mm(
 ) -> torch.Tensor:
     """``a @ b.T`` through ``MXFP4LinearFunction`` with a fresh random Hadamard per call (mxfp_linear.py:573-602)."""
     hadamard_transform = HadamardFactory.create_transform(device=b.device) if use_hadamard else None
-    return MXFP4LinearFunction.apply(a, b, use_2dblock_x, use_2dblock_w, use_sr_grad, use_dge, clip_mode,
+    everyday = use_2dblock_w and clip_mode in ("none", "static") and not (use_2dblock_x or use_macro_block_scaling or _WEIGHT_CACHE_ENABLED)
+    return (MXFP4LinearStep if everyday else MXFP4LinearFunction).apply(a, b, use_2dblock_x, use_2dblock_w, use_sr_grad, use_dge, clip_mode,
                                      use_macro_block_scaling, hadamard_transform, use_uos)

@@ -320,6 +320,12 @@ int alto_mxfp4_grouped_gemm_ps(const uint8_t* a, int64_t lda, const uint8_t* a_p
                                void* workspace, int64_t workspace_bytes, int plan_built, void* stream);
 
 /*
+ * Cumulative group ends (the convention of torch._grouped_mm) to the offsets the grouped entries take: offs[0] = 0, offs[g + 1] =
+ * ends[g] for g < num_groups.
+ */
+int alto_mxfp4_grouped_gemm_offsets(const int32_t* ends, int num_groups, int32_t* offs, void* stream);
+
+/*
  * Per-device set-up that the entry points otherwise do on first use: resolves, for the CURRENT device, the address of the
  * library's built-in pass-list array.  Call it once per device (with that device current) before capturing a HIP graph
  * that contains alto_mxfp4_grouped_gemm_noalloc.  Idempotent, thread-safe, allocates nothing.  No counterpart in the

@@ -292,6 +292,8 @@ Entry g_bf16q_entries[] = {
      [](const Args& a) { return call_bf16q(a, nullptr); }},
     {"attention_fwd_bf16q_packed", 16, 2, 7, {{1, 8, 2, 256, 288, 128, 64, 0, 64, 512, 0, 1, 8, 0, 128, 1024}, {0, 1}, {D, D, D, D, D, D, D}, 0.088388f, {0, 0}, g_signs, g_perm},
      [](const Args& a) { return call_bf16q(a, &g_bounds[(unsigned)a.i[0] % (kManySequences + 1)]); }},
+    {"grouped_gemm_offsets", 0, 1, 2, {{}, {32}, {D, D}, 1.0f, {0, 0}, g_signs, g_perm},
+     [](const Args& a) { return alto_mxfp4_grouped_gemm_offsets(P(const int32_t, 0), a.i[0], P(int32_t, 1), nullptr); }},
 };
 constexpr int kBf16qEntries = sizeof(g_bf16q_entries) / sizeof(g_bf16q_entries[0]);
 

@@ -1,0 +1,184 @@
+"""A layer's training step in one native call per direction against the general autograd functions: the same launches on the same
+operands, so outputs and gradients are the same bit for bit, with the same draws from torch's CPU generator."""
+import pytest
+import torch
+
+from tests.helpers import hadamard_from_seed, randn_outliers
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+@pytest.fixture(scope="module")
+def m():
+    import alto_amd.mxfp4 as mod
+    assert torch.cuda.is_available()
+    return mod
+
+
+def _same(got, want, what=""):
+    for a, b, name in zip(got, want, ("y", "dx", "dw")):
+        assert a.shape == b.shape and a.dtype == b.dtype and torch.equal(a, b), (what, name)
+
+
+def _linear(fn, x, w, go, h, clip="none", sr=True, uos=False, dge=False, seed=5):
+    torch.manual_seed(seed)
+    xg, wg = x.detach().requires_grad_(True), w.detach().requires_grad_(True)
+    y = fn.apply(xg, wg, False, True, sr, dge, clip, False, h, uos)
+    dx, dw = torch.autograd.grad(y, (xg, wg), go)
+    return y.detach(), dx, dw, torch.randint(0, 2 ** 62, (1,))
+
+
+# packed scales for all three products, for some, for none (below 128 rows, 512 K, N % 8); direct, few-row, small-tile and large-tile kernels
+SHAPES = [(512, 768, 1024), (256, 160, 544), (96, 256, 512), (128, 512, 160), (32, 32, 32), (1376, 2144, 2880), (2304, 2560, 512), (64, 96, 1056)]
+
+
+@pytest.mark.parametrize("M,N,K", SHAPES)
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("clip,uos,dge,sr,had", [("none", False, False, True, True), ("static", False, True, True, False), ("none", True, False, False, True)])
+def test_linear_step_equals_the_general_function(m, M, N, K, dtype, clip, uos, dge, sr, had):
+    from alto_amd.mxfp4.linear import MXFP4LinearStep
+    x, w = randn_outliers((M, K), dtype, seed=1).to(DEV), randn_outliers((N, K), dtype, seed=2).to(DEV)
+    go = (randn_outliers((M, N), dtype, seed=3) / (M * N)).to(DEV)
+    h = m.HadamardTransform(*hadamard_from_seed(11)) if had else None
+    a, b = (_linear(f, x, w, go, h, clip, sr, uos, dge) for f in (MXFP4LinearStep, m.MXFP4LinearFunction))
+    _same(a[:3], b[:3])
+    assert torch.equal(a[3], b[3])   # as many words taken from the generator
+
+
+def test_linear_step_operand_forms(m):
+    """Three-dimensional and strided activations, a strided weight, expanded and strided gradients, an fp32 weight under bf16
+    activations: taken, or declined and then served by the general function; a token count off the blocks of 32 is refused by both."""
+    from alto_amd.mxfp4.linear import MXFP4LinearStep
+    M, N, K = 256, 160, 544
+    big = randn_outliers((M, 2 * K), torch.bfloat16, seed=4).to(DEV)
+    w = randn_outliers((N, K), torch.bfloat16, seed=2).to(DEV)
+    go = (randn_outliers((M, N), torch.bfloat16, seed=3) / M).to(DEV)
+    h = m.HadamardTransform(*hadamard_from_seed(3))
+    xs = {"3d": big[:, :K].contiguous().view(4, 64, K), "rows strided": big[:, 8:K + 8], "off alignment": big[:, 1:K + 1], "columns strided": big[:, ::2],
+          "transposed": big[:, :K].contiguous().t().contiguous().t()}
+    for name, x in xs.items():
+        g = go.view(*x.shape[:-1], N)
+        _same(_linear(MXFP4LinearStep, x, w, g, h)[:3], _linear(m.MXFP4LinearFunction, x, w, g, h)[:3], name)
+    x = xs["rows strided"]
+    for name, g in {"expanded": go[:1, :1].expand(M, N), "transposed": go.t().contiguous().t()}.items():
+        _same(_linear(MXFP4LinearStep, x, w, g, h)[:3], _linear(m.MXFP4LinearFunction, x, w, g, h)[:3], name)
+    for name, ww in {"strided": torch.nn.functional.pad(w, (8, 8))[:, 8:K + 8], "transposed": w.t().contiguous().t(), "fp32": w.float()}.items():
+        _same(_linear(MXFP4LinearStep, x, ww, go, h)[:3], _linear(m.MXFP4LinearFunction, x, ww, go, h)[:3], name)
+    for fn in (MXFP4LinearStep, m.MXFP4LinearFunction):   # (the weight gradient's operand has blocks of 32 tokens)
+        with pytest.raises(RuntimeError):
+            fn.apply(x[:40], w, False, True, False, False, "none", False, None, False)
+
+
+def test_linear_step_saved_tensor_hooks_modes_and_repeats(m):
+    """Saved buffers that went through host memory; another rounding source than the forward saw; two backward passes over one graph."""
+    from alto_amd.mxfp4.linear import MXFP4LinearStep
+    x, w = randn_outliers((256, 544), torch.bfloat16, seed=1).to(DEV), randn_outliers((160, 544), torch.bfloat16, seed=2).to(DEV)
+    go = (randn_outliers((256, 160), torch.bfloat16, seed=3) / 256).to(DEV)
+    h = m.HadamardTransform(*hadamard_from_seed(5))
+    with torch.autograd.graph.save_on_cpu():
+        a = _linear(MXFP4LinearStep, x, w, go, h)
+    _same(a[:3], _linear(m.MXFP4LinearFunction, x, w, go, h)[:3], "saved on the host")
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: t, lambda t: torch.cat([t.new_zeros(3), t])[3:]):   # back at an odd address
+        a = _linear(MXFP4LinearStep, x, w, go, h)
+    _same(a[:3], _linear(m.MXFP4LinearFunction, x, w, go, h)[:3], "saved off alignment")
+    m.use_hardware_stochastic_rounding(False)
+    try:
+        _same(_linear(MXFP4LinearStep, x, w, go, h)[:3], _linear(m.MXFP4LinearFunction, x, w, go, h)[:3], "software rounding")
+    finally:
+        m.use_hardware_stochastic_rounding(True)
+    r = torch.randint(-2 ** 31, 2 ** 31, (256, 160), dtype=torch.int64).to(torch.int32).to(DEV)
+    m.set_rand_bits_source(lambda shape, d: r)
+    try:
+        _same(_linear(MXFP4LinearStep, x, w, go, h)[:3], _linear(m.MXFP4LinearFunction, x, w, go, h)[:3], "words from a source")
+    finally:
+        m.set_rand_bits_source(None)
+    m.enable_device_philox_state(seed=9)
+    try:
+        a = _linear(MXFP4LinearStep, x, w, go, h)
+        m.enable_device_philox_state(seed=9)
+        _same(a[:3], _linear(m.MXFP4LinearFunction, x, w, go, h)[:3], "device state")
+    finally:
+        m.enable_device_philox_state(False)
+    xg, wg = x.clone().requires_grad_(True), w.clone().requires_grad_(True)
+    y = MXFP4LinearStep.apply(xg, wg, False, True, False, False, "none", False, h, False)
+    first = torch.autograd.grad(y, (xg, wg), go, retain_graph=True)
+    _same(torch.autograd.grad(y, (xg, wg), go), first, "again")
+
+
+def _grouped(m, fn, x, w, go, offs, trans, seed=5, **kw):
+    from alto_amd.mxfp4 import grouped_gemm as G
+    torch.manual_seed(seed)
+    h = m.HadamardTransform(*hadamard_from_seed(7)) if kw.get("had", True) else None
+    sr, dge, clip, uos = kw.get("sr", True), kw.get("dge", False), kw.get("clip", "none"), kw.get("uos", False)
+    xg, wg = x.detach().requires_grad_(True), w.detach().requires_grad_(True)
+    if fn == "step":
+        out = G.MXFP4GroupedStep.apply(xg, wg, offs, False, trans, sr, dge, clip, h, uos)
+    elif fn == "ends":
+        out = G.MXFP4GroupedStep.apply(xg, wg, offs[1:].contiguous() if kw.get("dense", True) else offs[1:].long(), True, trans, sr, dge, clip, h, uos)
+    else:
+        out = G.MXFP4GroupedGEMM.apply(xg, wg, None, trans, False, True, sr, dge, clip, False, h, uos, offs)
+    dx, dw = torch.autograd.grad(out, (xg, wg), go)
+    return out.detach(), dx, dw, torch.randint(0, 2 ** 62, (1,))
+
+
+@pytest.mark.parametrize("N,K", [(768, 1280), (512, 2880), (288, 512), (128, 96)])
+@pytest.mark.parametrize("trans", [True, False])
+@pytest.mark.parametrize("kw", [{}, dict(clip="static", dge=True, had=False), dict(uos=True, sr=False)], ids=["sr", "static", "uos"])
+def test_grouped_step_equals_the_general_function(m, N, K, trans, kw):
+    offs = torch.tensor([0, 96, 96, 800, 832, 1024], dtype=torch.int32, device=DEV)   # ragged groups, one empty
+    x = randn_outliers((1024, K), torch.bfloat16, seed=31).to(DEV)
+    w = randn_outliers((5, N, K) if trans else (5, K, N), torch.bfloat16, seed=32).to(DEV)
+    go = (randn_outliers((1024, N), torch.bfloat16, seed=34) / (1024 * N)).to(DEV)
+    ref = _grouped(m, "general", x, w, go, offs, trans, **kw)
+    for fn, more in (("step", {}), ("ends", {}), ("ends", dict(dense=False))):
+        got = _grouped(m, fn, x, w, go, offs, trans, **kw, **more)
+        _same(got[:3], ref[:3], (fn, more))
+        assert torch.equal(got[3], ref[3])
+
+
+def test_grouped_step_forms_and_hooks(m):
+    """Row counts below the packed kernels' 512, fp32 and strided operands (declined), gradients that are expanded, saved buffers through
+    host memory, software rounding in the backward."""
+    N, K = 288, 512
+    offs = torch.tensor([0, 96, 800, 1024], dtype=torch.int32, device=DEV)
+    x = randn_outliers((1024, K), torch.bfloat16, seed=31).to(DEV)
+    w = randn_outliers((3, N, K), torch.bfloat16, seed=32).to(DEV)
+    go = (randn_outliers((1024, N), torch.bfloat16, seed=34) / 1024).to(DEV)
+    both = lambda *a, **k: (_grouped(m, "step", *a, **k)[:3], _grouped(m, "general", *a, **k)[:3])
+    for name, args in {"fp32": (x.float(), w.float(), go.float(), offs), "strided": (torch.nn.functional.pad(x, (8, 8))[:, 8:K + 8], w, go, offs),
+                       "expanded": (x, w, go[:1, :1].expand(1024, N), offs), "few rows": (x[:256], w, go[:256], (offs / 4).int() // 32 * 32)}.items():
+        _same(*both(*args, True), name)
+    ref = _grouped(m, "general", x, w, go, offs, True)
+    with torch.autograd.graph.save_on_cpu():
+        _same(_grouped(m, "step", x, w, go, offs, True)[:3], ref[:3], "saved on the host")
+    m.use_hardware_stochastic_rounding(False)
+    try:
+        _same(*both(x, w, go, offs, True), "software rounding")
+    finally:
+        m.use_hardware_stochastic_rounding(True)
+
+
+def test_steps_run_on_the_callers_stream_and_replay(m):
+    """A linear forward and backward captured into a graph and replayed with new values (round to nearest: no draw is frozen in)."""
+    from alto_amd.mxfp4.linear import MXFP4LinearStep
+    x, w = randn_outliers((256, 544), torch.bfloat16, seed=1).to(DEV), randn_outliers((160, 544), torch.bfloat16, seed=2).to(DEV)
+    go = (randn_outliers((256, 160), torch.bfloat16, seed=3) / 256).to(DEV)
+    h = m.HadamardTransform(*hadamard_from_seed(5))
+    def step():
+        xg, wg = x.detach().requires_grad_(True), w.detach().requires_grad_(True)
+        y = MXFP4LinearStep.apply(xg, wg, False, True, False, False, "none", False, h, False)
+        return (y.detach(), *torch.autograd.grad(y, (xg, wg), go))
+    s = torch.cuda.Stream()
+    s.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(s):
+        step()
+    torch.cuda.current_stream().wait_stream(s)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        got = step()
+    for seed in (7, 8, 9):
+        x.copy_(randn_outliers((256, 544), torch.bfloat16, seed=seed).to(DEV))
+        graph.replay()
+        _same([t.clone() for t in got], step(), seed)
