@@ -42,6 +42,7 @@ struct Api {
   ALTO_FN(attention_quantize_kv);
   ALTO_FN(attention_fwd_bf16q);
   ALTO_FN(grouped_gemm_offsets);
+  ALTO_FN(quantize_operands);
 #undef ALTO_FN
 } api;
 py::object* check_fn = nullptr;   // _lib.check(rc, name): raises for rc != 0 (never freed: the interpreter may be gone by then)
@@ -63,6 +64,7 @@ void bind(const py::dict& address, py::object check) {
   ALTO_FN(attention_quantize_kv);
   ALTO_FN(attention_fwd_bf16q);
   ALTO_FN(grouped_gemm_offsets);
+  ALTO_FN(quantize_operands);
 #undef ALTO_FN
   delete check_fn;
   check_fn = new py::object(std::move(check));
@@ -335,18 +337,30 @@ struct Hadamard {
   }
 };
 
-// both copies of x (rows `row.rows`, columns `col.rows`); sr_mode 0 (nearest) or 3 (the hardware's stochastic converts)
-bool quantize_both(Failure& f, const Tensor& x, const Copy& row, const Tensor& row_buf, const Copy& col, const Tensor& col_buf, bool is_2d, int sr_mode, uint64_t seed,
-                   const Hadamard& h, int clip, bool uos, void* s) {
-  const int64_t B = row.batch, M = row.rows, C = col.rows, ld = M > 1 ? x.stride(-2) : C, bs = B > 1 ? x.stride(0) : M * ld;
+// both copies of a gradient [row.rows, col.rows], 1D blocks; sr_mode 0 (nearest) or 3 (the hardware's stochastic converts)
+bool quantize_gradient(Failure& f, const Tensor& x, const Copy& row, const Tensor& row_buf, const Copy& col, const Tensor& col_buf, int sr_mode, uint64_t seed,
+                       const Hadamard& h, int clip, bool uos, void* s) {
+  const int64_t M = row.rows, C = col.rows, ld = M > 1 ? x.stride(-2) : C, bs = M * ld;
   const int dt = dtype_code(x.scalar_type());
   if (sr_mode == 3 && !row.packed && !col.packed)
-    return f.ok("alto_mxfp4_quantize_sr_hw", api.quantize_sr_hw(x.data_ptr(), dt, B, M, C, ld, bs, row.codes(row_buf), row.scales(row_buf), col.codes(col_buf),
-                                                                col.scales(col_buf), row.ld(), col.ld(), (int)is_2d, seed, 0, nullptr, h.on, h.signs, h.perm, clip, (int)uos, s));
+    return f.ok("alto_mxfp4_quantize_sr_hw", api.quantize_sr_hw(x.data_ptr(), dt, 1, M, C, ld, bs, row.codes(row_buf), row.scales(row_buf), col.codes(col_buf),
+                                                                col.scales(col_buf), row.ld(), col.ld(), 0, seed, 0, nullptr, h.on, h.signs, h.perm, clip, (int)uos, s));
   return f.ok("alto_mxfp4_quantize_ex",
-              api.quantize_ex(x.data_ptr(), dt, B, M, C, ld, bs, row.codes(row_buf), row.scales(row_buf), col.codes(col_buf), col.scales(col_buf), row.ld(), col.ld(),
-                              (int)is_2d, sr_mode, nullptr, 0, 0, seed, 0, nullptr, h.on, h.signs, h.perm, clip, (int)uos,
+              api.quantize_ex(x.data_ptr(), dt, 1, M, C, ld, bs, row.codes(row_buf), row.scales(row_buf), col.codes(col_buf), col.scales(col_buf), row.ld(), col.ld(),
+                              0, sr_mode, nullptr, 0, 0, seed, 0, nullptr, h.on, h.signs, h.perm, clip, (int)uos,
                               (row.packed ? ALTO_QUANT_PACK_ROW_SCALES : 0) | (col.packed ? ALTO_QUANT_PACK_COL_SCALES : 0), s));
+}
+
+// both copies of x (1D blocks) and of W (2D blocks), round to nearest; w_row / w_col: the copies along W's columns and along its rows
+bool quantize_operands(Failure& f, const Tensor& x, const Copy& x_row, const Tensor& x_row_buf, const Copy& x_col, const Tensor& x_col_buf, const Hadamard& h, int clip,
+                       const Tensor& w, const Copy& w_row, const Tensor& w_row_buf, const Copy& w_col, const Tensor& w_col_buf, bool uos, void* s) {
+  const int64_t M = x_row.rows, K = x_col.rows, B = w_row.batch, R = w_row.rows, C = w_col.rows, ld_w = R > 1 ? w.stride(-2) : C;
+  auto flags = [](const Copy& r, const Copy& c) { return (r.packed ? ALTO_QUANT_PACK_ROW_SCALES : 0) | (c.packed ? ALTO_QUANT_PACK_COL_SCALES : 0); };
+  return f.ok("alto_mxfp4_quantize_operands",
+              api.quantize_operands(x.data_ptr(), dtype_code(x.scalar_type()), M, K, M > 1 ? x.stride(-2) : K, x_row.codes(x_row_buf), x_row.scales(x_row_buf),
+                                    x_col.codes(x_col_buf), x_col.scales(x_col_buf), x_row.ld(), x_col.ld(), h.on, h.signs, h.perm, clip, flags(x_row, x_col), w.data_ptr(),
+                                    dtype_code(w.scalar_type()), B, R, C, ld_w, B > 1 ? w.stride(0) : R * ld_w, w_row.codes(w_row_buf), w_row.scales(w_row_buf),
+                                    w_col.codes(w_col_buf), w_col.scales(w_col_buf), w_row.ld(), w_col.ld(), flags(w_row, w_col), (int)uos, s));
 }
 
 bool product(Failure& f, const Copy& a, const Tensor& a_buf, const Copy& b, const Tensor& b_buf, const Tensor& c, double out_scale, void* s) {
@@ -390,7 +404,7 @@ py::object linear_forward(const Tensor& x_in, const Tensor& w, const OptTensor& 
   if (allow_packed && x.scalar_type() == at::kBFloat16 && M * std::max(N, K) < (1ll << 36) && N * K < (1ll << 36))
     packed = (int)packed_gemm_supported(M, N, K) | (int)packed_gemm_supported(M, K, N) << 1 | (int)packed_gemm_supported(N, K, M) << 2;
   const LinearCopies c(M, N, K, packed);
-  const Hadamard h(signs, perm), none(std::nullopt, std::nullopt);
+  const Hadamard h(signs, perm);
   Tensor xs, ws, y;
   Failure f;
   {
@@ -401,8 +415,7 @@ py::object linear_forward(const Tensor& x_in, const Tensor& w, const OptTensor& 
     ws = a.dense({c.w_col.end()});
     y = at::empty({M, N}, x.options());
     void* s = reinterpret_cast<void*>(stream);
-    quantize_both(f, x, c.x_row, tmp, c.x_col, xs, false, 0, 0, h, clip, uos, s) &&
-        quantize_both(f, w, c.w_row, tmp, c.w_col, ws, true, 0, 0, none, 0, uos, s) && product(f, c.x_row, tmp, c.w_row, tmp, y, 1.0, s);
+    quantize_operands(f, x, c.x_row, tmp, c.x_col, xs, h, clip, w, c.w_row, tmp, c.w_col, ws, uos, s) && product(f, c.x_row, tmp, c.w_row, tmp, y, 1.0, s);
     if (x_in.dim() != 2) {
       auto shape = x_in.sizes().vec();
       shape.back() = N;
@@ -437,7 +450,7 @@ py::object linear_backward(const Tensor& go_in, const Tensor& xs, const Tensor& 
     dx = at::empty({M, K}, go.options());
     dw = at::empty({N, K}, go.options());
     void* s = reinterpret_cast<void*>(stream);
-    quantize_both(f, go, c.go_row, tmp, c.go_col, tmp, false, sr ? 3 : 0, seed, h, clip, uos, s) && product(f, c.go_row, tmp, c.w_col, ws, dx, 1.0, s) &&
+    quantize_gradient(f, go, c.go_row, tmp, c.go_col, tmp, sr ? 3 : 0, seed, h, clip, uos, s) && product(f, c.go_row, tmp, c.w_col, ws, dx, 1.0, s) &&
         product(f, c.go_col, tmp, c.x_col, xs, dw, out_scale, s);
     if (go_in.dim() != 2) {
       auto shape = go_in.sizes().vec();
@@ -511,7 +524,7 @@ py::object grouped_forward(const Tensor& x, const Tensor& w, const Tensor& offs_
       !grouped_dw_packed_supported(M, N, K, E, E))
     return py::none();
   const GroupedCopies c(M, E, N, K);
-  const Hadamard h(signs, perm), none(std::nullopt, std::nullopt);
+  const Hadamard h(signs, perm);
   Tensor xs, ws, out, offs = offs_in, plan;
   Failure f;
   {
@@ -528,8 +541,8 @@ py::object grouped_forward(const Tensor& x, const Tensor& w, const Tensor& offs_
       offs = at::empty({E + 1}, offs_in.options());
       ok = f.ok("alto_mxfp4_grouped_gemm_offsets", api.grouped_gemm_offsets(static_cast<const int32_t*>(offs_in.data_ptr()), (int)E, static_cast<int32_t*>(offs.data_ptr()), s));
     }
-    ok = ok && quantize_both(f, x, c.x_row, tmp, c.x_col, xs, false, 0, 0, h, clip, uos, s);
-    ok = ok && (trans_weights ? quantize_both(f, w, c.wf, tmp, c.wd, ws, true, 0, 0, none, 0, uos, s) : quantize_both(f, w, c.wd, ws, c.wf, tmp, true, 0, 0, none, 0, uos, s));
+    ok = ok && (trans_weights ? quantize_operands(f, x, c.x_row, tmp, c.x_col, xs, h, clip, w, c.wf, tmp, c.wd, ws, uos, s)
+                              : quantize_operands(f, x, c.x_row, tmp, c.x_col, xs, h, clip, w, c.wd, ws, c.wf, tmp, uos, s));
     ok = ok && grouped_product(f, c.x_row, tmp, c.wf, tmp, offs, plan, false, out, s);
   }
   f.raise();
@@ -554,7 +567,7 @@ py::object grouped_backward(const Tensor& go, const Tensor& xs, const Tensor& ws
     const Tensor tmp = Alloc(go).dense({c.go_col.end()});
     dx = at::empty({M, K}, go.options());
     dw = trans_weights ? at::empty({E, N, K}, go.options()) : at::empty({E, K, N}, go.options());
-    quantize_both(f, go, c.go_row, tmp, c.go_col, tmp, false, sr ? 3 : 0, seed, h, clip, uos, s) &&
+    quantize_gradient(f, go, c.go_row, tmp, c.go_col, tmp, sr ? 3 : 0, seed, h, clip, uos, s) &&
         grouped_product(f, c.go_row, tmp, c.wd, ws, offs, plan, true, dx, s) &&
         f.ok("alto_mxfp4_grouped_gemm_dw_ps",
              api.grouped_gemm_dw_ps(c.go_col.codes(tmp), c.go_col.ld(), c.go_col.scales(tmp), c.x_col.codes(xs), c.x_col.ld(), c.x_col.scales(xs),

@@ -110,8 +110,21 @@ __device__ __forceinline__ float round_to_T(float v) {
 // 16-byte pieces of a 128-byte line of every column's codes and stores whole lines, eight columns per wave instruction,
 // instead of one piece of 64 different lines per instruction).
 // STREAM: loads of x, row-code stores and (BPW = 8) column-code stores are non-temporal.
-template <typename T, bool DO_ROW, bool DO_COL, int SR, bool RHT, bool B2D, bool GEN, int BPW = 1, bool STREAM = false>
-__global__ __launch_bounds__(256) void quant_kernel(const QuantParams p) {
+// The tile of one workgroup in LDS (`smem` of quant_tile).
+template <typename T, bool DO_COL, int SR, bool RHT, bool B2D>
+struct QuantTile {
+  // the column phase of the hardware mode brings its transformed values back to row order through a private strip per
+  // thread (17 dwords of bf16 pairs or 33 dwords of fp32: odd pitches, conflict-free), which reuses the tile's memory
+  static constexpr int STRIP = sizeof(T) == 2 ? 17 : 33;
+  // the column phase hands the hardware converts two rows at a time (stochastic mode with 1D blocks, round to nearest always)
+  static constexpr bool PAIRS = (SR == 3 && !B2D) || SR == 0;
+  static constexpr int BYTES = !DO_COL ? 8 * (int)sizeof(T) : ((PAIRS && RHT) ? 256 * STRIP * 4 : 32 * TILE_C * (int)sizeof(T));
+};
+
+// One workgroup's tile(s): `wg` counts the workgroups of a launch with a column output (others take their place from the grid),
+// `bz` the matrices of a batch.
+template <typename T, bool DO_ROW, bool DO_COL, int SR, bool RHT, bool B2D, bool GEN, int BPW, bool STREAM>
+__device__ __forceinline__ void quant_tile(const QuantParams& p, unsigned wg, unsigned bz, uint8_t* smem) {
   static_assert(BPW == 1 || (BPW == 8 && DO_COL && B2D), "bands per workgroup: 1, or 8 for the column output of 2D blocks");
   constexpr bool BF = sizeof(T) == 2;
   constexpr int NT = STREAM ? 2 : 0;   // cache policy operand of the buffer instructions
@@ -126,13 +139,10 @@ __global__ __launch_bounds__(256) void quant_kernel(const QuantParams p) {
   constexpr bool DEFER_FLIP = RHT && DO_COL && !HW;   // the Hadamard signs go onto the finished column codes
   constexpr bool XCODES = HW && B2D && DO_COL;   // 2D blocks: the column packing takes the row phase's codes through LDS
   constexpr int OOB = (int)0x80000000;
-  // the column phase of the hardware mode brings its transformed values back to row order through a private strip per
-  // thread (17 dwords of bf16 pairs or 33 dwords of fp32: odd pitches, conflict-free), which reuses the tile's memory
-  constexpr int STRIP = BF ? 17 : 33;
-  // the column phase hands the hardware converts two rows at a time (stochastic mode with 1D blocks, round to nearest always)
-  constexpr bool PAIRS = (HW && !B2D) || SR == 0;
-  constexpr int TILE_ELEMS = !DO_COL ? 8 : ((PAIRS && RHT) ? (256 * STRIP * 4 + (int)sizeof(T) - 1) / (int)sizeof(T) : 32 * TILE_C);
-  __shared__ __align__(16) T tile[TILE_ELEMS];
+  constexpr int STRIP = QuantTile<T, DO_COL, SR, RHT, B2D>::STRIP;
+  constexpr bool PAIRS = QuantTile<T, DO_COL, SR, RHT, B2D>::PAIRS;
+  constexpr int TILE_BYTES = QuantTile<T, DO_COL, SR, RHT, B2D>::BYTES;
+  T* tile = reinterpret_cast<T*>(smem);
   __shared__ __align__(8) uint8_t xcodes[XCODES ? 32 * TILE_C : 8];
   __shared__ __align__(16) uint32_t stash[STASH ? 32 * TILE_C : 4];
   __shared__ uint32_t blkmax[8];
@@ -150,7 +160,7 @@ __global__ __launch_bounds__(256) void quant_kernel(const QuantParams p) {
   const int nby = (M + 31) >> 5;
   int bx, by0;   // column tile; first band of this workgroup
   if constexpr (DO_COL) {
-    const unsigned wg = blockIdx.x, us = (unsigned)p.unit_shift;
+    const unsigned us = (unsigned)p.unit_shift;
     const unsigned unit = (wg >> (3 + us)) * 8 + (wg & 7), tiles_x = (unsigned)(C + TILE_C - 1) / TILE_C;
     bx = (int)(unit % tiles_x);
     by0 = (int)(((unit / tiles_x) << us) + ((wg >> 3) & ((1u << us) - 1))) * BPW;
@@ -160,7 +170,7 @@ __global__ __launch_bounds__(256) void quant_kernel(const QuantParams p) {
     by0 = (int)blockIdx.y;
   }
   const int col0 = bx * TILE_C;
-  const int64_t b = blockIdx.z;
+  const int64_t b = bz;
 
   if (RHT || B2D) {
     if (tid < 32) sperm[tid] = (uint8_t)((p.perm4[tid >> 2] >> (8 * (tid & 3))) & 0xFFu);
@@ -629,7 +639,7 @@ __global__ __launch_bounds__(256) void quant_kernel(const QuantParams p) {
     // XORed with the column so that neighbouring columns spread over the banks), then lane l of a wave takes piece l % 8
     // of column l / 8: one store instruction covers 8 columns x 128 bytes.
     uint4* stage = reinterpret_cast<uint4*>(tile);
-    static_assert(sizeof(tile) >= 128 * BPW * 16, "the column-code staging reuses the tile");
+    static_assert(TILE_BYTES >= 128 * BPW * 16, "the column-code staging reuses the tile");
     const __amdgpu_buffer_rsrc_t rsrc_cc = __builtin_amdgcn_make_buffer_rsrc(
         p.col_codes + (b * C + col0) * p.ld_cc + by0 * 16, 0, 0x7FFFFFFF, 0x00020000);
     const int first = BPW - bands_done;   // pieces below this index hold nothing
@@ -651,6 +661,26 @@ __global__ __launch_bounds__(256) void quant_kernel(const QuantParams p) {
                                                (ccol < C && q >= first) ? (half * 128 + cl) * (int)p.ld_cc + (q - first) * 16 : OOB, 0, NT);
       }
     }
+  }
+}
+
+template <typename T, bool DO_ROW, bool DO_COL, int SR, bool RHT, bool B2D, bool GEN, int BPW = 1, bool STREAM = false>
+__global__ __launch_bounds__(256) void quant_kernel(const QuantParams p) {
+  __shared__ __align__(16) uint8_t smem[QuantTile<T, DO_COL, SR, RHT, B2D>::BYTES];
+  quant_tile<T, DO_ROW, DO_COL, SR, RHT, B2D, GEN, BPW, STREAM>(p, blockIdx.x, blockIdx.z, smem);
+}
+
+// Both operands of a product in one launch, both copies of each, round to nearest: the activation's workgroups (1D blocks; a multiple
+// of 8 of them, so that the second operand's meet the XCDs in the same order), then those of the weight matrices (2D blocks).
+template <typename T, bool RHT, bool GEN>
+__global__ __launch_bounds__(256) void quant_operands_kernel(const QuantParams x, const QuantParams w, unsigned x_wgs, unsigned w_wgs) {
+  constexpr int X = QuantTile<T, true, 0, RHT, false>::BYTES, W = QuantTile<T, true, 0, false, true>::BYTES;
+  __shared__ __align__(16) uint8_t smem[X > W ? X : W];
+  if (blockIdx.x < x_wgs) {
+    quant_tile<T, true, true, 0, RHT, false, GEN, 1, false>(x, blockIdx.x, 0, smem);
+  } else {
+    const unsigned i = blockIdx.x - x_wgs;
+    quant_tile<T, true, true, 0, false, true, false, 1, false>(w, i % w_wgs, i / w_wgs, smem);
   }
 }
 
@@ -825,13 +855,21 @@ namespace {
 // one-thread kernel: moves the counter of a device-resident Philox state past the blocks a quantizer call consumed
 __global__ void philox_advance_kernel(uint64_t* state, uint64_t blocks) { state[1] += blocks; }
 
+// A quantizer call past its checks: what to launch.
+struct QuantCall {
+  QuantParams p;
+  dim3 grid;
+  int dtype, sr;
+  bool empty, do_row, do_col, rht, is_2d, gen, bpw8, streaming;
+};
+
 // sr_mode: 0 round to nearest even, 1 stochastic with the words in rand_bits, 2 stochastic with Philox words made in the kernel,
 // 3 stochastic with the hardware converts (dwords cut from Philox words made in the kernel)
-int quantize_impl(const void* x, int dtype, int64_t batch, int64_t M, int64_t C, int64_t ld_x, int64_t bs_x,
+int plan_quantize(QuantCall& q, const void* x, int dtype, int64_t batch, int64_t M, int64_t C, int64_t ld_x, int64_t bs_x,
                   uint8_t* row_codes, uint8_t* row_scales, uint8_t* col_codes, uint8_t* col_scales,
                   int64_t ld_row_codes, int64_t ld_col_codes, int is_2d, int sr_mode,
                   const uint32_t* rand_bits, int64_t ld_rand, int64_t bs_rand, uint64_t seed, uint64_t offset, const uint64_t* philox_state,
-                  int hadamard, const int8_t* signs, const uint8_t* perm, int clip_mode, int use_uos, void* stream, int flags = 0) {
+                  int hadamard, const int8_t* signs, const uint8_t* perm, int clip_mode, int use_uos, int flags) {
   if (ld_row_codes == 0) ld_row_codes = C / 2;
   if (ld_col_codes == 0) ld_col_codes = M / 2;
   ALTO_REQUIRE(row_codes == nullptr || (ld_row_codes >= C / 2 && ld_row_codes % 4 == 0), "quantize: ld_row_codes must be >= C/2 and a multiple of 4 bytes");
@@ -868,21 +906,10 @@ int quantize_impl(const void* x, int dtype, int64_t batch, int64_t M, int64_t C,
     ALTO_REQUIRE(((reinterpret_cast<uintptr_t>(pack_rs ? row_scales : nullptr) | reinterpret_cast<uintptr_t>(pack_cs ? col_scales : nullptr)) & 15) == 0,
                  "quantize: packed scales must be 16-byte aligned");
   }
-  if (batch == 0 || M == 0 || C == 0) return ALTO_MXFP4_OK;
-  if (clip_mode == ALTO_CLIP_DYNAMIC) {   // std-based scale: separate plain kernel, quantisation along the contiguous dim
-    ALTO_REQUIRE(do_row && !do_col && !hadamard,
-                 "quantize: clip_mode=dynamic gives the row output only (no column output, no Hadamard); transpose on the host");
-    if (sr_mode >= 2) {
-      set_error("quantize: clip_mode=dynamic takes its random words from a tensor (fill one with alto_mxfp4_random_bits)");
-      return ALTO_MXFP4_ENOTIMPL;
-    }
-    ALTO_REQUIRE(ld_row_codes % 16 == 0, "quantize: clip_mode=dynamic needs 16-byte aligned code rows");
-    ALTO_REQUIRE((M + 31) / 32 <= 65535, "quantize: M (%lld) exceeds 65535 row blocks", (long long)M);
-    return quantize_dynamic_launch(x, dtype, batch, M, C, ld_x, bs_x, row_codes, row_scales, ld_row_codes, is_2d, sr_mode == 1,
-                                   rand_bits, ld_rand, bs_rand, use_uos, reinterpret_cast<hipStream_t>(stream));
-  }
+  q.empty = batch == 0 || M == 0 || C == 0;
+  if (q.empty || clip_mode == ALTO_CLIP_DYNAMIC) return ALTO_MXFP4_OK;
 
-  QuantParams p;
+  QuantParams& p = q.p;
   p.x = x; p.ld_x = ld_x; p.bs_x = bs_x; p.M = (int)M; p.C = (int)C;
   p.rand = rand_bits; p.ld_r = ld_rand; p.bs_r = bs_rand;
   p.seed = seed; p.ctr0 = offset; p.philox_state = philox_state;
@@ -932,11 +959,60 @@ int quantize_impl(const void* x, int dtype, int64_t batch, int64_t M, int64_t C,
   while (us > us_min && padded(us) * 20 > tiles_x * wrows * 21) --us;
   p.unit_shift = us;
   ALTO_REQUIRE(do_col ? padded(us) < (1ll << 31) : (tiles_x < (1ll << 31) && bands <= 65535), "quantize: %lld x %lld exceeds the grid", (long long)M, (long long)C);
-  const dim3 grid = do_col ? dim3((unsigned)padded(us), 1, (unsigned)batch) : dim3((unsigned)tiles_x, (unsigned)bands, (unsigned)batch);
-  hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-  if (dtype == ALTO_DT_BF16) dispatch<__bf16>(p, grid, st, do_row, do_col, hadamard != 0, is_2d != 0, sr_mode, gen, bpw8, streaming);
-  else dispatch<float>(p, grid, st, do_row, do_col, hadamard != 0, is_2d != 0, sr_mode, gen, bpw8, streaming);
+  q.grid = do_col ? dim3((unsigned)padded(us), 1, (unsigned)batch) : dim3((unsigned)tiles_x, (unsigned)bands, (unsigned)batch);
+  q.dtype = dtype; q.sr = sr_mode;
+  q.do_row = do_row; q.do_col = do_col; q.rht = hadamard != 0; q.is_2d = is_2d != 0; q.gen = gen; q.bpw8 = bpw8; q.streaming = streaming;
+  return ALTO_MXFP4_OK;
+}
+
+void launch_quantize(const QuantCall& q, hipStream_t st) {
+  if (q.dtype == ALTO_DT_BF16) dispatch<__bf16>(q.p, q.grid, st, q.do_row, q.do_col, q.rht, q.is_2d, q.sr, q.gen, q.bpw8, q.streaming);
+  else dispatch<float>(q.p, q.grid, st, q.do_row, q.do_col, q.rht, q.is_2d, q.sr, q.gen, q.bpw8, q.streaming);
+}
+
+int quantize_impl(const void* x, int dtype, int64_t batch, int64_t M, int64_t C, int64_t ld_x, int64_t bs_x,
+                  uint8_t* row_codes, uint8_t* row_scales, uint8_t* col_codes, uint8_t* col_scales,
+                  int64_t ld_row_codes, int64_t ld_col_codes, int is_2d, int sr_mode,
+                  const uint32_t* rand_bits, int64_t ld_rand, int64_t bs_rand, uint64_t seed, uint64_t offset, const uint64_t* philox_state,
+                  int hadamard, const int8_t* signs, const uint8_t* perm, int clip_mode, int use_uos, void* stream, int flags = 0) {
+  QuantCall q;
+  const int rc = plan_quantize(q, x, dtype, batch, M, C, ld_x, bs_x, row_codes, row_scales, col_codes, col_scales, ld_row_codes, ld_col_codes, is_2d, sr_mode, rand_bits,
+                               ld_rand, bs_rand, seed, offset, philox_state, hadamard, signs, perm, clip_mode, use_uos, flags);
+  if (rc != ALTO_MXFP4_OK || q.empty) return rc;
+  if (clip_mode == ALTO_CLIP_DYNAMIC) {   // std-based scale: separate plain kernel, quantisation along the contiguous dim
+    ALTO_REQUIRE(row_codes && !col_codes && !hadamard,
+                 "quantize: clip_mode=dynamic gives the row output only (no column output, no Hadamard); transpose on the host");
+    if (sr_mode >= 2) {
+      set_error("quantize: clip_mode=dynamic takes its random words from a tensor (fill one with alto_mxfp4_random_bits)");
+      return ALTO_MXFP4_ENOTIMPL;
+    }
+    if (ld_row_codes == 0) ld_row_codes = C / 2;
+    ALTO_REQUIRE(ld_row_codes % 16 == 0, "quantize: clip_mode=dynamic needs 16-byte aligned code rows");
+    ALTO_REQUIRE((M + 31) / 32 <= 65535, "quantize: M (%lld) exceeds 65535 row blocks", (long long)M);
+    return quantize_dynamic_launch(x, dtype, batch, M, C, ld_x, bs_x, row_codes, row_scales, ld_row_codes, is_2d, sr_mode == 1,
+                                   rand_bits, ld_rand, bs_rand, use_uos, reinterpret_cast<hipStream_t>(stream));
+  }
+
+  launch_quantize(q, reinterpret_cast<hipStream_t>(stream));
   return check_launch("quantize");
+}
+
+// Both operands of a product: one launch wherever both run with one band a workgroup and through the caches.  What bounds small
+// operands is not memory but the launches themselves and a chip that the second one finds half empty.  Quantizers and product of
+// a layer's forward, device time, two launches -> one, us: 512 x 1024 x 1024 12.2 -> 9.2, 1024 x 2048 x 2048 19.4 -> 16.2, 2048 x 4096
+// x 4096 47.2 -> 44.1, 4096 x 4096 x 4096 66.1 -> 59.5, 8192 x 14336 x 4096 284.8 -> 279.1, 4096 x 14336 x 8192 322.2 -> 322.0; fp32 1376 x
+// 2144 x 2880 32.4 -> 29.0; 8 experts of 2560 x 1440 x 1024 29.5 -> 26.2.
+bool one_launch(const QuantCall& x, const QuantCall& w) {
+  if (x.empty || w.empty || x.dtype != w.dtype || x.streaming || w.streaming || w.bpw8 || w.gen) return false;
+  return (uint64_t)x.grid.x + (uint64_t)w.grid.x * w.grid.z < (1ull << 31);
+}
+
+template <typename T>
+void launch_operands(const QuantCall& x, const QuantCall& w, hipStream_t st) {
+  const dim3 grid(x.grid.x + w.grid.x * w.grid.z);
+  auto go = [&](auto kern) { hipLaunchKernelGGL(kern, grid, dim3(256), 0, st, x.p, w.p, x.grid.x, w.grid.x); };
+  if (x.rht) x.gen ? go(quant_operands_kernel<T, true, true>) : go(quant_operands_kernel<T, true, false>);
+  else x.gen ? go(quant_operands_kernel<T, false, true>) : go(quant_operands_kernel<T, false, false>);
 }
 
 }  // namespace
@@ -1060,4 +1136,31 @@ extern "C" int alto_mxfp4_hadamard_apply(const void* x, int dtype, int64_t M, in
 extern "C" int alto_mxfp4_hadamard(const void* x, int dtype, int64_t M, int64_t C, int64_t ld_x, void* y, int64_t ld_y,
                                    const int8_t* signs, const uint8_t* perm, void* stream) {
   return alto_mxfp4_hadamard_apply(x, dtype, M, C, ld_x, y, ld_y, signs, perm, 0, 1, stream);
+}
+
+extern "C" int alto_mxfp4_quantize_operands(const void* x, int x_dtype, int64_t M, int64_t K, int64_t ld_x, uint8_t* x_row_codes, uint8_t* x_row_scales,
+                                            uint8_t* x_col_codes, uint8_t* x_col_scales, int64_t ld_x_row, int64_t ld_x_col, int hadamard, const int8_t* signs,
+                                            const uint8_t* perm, int clip_mode, int x_flags, const void* w, int w_dtype, int64_t batch, int64_t R, int64_t C, int64_t ld_w,
+                                            int64_t bs_w, uint8_t* w_row_codes, uint8_t* w_row_scales, uint8_t* w_col_codes, uint8_t* w_col_scales, int64_t ld_w_row,
+                                            int64_t ld_w_col, int w_flags, int use_uos, void* stream) {
+  using namespace alto;
+  ALTO_REQUIRE(x_row_codes && x_col_codes && w_row_codes && w_col_codes, "quantize_operands: both copies of both operands are written");
+  ALTO_REQUIRE(clip_mode == ALTO_CLIP_NONE || clip_mode == ALTO_CLIP_STATIC, "quantize_operands: clip_mode %d is neither none nor static", clip_mode);
+  ALTO_REQUIRE(((x_flags | w_flags) & ~3) == 0, "quantize_operands: unknown flags 0x%x", x_flags | w_flags);
+  QuantCall a, b;
+  int rc = plan_quantize(a, x, x_dtype, 1, M, K, ld_x, 0, x_row_codes, x_row_scales, x_col_codes, x_col_scales, ld_x_row, ld_x_col, 0, 0, nullptr, 0, 0, 0, 0, nullptr,
+                         hadamard, signs, perm, clip_mode, use_uos, x_flags);
+  if (rc != ALTO_MXFP4_OK) return rc;
+  rc = plan_quantize(b, w, w_dtype, batch, R, C, ld_w, bs_w, w_row_codes, w_row_scales, w_col_codes, w_col_scales, ld_w_row, ld_w_col, 1, 0, nullptr, 0, 0, 0, 0, nullptr, 0,
+                     nullptr, nullptr, ALTO_CLIP_NONE, use_uos, w_flags);
+  if (rc != ALTO_MXFP4_OK) return rc;
+  hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+  if (one_launch(a, b)) {
+    if (x_dtype == ALTO_DT_BF16) launch_operands<__bf16>(a, b, st);
+    else launch_operands<float>(a, b, st);
+  } else {
+    if (!a.empty) launch_quantize(a, st);
+    if (!b.empty) launch_quantize(b, st);
+  }
+  return check_launch("quantize_operands");
 }

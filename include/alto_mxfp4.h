@@ -176,6 +176,17 @@ int alto_mxfp4_quantize_ex(const void* x, int dtype, int64_t batch, int64_t M, i
                            int clip_mode, int use_uos, int flags, void* stream);
 
 /*
+ * Both operands of a layer's product in one call, both copies of each, round to nearest: what two calls of alto_mxfp4_quantize_ex
+ * write, the activation x [M][K] with 1D blocks (Hadamard transform and clip on its column copy) and `batch` weight matrices
+ * w [R][C] with 2D blocks, no clip; one launch for both unless one is too large for the caches.
+ */
+int alto_mxfp4_quantize_operands(const void* x, int x_dtype, int64_t M, int64_t K, int64_t ld_x, uint8_t* x_row_codes, uint8_t* x_row_scales,
+                                 uint8_t* x_col_codes, uint8_t* x_col_scales, int64_t ld_x_row, int64_t ld_x_col, int hadamard, const int8_t* signs,
+                                 const uint8_t* perm, int clip_mode, int x_flags, const void* w, int w_dtype, int64_t batch, int64_t R, int64_t C, int64_t ld_w,
+                                 int64_t bs_w, uint8_t* w_row_codes, uint8_t* w_row_scales, uint8_t* w_col_codes, uint8_t* w_col_scales, int64_t ld_w_row,
+                                 int64_t ld_w_col, int w_flags, int use_uos, void* stream);
+
+/*
  * Moves the counter of a device-resident Philox state {key, counter} past `words` random words (counter += ceil(words / 4)),
  * enqueued on `stream` after the quantizer call that consumed them.  A one-thread kernel; it can be captured together
  * with that call.  No counterpart in the reference (its Philox offsets are host integers).

@@ -292,6 +292,13 @@ Entry g_bf16q_entries[] = {
      [](const Args& a) { return call_bf16q(a, nullptr); }},
     {"attention_fwd_bf16q_packed", 16, 2, 7, {{1, 8, 2, 256, 288, 128, 64, 0, 64, 512, 0, 1, 8, 0, 128, 1024}, {0, 1}, {D, D, D, D, D, D, D}, 0.088388f, {0, 0}, g_signs, g_perm},
      [](const Args& a) { return call_bf16q(a, &g_bounds[(unsigned)a.i[0] % (kManySequences + 1)]); }},
+    // M, K, ld_x, x code pitches, batch, R, C, ld_w, bs_w, w code pitches; x_dtype, hadamard, clip, x_flags, w_dtype, w_flags, uos
+    {"quantize_operands", 12, 7, 10, {{64, 256, 256, 128, 32, 2, 96, 256, 256, 96 * 256, 128, 48}, {0, 1, 0, 1, 0, 2, 0}, {D, D, D, D, D, D, D, D, D, D}, 1.0f, {0, 0}, g_signs, g_perm},
+     [](const Args& a) {
+       return alto_mxfp4_quantize_operands(a.p[0], a.i[0], a.s[0], a.s[1], a.s[2], P(uint8_t, 1), P(uint8_t, 2), P(uint8_t, 3), P(uint8_t, 4), a.s[3], a.s[4], a.i[1],
+                                           a.signs, a.perm, a.i[2], a.i[3], a.p[5], a.i[4], a.s[5], a.s[6], a.s[7], a.s[8], a.s[9], P(uint8_t, 6), P(uint8_t, 7),
+                                           P(uint8_t, 8), P(uint8_t, 9), a.s[10], a.s[11], a.i[5], a.i[6], nullptr);
+     }},
     {"grouped_gemm_offsets", 0, 1, 2, {{}, {32}, {D, D}, 1.0f, {0, 0}, g_signs, g_perm},
      [](const Args& a) { return alto_mxfp4_grouped_gemm_offsets(P(const int32_t, 0), a.i[0], P(int32_t, 1), nullptr); }},
 };

@@ -182,3 +182,31 @@ def test_steps_run_on_the_callers_stream_and_replay(m):
         x.copy_(randn_outliers((256, 544), torch.bfloat16, seed=seed).to(DEV))
         graph.replay()
         _same([t.clone() for t in got], step(), seed)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("had,clip,uos", [(True, "none", False), (False, "static", False), (True, "static", True)])
+@pytest.mark.parametrize("x_shape,w_shape", [((32, 32), (1, 32, 32)), ((96, 544), (3, 288, 544)), ((1056, 256), (1, 160, 512)), ((64, 2080), (2, 1056, 96))])
+def test_operands_quantized_in_one_call(m, dtype, had, clip, uos, x_shape, w_shape):
+    """alto_mxfp4_quantize_operands writes what two quantizer calls write, plain and packed scales, also for operands of different
+    widths and types (then in two launches)."""
+    from alto_amd import _lib
+    from alto_amd.mxfp4.quantization import _quantize_call
+    from alto_amd.mxfp4 import _runtime as rt
+    h = m.HadamardTransform(*hadamard_from_seed(4)) if had else None
+    M, K = x_shape
+    E, R, C = w_shape
+    for w_dtype in (dtype, torch.float32):
+        x, w = randn_outliers(x_shape, dtype, seed=1).to(DEV), randn_outliers(w_shape, w_dtype, seed=2).to(DEV)
+        for pack in (False, True):
+            xr, xrs, xc, xcs = _quantize_call(x[None], True, True, False, False, None, h, rt.CLIP[clip], uos, True, pack_row_scales=pack, pack_col_scales=pack)
+            wr, wrs, wc, wcs = _quantize_call(w, True, True, True, False, None, None, 0, uos, True, pack_row_scales=pack, pack_col_scales=pack)
+            got = [torch.empty_strided(t.shape, t.stride(), dtype=torch.uint8, device=DEV).zero_() for t in (xr, xrs, xc, xcs, wr, wrs, wc, wcs)]
+            g = [t.data_ptr() for t in got]
+            flags = 3 if pack else 0
+            _lib.check(_lib.load().alto_mxfp4_quantize_operands(
+                x.data_ptr(), rt.dtype_code(dtype), M, K, K, *g[:4], xr.stride(1), xc.stride(1), int(had), h.signs.data_ptr() if had else None,
+                h.perm.data_ptr() if had else None, rt.CLIP[clip], flags, w.data_ptr(), rt.dtype_code(w_dtype), E, R, C, C, R * C, *g[4:], wr.stride(1), wc.stride(1), flags,
+                int(uos), rt.stream_ptr(x.device)), "alto_mxfp4_quantize_operands")
+            for a, b, what in zip(got, (xr, xrs, xc, xcs, wr, wrs, wc, wcs), "xr xrs xc xcs wr wrs wc wcs".split()):
+                assert torch.equal(a, b), (what, pack, w_dtype)
