@@ -273,10 +273,11 @@ struct TileLoader {
 // in the order of the LDS row below, bytes beyond K = 127] -- with OperandView::scales the base of it and
 // OperandView::ss_k the bytes from one block to the next (rows x 16).  A block of a tile's 256 + 256 rows is then 8 runs of
 // 1 KB, which the eight waves move straight into LDS with one load each (no registers, no fix-up, no ds_write; 8 cache
-// lines per load instead of the 64 of per-row scale rows).  Needs the end of K at compile time (LMS >= 0, or no K tail).
+// lines per load instead of the 64 of per-row scale rows).  Needs the end of K at compile time (LMS >= 0, or no K tail) or
+// LMS = -2.
 template <bool KTAIL, int LMS = -1, int NST = 4, int PS = 0>
 __device__ __forceinline__ void gemm_tile_mainloop(const TileArgs& ta, TileAcc& acc, uint8_t* smem) {
-  static_assert(PS != 1 || !KTAIL || LMS >= 0, "packed scales: the end of K must be known at compile time");
+  static_assert(PS != 1 || !KTAIL || LMS >= 0 || LMS == -2, "packed scales: the end of K is known at compile time, or whole stages run (-2)");
   static_assert(PS != 2 || (KTAIL && LMS < 0), "packed scales of a sub-range of K: the generic endings only");
   constexpr int SP = PS ? 4 : GT_SCALE_PITCH;   // dwords per row of a scale buffer in LDS
   TileLoader ld;
@@ -373,8 +374,10 @@ __device__ __forceinline__ void gemm_tile_mainloop(const TileArgs& ta, TileAcc& 
   const int ps_q0 = PS == 2 ? ta.ps_q0 : 0;
   auto sdma = [&](int kb) {   // packed block ps_q0 + kb -> scale buffer kb & 1
     typedef __attribute__((address_space(3))) uint8_t lds_u8s;
+    const int buf = kb & 1;
+    if constexpr (PS == 1 && KTAIL && LMS == -2) kb = kb < KB ? kb : KB - 1;   // (a block beyond K is loaded but not used; the end of the buffer is never passed)
     const int so = __builtin_amdgcn_readfirstlane((kb + ps_q0) * ps_blk + ps_row0);
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_ps, (__attribute__((address_space(3))) void*)((lds_u8s*)sscale + (kb & 1) * (GT_TM + GT_TN) * SP * 4 + wave * 1024), 16,
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_ps, (__attribute__((address_space(3))) void*)((lds_u8s*)sscale + buf * (GT_TM + GT_TN) * SP * 4 + wave * 1024), 16,
                                              lane * 16, so, 0, 0);
   };
   // 8 MFMAs of K step J (0..3) of macro stage MS (0..1 inside its 512-K block): scale byte J of dword MS

@@ -20,6 +20,22 @@ __global__ __launch_bounds__(GT_THREADS) void gemm_tiled_kernel(OperandView A, O
   gemm_tile_256x256<OutT, KTAIL, LMS, NST, PS>(ta, c, ldc, smem);
 }
 
+// Two products on packed scales, bf16 results (no KTAIL: K a multiple of 512 in both).  The tiles of the second fill the units that
+// the first one's last round leaves idle: 128 + 256 tiles of 2048 x 4096 x 4096 are two rounds of work and took 52.5 us in two launches, 40.3
+// in one.  Where K ends differs between the two, so a reduction runs its last 256-K stage in full (LMS = -2).
+template <bool KTAIL>
+__global__ __launch_bounds__(GT_THREADS) void gemm_tiled_two_kernel(GemmPair p) {
+  extern __shared__ __align__(16) uint8_t smem[];
+  const int k = (int)blockIdx.x >= p.before;
+  const GemmProblem& q = p.g[k];
+  int tm, tn;
+  if (!tile_coords((int)blockIdx.x - (k ? p.before : 0), p.tiles_m[k], p.tiles_n[k], tm, tn)) return;
+  const int KB = (q.G + 15) / 16;
+  TileArgs ta{q.A, q.B, (int64_t)tm * GT_TM, (int64_t)tn * GT_TN, 0, q.M, q.N, q.G, q.out_scale, (q.M - 1) * q.A.ld + q.G * 16, (q.N - 1) * q.B.ld + q.G * 16,
+              KB * q.A.ss_k, KB * q.B.ss_k, 0, q.G};
+  gemm_tile_256x256<__bf16, KTAIL, -2, 4, 1>(ta, static_cast<__bf16*>(q.c), q.ldc, smem);
+}
+
 // Plain scales of one operand -> the packed form the PS kernels read: dst[(kb * rows + row) * 16 + 4 (2 h + ms) + j] =
 // scale of group 16 kb + 8 ms + 2 j + h of that row, 127 beyond G.  One thread per (row, block).
 __global__ __launch_bounds__(256) void pack_scales_kernel(const uint8_t* __restrict__ src, int64_t ss_r, int64_t ss_k, int is_2d, int64_t rows, int G,
@@ -123,6 +139,23 @@ void gemm_tiled_launch_ps(const OperandView& A, const OperandView& B, int64_t M,
     }
   }
 #undef ALTO_TILED_LAUNCH
+}
+
+template <bool KTAIL>
+static void launch_two(const GemmProblem& p, const GemmProblem& q, hipStream_t st) {
+  auto kern = gemm_tiled_two_kernel<KTAIL>;
+  static std::once_flag once;
+  static hipError_t attr_rc = hipSuccess;
+  std::call_once(once, [&] { attr_rc = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, GT_LDS_BYTES); });
+  if (attr_rc != hipSuccess) return;
+  unsigned workgroups;
+  const GemmPair pair = pair_of(p, q, GT_TM, GT_TN, workgroups);
+  hipLaunchKernelGGL(kern, dim3(workgroups), dim3(GT_THREADS), GT_LDS_BYTES, st, pair);
+}
+
+void gemm_tiled_launch_two(const GemmProblem& first, const GemmProblem& second, hipStream_t st) {
+  if (first.G % 16 == 0 && second.G % 16 == 0) launch_two<false>(first, second, st);
+  else launch_two<true>(first, second, st);
 }
 
 void pack_scales_launch(const uint8_t* src, int64_t ss_r, int64_t ss_k, int is_2d, int64_t rows, int64_t G, uint8_t* dst, hipStream_t st) {

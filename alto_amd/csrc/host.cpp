@@ -43,6 +43,7 @@ struct Api {
   ALTO_FN(attention_fwd_bf16q);
   ALTO_FN(grouped_gemm_offsets);
   ALTO_FN(quantize_operands);
+  ALTO_FN(gemm_two);
 #undef ALTO_FN
 } api;
 py::object* check_fn = nullptr;   // _lib.check(rc, name): raises for rc != 0 (never freed: the interpreter may be gone by then)
@@ -65,6 +66,7 @@ void bind(const py::dict& address, py::object check) {
   ALTO_FN(attention_fwd_bf16q);
   ALTO_FN(grouped_gemm_offsets);
   ALTO_FN(quantize_operands);
+  ALTO_FN(gemm_two);
 #undef ALTO_FN
   delete check_fn;
   check_fn = new py::object(std::move(check));
@@ -363,13 +365,16 @@ bool quantize_operands(Failure& f, const Tensor& x, const Copy& x_row, const Ten
                                     w_col.codes(w_col_buf), w_col.scales(w_col_buf), w_row.ld(), w_col.ld(), flags(w_row, w_col), (int)uos, s));
 }
 
+alto_mxfp4_product product_of(const Copy& a, const Tensor& a_buf, const Copy& b, const Tensor& b_buf, const Tensor& c, double out_scale) {
+  return {a.codes(a_buf), a.scales(a_buf), b.codes(b_buf), b.scales(b_buf), a.ld(), a.scale_ld(), 1, b.ld(), b.scale_ld(), 1, a.rows, b.rows, a.K, c.data_ptr(), b.rows,
+          (float)out_scale, (int)a.is_2d, (int)b.is_2d, dtype_code(c.scalar_type()), (int)a.packed};
+}
 bool product(Failure& f, const Copy& a, const Tensor& a_buf, const Copy& b, const Tensor& b_buf, const Tensor& c, double out_scale, void* s) {
-  const int64_t N = b.rows;
-  if (a.packed)
-    return f.ok("alto_mxfp4_gemm_ps", api.gemm_ps(a.codes(a_buf), a.ld(), a.scales(a_buf), b.codes(b_buf), b.ld(), b.scales(b_buf), a.rows, N, a.K, c.data_ptr(), N,
-                                                  (float)out_scale, s));
-  return f.ok("alto_mxfp4_gemm", api.gemm(a.codes(a_buf), a.ld(), a.scales(a_buf), a.scale_ld(), 1, (int)a.is_2d, b.codes(b_buf), b.ld(), b.scales(b_buf), b.scale_ld(), 1,
-                                          (int)b.is_2d, a.rows, N, a.K, c.data_ptr(), dtype_code(c.scalar_type()), N, (float)out_scale, s));
+  const alto_mxfp4_product p = product_of(a, a_buf, b, b_buf, c, out_scale);
+  if (p.packed)
+    return f.ok("alto_mxfp4_gemm_ps", api.gemm_ps(p.a, p.lda, p.a_scales, p.b, p.ldb, p.b_scales, p.M, p.N, p.K, p.c, p.ldc, p.out_scale, s));
+  return f.ok("alto_mxfp4_gemm", api.gemm(p.a, p.lda, p.a_scales, p.a_ss_r, p.a_ss_k, p.a_is_2d, p.b, p.ldb, p.b_scales, p.b_ss_r, p.b_ss_k, p.b_is_2d, p.M, p.N, p.K, p.c,
+                                          p.c_dtype, p.ldc, p.out_scale, s));
 }
 
 // linear.py:packed_gemm_supported
@@ -450,8 +455,10 @@ py::object linear_backward(const Tensor& go_in, const Tensor& xs, const Tensor& 
     dx = at::empty({M, K}, go.options());
     dw = at::empty({N, K}, go.options());
     void* s = reinterpret_cast<void*>(stream);
-    quantize_gradient(f, go, c.go_row, tmp, c.go_col, tmp, sr ? 3 : 0, seed, h, clip, uos, s) && product(f, c.go_row, tmp, c.w_col, ws, dx, 1.0, s) &&
-        product(f, c.go_col, tmp, c.x_col, xs, dw, out_scale, s);
+    quantize_gradient(f, go, c.go_row, tmp, c.go_col, tmp, sr ? 3 : 0, seed, h, clip, uos, s) && [&] {
+      const alto_mxfp4_product x = product_of(c.go_row, tmp, c.w_col, ws, dx, 1.0), w = product_of(c.go_col, tmp, c.x_col, xs, dw, out_scale);
+      return f.ok("alto_mxfp4_gemm_two", api.gemm_two(&x, &w, s));
+    }();
     if (go_in.dim() != 2) {
       auto shape = go_in.sizes().vec();
       shape.back() = K;

@@ -275,6 +275,22 @@ int alto_mxfp4_gemm_ps(const uint8_t* a, int64_t lda, const uint8_t* a_packed, c
                        int64_t M, int64_t N, int64_t K, void* c, int64_t ldc, float out_scale, void* stream);
 
 /*
+ * Two independent products in one call: what alto_mxfp4_gemm (packed == 0) or alto_mxfp4_gemm_ps (packed != 0: a_scales / b_scales are the
+ * packed scales, the scale strides and is_2d flags are not read, c is bf16) make of each, the arguments as there.  Products
+ * that take the same kernel share one launch.  The input and weight gradients of a layer are such a pair.
+ */
+typedef struct {
+  const uint8_t *a, *a_scales, *b, *b_scales;
+  int64_t lda, a_ss_r, a_ss_k, ldb, b_ss_r, b_ss_k;
+  int64_t M, N, K;
+  void* c;
+  int64_t ldc;
+  float out_scale;
+  int a_is_2d, b_is_2d, c_dtype, packed;
+} alto_mxfp4_product;
+int alto_mxfp4_gemm_two(const alto_mxfp4_product* first, const alto_mxfp4_product* second, void* stream);
+
+/*
  * Ragged grouped GEMM for MoE experts.  Rows [offs[g], offs[g+1]) of A form group g and use
  * expert e(g) = group_expert ? group_expert[g] : g:
  *   out[r][:] = A[r][:] . W[e]^T,   W[e] = w + e * w_stride_e  ([N][K/2] bytes, row stride ldw),

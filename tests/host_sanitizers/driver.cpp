@@ -299,6 +299,15 @@ Entry g_bf16q_entries[] = {
                                            a.signs, a.perm, a.i[2], a.i[3], a.p[5], a.i[4], a.s[5], a.s[6], a.s[7], a.s[8], a.s[9], P(uint8_t, 6), P(uint8_t, 7),
                                            P(uint8_t, 8), P(uint8_t, 9), a.s[10], a.s[11], a.i[5], a.i[6], nullptr);
      }},
+    // lda, strides of its scales, ldb, strides of its scales, M, N, K, ldc; 2D flags, c_dtype, which product has packed scales
+    {"gemm_two", 10, 4, 10, {{256, 16, 1, 256, 16, 1, 512, 512, 512, 512}, {0, 0, 0, 2}, {D, D, D, D, D, D, D, D, D, D}, 1.0f, {0, 0}, g_signs, g_perm},
+     [](const Args& a) {
+       alto_mxfp4_product q[2];
+       for (int k = 0; k < 2; ++k)
+         q[k] = {P(const uint8_t, 5 * k), P(const uint8_t, 5 * k + 1), P(const uint8_t, 5 * k + 2), P(const uint8_t, 5 * k + 3), k ? a.s[3] : a.s[0], a.s[1], a.s[2],
+                 k ? a.s[0] : a.s[3], a.s[4], a.s[5], a.s[6], a.s[7], a.s[8], a.p[5 * k + 4], a.s[9], a.f, a.i[0], a.i[1], a.i[2], a.i[3] == k};
+       return alto_mxfp4_gemm_two(a.signs ? &q[0] : nullptr, a.perm ? &q[1] : nullptr, nullptr);
+     }},
     {"grouped_gemm_offsets", 0, 1, 2, {{}, {32}, {D, D}, 1.0f, {0, 0}, g_signs, g_perm},
      [](const Args& a) { return alto_mxfp4_grouped_gemm_offsets(P(const int32_t, 0), a.i[0], P(int32_t, 1), nullptr); }},
 };
