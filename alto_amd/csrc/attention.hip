@@ -42,7 +42,7 @@ struct AttnTile {
 // and reading them back and leaves the operand quantizer K and V only.  4 x 2048 tokens, 64 / 8 heads of 128, causal (134 of the
 // 168 MB are Q), operand quantizer + this kernel, us: on codes 38.9 + 181.5; every lane fetching the 64 bytes it multiplies
 // 10.6 + 201, whole lines (quantize_q) 10.9 + 197, at raised wave priority 10.6 + 195 (the two other workgroups of the compute unit
-// hide the wait, the priority lets the arithmetic behind it through), with the heads dealt as below 10.3 + 187, with the
+// hide the wait, the priority lets the arithmetic behind it through), with the heads dealt to the XCDs in ranges 10.3 + 187, with the
 // results stored as whole rows 10.7 + 181, Q read non-temporally 8.7 + 179.
 // SEQS: AttnSeqs, or AttnNoSeqs for B sequences of one length.
 template <int NK, int ND, bool BIASED, bool QBF, typename SEQS>

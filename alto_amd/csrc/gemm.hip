@@ -110,12 +110,12 @@ int own_tile_size(const GemmCall& g) { return g.route == Route::MID64 ? 64 : g.r
 // The tile of two packed products that share a launch, or 0: a launch each.  The bits are the same with every tile.
 // Time of a tile size: what a launch costs, and then either the longest reduction, which one workgroup walks through, or
 // all the work spread over the 256 compute units, whichever takes longer.  The constants are a least-squares fit to 346
-// pairs of 512..16384 x 512..14336 x 512..14336, three tile sizes each (10 % rms).  With the tile it names a pair takes 0.80 of
-// the time of two launches with a tile each, 1.5 % more than with the best tile (512 x 1024 x 1024 7.8 -> 5.0 us, 2048 x 4096 x 4096
-// 52.5 -> 41, 4096 x 2880 x 2880 56 -> 51, 8192 x 4096 x 14336 438 -> 432); one launch where both have the same tile anyway would
-// give 0.88.  A rule by the number of tiles alone is 7 % or more behind: a few tiles with a long reduction want them small.
+// pairs of 512..16384 x 512..14336 x 512..14336, three tile sizes each (10 % rms); the tile it names takes 1.5 % longer than the
+// best one.  A pair takes 0.84 of the time of two launches with a tile each (512 x 1024 x 1024 7.4 -> 5.1 us, 2048 x 4096 x 1024 22.0 -> 19.1,
+// 2048 x 4096 x 4096 50.7 -> 41.6, 4096 x 4096 x 4096 72.8 -> 71.3, 8192 x 4096 x 14336 441 -> 441), of which half comes from the tiles: a rule
+// by their number alone is 7 % or more behind, because a few tiles with a long reduction want them small.
 // Beyond a factor of 16 between the reductions no tile suits both unless both ask for the same one (512 x 3840 x 13440, 128 and 256:
-// 73 us apart, 79..90 together).
+// 69 us apart, 79..90 together).
 int shared_tile_size(const GemmCall& x, const GemmCall& y) {
   const double kx = (double)x.K, ky = (double)y.K;   // kx >= ky
   if (kx > 16 * ky) return x.route == y.route ? own_tile_size(x) : 0;

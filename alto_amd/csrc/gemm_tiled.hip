@@ -21,8 +21,8 @@ __global__ __launch_bounds__(GT_THREADS) void gemm_tiled_kernel(OperandView A, O
 }
 
 // Two products on packed scales, bf16 results (no KTAIL: K a multiple of 512 in both).  The tiles of the second fill the units that
-// the first one's last round leaves idle: 128 + 256 tiles of 2048 x 4096 x 4096 are two rounds of work and took 52.5 us in two launches, 40.3
-// in one.  Where K ends differs between the two, so a reduction runs its last 256-K stage in full (LMS = -2).
+// the first one's last round leaves idle: 128 + 256 tiles of 2048 x 4096 x 4096 take 50.7 us in two launches, 41.6 in
+// one.  Where K ends differs between the two, so a reduction runs its last 256-K stage in full (LMS = -2).
 template <bool KTAIL>
 __global__ __launch_bounds__(GT_THREADS) void gemm_tiled_two_kernel(GemmPair p) {
   extern __shared__ __align__(16) uint8_t smem[];

@@ -1,8 +1,9 @@
 """MXFP4 flash-attention forward, named as in ``alto/kernels/fp4/mxfp4/triton_flash_attention_mxfp4.py``.
 
 ``triton_attention_mxfp4`` keeps the reference's name and argument list (:1206-1239) so that
-``alto/kernels/dispatch/attention.py:22`` can point at it; here it quantises Q, K, V with one launch (2D blocks along the
-head dim, :1105-1107; V packed along the keys), read in the layout they come in, and runs one HIP kernel.
+``alto/kernels/dispatch/attention.py:22`` can point at it; here it quantises K and V with one launch (2D blocks along the
+head dim, :1105-1107; V packed along the keys), read in the layout they come in, and runs one HIP kernel, which quantises
+a bf16 Q itself (an fp32 one goes through that launch as well).
 Like the reference (:1143-1145) it has no backward.  Options outside the path ALTO's dispatch layer uses
 (``alto/kernels/dispatch/attention.py:61-77``: layout "bhsd", no bias, no alibi, no dropout, fixed lengths) raise.
 """
