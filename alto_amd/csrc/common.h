@@ -5,6 +5,8 @@
 #include <stdio.h>
 #include <stdarg.h>
 
+#include <atomic>
+
 #include "../../include/alto_mxfp4.h"
 
 namespace alto {
@@ -12,6 +14,24 @@ namespace alto {
 // ----------------------------------------------------------------------------- host: error reporting
 void set_error(const char* fmt, ...);
 int check_launch(const char* what);
+// More than 64 KB of dynamic LDS are asked for once per kernel and process.  A refusal is an error of every call that needs the kernel
+// (each asks again): a launch left out would leave the caller with results that nobody wrote.
+class LdsLimit {
+  std::atomic<bool> raised{false};   // (two host threads may make their first calls together: asking twice is harmless)
+
+ public:
+  int raise(const void* kernel, int bytes, const char* what) {
+    if (raised.load(std::memory_order_acquire)) return ALTO_MXFP4_OK;
+    const hipError_t e = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+    if (e != hipSuccess) {
+      (void)hipGetLastError();   // (not left for the next call's check)
+      set_error("%s: could not reserve %d bytes of LDS: %s", what, bytes, hipGetErrorString(e));
+      return ALTO_MXFP4_ELAUNCH;
+    }
+    raised.store(true, std::memory_order_release);
+    return ALTO_MXFP4_OK;
+  }
+};
 int quantize_dynamic_launch(const void* x, int dtype, int64_t batch, int64_t M, int64_t C, int64_t ld_x, int64_t bs_x, uint8_t* codes,
                             uint8_t* scales, int64_t ld_codes, int is_2d, int sr, const uint32_t* rand_bits, int64_t ld_rand,
                             int64_t bs_rand, int use_uos, hipStream_t st);

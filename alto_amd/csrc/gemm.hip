@@ -138,9 +138,8 @@ int launch_gemm(const GemmCall& g, hipStream_t st) {
     case Route::SKINNY: gemm_skinny_launch(q.A, q.B, q.M, q.N, g.K, q.c, g.c_dtype, q.ldc, q.out_scale, st); break;
     case Route::MID64: case Route::MID128: gemm_mid_launch(g.route == Route::MID64 ? 64 : 128, q, nullptr, g.c_dtype, g.packed, st); break;
     case Route::TILED:
-      if (g.packed) gemm_tiled_launch_ps(q.A, q.B, q.M, q.N, g.K, q.c, q.ldc, q.out_scale, st);
-      else gemm_tiled_launch(q.A, q.B, q.M, q.N, g.K, q.c, g.c_dtype, q.ldc, q.out_scale, st);
-      break;
+      if (g.packed) return gemm_tiled_launch_ps(q.A, q.B, q.M, q.N, g.K, q.c, q.ldc, q.out_scale, st);
+      return gemm_tiled_launch(q.A, q.B, q.M, q.N, g.K, q.c, g.c_dtype, q.ldc, q.out_scale, st);
     case Route::DIRECT: {
       const dim3 grid((unsigned)((q.N + 63) / 64), (unsigned)((q.M + 63) / 64));
       if (g.c_dtype == ALTO_DT_BF16)
@@ -181,8 +180,8 @@ extern "C" int alto_mxfp4_gemm_two(const alto_mxfp4_product* first, const alto_m
     const int own = x.route == y.route ? own_tile_size(x) : 0;
     const int tile = x.packed ? shared_tile_size(x, y) : own == 256 ? 0 : own;
     if (tile != 0) {
-      if (tile == 256) gemm_tiled_launch_two(x.q, y.q, st);
-      else gemm_mid_launch(tile, x.q, &y.q, x.c_dtype, x.packed, st);
+      if (tile == 256) return gemm_tiled_launch_two(x.q, y.q, st);
+      gemm_mid_launch(tile, x.q, &y.q, x.c_dtype, x.packed, st);
       return check_launch("gemm_two");
     }
   }

@@ -1,5 +1,4 @@
 // Tuned LDS-tiled MXFP4 GEMM for gfx950: dense entry (one 256x256 tile per 512-thread workgroup, XCD-aware tile order).
-#include <mutex>
 
 #include "gemm_tiled.h"
 #include "gemm_tile.h"
@@ -61,18 +60,14 @@ __global__ __launch_bounds__(256) void pack_scales_kernel(const uint8_t* __restr
 
 template <typename OutT, bool KTAIL, int LMS = -1, int NST = 4, bool PS = false>
 int launch_tiled(const OperandView& A, const OperandView& B, int64_t M, int64_t N, int64_t K, void* c, int64_t ldc, float out_scale, hipStream_t st) {
-  // the opt-in for > 64 KB of dynamic LDS is per function, set once per process (two host threads may make their first
-  // call together: forward on the caller's thread, backward on the autograd thread)
   auto kern = gemm_tiled_kernel<OutT, KTAIL, LMS, NST, PS>;
-  static std::once_flag once;
-  static hipError_t attr_rc = hipSuccess;
-  std::call_once(once, [&] { attr_rc = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, GT_LDS_BYTES); });
-  if (attr_rc != hipSuccess) return -1;
+  static LdsLimit lds;
+  if (const int rc = lds.raise(reinterpret_cast<const void*>(kern), GT_LDS_BYTES, "gemm")) return rc;
   const int tiles_m = (int)((M + GT_TM - 1) / GT_TM), tiles_n = (int)((N + GT_TN - 1) / GT_TN);
   const int T = tiles_m * tiles_n;
   const int per_xcd = (T + 7) / 8;
   hipLaunchKernelGGL(kern, dim3((unsigned)(per_xcd * 8)), dim3(GT_THREADS), GT_LDS_BYTES, st, A, B, M, N, (int)(K / 32), (OutT*)c, ldc, out_scale, tiles_m, tiles_n);
-  return 0;
+  return check_launch("gemm");
 }
 
 }  // namespace
@@ -90,72 +85,70 @@ bool gemm_tiled_supported(const OperandView& A, const OperandView& B, int64_t M,
   return tiles < (1ll << 28);
 }
 
-void gemm_tiled_launch(const OperandView& A, const OperandView& B, int64_t M, int64_t N, int64_t K, void* c, int c_dtype, int64_t ldc,
-                       float out_scale, hipStream_t st) {
+int gemm_tiled_launch(const OperandView& A, const OperandView& B, int64_t M, int64_t N, int64_t K, void* c, int c_dtype, int64_t ldc,
+                      float out_scale, hipStream_t st) {
   const bool tail = (K / 32) % 16 != 0;   // K not a multiple of 512: the last scale block of a row is partial
 #define ALTO_TILED_LAUNCH(T, ...) launch_tiled<T, __VA_ARGS__>(A, B, M, N, K, c, ldc, out_scale, st)
   if (!tail) {
-    if (c_dtype == ALTO_DT_BF16) ALTO_TILED_LAUNCH(__bf16, false);
-    else ALTO_TILED_LAUNCH(float, false);
+    if (c_dtype == ALTO_DT_BF16) return ALTO_TILED_LAUNCH(__bf16, false);
+    else return ALTO_TILED_LAUNCH(float, false);
   } else if (c_dtype != ALTO_DT_BF16) {
-    ALTO_TILED_LAUNCH(float, true);   // (fp32 output: the general ending)
+    return ALTO_TILED_LAUNCH(float, true);   // (fp32 output: the general ending)
   } else {
     // K is known here: the kernel that ends the reduction exactly where K ends
     int lms, nst;
     gemm_tile_last_stage(K / 32, lms, nst);
     switch (lms * 4 + nst - 1) {
-      case 0: ALTO_TILED_LAUNCH(__bf16, true, 0, 1); break;
-      case 1: ALTO_TILED_LAUNCH(__bf16, true, 0, 2); break;
-      case 2: ALTO_TILED_LAUNCH(__bf16, true, 0, 3); break;
-      case 3: ALTO_TILED_LAUNCH(__bf16, true, 0, 4); break;
-      case 4: ALTO_TILED_LAUNCH(__bf16, true, 1, 1); break;
-      case 5: ALTO_TILED_LAUNCH(__bf16, true, 1, 2); break;
-      case 6: ALTO_TILED_LAUNCH(__bf16, true, 1, 3); break;
-      default: ALTO_TILED_LAUNCH(__bf16, true, 1, 4); break;
+      case 0: return ALTO_TILED_LAUNCH(__bf16, true, 0, 1);
+      case 1: return ALTO_TILED_LAUNCH(__bf16, true, 0, 2);
+      case 2: return ALTO_TILED_LAUNCH(__bf16, true, 0, 3);
+      case 3: return ALTO_TILED_LAUNCH(__bf16, true, 0, 4);
+      case 4: return ALTO_TILED_LAUNCH(__bf16, true, 1, 1);
+      case 5: return ALTO_TILED_LAUNCH(__bf16, true, 1, 2);
+      case 6: return ALTO_TILED_LAUNCH(__bf16, true, 1, 3);
+      default: return ALTO_TILED_LAUNCH(__bf16, true, 1, 4);
     }
   }
 #undef ALTO_TILED_LAUNCH
 }
 
 // Both operands with packed scales (A.scales / B.scales = packed base, ss_k = bytes per block), bf16 output.
-void gemm_tiled_launch_ps(const OperandView& A, const OperandView& B, int64_t M, int64_t N, int64_t K, void* c, int64_t ldc, float out_scale,
-                          hipStream_t st) {
+int gemm_tiled_launch_ps(const OperandView& A, const OperandView& B, int64_t M, int64_t N, int64_t K, void* c, int64_t ldc, float out_scale,
+                         hipStream_t st) {
   const bool tail = (K / 32) % 16 != 0;
 #define ALTO_TILED_LAUNCH(...) launch_tiled<__bf16, __VA_ARGS__, true>(A, B, M, N, K, c, ldc, out_scale, st)
   if (!tail) {
-    ALTO_TILED_LAUNCH(false, -1, 4);
+    return ALTO_TILED_LAUNCH(false, -1, 4);
   } else {
     int lms, nst;
     gemm_tile_last_stage(K / 32, lms, nst);
     switch (lms * 4 + nst - 1) {
-      case 0: ALTO_TILED_LAUNCH(true, 0, 1); break;
-      case 1: ALTO_TILED_LAUNCH(true, 0, 2); break;
-      case 2: ALTO_TILED_LAUNCH(true, 0, 3); break;
-      case 3: ALTO_TILED_LAUNCH(true, 0, 4); break;
-      case 4: ALTO_TILED_LAUNCH(true, 1, 1); break;
-      case 5: ALTO_TILED_LAUNCH(true, 1, 2); break;
-      case 6: ALTO_TILED_LAUNCH(true, 1, 3); break;
-      default: ALTO_TILED_LAUNCH(true, 1, 4); break;
+      case 0: return ALTO_TILED_LAUNCH(true, 0, 1);
+      case 1: return ALTO_TILED_LAUNCH(true, 0, 2);
+      case 2: return ALTO_TILED_LAUNCH(true, 0, 3);
+      case 3: return ALTO_TILED_LAUNCH(true, 0, 4);
+      case 4: return ALTO_TILED_LAUNCH(true, 1, 1);
+      case 5: return ALTO_TILED_LAUNCH(true, 1, 2);
+      case 6: return ALTO_TILED_LAUNCH(true, 1, 3);
+      default: return ALTO_TILED_LAUNCH(true, 1, 4);
     }
   }
 #undef ALTO_TILED_LAUNCH
 }
 
 template <bool KTAIL>
-static void launch_two(const GemmProblem& p, const GemmProblem& q, hipStream_t st) {
+static int launch_two(const GemmProblem& p, const GemmProblem& q, hipStream_t st) {
   auto kern = gemm_tiled_two_kernel<KTAIL>;
-  static std::once_flag once;
-  static hipError_t attr_rc = hipSuccess;
-  std::call_once(once, [&] { attr_rc = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, GT_LDS_BYTES); });
-  if (attr_rc != hipSuccess) return;
+  static LdsLimit lds;
+  if (const int rc = lds.raise(reinterpret_cast<const void*>(kern), GT_LDS_BYTES, "gemm_two")) return rc;
   unsigned workgroups;
   const GemmPair pair = pair_of(p, q, GT_TM, GT_TN, workgroups);
   hipLaunchKernelGGL(kern, dim3(workgroups), dim3(GT_THREADS), GT_LDS_BYTES, st, pair);
+  return check_launch("gemm_two");
 }
 
-void gemm_tiled_launch_two(const GemmProblem& first, const GemmProblem& second, hipStream_t st) {
-  if (first.G % 16 == 0 && second.G % 16 == 0) launch_two<false>(first, second, st);
-  else launch_two<true>(first, second, st);
+int gemm_tiled_launch_two(const GemmProblem& first, const GemmProblem& second, hipStream_t st) {
+  return first.G % 16 == 0 && second.G % 16 == 0 ? launch_two<false>(first, second, st) : launch_two<true>(first, second, st);
 }
 
 void pack_scales_launch(const uint8_t* src, int64_t ss_r, int64_t ss_k, int is_2d, int64_t rows, int64_t G, uint8_t* dst, hipStream_t st) {

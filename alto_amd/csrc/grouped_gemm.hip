@@ -474,30 +474,24 @@ template <typename OutT, bool KTAIL, int LMS = -1, int NST = 4, bool PS = false>
 int launch_grouped_tiled(const OperandView& A, const uint8_t* w, int64_t w_stride_e, int64_t ldw, const uint8_t* w_scales, int64_t ws_stride_e,
                          int64_t ws_r, int w_is_2d, const int32_t* offs, const int32_t* group_expert, int num_groups, int num_experts,
                          int64_t M_total, int64_t N, int64_t K, void* out, int64_t ldo, int32_t* plan, bool build_plan, hipStream_t st) {
-  // the opt-in for > 64 KB of dynamic LDS is per function, set once per process (thread-safe: forward and backward may
-  // make their first calls from two host threads)
   auto kern = grouped_tiled_kernel<OutT, KTAIL, LMS, NST, PS>;
-  static std::once_flag once;
-  static hipError_t attr_rc = hipSuccess;
-  std::call_once(once, [&] { attr_rc = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, GT_LDS_BYTES); });
-  if (attr_rc != hipSuccess) return -1;
+  static LdsLimit lds;
+  if (const int rc = lds.raise(reinterpret_cast<const void*>(kern), GT_LDS_BYTES, "grouped_gemm")) return rc;
   const int tiles_m = (int)((M_total + GT_TM - 1) / GT_TM), tiles_n = (int)((N + GT_TN - 1) / GT_TN);
   const int max_pass = (int)grouped_max_passes(M_total, num_groups);
   PassWalk wk{offs, group_expert, num_groups, num_experts, M_total};
   if (build_plan) hipLaunchKernelGGL(grouped_plan_kernel, dim3(1), dim3(PLAN_THREADS), 0, st, wk, tiles_m, plan, max_pass);
   hipLaunchKernelGGL(kern, dim3((unsigned)grouped_grid_size(max_pass, tiles_n)), dim3(GT_THREADS), GT_LDS_BYTES, st, A, w, w_stride_e, ldw, w_scales, ws_stride_e, ws_r,
                      w_is_2d, plan, M_total, N, (int)(K / 32), (OutT*)out, ldo, tiles_n, M_total >= 4ll * GT_TM * num_experts ? 2 : 0);
-  return 0;
+  return check_launch("grouped_gemm");
 }
 
 template <typename OutT, bool PS = false>
 int launch_dw_tiled(const OperandView& P, const OperandView& Q, int64_t NP, int64_t NQ, const int32_t* offs, const int32_t* group_expert,
                     int num_groups, int num_experts, int64_t M_total, void* dw, int64_t s_e, int64_t ld, float out_scale, hipStream_t st) {
   auto kern = grouped_dw_tiled_kernel<OutT, PS>;
-  static std::once_flag once;
-  static hipError_t attr_rc = hipSuccess;
-  std::call_once(once, [&] { attr_rc = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, GT_DW_LDS_BYTES); });
-  if (attr_rc != hipSuccess) return -1;
+  static LdsLimit lds;
+  if (const int rc = lds.raise(reinterpret_cast<const void*>(kern), GT_DW_LDS_BYTES, "grouped_gemm_dw")) return rc;
   const int tiles_p = (int)((NP + GT_TM - 1) / GT_TM), tiles_q = (int)((NQ + GT_TN - 1) / GT_TN);
   // split of the 8 XCDs over the tile grid: the smallest blocks (least idle workgroups), then the smallest perimeter
   int xq_log2 = 0;
@@ -513,7 +507,7 @@ int launch_dw_tiled(const OperandView& P, const OperandView& Q, int64_t NP, int6
   }
   hipLaunchKernelGGL(kern, dim3((unsigned)(8 * best_area), (unsigned)num_experts), dim3(GT_THREADS), GT_DW_LDS_BYTES, st, P, Q, NP, NQ, offs,
                      group_expert, num_groups, M_total, (OutT*)dw, s_e, ld, out_scale, tiles_p, tiles_q, xq_log2);
-  return 0;
+  return check_launch("grouped_gemm_dw");
 }
 
 }  // namespace
@@ -565,7 +559,7 @@ int grouped_gemm_impl(const uint8_t* a, int64_t lda, const uint8_t* a_scales, in
                  (long long)plan_bytes, (long long)M_total, num_groups, (long long)need);
     const bool tail = (K / 32) % 16 != 0;
     int32_t* pl = reinterpret_cast<int32_t*>(plan);
-    int rc = -1;
+    int rc = ALTO_MXFP4_EINVAL;
 #define ALTO_GROUPED_LAUNCH(T, ...) launch_grouped_tiled<T, __VA_ARGS__>(A, w, w_stride_e, ldw, w_scales, ws_stride_e, ws_r, w_is_2d, offs, group_expert, num_groups, num_experts, M_total, N, K, out, ldo, pl, build_plan, st)
     if (ps) {
       int lms = -1, nst = 4;
@@ -601,11 +595,7 @@ int grouped_gemm_impl(const uint8_t* a, int64_t lda, const uint8_t* a_scales, in
       }
     }
 #undef ALTO_GROUPED_LAUNCH
-    if (rc != 0) {
-      set_error("grouped_gemm: could not reserve %d bytes of LDS", GT_LDS_BYTES);
-      return ALTO_MXFP4_ELAUNCH;
-    }
-    return check_launch("grouped_gemm");
+    return rc;
   }
   // upper bound on row tiles: every expert (and the zero tail) may end with one partial tile
   const int64_t tiles = M_total / 64 + num_groups + 2;
@@ -801,11 +791,7 @@ int grouped_dw_impl(const uint8_t* go, int64_t ld_go, const uint8_t* go_scales, 
                      : dw_dtype == ALTO_DT_BF16
                          ? launch_dw_tiled<__bf16>(P, Q, NP, NQ, offs, group_expert, num_groups, num_experts, M_total, dw, dw_stride_e, ld, out_scale, st)
                          : launch_dw_tiled<float>(P, Q, NP, NQ, offs, group_expert, num_groups, num_experts, M_total, dw, dw_stride_e, ld, out_scale, st);
-      if (rc != 0) {
-        set_error("grouped_gemm_dw: could not reserve %d bytes of LDS", GT_DW_LDS_BYTES);
-        return ALTO_MXFP4_ELAUNCH;
-      }
-      return check_launch("grouped_gemm_dw");
+      return rc;
     }
   }
   dim3 grid((unsigned)((K + 63) / 64), (unsigned)((N + 63) / 64), (unsigned)num_experts);
