@@ -97,6 +97,14 @@ __device__ __forceinline__ uint32_t encode8(const uint32_t* w, float scale) {
 }
 
 
+// Between a wave's LDS writes and its own lanes' reads of them.  The LDS keeps a wave's accesses in order, so this is no instruction;
+// it keeps the compiler from moving either side past the other.
+__device__ __forceinline__ void wave_lds_order() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
+}
+
 // A wave's 32 rows of Q, straight from bf16, as the score product takes them: lane (r = lane % 32, h = lane / 32) gets the codes of
 // row r, columns 64 s + 32 h .. + 32, and the scale byte of that 32 x 32 block.  The loads are whole 128-byte lines (8 lanes a row,
 // 8 rows an instruction; a lane that fetched its own 64 bytes cost 32 line lookups an instruction instead of 8); the codes change
@@ -127,6 +135,7 @@ __device__ __forceinline__ void quantize_q(const __bf16* x, int64_t row_stride, 
     for (int i = 0; i < 4; ++i) *reinterpret_cast<uint32_t*>(scratch + 1024 * s + 256 * i + 4 * lane) = encode8<__bf16>(w[s][i], u2f(e << 23));
     qsc[s] = lane < 32 ? __builtin_amdgcn_readlane((int)e, 0) : __builtin_amdgcn_readlane((int)e, 4);
   }
+  wave_lds_order();
 #pragma unroll
   for (int s = 0; s < NK; ++s) qf[s] = frag16(scratch + 1024 * s + (lane & 31) * 32 + (lane >> 5) * 16);
 }

@@ -325,6 +325,7 @@ __device__ __forceinline__ void attn_fwd_body(const AttnArgs& a, const SEQS& seq
       w.y = pack_bf16x2(acc_o[d][4 * g + 2] * rl, acc_o[d][4 * g + 3] * rl);
       *reinterpret_cast<uint2*>(rows + r * (DV * 2) + (((4 * d + g) ^ ((r / (16 / PR)) % PR)) * 16 + 8 * h)) = w;
     }
+  wave_lds_order();
   __bf16* o_first = out + b * a.o_sb + hq * a.o_sh + (int64_t)(q_first + q0) * a.o_ss;
 #pragma unroll
   for (int i = 0; i < PR / 2; ++i) {
