@@ -84,6 +84,8 @@ SIGNATURES = {
     "alto_mxfp4_attention_quantize": (c_int, [c_vp, c_vp, c_vp, c_int] + [c_i64] * 16 + [c_vp] * 7),
     "alto_mxfp4_attention_fwd_strided": (c_int, [c_vp] * 8 + [c_i64] * 13 + [c_int, c_vp, c_vp, c_f32, c_int, c_vp, c_i64, c_i64, c_vp]),
     "alto_mxfp4_gemm_two": (c_int, [c_vp, c_vp, c_vp]),
+    "alto_mxfp4_gemm_two_tile": (c_int, [c_vp, c_vp]),
+    "alto_mxfp4_attention_rows_per_workgroup": (c_int, [c_i64] * 5 + [c_int, c_vp, c_vp, c_int]),
     "alto_mxfp4_quantize_operands": (c_int, [c_vp, c_int] + [c_i64] * 3 + [c_vp] * 4 + [c_i64] * 2 + [c_int, c_vp, c_vp, c_int, c_int, c_vp, c_int] + [c_i64] * 5
                                      + [c_vp] * 4 + [c_i64] * 2 + [c_int, c_int, c_vp]),
     "alto_mxfp4_attention_quantize_kv": (c_int, [c_vp, c_vp, c_int] + [c_i64] * 11 + [c_vp] * 5),

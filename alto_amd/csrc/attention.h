@@ -218,8 +218,7 @@ __device__ __forceinline__ void quantize_probabilities(v16f_t (&S)[2], const flo
   pscale = h ? psc[1] : psc[0];
 }
 
-// Launches of the two kernels (attention.hip: four waves walk the keys of 128 rows; attention_split.hip: they deal out the keys of
-// 32 rows); `row_blocks` in units of 128 and of 32 rows.
+// Launch of the kernel whose four waves deal out the keys of 32 rows (attention_split.hip); `row_blocks` in units of 32 rows.
 template <typename SEQS>
 int launch_attn_split(const AttnArgs& a, const SEQS& seqs, int B, int row_blocks, int64_t D, int64_t Dv, hipStream_t st);
 

@@ -364,6 +364,8 @@ static int launch_attn(const AttnArgs& a, const SEQS& seqs, int B, int row_block
 //   short: 32 x 256 11.8 / 9.2 (.14), 4 x 16 x 512 18.4 / 18.2 (1.0), 4 x 32 x 256 15.0 / 16.5 (1.13);
 //   D = 64: 16 x 2048 causal 36.3 / 23.0 (.59), 28 x 2048 36.8 / 33.0 (1.04), 32 x 2048 37.5 / 35.1 (1.18), 56 x 1024 23.0 / 23.7 (1.15);
 //   D = 192: 16 x 1024 causal 30.3 / 18.1 (.66), D = 256: 16 x 1024 all keys 27.6 / 23.4 (1.0), 32 x 1024 causal 30.5 / 30.6 (1.32).
+// Packed sequences are weighed all together, also where there are more than one launch holds (64): such a call keeps to 128 rows
+// sooner than each of its launches by itself would have to.
 static int rows_per_workgroup(const AttnArgs& a, int64_t B, int64_t D, int n_seqs, const int32_t* cu_q, const int32_t* cu_k) {
   if (a.bias || a.alibi || a.Sq / 32 > 65535) return 128;
   double work = 0.0;
@@ -443,6 +445,18 @@ struct QueryOperand {
   int64_t sb, sh, ss;
 };
 
+static int check_boundaries(int64_t B, int64_t Sq, int64_t Sk, int n_seqs, const int32_t* cu_q, const int32_t* cu_k, int causal) {
+  ALTO_REQUIRE(n_seqs > 0 && cu_q && cu_k && B == 1, "attention_fwd: packed sequences need their boundaries and B = 1");
+  ALTO_REQUIRE(cu_q[0] == 0 && cu_k[0] == 0 && cu_q[n_seqs] == Sq && cu_k[n_seqs] == Sk, "attention_fwd: the sequence boundaries must run from 0 to the token counts");
+  for (int i = 0; i < n_seqs; ++i) {
+    ALTO_REQUIRE(cu_q[i + 1] > cu_q[i] && cu_k[i + 1] > cu_k[i] && cu_q[i + 1] % 32 == 0 && cu_k[i + 1] % 32 == 0,
+                 "attention_fwd: sequence boundaries must be increasing multiples of 32 tokens");
+    ALTO_REQUIRE(!causal || cu_q[i + 1] - cu_q[i] <= cu_k[i + 1] - cu_k[i], "attention_fwd: causal attention needs Sq <= Sk (got %d > %d)", cu_q[i + 1] - cu_q[i],
+                 cu_k[i + 1] - cu_k[i]);
+  }
+  return ALTO_MXFP4_OK;
+}
+
 static int attention_fwd_strided(const QueryOperand& q, const void* k_codes, const void* k_scales, const void* vt_codes, const void* v_scales, void* out,
                                  float* lse, int64_t B, int64_t Hq, int64_t Hk, int64_t Sq, int64_t Sk, int64_t D, int64_t Dv, int64_t o_sb, int64_t o_sh,
                                  int64_t o_ss, int64_t l_sb, int64_t l_sh, int64_t l_ss, int n_seqs, const int32_t* cu_q, const int32_t* cu_k, float sm_scale,
@@ -470,14 +484,7 @@ static int attention_fwd_strided(const QueryOperand& q, const void* k_codes, con
     const int rows = rows_per_workgroup(a, B, D, 0, nullptr, nullptr);
     return launch_attn_dims(a, AttnNoSeqs{}, (int)B, (int)((Sq + rows - 1) / rows), rows, D, Dv, st);
   }
-  ALTO_REQUIRE(n_seqs > 0 && cu_q && cu_k && B == 1, "attention_fwd: packed sequences need their boundaries and B = 1");
-  ALTO_REQUIRE(cu_q[0] == 0 && cu_k[0] == 0 && cu_q[n_seqs] == Sq && cu_k[n_seqs] == Sk, "attention_fwd: the sequence boundaries must run from 0 to the token counts");
-  for (int i = 0; i < n_seqs; ++i) {
-    ALTO_REQUIRE(cu_q[i + 1] > cu_q[i] && cu_k[i + 1] > cu_k[i] && cu_q[i + 1] % 32 == 0 && cu_k[i + 1] % 32 == 0,
-                 "attention_fwd: sequence boundaries must be increasing multiples of 32 tokens");
-    ALTO_REQUIRE(!causal || cu_q[i + 1] - cu_q[i] <= cu_k[i + 1] - cu_k[i], "attention_fwd: causal attention needs Sq <= Sk (got %d > %d)", cu_q[i + 1] - cu_q[i],
-                 cu_k[i + 1] - cu_k[i]);
-  }
+  if (const int rc = check_boundaries(B, Sq, Sk, n_seqs, cu_q, cu_k, causal)) return rc;
   // longest sequences first, up to ATTN_MAX_SEQS of them and 65535 row blocks per launch
   std::unique_ptr<int[]> order(new (std::nothrow) int[(size_t)n_seqs]);   // (no exception may leave a C entry)
   if (!order) {
@@ -530,6 +537,18 @@ extern "C" int alto_mxfp4_attention_fwd_bf16q(const void* q, int64_t q_sb, int64
     ALTO_REQUIRE(s >= 0 && s < (1ll << 44) && s % 8 == 0, "attention_fwd: strides of q must be non-negative multiples of 8 elements");
   return alto::attention_fwd_strided({nullptr, nullptr, q, q_sb, q_sh, q_ss}, k_codes, k_scales, vt_codes, v_scales, out, lse, B, Hq, Hk, Sq, Sk, D, Dv, o_sb, o_sh, o_ss,
                                      l_sb, l_sh, l_ss, n_seqs, cu_q, cu_k, sm_scale, causal, nullptr, 0, 0, (hipStream_t)stream);
+}
+
+extern "C" int alto_mxfp4_attention_rows_per_workgroup(int64_t B, int64_t Hq, int64_t Sq, int64_t Sk, int64_t D, int n_seqs, const int32_t* cu_q, const int32_t* cu_k,
+                                                       int causal) {
+  using namespace alto;
+  ALTO_REQUIRE(B > 0 && Hq > 0 && Sq > 0 && Sk > 0, "attention_rows_per_workgroup: sizes must be positive");
+  ALTO_REQUIRE(B < (1ll << 31) && Hq < (1ll << 31) && Sq < (1ll << 31) && Sk < (1ll << 31), "attention_rows_per_workgroup: size out of range");
+  if (n_seqs != 0)
+    if (const int rc = check_boundaries(B, Sq, Sk, n_seqs, cu_q, cu_k, causal)) return rc;
+  AttnArgs a{};
+  a.Hq = (int)Hq; a.Sq = (int)Sq; a.Sk_used = (int)Sk; a.causal = causal ? 1 : 0;
+  return rows_per_workgroup(a, B, D, n_seqs, cu_q, cu_k);
 }
 
 extern "C" int alto_mxfp4_attention_fwd(const void* q_codes, const void* q_scales, const void* k_codes, const void* k_scales,

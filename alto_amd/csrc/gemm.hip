@@ -131,6 +131,24 @@ int shared_tile_size(const GemmCall& x, const GemmCall& y) {
   return best;
 }
 
+// The tile of the launch that two products share, longer reduction first, or 0: a launch each.
+int tile_of_two(const GemmCall& x, const GemmCall& y) {
+  if (x.route == Route::NONE || y.route == Route::NONE || x.packed != y.packed || x.c_dtype != y.c_dtype) return 0;
+  if (x.packed) return shared_tile_size(x, y);
+  const int own = x.route == y.route ? own_tile_size(x) : 0;   // (plain scales: the two small tiles, where both ask for the same one)
+  return own == 256 ? 0 : own;
+}
+
+int plan_gemm_two(const alto_mxfp4_product* first, const alto_mxfp4_product* second, GemmCall (&g)[2]) {
+  ALTO_REQUIRE(first && second, "gemm_two: NULL product");
+  for (int i = 0; i < 2; ++i) {
+    const alto_mxfp4_product& p = i ? *second : *first;
+    const int rc = p.packed ? plan_gemm_ps(p, g[i]) : plan_gemm(p, g[i]);
+    if (rc != ALTO_MXFP4_OK) return rc;
+  }
+  return ALTO_MXFP4_OK;
+}
+
 int launch_gemm(const GemmCall& g, hipStream_t st) {
   const GemmProblem& q = g.q;
   switch (g.route) {
@@ -165,28 +183,29 @@ extern "C" int alto_mxfp4_gemm(const uint8_t* a, int64_t lda, const uint8_t* a_s
 
 extern "C" int alto_mxfp4_gemm_two(const alto_mxfp4_product* first, const alto_mxfp4_product* second, void* stream) {
   using namespace alto;
-  ALTO_REQUIRE(first && second, "gemm_two: NULL product");
   GemmCall g[2];
-  for (int i = 0; i < 2; ++i) {
-    const alto_mxfp4_product& p = i ? *second : *first;
-    const int rc = p.packed ? plan_gemm_ps(p, g[i]) : plan_gemm(p, g[i]);
-    if (rc != ALTO_MXFP4_OK) return rc;
-  }
+  int rc = plan_gemm_two(first, second, g);
+  if (rc != ALTO_MXFP4_OK) return rc;
   hipStream_t st = (hipStream_t)stream;
   const bool swap = g[1].K > g[0].K;   // the longer tiles first
   const GemmCall &x = g[swap], &y = g[!swap];
-  if (x.route != Route::NONE && y.route != Route::NONE && x.packed == y.packed && x.c_dtype == y.c_dtype) {
-    // (plain scales: the two small tiles, where both ask for the same one)
-    const int own = x.route == y.route ? own_tile_size(x) : 0;
-    const int tile = x.packed ? shared_tile_size(x, y) : own == 256 ? 0 : own;
-    if (tile != 0) {
-      if (tile == 256) return gemm_tiled_launch_two(x.q, y.q, st);
-      gemm_mid_launch(tile, x.q, &y.q, x.c_dtype, x.packed, st);
-      return check_launch("gemm_two");
-    }
+  const int tile = tile_of_two(x, y);
+  if (tile == 256) return gemm_tiled_launch_two(x.q, y.q, st);
+  if (tile != 0) {
+    gemm_mid_launch(tile, x.q, &y.q, x.c_dtype, x.packed, st);
+    return check_launch("gemm_two");
   }
-  const int rc = launch_gemm(g[0], st);
+  rc = launch_gemm(g[0], st);
   return rc != ALTO_MXFP4_OK ? rc : launch_gemm(g[1], st);
+}
+
+extern "C" int alto_mxfp4_gemm_two_tile(const alto_mxfp4_product* first, const alto_mxfp4_product* second) {
+  using namespace alto;
+  GemmCall g[2];
+  const int rc = plan_gemm_two(first, second, g);
+  if (rc != ALTO_MXFP4_OK) return rc;
+  const bool swap = g[1].K > g[0].K;
+  return tile_of_two(g[swap], g[!swap]);
 }
 
 extern "C" int64_t alto_mxfp4_packed_scales_bytes(int64_t rows, int64_t K) {

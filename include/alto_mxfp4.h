@@ -178,7 +178,8 @@ int alto_mxfp4_quantize_ex(const void* x, int dtype, int64_t batch, int64_t M, i
 /*
  * Both operands of a layer's product in one call, both copies of each, round to nearest: what two calls of alto_mxfp4_quantize_ex
  * write, the activation x [M][K] with 1D blocks (Hadamard transform and clip on its column copy) and `batch` weight matrices
- * w [R][C] with 2D blocks, no clip; one launch for both unless one is too large for the caches.
+ * w [R][C] with 2D blocks, no clip.  One launch for both where they have the same type, use_uos is 0, neither moves more than the
+ * last-level cache holds and the weights are not so many that a workgroup takes eight bands of 32 rows; otherwise two.
  */
 int alto_mxfp4_quantize_operands(const void* x, int x_dtype, int64_t M, int64_t K, int64_t ld_x, uint8_t* x_row_codes, uint8_t* x_row_scales,
                                  uint8_t* x_col_codes, uint8_t* x_col_scales, int64_t ld_x_row, int64_t ld_x_col, int hadamard, const int8_t* signs,
@@ -276,8 +277,10 @@ int alto_mxfp4_gemm_ps(const uint8_t* a, int64_t lda, const uint8_t* a_packed, c
 
 /*
  * Two independent products in one call: what alto_mxfp4_gemm (packed == 0) or alto_mxfp4_gemm_ps (packed != 0: a_scales / b_scales are the
- * packed scales, the scale strides and is_2d flags are not read, c is bf16) make of each, the arguments as there.  Products
- * that take the same kernel share one launch.  The input and weight gradients of a layer are such a pair.
+ * packed scales, the scale strides and is_2d flags are not read, c is bf16) make of each, the arguments as there.  The input and weight
+ * gradients of a layer are such a pair.  They share one launch where both have packed scales, on the tile that suits the pair (unless
+ * one reduction is more than 16 times the other and the two would not take the same tile), and where both have plain scales, the
+ * same result type and the same tile of 64 or 128; otherwise they get a launch each.
  */
 typedef struct {
   const uint8_t *a, *a_scales, *b, *b_scales;
@@ -289,6 +292,8 @@ typedef struct {
   int a_is_2d, b_is_2d, c_dtype, packed;
 } alto_mxfp4_product;
 int alto_mxfp4_gemm_two(const alto_mxfp4_product* first, const alto_mxfp4_product* second, void* stream);
+/* What that call does with the two: the tile (64, 128 or 256) of the launch they share, 0: a launch each, negative: refused.  Host only. */
+int alto_mxfp4_gemm_two_tile(const alto_mxfp4_product* first, const alto_mxfp4_product* second);
 
 /*
  * Ragged grouped GEMM for MoE experts.  Rows [offs[g], offs[g+1]) of A form group g and use
@@ -505,6 +510,14 @@ int alto_mxfp4_attention_fwd_bf16q(const void* q, int64_t q_sb, int64_t q_sh, in
                                    int64_t Sq, int64_t Sk, int64_t D, int64_t Dv, int64_t o_sb, int64_t o_sh, int64_t o_ss, int64_t l_sb,
                                    int64_t l_sh, int64_t l_ss, int n_seqs, const int32_t* cu_q, const int32_t* cu_k, float sm_scale, int causal,
                                    void* stream);
+
+/*
+ * Rows of one workgroup of the attention kernel that the entries above take for a call without bias or ALiBi slopes: 32 (its waves
+ * deal out the keys) or 128 (each walks them all; always with bias or slopes).  Same bits either way.  Sk: the keys that exist; n_seqs, cu_q,
+ * cu_k as above.  Host only; negative: refused.
+ */
+int alto_mxfp4_attention_rows_per_workgroup(int64_t B, int64_t Hq, int64_t Sq, int64_t Sk, int64_t D, int n_seqs, const int32_t* cu_q, const int32_t* cu_k,
+                                            int causal);
 
 /*
  * Fills out[0 .. n) with random 32-bit words for stochastic rounding: word 4 c + j is word j of Philox4x32-10 (Salmon et

@@ -308,6 +308,22 @@ Entry g_bf16q_entries[] = {
                  k ? a.s[0] : a.s[3], a.s[4], a.s[5], a.s[6], a.s[7], a.s[8], a.p[5 * k + 4], a.s[9], a.f, a.i[0], a.i[1], a.i[2], a.i[3] == k};
        return alto_mxfp4_gemm_two(a.signs ? &q[0] : nullptr, a.perm ? &q[1] : nullptr, nullptr);
      }},
+    {"gemm_two_tile", 10, 4, 10, {{256, 16, 1, 256, 16, 1, 512, 512, 512, 512}, {0, 0, 0, 2}, {D, D, D, D, D, D, D, D, D, D}, 1.0f, {0, 0}, g_signs, g_perm},
+     [](const Args& a) {
+       alto_mxfp4_product q[2];
+       for (int k = 0; k < 2; ++k)
+         q[k] = {P(const uint8_t, 5 * k), P(const uint8_t, 5 * k + 1), P(const uint8_t, 5 * k + 2), P(const uint8_t, 5 * k + 3), k ? a.s[3] : a.s[0], a.s[1], a.s[2],
+                 k ? a.s[0] : a.s[3], a.s[4], a.s[5], a.s[6], a.s[7], a.s[8], a.p[5 * k + 4], a.s[9], a.f, a.i[0], a.i[1], a.i[2], a.i[3] == k};
+       const int tile = alto_mxfp4_gemm_two_tile(a.signs ? &q[0] : nullptr, a.perm ? &q[1] : nullptr);
+       return tile == 0 || tile == 64 || tile == 128 || tile == 256 ? 0 : tile;
+     }},
+    // B, Hq, Sq, Sk, D; boundaries, causal
+    {"attention_rows_per_workgroup", 5, 2, 0, {{1, 8, 256, 288, 128}, {0, 1}, {}, 1.0f, {0, 0}, g_signs, g_perm},
+     [](const Args& a) {
+       const Boundaries& b = g_bounds[(unsigned)a.i[0] % (kManySequences + 1)];
+       const int rows = alto_mxfp4_attention_rows_per_workgroup(a.s[0], a.s[1], a.s[2], a.s[3], a.s[4], b.n, b.q, b.k, a.i[1]);
+       return rows == 32 || rows == 128 ? 0 : rows;
+     }},
     {"grouped_gemm_offsets", 0, 1, 2, {{}, {32}, {D, D}, 1.0f, {0, 0}, g_signs, g_perm},
      [](const Args& a) { return alto_mxfp4_grouped_gemm_offsets(P(const int32_t, 0), a.i[0], P(int32_t, 1), nullptr); }},
 };

@@ -344,3 +344,34 @@ def test_host_module_is_stale_for_another_torch_interpreter_or_source(monkeypatc
         with pytest.raises(_lib.AltoMxfp4Error, match="was not built"):
             _lib.host()
     assert not B.host_is_stale()
+
+
+def test_host_only_queries_of_the_dispatch():
+    """Which attention kernel and which shared tile a call takes: both sides of each rule (sizes from the tables beside them), and the
+    argument checks of the calls themselves."""
+    from alto_amd import _lib
+    from tests.test_gpu_gemm_two import Product
+    lib = _lib.load()
+
+    def rows(B, Hq, Sq, Sk, D, causal, cu=None):
+        n = 0 if cu is None else len(cu) - 1
+        c = None if cu is None else (ctypes.c_int32 * (n + 1))(*cu)
+        return lib.alto_mxfp4_attention_rows_per_workgroup(B, Hq, Sq, Sk, D, n, c, c, int(causal))
+
+    assert [rows(1, h, s, s, 128, True) for h, s in ((8, 1024), (12, 4096), (24, 2048), (32, 2048))] == [32, 32, 128, 128]
+    assert [rows(1, h, s, s, 128, False) for h, s in ((24, 1024), (28, 1024), (8, 4096))] == [32, 128, 128]
+    assert rows(4, 32, 2048, 2048, 128, True) == 128 and rows(1, 16, 2048, 2048, 64, True) == 32 and rows(1, 16, 1024, 1024, 256, False) == 32
+    assert rows(1, 4, 544, 544, 64, True, [0, 96, 544]) == 32 and rows(1, 4, 96 * 800, 96 * 800, 64, True, list(range(0, 96 * 801, 96))) == 128
+    assert rows(1, 4, 96, 96, 64, True, [0, 40, 96]) == -1 and b"multiples of 32" in lib.alto_mxfp4_last_error()
+    assert rows(0, 4, 96, 96, 64, True) == -1
+
+    p = 4096   # (an address no call here reads)
+
+    def tile(T, K, N, packed=(1, 1), dtype=0):
+        def one(M, N, K, packed):
+            return Product(p, p, p, p, K // 2, K // 32, 1, K // 2, K // 32, 1, M, N, K, p, N, 1.0, 0, 0, dtype, packed)
+        return lib.alto_mxfp4_gemm_two_tile(ctypes.byref(one(T, K, N, packed[0])), ctypes.byref(one(N, K, T, packed[1])))
+
+    assert [tile(*s) for s in ((512, 512, 512), (1024, 2048, 2048), (2048, 2048, 2048), (512, 1024, 13440))] == [64, 128, 256, 0]
+    assert tile(512, 1024, 1024, (0, 0)) == 64 and tile(8192, 4096, 4096, (0, 0)) == 0 and tile(544, 1024, 512, (1, 0)) == 0
+    assert tile(512, 512, 520) == -1 and tile(96, 512, 512) == -3   # a reduction that is not whole blocks; fewer rows than packed scales serve
