@@ -52,3 +52,13 @@ def snr_db(ref: torch.Tensor, got: torch.Tensor) -> float:
     r, g = ref.double().cpu(), got.double().cpu()
     noise = ((r - g) ** 2).sum()
     return float("inf") if noise == 0 else float(10 * torch.log10((r ** 2).sum() / noise))
+
+
+def attention_rows(B, Hq, Sq, Sk, D, causal, cu_q=None, cu_k=None):
+    """32 or 128: which of the two attention kernels a call without bias or ALiBi slopes takes (rows of one workgroup)."""
+    import ctypes
+
+    from alto_amd import _lib
+    n = 0 if cu_q is None else len(cu_q) - 1
+    c = [None, None] if cu_q is None else [(ctypes.c_int32 * (n + 1))(*b) for b in (cu_q, cu_k)]
+    return _lib.load().alto_mxfp4_attention_rows_per_workgroup(B, Hq, Sq, Sk, D, n, *c, int(causal))

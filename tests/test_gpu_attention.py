@@ -10,6 +10,7 @@ import torch
 
 from oracle import mxfp4_oracle as O
 from oracle.attention_oracle import attention_fp32_ref, attention_fwd_ref
+from tests.helpers import attention_rows
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
@@ -251,7 +252,7 @@ def test_reference_attention_configs(m, cfg):
     similarity without a threshold (test_mxfp_attention.py:122-128).  Here the same comparison carries floors chosen
     below what MXFP4 operands and probabilities give on this data (observed 12.1 to 12.3 dB, cosine 0.970 to 0.972): a wrong mask
     offset, head mapping or scale block would fall far below them."""
-    from tests.helpers import snr_db
+    from tests.helpers import attention_rows, snr_db
     S, Hq, Hk, D, Dv = cfg
     B = 4
     g = torch.Generator(device=DEV).manual_seed(1234)
@@ -348,6 +349,54 @@ def test_scale_bytes_behind_the_keys_are_not_used(m, D, Dv, causal):
             ref, ref_lse = attention_fwd_ref(q[:, :, q0:q1], k[:, :, k0:k1], v[:, :, k0:k1], causal=causal)
             assert _rel(out[:, :, q0:q1].cpu(), ref) <= REL_L2
             assert float((lse[:, :, q0:q1].cpu() - ref_lse).abs().max()) <= 1e-4
+
+
+@pytest.mark.parametrize("D,Dv", [(64, 64), (64, 128), (128, 64), (128, 128), (192, 64), (256, 128)])
+@pytest.mark.parametrize("causal", [True, False])
+def test_scale_bytes_behind_the_keys_are_not_used_by_large_launches(m, D, Dv, causal):
+    """The same for launches with so many rows that every wave walks all keys.  Behind the last head's bands lie the 16 bytes of the
+    buffer's end; behind every other head's last band lie the next head's first scales, here the E8M0 NaN for one of them."""
+    for Hq, Hk, Sq, Sk, lens in ((2, 1, 32, 32, None), (4, 2, 96, 96, None), (2, 2, 160, 288, None), (4, 2, 0, 0, [96, 160, 32])):
+        B = 1
+        if lens is None:
+            while attention_rows(B, Hq, Sq, Sk, D, causal) == 32:
+                B += 64
+            seqs = None
+        else:   # packed sequences of odd numbers of bands
+            cu = [0]
+            while attention_rows(1, Hq, cu[-1] or 32, cu[-1] or 32, D, causal, cu if cu[-1] else [0, 32], cu if cu[-1] else [0, 32]) == 32:
+                cu += (torch.tensor(lens * 64).cumsum(0) + cu[-1]).tolist()
+            Sq = Sk = cu[-1]
+            seqs = (cu, cu)
+        g = torch.Generator(device=DEV).manual_seed(Sq + D)
+        q, k, v = (torch.randn(B, H, S, d, generator=g, device=DEV).to(torch.bfloat16) for H, S, d in ((Hq, Sq, D), (Hk, Sk, D), (Hk, Sk, Dv)))
+        operands = m.quantize_qkv(q, k, v)
+        dims = (B, Hq, Hk, Sq, Sk, D, Dv)
+        out, lse = _strided_call(operands, dims, causal, 0x7F, seqs)
+        for fill in (0xFF, 0):
+            o, l = _strided_call(operands, dims, causal, fill, seqs)
+            assert torch.equal(o, out) and torch.equal(l, lse), (dims, fill)
+        # the small launches' kernel, which the test above checks against the oracle, has the same bits
+        last = cu[-2] if seqs else 0
+        if seqs is None:
+            o, l = _strided_call([t[-1:].contiguous() for t in operands], (1, *dims[1:]), causal, 0xFF)
+        else:
+            qq, qs, kq, ks, vq, vs = operands
+            part = (qq[:, :, last:], qs[:, :, last // 32:], kq[:, :, last:], ks[:, :, last // 32:], vq[..., last // 2:], vs[:, :, last // 32:])
+            o, l = _strided_call([t.contiguous() for t in part], (1, Hq, Hk, Sq - last, Sk - last, D, Dv), causal, 0xFF)
+        assert torch.equal(o[0], out[-1, :, last:]) and torch.equal(l[0], lse[-1, :, last:]), dims
+        qq, qs, kq, ks, vq, vs = operands
+        bad = vs.clone()
+        if seqs is None:   # the first band of the second head of the buffer
+            bad[1 if Hk == 1 else 0, 0 if Hk == 1 else 1, 0] = 0xFF
+            rows = (1, slice(None)) if Hk == 1 else (0, slice(Hq // Hk, 2 * Hq // Hk))
+        else:              # the first band of the second sequence
+            bad[:, :, cu[1] // 32] = 0xFF
+            rows = (slice(None), slice(None), slice(cu[1], cu[2]))
+        o, l = _strided_call((qq, qs, kq, ks, vq, bad), dims, causal, 0x7F, seqs)
+        assert o[rows].isnan().any()
+        o[rows] = out[rows]
+        assert torch.equal(o, out) and torch.equal(l, lse), dims
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])

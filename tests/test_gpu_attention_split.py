@@ -4,6 +4,8 @@ Every case runs a few sequences alone and the same ones inside a batch that is t
 import pytest
 import torch
 
+from tests.helpers import attention_rows
+
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
 
@@ -40,6 +42,7 @@ def test_split_kernel_equals_the_unsplit_one(m, dims, causal, dtype):
         for i in (0, B - 1):
             out, lse, _ = m.triton_attention_mxfp4(q[i:i + 1], k[i:i + 1], v[i:i + 1], causal=causal)
             assert torch.equal(out[0], big[i]) and torch.equal(lse[0], big_lse[i]), (Sq, Sk, i)
+        assert attention_rows(1, Hq, Sq, Sk, D, causal) == 32 and attention_rows(B, Hq, Sq, Sk, D, causal) == 128, (Sq, Sk)
 
 
 @pytest.mark.parametrize("D", [64, 128, 256])
@@ -55,6 +58,7 @@ def test_split_kernel_packed_sequences(m, D):
         big, big_lse, _ = m.triton_attention_mxfp4(*(t.repeat(times, 1, 1) for t in (q, k, v)), cu_seqlens_q=many, cu_seqlens_k=many, causal=causal, layout="thd")
         assert torch.equal(big[:one[-1]], out) and torch.equal(big_lse[:one[-1]], lse)
         assert torch.equal(big[-one[-1]:], out) and torch.equal(big_lse[-one[-1]:], lse)
+        assert attention_rows(1, 4, one[-1], one[-1], D, causal, one, one) == 32 and attention_rows(1, 4, many[-1], many[-1], D, causal, many, many) == 128
 
 
 def test_split_kernel_special_values(m):
@@ -73,3 +77,4 @@ def test_split_kernel_special_values(m):
         big, big_lse, _ = m.triton_attention_mxfp4(*(t.repeat(B, 1, 1, 1) for t in (q, k, v)), causal=causal)
         assert torch.equal(out[0].view(torch.int16), big[1].view(torch.int16)) and torch.equal(lse[0].isnan(), big_lse[1].isnan())
         assert torch.equal(lse[0].nan_to_num(0.0), big_lse[1].nan_to_num(0.0))
+        assert attention_rows(1, Hq, S, S, D, causal) == 32 and attention_rows(B, Hq, S, S, D, causal) == 128
