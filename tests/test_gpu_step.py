@@ -1,5 +1,7 @@
 """A layer's training step in one native call per direction against the general autograd functions: the same launches on the same
 operands, so outputs and gradients are the same bit for bit, with the same draws from torch's CPU generator."""
+import contextlib
+
 import pytest
 import torch
 
@@ -21,11 +23,35 @@ def _same(got, want, what=""):
         assert a.shape == b.shape and a.dtype == b.dtype and torch.equal(a, b), (what, name)
 
 
-def _linear(fn, x, w, go, h, clip="none", sr=True, uos=False, dge=False, seed=5):
+@contextlib.contextmanager
+def _routes():
+    """Counts the directions of steps that the native calls declined (the general functions' own calls among them)."""
+    from alto_amd.mxfp4 import grouped_gemm as G
+    from alto_amd.mxfp4 import linear as L
+    count = dict(forward=0, backward=0)
+
+    def counted(fn, what):
+        def call(*a, **k):
+            count[what] += 1
+            return fn(*a, **k)
+        return call
+
+    with pytest.MonkeyPatch.context() as p:
+        for owner, fwd, bwd in ((L, L.MXFP4LinearFunction, "_linear_backward"), (G, G.MXFP4GroupedGEMM, "_grouped_backward")):
+            p.setattr(fwd, "forward", staticmethod(counted(fwd.forward, "forward")))
+            p.setattr(owner, bwd, counted(getattr(owner, bwd), "backward"))
+        yield count
+
+
+def _linear(fn, x, w, go, h, clip="none", sr=True, uos=False, dge=False, seed=5, native=None):
+    """native: what the native calls of a step must have served, (forward, backward)."""
     torch.manual_seed(seed)
     xg, wg = x.detach().requires_grad_(True), w.detach().requires_grad_(True)
-    y = fn.apply(xg, wg, False, True, sr, dge, clip, False, h, uos)
-    dx, dw = torch.autograd.grad(y, (xg, wg), go)
+    with _routes() as declined:
+        y = fn.apply(xg, wg, False, True, sr, dge, clip, False, h, uos)
+        dx, dw = torch.autograd.grad(y, (xg, wg), go)
+    if native is not None:
+        assert (declined["forward"] == 0, declined["backward"] == 0) == native
     return y.detach(), dx, dw, torch.randint(0, 2 ** 62, (1,))
 
 
@@ -41,7 +67,8 @@ def test_linear_step_equals_the_general_function(m, M, N, K, dtype, clip, uos, d
     x, w = randn_outliers((M, K), dtype, seed=1).to(DEV), randn_outliers((N, K), dtype, seed=2).to(DEV)
     go = (randn_outliers((M, N), dtype, seed=3) / (M * N)).to(DEV)
     h = m.HadamardTransform(*hadamard_from_seed(11)) if had else None
-    a, b = (_linear(f, x, w, go, h, clip, sr, uos, dge) for f in (MXFP4LinearStep, m.MXFP4LinearFunction))
+    a = _linear(MXFP4LinearStep, x, w, go, h, clip, sr, uos, dge, native=(True, True))
+    b = _linear(m.MXFP4LinearFunction, x, w, go, h, clip, sr, uos, dge, native=(False, False))
     _same(a[:3], b[:3])
     assert torch.equal(a[3], b[3])   # as many words taken from the generator
 
@@ -59,12 +86,14 @@ def test_linear_step_operand_forms(m):
           "transposed": big[:, :K].contiguous().t().contiguous().t()}
     for name, x in xs.items():
         g = go.view(*x.shape[:-1], N)
-        _same(_linear(MXFP4LinearStep, x, w, g, h)[:3], _linear(m.MXFP4LinearFunction, x, w, g, h)[:3], name)
+        served = name in ("3d", "rows strided")
+        _same(_linear(MXFP4LinearStep, x, w, g, h, native=(served, served))[:3], _linear(m.MXFP4LinearFunction, x, w, g, h)[:3], name)
     x = xs["rows strided"]
     for name, g in {"expanded": go[:1, :1].expand(M, N), "transposed": go.t().contiguous().t()}.items():
-        _same(_linear(MXFP4LinearStep, x, w, g, h)[:3], _linear(m.MXFP4LinearFunction, x, w, g, h)[:3], name)
+        _same(_linear(MXFP4LinearStep, x, w, g, h, native=(True, False))[:3], _linear(m.MXFP4LinearFunction, x, w, g, h)[:3], name)
     for name, ww in {"strided": torch.nn.functional.pad(w, (8, 8))[:, 8:K + 8], "transposed": w.t().contiguous().t(), "fp32": w.float()}.items():
-        _same(_linear(MXFP4LinearStep, x, ww, go, h)[:3], _linear(m.MXFP4LinearFunction, x, ww, go, h)[:3], name)
+        served = name != "transposed"
+        _same(_linear(MXFP4LinearStep, x, ww, go, h, native=(served, served))[:3], _linear(m.MXFP4LinearFunction, x, ww, go, h)[:3], name)
     for fn in (MXFP4LinearStep, m.MXFP4LinearFunction):   # (the weight gradient's operand has blocks of 32 tokens)
         with pytest.raises(RuntimeError):
             fn.apply(x[:40], w, False, True, False, False, "none", False, None, False)
@@ -77,25 +106,25 @@ def test_linear_step_saved_tensor_hooks_modes_and_repeats(m):
     go = (randn_outliers((256, 160), torch.bfloat16, seed=3) / 256).to(DEV)
     h = m.HadamardTransform(*hadamard_from_seed(5))
     with torch.autograd.graph.save_on_cpu():
-        a = _linear(MXFP4LinearStep, x, w, go, h)
+        a = _linear(MXFP4LinearStep, x, w, go, h, native=(True, True))
     _same(a[:3], _linear(m.MXFP4LinearFunction, x, w, go, h)[:3], "saved on the host")
     with torch.autograd.graph.saved_tensors_hooks(lambda t: t, lambda t: torch.cat([t.new_zeros(3), t])[3:]):   # back at an odd address
-        a = _linear(MXFP4LinearStep, x, w, go, h)
+        a = _linear(MXFP4LinearStep, x, w, go, h, native=(True, False))
     _same(a[:3], _linear(m.MXFP4LinearFunction, x, w, go, h)[:3], "saved off alignment")
     m.use_hardware_stochastic_rounding(False)
     try:
-        _same(_linear(MXFP4LinearStep, x, w, go, h)[:3], _linear(m.MXFP4LinearFunction, x, w, go, h)[:3], "software rounding")
+        _same(_linear(MXFP4LinearStep, x, w, go, h, native=(True, False))[:3], _linear(m.MXFP4LinearFunction, x, w, go, h)[:3], "software rounding")
     finally:
         m.use_hardware_stochastic_rounding(True)
     r = torch.randint(-2 ** 31, 2 ** 31, (256, 160), dtype=torch.int64).to(torch.int32).to(DEV)
     m.set_rand_bits_source(lambda shape, d: r)
     try:
-        _same(_linear(MXFP4LinearStep, x, w, go, h)[:3], _linear(m.MXFP4LinearFunction, x, w, go, h)[:3], "words from a source")
+        _same(_linear(MXFP4LinearStep, x, w, go, h, native=(True, False))[:3], _linear(m.MXFP4LinearFunction, x, w, go, h)[:3], "words from a source")
     finally:
         m.set_rand_bits_source(None)
     m.enable_device_philox_state(seed=9)
     try:
-        a = _linear(MXFP4LinearStep, x, w, go, h)
+        a = _linear(MXFP4LinearStep, x, w, go, h, native=(True, False))
         m.enable_device_philox_state(seed=9)
         _same(a[:3], _linear(m.MXFP4LinearFunction, x, w, go, h)[:3], "device state")
     finally:
@@ -112,14 +141,21 @@ def _grouped(m, fn, x, w, go, offs, trans, seed=5, **kw):
     h = m.HadamardTransform(*hadamard_from_seed(7)) if kw.get("had", True) else None
     sr, dge, clip, uos = kw.get("sr", True), kw.get("dge", False), kw.get("clip", "none"), kw.get("uos", False)
     xg, wg = x.detach().requires_grad_(True), w.detach().requires_grad_(True)
+    with _routes() as declined:
+        out, dx, dw = _grouped_call(G, fn, xg, wg, go, offs, trans, sr, dge, clip, h, uos, kw.get("dense", True))
+    if kw.get("native") is not None:
+        assert (declined["forward"] == 0, declined["backward"] == 0) == kw["native"]
+    return out.detach(), dx, dw, torch.randint(0, 2 ** 62, (1,))
+
+
+def _grouped_call(G, fn, xg, wg, go, offs, trans, sr, dge, clip, h, uos, dense):
     if fn == "step":
         out = G.MXFP4GroupedStep.apply(xg, wg, offs, False, trans, sr, dge, clip, h, uos)
     elif fn == "ends":
-        out = G.MXFP4GroupedStep.apply(xg, wg, offs[1:].contiguous() if kw.get("dense", True) else offs[1:].long(), True, trans, sr, dge, clip, h, uos)
+        out = G.MXFP4GroupedStep.apply(xg, wg, offs[1:].contiguous() if dense else offs[1:].long(), True, trans, sr, dge, clip, h, uos)
     else:
         out = G.MXFP4GroupedGEMM.apply(xg, wg, None, trans, False, True, sr, dge, clip, False, h, uos, offs)
-    dx, dw = torch.autograd.grad(out, (xg, wg), go)
-    return out.detach(), dx, dw, torch.randint(0, 2 ** 62, (1,))
+    return (out, *torch.autograd.grad(out, (xg, wg), go))
 
 
 @pytest.mark.parametrize("N,K", [(768, 1280), (512, 2880), (288, 512), (128, 96)])
@@ -132,9 +168,57 @@ def test_grouped_step_equals_the_general_function(m, N, K, trans, kw):
     go = (randn_outliers((1024, N), torch.bfloat16, seed=34) / (1024 * N)).to(DEV)
     ref = _grouped(m, "general", x, w, go, offs, trans, **kw)
     for fn, more in (("step", {}), ("ends", {}), ("ends", dict(dense=False))):
-        got = _grouped(m, fn, x, w, go, offs, trans, **kw, **more)
+        served = min(N, K) >= 512 and "dense" not in more   # (both directions' reductions are long enough for packed scales; ends are int32)
+        got = _grouped(m, fn, x, w, go, offs, trans, **kw, **more, native=(served, served))
         _same(got[:3], ref[:3], (fn, more))
         assert torch.equal(got[3], ref[3])
+
+
+def test_grouped_step_forms_and_hooks_of_native_calls(m):
+    """Shapes that the native calls serve: what else makes them decline, in the forward or in the backward alone."""
+    N, K = 544, 800
+    offs = torch.tensor([0, 96, 800, 1024], dtype=torch.int32, device=DEV)
+    x = randn_outliers((1024, K), torch.bfloat16, seed=31).to(DEV)
+    w = randn_outliers((3, N, K), torch.bfloat16, seed=32).to(DEV)
+    go = (randn_outliers((1024, N), torch.bfloat16, seed=34) / 1024).to(DEV)
+    ref = _grouped(m, "general", x, w, go, offs, True, native=(False, False))
+    step = lambda *a, native: _grouped(m, "step", *a, native=native)[:3]
+    _same(step(x, w, go, offs, True, native=(True, True)), ref[:3], "plain")
+    with torch.autograd.graph.save_on_cpu():
+        _same(step(x, w, go, offs, True, native=(True, True)), ref[:3], "saved on the host")
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: t, lambda t: torch.cat([t.new_zeros(1), t])[1:] if t.dtype == torch.uint8 and t.numel() > 1 << 16 else t):
+        _same(step(x, w, go, offs, True, native=(True, False)), ref[:3], "codes saved off alignment")
+    for name, args, native in (("fp32", (x.float(), w.float(), go.float(), offs), (False, False)), ("fp32 weights", (x, w.float(), go, offs), (True, True)),
+                               ("rows strided", (torch.nn.functional.pad(x, (8, 8))[:, 8:K + 8], w, go, offs), (False, False)),
+                               ("expanded", (x, w, go[:1, :1].expand(1024, N), offs), (True, False)), ("transposed", (x, w, go.t().contiguous().t(), offs), (True, False)),
+                               ("few rows", (x[:256], w, go[:256], (offs / 4).int() // 32 * 32), (False, False))):
+        _same(step(*args, True, native=native), _grouped(m, "general", *args, True)[:3], name)
+    m.use_hardware_stochastic_rounding(False)
+    try:
+        _same(step(x, w, go, offs, True, native=(True, False)), _grouped(m, "general", x, w, go, offs, True)[:3], "software rounding")
+    finally:
+        m.use_hardware_stochastic_rounding(True)
+
+
+def test_public_calls_take_the_native_steps(m):
+    """A wrapped linear layer and both grouped entries, as a program calls them; the options outside the everyday call do not."""
+    x, w = randn_outliers((512, 544), torch.bfloat16, seed=1).to(DEV), randn_outliers((640, 544), torch.bfloat16, seed=2).to(DEV)
+    offs = torch.tensor([0, 96, 320, 512], dtype=torch.int32, device=DEV)
+    e = randn_outliers((3, 544, 640), torch.bfloat16, seed=3).to(DEV)
+
+    def step(config):
+        p, pe = (torch.nn.Parameter(m.MXFP4TrainingWeightWrapperTensor(t.clone(), config)) for t in (w, e))
+        torch.nn.functional.linear(x, p).sum().backward()
+        torch._grouped_mm(x.clone().requires_grad_(True), pe, offs=offs[1:].contiguous()).backward(torch.ones(512, 640, device=DEV, dtype=torch.bfloat16))
+
+    with _routes() as declined:
+        step(m.TrainingOpConfig())
+        out = m.mxfp4_grouped_gemm(x.clone().requires_grad_(True), e, None, trans_weights=False, offsets=offs)
+        out.backward(torch.ones_like(out))
+    assert declined == dict(forward=0, backward=1)   # (the gradient of a sum is expanded, with no strides)
+    with _routes() as declined:
+        step(m.TrainingOpConfig(use_2dblock_x=True, use_hadamard=False))
+    assert declined == dict(forward=2, backward=2)
 
 
 def test_grouped_step_forms_and_hooks(m):
