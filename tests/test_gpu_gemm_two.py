@@ -54,24 +54,26 @@ def alone(p):
 BF, F32 = torch.bfloat16, torch.float32
 
 
-@pytest.mark.parametrize("T,K,N,packed,dtype", [
-    (512, 512, 512, (1, 1), BF),       # 64x64 tiles, one block of K
-    (544, 520, 1056, (1, 1), BF),      # ragged in every direction
-    (1024, 4096, 4096, (1, 1), BF),    # 128x128
-    (672, 2528, 7488, (1, 1), BF),     # 128x128, ragged
-    (2048, 4096, 4096, (1, 1), BF),    # 256x256, K a multiple of 512 in both
-    (4096, 2592, 2592, (1, 1), BF),    # 256x256, the last block of one reduction half empty
-    (2144, 5696, 3008, (1, 1), BF),    # 256x256, both reductions end inside a block
-    (2336, 4096, 4608, (1, 1), BF),    # 256x256, one of them
-    (512, 1024, 13440, (1, 1), BF),    # reductions more than 16 times apart: a launch each
-    (512, 10208, 13440, (1, 1), BF),   # ... but both on the large tile
-    (512, 1024, 1024, (0, 0), BF),     # plain scales
-    (1376, 2880, 2144, (0, 0), F32),
-    (96, 64, 1024, (0, 0), BF),        # few rows and the direct kernel
-    (544, 1024, 512, (1, 0), BF),      # one of each
-    (0, 512, 512, (0, 0), BF),         # an empty product
+@pytest.mark.parametrize("T,K,N,packed,dtype,tile", [   # tile: of the launch they share, 0: a launch each
+    (512, 512, 512, (1, 1), BF, 64),       # one block of K
+    (544, 520, 1056, (1, 1), BF, 64),      # ragged in every direction
+    (1024, 2048, 4096, (1, 1), BF, 128),   # K a multiple of 512 in both
+    (672, 2528, 7488, (1, 1), BF, 128),    # ragged
+    (1024, 4096, 4096, (1, 1), BF, 256),   # K a multiple of 512 in both
+    (2048, 4096, 4096, (1, 1), BF, 256),
+    (4096, 2592, 2592, (1, 1), BF, 256),   # the last block of one reduction half empty
+    (2144, 5696, 3008, (1, 1), BF, 256),   # both reductions end inside a block
+    (2336, 4096, 4608, (1, 1), BF, 256),   # one of them
+    (512, 1024, 13440, (1, 1), BF, 0),     # reductions more than 16 times apart
+    (512, 10208, 13440, (1, 1), BF, 256),  # ... but both ask for the large tile
+    (512, 1024, 1024, (0, 0), BF, 64),     # plain scales
+    (1376, 2880, 2144, (0, 0), F32, 128),
+    (2048, 4096, 4096, (0, 0), BF, 0),     # both on the large tile
+    (96, 64, 1024, (0, 0), BF, 0),         # few rows and the direct kernel
+    (544, 1024, 512, (1, 0), BF, 0),       # one of each
+    (0, 512, 512, (0, 0), BF, 0),          # an empty product
 ])
-def test_two_products_are_the_two_calls(T, K, N, packed, dtype):
+def test_two_products_are_the_two_calls(T, K, N, packed, dtype, tile):
     g = torch.Generator(device="cuda").manual_seed(T + K + N)
     x, dx, keep_x = product(T, K, N, packed[0], dtype, 1.0, g)
     w, dw, keep_w = product(N, K, T, packed[1], dtype, 0.25, g) if T else product(N, K, 512, packed[1], dtype, 0.25, g)
@@ -79,6 +81,7 @@ def test_two_products_are_the_two_calls(T, K, N, packed, dtype):
     alone(w)
     want = dx.clone(), dw.clone()
     for first, second in ((x, w), (w, x)):
+        assert _lib.load().alto_mxfp4_gemm_two_tile(ctypes.byref(first), ctypes.byref(second)) == tile
         dx.fill_(7.0)
         dw.fill_(7.0)
         _lib.check(_lib.load().alto_mxfp4_gemm_two(ctypes.byref(first), ctypes.byref(second), stream()), "gemm_two")
