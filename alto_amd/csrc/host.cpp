@@ -633,4 +633,8 @@ PYBIND11_MODULE(alto_mxfp4_host, m) {
   m.def("grouped_backward", &grouped_backward);
   m.def("grouped_saved", &grouped_saved);
   m.def("draw_hadamard", &draw_hadamard);
+  // (the rules that linear.py and grouped_gemm.py state as well, for a comparison of the two)
+  m.def("packed_gemm_supported", &packed_gemm_supported);
+  m.def("grouped_packed_supported", &grouped_packed_supported);
+  m.def("grouped_dw_packed_supported", &grouped_dw_packed_supported);
 }

@@ -375,3 +375,29 @@ def test_host_only_queries_of_the_dispatch():
     assert [tile(*s) for s in ((512, 512, 512), (1024, 2048, 2048), (2048, 2048, 2048), (512, 1024, 13440))] == [64, 128, 256, 0]
     assert tile(512, 1024, 1024, (0, 0)) == 64 and tile(8192, 4096, 4096, (0, 0)) == 0 and tile(544, 1024, 512, (1, 0)) == 0
     assert tile(512, 512, 520) == -1 and tile(96, 512, 512) == -3   # a reduction that is not whole blocks; fewer rows than packed scales serve
+
+
+def test_native_and_python_rules_for_packed_scales_agree():
+    """The native steps choose between packed and plain scales by the same rules as the general functions: compared at the limits of every
+    condition, alone and with each other, and over the sizes between."""
+    import itertools
+    import random
+
+    from alto_amd import _lib
+    from alto_amd.mxfp4 import grouped_gemm as G
+    from alto_amd.mxfp4 import linear as L
+    host = _lib.host()
+    edges = [8, 96, 120, 127, 128, 136, 480, 511, 512, 520, 544, 1024, 2880, 4100, 14336, 65536, 2 ** 20, 2 ** 22, 2 ** 22 + 32, 2 ** 25, 2 ** 28, 2 ** 31 - 32]
+    rng = random.Random(5)
+    drawn = [tuple(int(2 ** rng.uniform(3, 31)) // 8 * 8 for _ in range(3)) for _ in range(4000)]
+    seen = {n: set() for n in ("linear", "grouped", "dw")}
+    for M, N, K in itertools.chain(itertools.product(edges, repeat=3), drawn):
+        a = L.packed_gemm_supported(M, N, K)
+        assert host.packed_gemm_supported(M, N, K) == a, (M, N, K)
+        seen["linear"].add(a)
+        for groups in (1, 32, 4096, 32768, 32769, 65535, 65536):
+            a, b = G.grouped_packed_supported(M, N, K, groups), G.grouped_dw_packed_supported(M, N, K, groups, groups)
+            assert host.grouped_packed_supported(M, N, K, groups) == a and host.grouped_dw_packed_supported(M, N, K, groups, groups) == b, (M, N, K, groups)
+            seen["grouped"].add(a)
+            seen["dw"].add(b)
+    assert all(s == {True, False} for s in seen.values())
