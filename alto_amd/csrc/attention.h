@@ -108,8 +108,8 @@ __device__ __forceinline__ void wave_lds_order() {
 // A wave's 32 rows of Q, straight from bf16, as the score product takes them: lane (r = lane % 32, h = lane / 32) gets the codes of
 // row r, columns 64 s + 32 h .. + 32, and the scale byte of that 32 x 32 block.  The loads are whole 128-byte lines (8 lanes a row,
 // 8 rows an instruction; a lane that fetched its own 64 bytes cost 32 line lookups an instruction instead of 8); the codes change
-// lanes through `scratch`, NK KB of LDS that only this wave uses, at consecutive addresses both ways.  Codes and scales are those
-// of alto_mxfp4_attention_quantize.
+// lanes through `scratch`, NK KB of LDS that only this wave uses, at consecutive addresses (two rows meet in a bank on the way out:
+// 4 cycles a read).  Codes and scales are those of alto_mxfp4_attention_quantize.
 template <int NK>
 __device__ __forceinline__ void quantize_q(const __bf16* x, int64_t row_stride, int lane, uint8_t* scratch, v8i_t (&qf)[NK], int (&qsc)[NK]) {
   uint32_t w[NK][4][4];

@@ -40,10 +40,11 @@ struct AttnTile {
 // before the running maximum (:288-308); a separate instantiation, the plain one carries none of it.
 // QBF: Q comes as bf16 values and every wave quantizes its own rows (no other wave reads them), which saves writing the codes
 // and reading them back and leaves the operand quantizer K and V only.  4 x 2048 tokens, 64 / 8 heads of 128, causal (134 of the
-// 168 MB are Q), operand quantizer + this kernel, us: on codes 38.9 + 181.5; every lane fetching the 64 bytes it multiplies
-// 10.6 + 201, whole lines (quantize_q) 10.9 + 197, at raised wave priority 10.6 + 195 (the two other workgroups of the compute unit
-// hide the wait, the priority lets the arithmetic behind it through), with the heads dealt to the XCDs in ranges 10.3 + 187, with the
-// results stored as whole rows 10.7 + 181, Q read non-temporally 8.7 + 179.
+// 168 MB are Q), changing inputs, us: quantizer and this kernel on codes 38.8 and 169.5, 201 together; with QBF 8.8 and 181, 187
+// together (another box: 38.6 and 162.7, 193.5; 8.8 and 171.8, 181).  How the kernel with QBF got there: every lane fetching the 64
+// bytes it multiplies 201, whole lines (quantize_q) 197, at raised wave priority 195 (the two other workgroups of the compute unit hide the
+// wait, the priority lets the arithmetic behind it through), Q read non-temporally 2 less; of use to the kernel on codes as well:
+// the heads dealt to the XCDs in ranges 195 -> 187, the results stored as whole rows 187 -> 181.
 // SEQS: AttnSeqs, or AttnNoSeqs for B sequences of one length.
 template <int NK, int ND, bool BIASED, bool QBF, typename SEQS>
 __device__ __forceinline__ void attn_fwd_body(const AttnArgs& a, const SEQS& seqs, __bf16* __restrict__ out, float* __restrict__ lse_out, uint8_t* ring) {
@@ -310,8 +311,9 @@ __device__ __forceinline__ void attn_fwd_body(const AttnArgs& a, const SEQS& seq
   if (!live) return;
 
   // ---- O = acc / l, bf16; log-sum-exp.  The rows change lanes through the LDS (the ring is no longer read: every wave has passed
-  // the loop's last barrier; each wave uses a part of its own), so that a store instruction writes whole rows (8-byte pieces of 32 rows an instruction before: 187 -> 181 us, QBF above).  16-byte piece c of
-  // row r goes to position c ^ (r / (16 / PR)) % PR, PR pieces per row: no bank conflicts either way.
+  // the loop's last barrier; each wave uses a part of its own), so that a store instruction writes whole rows (8-byte pieces of 32 rows
+  // an instruction before: 187 -> 181 us, QBF above).  16-byte piece c of row r goes to position c ^ (r / (16 / PR)) % PR, PR pieces per
+  // row: the reads are free of bank conflicts, in the writes two rows meet (Dv = 128: 4 cycles each, 64 a wave; 1 % of the kernel's).
   const float l = acc_l[0];
   const float rl = 1.0f / l;
   constexpr int PR = DV / 8;
