@@ -12,6 +12,7 @@
 #include <torch/csrc/utils/pybind.h>
 
 #include <ATen/ATen.h>
+#include <c10/core/impl/LocalDispatchKeySet.h>
 
 #include <algorithm>
 #include <optional>
@@ -301,6 +302,9 @@ struct Failure {
   }
 };
 
+// (torch.jit.trace would record the outputs' allocation and none of the launches: the general functions end in an error there)
+bool being_traced() { return c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::Tracer); }
+
 int64_t pitch128(int64_t n) { return div_up(n, 128) * 128; }
 int64_t up256(int64_t n) { return div_up(n, 256) * 256; }
 int64_t packed_bytes(int64_t K, int64_t rows) { return div_up(K / 32, 16) * rows * 16; }
@@ -399,7 +403,7 @@ struct LinearCopies {
 
 // linear.py:MXFP4LinearStep.forward -> (y, buffer of x's column copy, buffer of W's column copy, packed bits)
 py::object linear_forward(const Tensor& x_in, const Tensor& w, const OptTensor& signs, const OptTensor& perm, int clip, bool uos, bool allow_packed, uintptr_t stream) {
-  if (!on_gpu(x_in) || x_in.dim() < 2 || w.dim() != 2 || !rows_readable(w)) return py::none();
+  if (!on_gpu(x_in) || x_in.dim() < 2 || w.dim() != 2 || !rows_readable(w) || being_traced()) return py::none();
   const int64_t N = w.size(0), K = w.size(1);
   if (x_in.size(-1) != K || x_in.numel() == 0 || N == 0 || N % 32 != 0 || K % 32 != 0) return py::none();
   const Tensor x = x_in.dim() == 2 ? x_in : x_in.reshape({-1, K});
@@ -524,7 +528,7 @@ bool grouped_product(Failure& f, const Copy& a, const Tensor& a_buf, const Copy&
 py::object grouped_forward(const Tensor& x, const Tensor& w, const Tensor& offs_in, bool ends, bool trans_weights, const OptTensor& signs, const OptTensor& perm, int clip,
                            bool uos, uintptr_t stream) {
   if (x.dim() != 2 || w.dim() != 3 || !rows_readable(x) || !rows_readable(w) || x.scalar_type() != at::kBFloat16 || !x.is_contiguous() || !w.is_contiguous()) return py::none();
-  if (!on_gpu(offs_in) || offs_in.dim() != 1 || offs_in.scalar_type() != at::kInt || !offs_in.is_contiguous()) return py::none();
+  if (being_traced() || !on_gpu(offs_in) || offs_in.dim() != 1 || offs_in.scalar_type() != at::kInt || !offs_in.is_contiguous()) return py::none();
   const int64_t M = x.size(0), E = w.size(0), N = w.size(trans_weights ? 1 : 2), K = w.size(trans_weights ? 2 : 1);
   if (x.size(1) != K || offs_in.numel() != E + !ends || M == 0 || E == 0 || N % 32 != 0 || K % 32 != 0) return py::none();
   if (M * std::max(N, K) >= (1ll << 36) || N * K >= (1ll << 36) || !grouped_packed_supported(M, N, K, E) || !grouped_packed_supported(M, K, N, E) ||

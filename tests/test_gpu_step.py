@@ -294,3 +294,21 @@ def test_operands_quantized_in_one_call(m, dtype, had, clip, uos, x_shape, w_sha
                 int(uos), rt.stream_ptr(x.device)), "alto_mxfp4_quantize_operands")
             for a, b, what in zip(got, (xr, xrs, xc, xcs, wr, wrs, wc, wcs), "xr xrs xc xcs wr wrs wc wcs".split()):
                 assert torch.equal(a, b), (what, pack, w_dtype)
+
+
+@pytest.mark.filterwarnings("ignore::torch.jit.TracerWarning")
+def test_steps_refuse_a_trace_as_the_general_functions_do(m):
+    """torch.jit.trace records no launch: the general functions end in an error under it, and the steps leave it to them."""
+    from alto_amd.mxfp4 import grouped_gemm as G
+    from alto_amd.mxfp4.linear import MXFP4LinearStep
+    x, w = randn_outliers((512, 544), torch.bfloat16, seed=1).to(DEV), randn_outliers((640, 544), torch.bfloat16, seed=2).to(DEV)
+    e = randn_outliers((3, 640, 544), torch.bfloat16, seed=3).to(DEV)
+    offs = torch.tensor([0, 96, 320, 512], dtype=torch.int32, device=DEV)
+    for fn in (lambda a: m.MXFP4LinearFunction.apply(a, w, False, True, False, False, "none", False, None, False),
+               lambda a: MXFP4LinearStep.apply(a, w, False, True, False, False, "none", False, None, False),
+               lambda a: G.MXFP4GroupedGEMM.apply(a, e, None, True, False, True, False, False, "none", False, None, False, offs),
+               lambda a: G.MXFP4GroupedStep.apply(a, e, offs, False, True, False, False, "none", None, False),
+               lambda a: G.MXFP4GroupedStep.apply(a, e, offs[1:].contiguous(), True, True, False, False, "none", None, False)):
+        with pytest.raises(TypeError, match="cond must be a bool"):
+            torch.jit.trace(fn, x, check_trace=False)
+        fn(x)
