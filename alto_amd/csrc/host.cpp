@@ -425,11 +425,10 @@ py::object linear_forward(const Tensor& x_in, const Tensor& w, const OptTensor& 
     y = at::empty({M, N}, x.options());
     void* s = reinterpret_cast<void*>(stream);
     quantize_operands(f, x, c.x_row, tmp, c.x_col, xs, h, clip, w, c.w_row, tmp, c.w_col, ws, uos, s) && product(f, c.x_row, tmp, c.w_row, tmp, y, 1.0, s);
-    if (x_in.dim() != 2) {
-      auto shape = x_in.sizes().vec();
-      shape.back() = N;
-      y = y.view(shape);
-    }
+    // a view for two dimensions as well, as the general function returns it: autograd refuses to change either in place
+    auto shape = x_in.sizes().vec();
+    shape.back() = N;
+    y = y.view(shape);
   }
   f.raise();
   return py::make_tuple(y, xs, ws, packed);

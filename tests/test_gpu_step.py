@@ -312,3 +312,23 @@ def test_steps_refuse_a_trace_as_the_general_functions_do(m):
         with pytest.raises(TypeError, match="cond must be a bool"):
             torch.jit.trace(fn, x, check_trace=False)
         fn(x)
+
+
+def test_a_step_result_is_changed_in_place_where_the_general_functions_allow_it(m):
+    from alto_amd.mxfp4 import grouped_gemm as G
+    from alto_amd.mxfp4.linear import MXFP4LinearStep
+    x, w = randn_outliers((512, 544), torch.bfloat16, seed=1).to(DEV), randn_outliers((640, 544), torch.bfloat16, seed=2).to(DEV)
+    e = randn_outliers((3, 640, 544), torch.bfloat16, seed=3).to(DEV)
+    offs = torch.tensor([0, 96, 320, 512], dtype=torch.int32, device=DEV)
+    for fn in (MXFP4LinearStep, m.MXFP4LinearFunction):   # (its result is a view made inside the function)
+        for shape in ((512,), (8, 64)):
+            y = fn.apply(x.view(*shape, 544).detach().requires_grad_(True), w, False, True, False, False, "none", False, None, False)
+            with pytest.raises(RuntimeError, match="is a view and is being modified inplace"):
+                y.mul_(2)
+    both = []
+    for fn in (lambda a: G.MXFP4GroupedStep.apply(a, e, offs, False, True, False, False, "none", None, False),
+               lambda a: G.MXFP4GroupedGEMM.apply(a, e, None, True, False, True, False, False, "none", False, None, False, offs)):
+        a = x.detach().requires_grad_(True)
+        y = fn(a).mul_(2)
+        both.append((y.detach(), torch.autograd.grad(y, a, torch.ones_like(y))[0]))
+    assert all(torch.equal(s, t) for s, t in zip(*both))
