@@ -56,10 +56,14 @@ typedef unsigned v2u_t __attribute__((ext_vector_type(2)));
 typedef int v4i_8_t __attribute__((ext_vector_type(4), aligned(8)));   // 16 bytes at an 8-byte boundary
 // v_permlane32_swap(a, b) returns {a of lanes 0..31 | b of lanes 0..31,  a of lanes 32..63 | b of lanes 32..63}
 // (first | second half of the wave): a value and its copy come back as the low half's and the high half's values.
-__device__ __forceinline__ float pair_max(float v) {   // max over the two lanes l and l ^ 32
-  const v2u_t p = __builtin_amdgcn_permlane32_swap(f2u(v), f2u(v), false, false);
-  return fmaxf(u2f(p[0]), u2f(p[1]));
+// fmaxf for values of which at most one is NaN, in one instruction: v_med3 with +infinity (opaque to the compiler, which would turn it
+// back into a maximum and put a canonicalizing copy of either operand in front of it).
+__device__ __forceinline__ float max_one(float x, float y) {
+  float inf = __builtin_inff();
+  asm("" : "+s"(inf));
+  return __builtin_amdgcn_fmed3f(x, y, inf);
 }
+__device__ __forceinline__ float max_of_pair(v2u_t p) { return max_one(u2f(p[0]), u2f(p[1])); }
 
 typedef unsigned short us2a_t __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ uint32_t pk_max_u16a(uint32_t a, uint32_t b) {
@@ -167,55 +171,81 @@ __device__ __forceinline__ int attn_head(const AttnArgs& a) {
   return a.Hq % 8 == 0 ? (int)((blockIdx.x & 7) * (a.Hq >> 3) + (blockIdx.x >> 3)) : (int)blockIdx.x;
 }
 
-// Hides the scores of keys that a lane's row may not see: `seen` = how many keys from the lane's first one (4 h of the block) on
-// it does.  (The empty assembly keeps each comparison next to its use: taken together, their 32 results spilled scalars that the
-// loop over the blocks needs.  In attention.hip, whose own form spills none, this one is 0 to 5 % faster with a causal mask and 2 to
-// 4 % slower without.)
+// Which key of a 32-key tile row i of the score product is: bits 2 and 3 of i change places, so that register v of half h holds key
+// 16 (v / 8) + 8 h + v % 8.  A half's eight codes of a dword are then eight consecutive keys, and the operand of the product with V
+// comes out of the half-wave swaps in key order (in the plain order, key 8 (v / 4) + 4 h + v % 4, it took four byte permutes more).
+__device__ __forceinline__ int score_key(int i) { return (i & 0x13) | (i & 4) << 1 | (i & 8) >> 1; }
+
+// Hides the scores of keys that a lane's row may not see: `seen` = how many keys from the lane's first one (8 h of the block) on
+// it does.  (The empty assembly keeps each four comparisons next to their uses: all 32 results taken together spilled scalars that the
+// loop over the blocks needs, and one at a time every use waits for its comparison.)
 __device__ __forceinline__ void mask_scores(v16f_t (&S)[2], int seen) {
 #pragma unroll
   for (int t = 0; t < 2; ++t)
 #pragma unroll
-    for (int v = 0; v < 16; ++v) {
-      float x = 32 * t + 8 * (v >> 2) + (v & 3) >= seen ? -__builtin_inff() : S[t][v];
-      asm volatile("" : "+v"(x));
-      S[t][v] = x;
+    for (int v = 0; v < 16; v += 4) {
+      float x[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) x[i] = 32 * t + 16 * (v >> 3) + (v & 7) + i >= seen ? -__builtin_inff() : S[t][v + i];
+      asm volatile("" : "+v"(x[0]), "+v"(x[1]), "+v"(x[2]), "+v"(x[3]));
+#pragma unroll
+      for (int i = 0; i < 4; ++i) S[t][v + i] = x[i];
     }
 }
 
-// Probabilities of a wave's 32 rows and 64 keys (S: scores of this lane's row, keys 8 g + 4 h + (0..3) of tiles of 32; tmx: the
-// row's largest score of each tile; cs: factor into the base-2 domain; m_new: running maximum there): one E8M0 scale per (row,
-// 32 keys), E2M1 codes (round to nearest even), as the second operand of the product with V.
-__device__ __forceinline__ void quantize_probabilities(v16f_t (&S)[2], const float (&tmx)[2], float cs, float m_new, int h, v8i_t& pf, int& pscale) {
-  uint32_t c[2][2];
-  int psc[2];
+// Largest score of row r = lane % 32 in the tile h = lane / 32 (S: two tiles of 32 keys, a row's keys over the lanes r and r + 32), and
+// in both tiles.  One swap hands either lane of a row the other one's part of its tile (a swap for each tile, as before, does the work
+// for both tiles in both lanes).
+__device__ __forceinline__ void row_maxima(const v16f_t (&S)[2], float& tile_max, float& row_max) {
+  float x[2];
 #pragma unroll
   for (int t = 0; t < 2; ++t) {
+    x[t] = -__builtin_inff();   // (and never NaN)
 #pragma unroll
-    for (int v = 0; v < 16; ++v) S[t][v] = __builtin_amdgcn_exp2f(__builtin_fmaf(S[t][v], cs, -m_new));
-    const float am = __builtin_amdgcn_exp2f(__builtin_fmaf(tmx[t], cs, -m_new));   // = max of the 32 values above
-    const uint32_t e = e8m0_from_f32_bits(f2u(am));
-    psc[t] = (int)e;
-    const float scale_f = u2f(e << 23);
+    for (int v = 0; v < 16; ++v) x[t] = fmaxf(x[t], S[t][v]);
+  }
+  tile_max = max_of_pair(__builtin_amdgcn_permlane32_swap(f2u(x[0]), f2u(x[1]), false, false));
+  row_max = max_of_pair(__builtin_amdgcn_permlane32_swap(f2u(tile_max), f2u(tile_max), false, false));
+}
+
+// Probabilities of a wave's 32 rows and 64 keys (S: scores of this lane's row, keys as score_key() deals them; tile_max: the row's
+// largest score in the tile h, whose probability is the tile's largest: exp2 is monotonic; cs: factor into the base-2 domain; m_new:
+// running maximum there): one E8M0 scale per (row, 32 keys), E2M1 codes (round to nearest even), as an operand of the product with V.
+// Lane (r, h) multiplies tile h: it has that tile's scale, and gets the 16 codes of it that the other lane of the row holds.
+__device__ __forceinline__ void quantize_probabilities(v16f_t (&S)[2], float tile_max, float cs, float m_new, v8i_t& pf, int& pscale) {
+  const float am = __builtin_amdgcn_exp2f(__builtin_fmaf(tile_max, cs, -m_new));
+  pscale = (int)e8m0_from_f32_bits(f2u(am));
+  const v2u_t scale = __builtin_amdgcn_permlane32_swap((unsigned)pscale << 23, (unsigned)pscale << 23, false, false);   // of tile 0, of tile 1
+  uint32_t c[2][2];
+#pragma unroll
+  for (int t = 0; t < 2; ++t) {
+    const float scale_f = u2f(scale[t]);
 #pragma unroll
     for (int w = 0; w < 2; ++w) {
-      uint32_t o = 0;
-      o = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(o, S[t][8 * w + 0], S[t][8 * w + 1], scale_f, 0);
-      o = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(o, S[t][8 * w + 2], S[t][8 * w + 3], scale_f, 1);
-      o = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(o, S[t][8 * w + 4], S[t][8 * w + 5], scale_f, 2);
-      o = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(o, S[t][8 * w + 6], S[t][8 * w + 7], scale_f, 3);
+      float p[8];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) p[i] = __builtin_amdgcn_exp2f(__builtin_fmaf(S[t][8 * w + i], cs, -m_new));
+      uint32_t o = f2u(p[0]);   // (every byte is replaced: starting from a register that ends here costs no move)
+      o = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(o, p[0], p[1], scale_f, 0);
+      o = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(o, p[2], p[3], scale_f, 1);
+      o = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(o, p[4], p[5], scale_f, 2);
+      o = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(o, p[6], p[7], scale_f, 3);
       c[t][w] = o;
     }
   }
-  // Lane (r, h) multiplies tile h of this block and needs that tile's 32 codes of row r in key order; it holds the
-  // keys 8 g + 4 h + (0..3) of both tiles.  One half-wave swap per dword hands lane (r, 0) the tile-0 codes of lane
-  // (r, 1) and lane (r, 1) the tile-1 codes of lane (r, 0); in both halves the swapped pair is then {keys 8 g + 0..3,
-  // keys 8 g + 4..7} = {p[0], p[1]}, interleaved 16 bits at a time.
-  const v2u_t p0 = __builtin_amdgcn_permlane32_swap(c[0][0], c[1][0], false, false);
-  const v2u_t p1 = __builtin_amdgcn_permlane32_swap(c[0][1], c[1][1], false, false);
-  pf = v8i_t{(int)__builtin_amdgcn_perm(p0[1], p0[0], 0x05040100u), (int)__builtin_amdgcn_perm(p0[1], p0[0], 0x07060302u),
-                         (int)__builtin_amdgcn_perm(p1[1], p1[0], 0x05040100u), (int)__builtin_amdgcn_perm(p1[1], p1[0], 0x07060302u),
-                         0, 0, 0, 0};
-  pscale = h ? psc[1] : psc[0];
+  const v2u_t p0 = __builtin_amdgcn_permlane32_swap(c[0][0], c[1][0], false, false);   // keys 0..7 and 8..15 of the tile
+  const v2u_t p1 = __builtin_amdgcn_permlane32_swap(c[0][1], c[1][1], false, false);   // keys 16..23 and 24..31
+  pf = v8i_t{(int)p0[0], (int)p0[1], (int)p1[0], (int)p1[1], 0, 0, 0, 0};
+}
+
+// Row sums of the quantised probabilities, in one product of 16 x 16 x 128 (4 accumulator registers a lane instead of 16, and half the
+// matrix time of a 32 x 32 x 64 product with a column of ones).  That product takes the operand of lane l for row l % 16 and keys
+// 32 (l / 16) .. + 32, while the lane holds row l % 32 and the tile l / 32: for row i < 16 the key ranges 0 and 2 are its two tiles and 1
+// and 3 those of row 16 + i.  Row n of the other operand is one where (n / 4) % 2 and the range agree in the lowest bit, so all
+// registers of lane l get the sum of row l % 32.
+__device__ __forceinline__ int row_sum_selector(int lane) { return ((lane >> 2) & 1) == ((lane >> 4) & 1) ? 0x22222222 : 0; }   // (E2M1 code 2 = 1.0)
+__device__ __forceinline__ v4f_t add_row_sums(int selector, const v8i_t& pf, int pscale, v4f_t l) {
+  return __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(v8i_t{selector, selector, selector, selector, 0, 0, 0, 0}, pf, l, 4, 4, 0, 127, 0, pscale);
 }
 
 // Launch of the kernel whose four waves deal out the keys of 32 rows (attention_split.hip); `row_blocks` in units of 32 rows.

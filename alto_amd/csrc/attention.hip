@@ -2,10 +2,22 @@
 // probabilities re-quantised to MXFP4 in registers and the row sums taken from the SAME quantised probabilities
 // (the recurrence of alto/kernels/fp4/mxfp4/triton_flash_attention_mxfp4.py:168-400,640-890, key blocks of 64).
 //
-// One wave owns 32 query rows of one head.  The MFMA is issued as (first = rows that land in registers, second = rows
-// that land in lanes): S tiles and O tiles keep the query row in the lane (lane % 32) and spread keys / value columns
-// over the 16 accumulator registers, so the per-row softmax state (running max, rescale factor) is one scalar per lane
-// and the only cross-lane traffic is between the two lanes (l, l ^ 32) that share a row.
+// One wave owns 32 query rows of one head.  The MFMA is issued as (first = rows that land in registers, second = rows that land in
+// lanes).  S tiles keep the query row in the lane (lane % 32) and spread keys over the 16 accumulator registers, so the per-row softmax
+// state (running max, rescale factor, sum) is one scalar per lane and the only cross-lane traffic is between the two lanes (l, l ^ 32)
+// that share a row.  O tiles have the rows in the registers and the value columns in the lanes: a block whose running maximum rises in
+// a few rows only rescales the registers of those rows, and a lane's columns are neighbours in memory.
+//
+// What bounds it: vector instructions (the matrix pipes are busy a fifth of the time).  Device time of changing inputs, us, against the
+// kernel with O's rows in lanes, a maximum and a scale of either tile in both lanes of a row, row sums by a 32 x 32 x 64 product of ones
+// and the plain key order, all with the same results bit for bit:
+//   4 x 2048 tokens, 64 / 8 heads of 128: causal 177.6 -> 162.1, all keys 304 -> 281; 4096 tokens, 32 heads of 128, all keys 151.6 -> 141.7;
+//   4 x 4096, 32 / 8 heads of 64: 428 -> 385, causal 230 -> 203; 2 x 2048, 32 / 8 heads of 192 / 256, causal: 61.0 -> 52.8, 63.3 -> 60.0.
+// Of that, the maxima, scales, key order and mask (row_maxima() .. mask_scores() in attention.h) gave 5 % (D = 128) to 8 % (64), the
+// rescale by rows 3 to 5 %, the smaller product for the sums 1 to 2 %.  The rescale factors take the way through the LDS: a product
+// with a row of ones on the matrix pipe and ds_bpermute were 2 to 4 % slower; groups of four rows instead of eight are 1 % faster with
+// long sequences of D = 128, 3 % slower with D = 64 and 1 % slower with 1024 tokens.  Four workgroups a compute unit do not fit D = 128
+// (12 registers spilled: 178), five are no faster with D = 64.
 #include <algorithm>
 #include <memory>
 #include <new>
@@ -30,7 +42,7 @@ struct AttnTile {
   static constexpr int D = NK * 64, DV = ND * 32;
   static constexpr int K_BYTES = 64 * (D / 2), V_BYTES = DV * 32;       // one block of K codes, of V codes
   static constexpr int SLOT = K_BYTES + V_BYTES;
-  static constexpr int LDS = ATTN_RING * SLOT > 128 * DV * 2 ? ATTN_RING * SLOT : 128 * DV * 2;         // the ring, then the 128 result rows
+  static constexpr int FACTORS = ATTN_RING * SLOT, QUERY = FACTORS + 4 * 128;   // behind the ring: 32 row factors a wave, then Q's codes on their way through the lanes
 };
 
 // The body of the kernel as a function of its own because of the `__restrict__` on the outputs: inlining then marks the
@@ -44,7 +56,7 @@ struct AttnTile {
 // together (another box: 38.6 and 162.7, 193.5; 8.8 and 171.8, 181).  How the kernel with QBF got there: every lane fetching the 64
 // bytes it multiplies 201, whole lines (quantize_q) 197, at raised wave priority 195 (the two other workgroups of the compute unit hide the
 // wait, the priority lets the arithmetic behind it through), Q read non-temporally 2 less; of use to the kernel on codes as well:
-// the heads dealt to the XCDs in ranges 195 -> 187, the results stored as whole rows 187 -> 181.
+// the heads dealt to the XCDs in ranges 195 -> 187, the results stored as whole rows 187 -> 181 (then through the LDS).
 // SEQS: AttnSeqs, or AttnNoSeqs for B sequences of one length.
 template <int NK, int ND, bool BIASED, bool QBF, typename SEQS>
 __device__ __forceinline__ void attn_fwd_body(const AttnArgs& a, const SEQS& seqs, __bf16* __restrict__ out, float* __restrict__ lse_out, uint8_t* ring) {
@@ -82,13 +94,12 @@ __device__ __forceinline__ void attn_fwd_body(const AttnArgs& a, const SEQS& seq
     }
   }
 
-  v16f_t acc_o[ND], acc_l;
+  v16f_t acc_o[ND];
+  v4f_t acc_l = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
   for (int d = 0; d < ND; ++d)
 #pragma unroll
     for (int v = 0; v < 16; ++v) acc_o[d][v] = 0.0f;
-#pragma unroll
-  for (int v = 0; v < 16; ++v) acc_l[v] = 0.0f;
   float m_i = -__builtin_inff();                   // running row max of S * sm_scale * log2(e)
   const float c2 = a.sm_scale * ATTN_RCP_LN2;
   const float cs = BIASED ? 1.0f : c2;   // what is left to multiply once the scores are in the base-2 domain
@@ -98,7 +109,8 @@ __device__ __forceinline__ void attn_fwd_body(const AttnArgs& a, const SEQS& seq
       (BIASED && a.bias) ? (int)(a.bias_bytes - (b * a.bias_sb + hq * a.bias_sh) * 4) : 0, 0x00020000);
   const float slope2 = (BIASED && a.alibi) ? a.alibi[b * a.alibi_sb + hq * a.alibi_sh] * ATTN_RCP_LN2 : 0.0f;
 
-  const v8i_t ones = v8i_t{0x22222222, 0x22222222, 0x22222222, 0x22222222, 0, 0, 0, 0};   // E2M1 code 2 = 1.0
+  const int selector = row_sum_selector(lane);
+  float* const factors = reinterpret_cast<float*>(ring + AttnTile<NK, ND>::FACTORS + wave * 128);   // of this wave's rows, on their way to the registers
 
   // blocks this wave needs, and the most any wave of the workgroup needs (the last wave's rows reach furthest)
   const int all_blk = (kn + 63) / 64;
@@ -141,13 +153,14 @@ __device__ __forceinline__ void attn_fwd_body(const AttnArgs& a, const SEQS& seq
         __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_k, (__attribute__((address_space(3))) void*)(base + p0 * 16), 16, (row * KPR + c) * 16,
                                                  __builtin_amdgcn_readfirstlane(kb * K_BYTES), 0, 0);
       } else {
-        const int p = p0 - K_PIECES + lane, row = p >> 1;
+        const int p = p0 - K_PIECES + lane, row = p >> 1, column = ND * (row & 31) + (row >> 5);
         __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_v, (__attribute__((address_space(3))) void*)(base + p0 * 16), 16,
-                                                 row * (a.Sk / 2) + (((p & 1) ^ ((row >> 3) & 1)) * 16), __builtin_amdgcn_readfirstlane(kb * 32), 0, 0);
+                                                 column * (a.Sk / 2) + (((p & 1) ^ ((row >> 3) & 1)) * 16), __builtin_amdgcn_readfirstlane(kb * 32), 0, 0);
       }
     }
   };
-  const int k_swz = KSW ? ((r / (KSW ? KSW : 1)) % KPR) * 16 : 0;   // XOR on the byte offset of a piece inside its K row
+  const int kr = score_key(r);                                      // this lane's key of a tile
+  const int k_swz = KSW ? ((kr / (KSW ? KSW : 1)) % KPR) * 16 : 0;  // XOR on the byte offset of a piece inside its K row
   const int v_swz = ((r >> 3) & 1) * 16;                            // and inside its 32-byte V row
   auto wait_dma = [&](bool one_block_in_flight) {   // this wave's loads are done, except the youngest block's if asked
     if (!one_block_in_flight) __builtin_amdgcn_s_waitcnt(0x0070 | 0x0F00 | 0);                      // vmcnt(0)
@@ -191,7 +204,7 @@ __device__ __forceinline__ void attn_fwd_body(const AttnArgs& a, const SEQS& seq
   }
   if constexpr (QBF) {   // behind the first blocks' loads, which then travel with it
     __builtin_amdgcn_s_setprio(3);
-    quantize_q<NK>(a.qx + b * a.qx_sb + hq * a.qx_sh + (int64_t)(q_first + (live ? q0 : 0)) * a.qx_ss, a.qx_ss, lane, ring + AttnTile<NK, ND>::LDS + wave * (NK * 1024), qf, qsc);
+    quantize_q<NK>(a.qx + b * a.qx_sb + hq * a.qx_sh + (int64_t)(q_first + (live ? q0 : 0)) * a.qx_ss, a.qx_ss, lane, ring + AttnTile<NK, ND>::QUERY + wave * (NK * 1024), qf, qsc);
     __builtin_amdgcn_s_setprio(0);
   }
   // (the bare barrier instruction: `__syncthreads()` would first wait for every outstanding load, the prefetched block's
@@ -218,13 +231,13 @@ __device__ __forceinline__ void attn_fwd_body(const AttnArgs& a, const SEQS& seq
     if (kb + 1 < wg_blk) fetch_scales(kb + 1, ksw_next, vsw_next);
     if (kb + 2 < wg_blk) dma(kb + 2, slot == 0 ? ATTN_RING - 1 : slot - 1);
     if (kb < nblk) {
-      v4f_t bb[BIASED ? 2 : 1][BIASED ? 4 : 1];   // bias of this lane's 32 scores: keys key0 + 32 t + 8 g + 4 h + (0..3)
+      v4f_t bb[BIASED ? 2 : 1][BIASED ? 4 : 1];   // bias of this lane's 32 scores: keys key0 + 32 t + 16 (g / 2) + 8 h + 4 (g % 2) + (0..3)
       if constexpr (BIASED) {
 #pragma unroll
         for (int t = 0; t < 2; ++t)
 #pragma unroll
           for (int g = 0; g < 4; ++g) {
-            const v4i_t w = __builtin_amdgcn_raw_buffer_load_b128(rsrc_bias, (int)((qrow * a.bias_sm + key0 + 32 * t + 8 * g + 4 * h) * 4), 0, 0);
+            const v4i_t w = __builtin_amdgcn_raw_buffer_load_b128(rsrc_bias, (int)((qrow * a.bias_sm + key0 + 32 * t + 16 * (g >> 1) + 8 * h + 4 * (g & 1)) * 4), 0, 0);
             bb[t][g] = __builtin_bit_cast(v4f_t, w);
           }
       }
@@ -240,7 +253,7 @@ __device__ __forceinline__ void attn_fwd_body(const AttnArgs& a, const SEQS& seq
         static_for<NK>([&](auto sc) {
           constexpr int s = decltype(sc)::value;
           constexpr int byte = t * (D / 32) + 2 * s;
-          const v8i_t kf = frag16(tile + (32 * t + r) * (D / 2) + ((32 * s + 16 * h) ^ k_swz));
+          const v8i_t kf = frag16(tile + (32 * t + kr) * (D / 2) + ((32 * s + 16 * h) ^ k_swz));
           S[t] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(kf, qf[s], S[t], 4, 4, byte % 4, ksh[byte / 4], 0, qsc[s]);
         });
       });
@@ -249,7 +262,7 @@ __device__ __forceinline__ void attn_fwd_body(const AttnArgs& a, const SEQS& seq
         for (int t = 0; t < 2; ++t)
 #pragma unroll
           for (int v = 0; v < 16; ++v) {
-            const int key = key0 + 32 * t + 8 * (v >> 2) + 4 * h + (v & 3);
+            const int key = key0 + 32 * t + 16 * (v >> 3) + 8 * h + (v & 7);
             float x = __builtin_fmaf(bb[t][v >> 2][v & 3], ATTN_RCP_LN2, S[t][v] * c2);
             x = __builtin_fmaf(-slope2, __builtin_fabsf((float)(qrow + shift - key)), x);
             S[t][v] = x;
@@ -258,24 +271,11 @@ __device__ __forceinline__ void attn_fwd_body(const AttnArgs& a, const SEQS& seq
       // ---- mask (only blocks the diagonal crosses or that reach past the last key), running max kept in the base-2 domain: m = max(S) * sm_scale * log2(e)
       if ((a.causal && key0 + 63 > q0 + shift) || key0 + 64 > kn) {
         asm volatile("" ::: "memory");   // keep this a branch: most blocks skip it
-#pragma unroll
-        for (int t = 0; t < 2; ++t)
-#pragma unroll
-          for (int v = 0; v < 16; ++v) {
-            const int key = key0 + 32 * t + 8 * (v >> 2) + 4 * h + (v & 3);
-            if ((a.causal && key > qrow + shift) || key >= kn) S[t][v] = -__builtin_inff();
-          }
+        mask_scores(S, (a.causal && qrow + shift + 1 < kn ? qrow + shift + 1 : kn) - key0 - 8 * h);
       }
-      float tmx[2];   // row maximum of each 32-key tile (exp2 is monotonic: its largest probability comes from this score)
-#pragma unroll
-      for (int t = 0; t < 2; ++t) {
-        float x = -__builtin_inff();
-#pragma unroll
-        for (int v = 0; v < 16; ++v) x = fmaxf(x, S[t][v]);
-        tmx[t] = pair_max(x);
-      }
-      const float mx = fmaxf(tmx[0], tmx[1]);
-      float m_new = fmaxf(m_i, mx * cs);
+      float tile_max, mx;
+      row_maxima(S, tile_max, mx);
+      float m_new = max_one(m_i, mx * cs);
       // a bias may hide every key a row has seen so far (-inf): such a row keeps m = -inf and takes exp2(-inf - 0) = 0
       // everywhere instead of exp2(-inf + inf)
       const float m_sub = (BIASED && m_new == -__builtin_inff()) ? 0.0f : m_new;
@@ -285,23 +285,35 @@ __device__ __forceinline__ void attn_fwd_body(const AttnArgs& a, const SEQS& seq
 
       v8i_t pf;
       int pscale;
-      quantize_probabilities(S, tmx, cs, m_new, h, pf, pscale);
+      quantize_probabilities(S, tile_max, cs, m_new, pf, pscale);
 
       // ---- row sums of the quantised probabilities (a column of ones) and O += P V
-      if (__builtin_amdgcn_ballot_w64(alpha != 1.0f) != 0) {   // the row maxima settle after a few blocks
-        acc_l[0] *= alpha;                                     // all 16 registers hold the row sum; only [0] is read
+      const uint32_t changed = (uint32_t)__builtin_amdgcn_ballot_w64(alpha != 1.0f);   // (both lanes of a row have its alpha)
+      if (changed != 0) {
+        acc_l[0] *= alpha;   // all registers hold the row sum; only [0] is read
+        factors[r] = alpha;
+        wave_lds_order();
+        v4f_t f[4];   // (all read before the first branch: read in the branches they cost 4 % with D = 128)
 #pragma unroll
-        for (int d = 0; d < ND; ++d)
+        for (int g = 0; g < 4; ++g) f[g] = *reinterpret_cast<const v4f_t*>(factors + 8 * g + 4 * h);
+        static_for<4>([&](auto gc) {
+          constexpr int g = decltype(gc)::value;   // registers 4 g .. + 4 of the two halves: rows 8 g .. + 8
+          if (changed & (0xFFu << (8 * g))) {
+            asm volatile("" ::: "memory");   // keep this a branch
 #pragma unroll
-          for (int v = 0; v < 16; ++v) acc_o[d][v] *= alpha;
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+              for (int d = 0; d < ND; ++d) acc_o[d][4 * g + i] *= f[g][i];
+          }
+        });
       }
-      acc_l = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(ones, pf, acc_l, 4, 4, 0, 127, 0, pscale);
-      // V scale of (key tile h, column block d) = byte h Dv/32 + d
-      const int vsh = DV == 128 ? (int)(h ? vsw[VS_DW - 1] : vsw[0]) : (int)(vsw[0] >> (16 * h));
+      acc_l = add_row_sums(selector, pf, pscale, acc_l);
+      // V scale of (key tile h, this lane's columns ND r .. + ND) = byte h Dv/32 + r / (32 / ND)
+      const int vsh = DV == 128 ? (int)((h ? vsw[VS_DW - 1] : vsw[0]) >> (8 * (r >> 3))) : (int)(vsw[0] >> (16 * h + 8 * (r >> 4)));
       static_for<ND>([&](auto dc) {
         constexpr int d = decltype(dc)::value;
         const v8i_t vf = frag16(tile + K_BYTES + (32 * d + r) * 32 + ((16 * h) ^ v_swz));
-        acc_o[d] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(vf, pf, acc_o[d], 4, 4, d, vsh, 0, pscale);
+        acc_o[d] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(pf, vf, acc_o[d], 4, 4, 0, pscale, 0, vsh);
       });
     }
     wait_dma(kb + 2 < wg_blk);   // block kb + 1 has landed (this wave's part; the barrier collects the others')
@@ -310,37 +322,29 @@ __device__ __forceinline__ void attn_fwd_body(const AttnArgs& a, const SEQS& seq
   }
   if (!live) return;
 
-  // ---- O = acc / l, bf16; log-sum-exp.  The rows change lanes through the LDS (the ring is no longer read: every wave has passed
-  // the loop's last barrier; each wave uses a part of its own), so that a store instruction writes whole rows (8-byte pieces of 32 rows
-  // an instruction before: 187 -> 181 us, QBF above).  16-byte piece c of row r goes to position c ^ (r / (16 / PR)) % PR, PR pieces per
-  // row: the reads are free of bank conflicts, in the writes two rows meet (Dv = 128: 4 cycles each, 64 a wave; 1 % of the kernel's).
+  // ---- O = acc / l, bf16; log-sum-exp.  A lane holds ND consecutive columns of 16 rows: a store instruction writes two whole rows.
   const float l = acc_l[0];
-  const float rl = 1.0f / l;
-  constexpr int PR = DV / 8;
-  uint8_t* rows = ring + wave * (32 * DV * 2);
-#pragma unroll
-  for (int d = 0; d < ND; ++d)
-#pragma unroll
-    for (int g = 0; g < 4; ++g) {
-      uint2 w;
-      w.x = pack_bf16x2(acc_o[d][4 * g + 0] * rl, acc_o[d][4 * g + 1] * rl);
-      w.y = pack_bf16x2(acc_o[d][4 * g + 2] * rl, acc_o[d][4 * g + 3] * rl);
-      *reinterpret_cast<uint2*>(rows + r * (DV * 2) + (((4 * d + g) ^ ((r / (16 / PR)) % PR)) * 16 + 8 * h)) = w;
-    }
+  factors[r] = 1.0f / l;
   wave_lds_order();
-  __bf16* o_first = out + b * a.o_sb + hq * a.o_sh + (int64_t)(q_first + q0) * a.o_ss;
+  __bf16* o_lane = out + b * a.o_sb + hq * a.o_sh + (int64_t)(q_first + q0 + 4 * h) * a.o_ss + ND * r;
 #pragma unroll
-  for (int i = 0; i < PR / 2; ++i) {
-    const int p = 64 * i + lane, row = p / PR, c = p % PR;
-    const v4i_t w = *reinterpret_cast<const v4i_t*>(rows + row * (DV * 2) + (c ^ ((row / (16 / PR)) % PR)) * 16);
-    *reinterpret_cast<v4i_8_t*>(o_first + row * a.o_ss + 8 * c) = w;
+  for (int g = 0; g < 4; ++g) {
+    const v4f_t rl = *reinterpret_cast<const v4f_t*>(factors + 8 * g + 4 * h);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      __bf16* o = o_lane + (8 * g + i) * a.o_ss;
+      const int v = 4 * g + i;
+      const uint32_t w = pack_bf16x2(acc_o[0][v] * rl[i], acc_o[1][v] * rl[i]);
+      if constexpr (ND == 4) *reinterpret_cast<uint2*>(o) = make_uint2(w, pack_bf16x2(acc_o[2][v] * rl[i], acc_o[3][v] * rl[i]));
+      else *reinterpret_cast<uint32_t*>(o) = w;
+    }
   }
   if (h == 0) lse_out[b * a.l_sb + hq * a.l_sh + (q_first + qrow) * a.l_ss] = (m_i + log2f(l)) * ATTN_LN2;
 }
 
 template <int NK, int ND, bool BIASED, bool QBF, typename SEQS>
 __global__ __launch_bounds__(256, BIASED ? 2 : ATTN_WG_PER_CU) void attn_fwd_kernel(AttnArgs a, SEQS seqs) {
-  __shared__ __attribute__((aligned(16))) uint8_t ring[AttnTile<NK, ND>::LDS + (QBF ? 4 * NK * 1024 : 0)];
+  __shared__ __attribute__((aligned(16))) uint8_t ring[AttnTile<NK, ND>::QUERY + (QBF ? 4 * NK * 1024 : 0)];
   attn_fwd_body<NK, ND, BIASED, QBF>(a, seqs, reinterpret_cast<__bf16*>(a.out), a.lse, ring);
 }
 

@@ -65,7 +65,7 @@ __device__ __forceinline__ void attn_split_body(const AttnArgs& a, const SEQS& s
 #pragma unroll
     for (int t = 0; t < 2; ++t)
 #pragma unroll
-      for (int s = 0; s < NK; ++s) kf[t][s] = __builtin_amdgcn_raw_buffer_load_b128(rsrc_k, (32 * t + r) * (D / 2) + 32 * s + 16 * h, kb * K_BYTES, 0);
+      for (int s = 0; s < NK; ++s) kf[t][s] = __builtin_amdgcn_raw_buffer_load_b128(rsrc_k, (32 * t + score_key(r)) * (D / 2) + 32 * s + 16 * h, kb * K_BYTES, 0);
     ksc = *reinterpret_cast<const KScales*>(a.ks + (k_base / 32 + kb * 2) * (D / 32));
   };
   load_k(wave);
@@ -94,12 +94,13 @@ __device__ __forceinline__ void attn_split_body(const AttnArgs& a, const SEQS& s
     }
   }
 
-  v16f_t acc_o, acc_l;
+  v16f_t acc_o;
 #pragma unroll
-  for (int v = 0; v < 16; ++v) acc_o[v] = acc_l[v] = 0.0f;
+  for (int v = 0; v < 16; ++v) acc_o[v] = 0.0f;
+  v4f_t acc_l = {0.0f, 0.0f, 0.0f, 0.0f};
   float m_i = -__builtin_inff();
   const float cs = a.sm_scale * ATTN_RCP_LN2;
-  const v8i_t ones = v8i_t{0x22222222, 0x22222222, 0x22222222, 0x22222222, 0, 0, 0, 0};
+  const int selector = row_sum_selector(lane);
 
   // ---- V pieces of this wave's columns: row 32 role + r of V^T; scale byte of (key tile h, column block role)
   v4i_t vf[4];
@@ -115,7 +116,7 @@ __device__ __forceinline__ void attn_split_body(const AttnArgs& a, const SEQS& s
     }
   };
   v16f_t S[2];
-  float tmx[2];
+  float tile_max;
   auto phase_a = [&](int first, int buf) {
     const int kb = first + wave, key0 = kb * 64;
     int ksh[KS_DW];
@@ -134,16 +135,11 @@ __device__ __forceinline__ void attn_split_body(const AttnArgs& a, const SEQS& s
     load_k(kb + 4);
     if ((a.causal && key0 + 63 > q0 + shift) || key0 + 64 > kn) {
       asm volatile("" ::: "memory");   // keep this a branch: most blocks skip it
-      mask_scores(S, (a.causal && qrow + shift + 1 < kn ? qrow + shift + 1 : kn) - key0 - 4 * h);
+      mask_scores(S, (a.causal && qrow + shift + 1 < kn ? qrow + shift + 1 : kn) - key0 - 8 * h);
     }
-#pragma unroll
-    for (int t = 0; t < 2; ++t) {
-      float x = -__builtin_inff();
-#pragma unroll
-      for (int v = 0; v < 16; ++v) x = fmaxf(x, S[t][v]);
-      tmx[t] = pair_max(x);
-    }
-    const float mx = kb < nblk ? fmaxf(tmx[0], tmx[1]) * cs : -__builtin_inff();
+    float mx;
+    row_maxima(S, tile_max, mx);
+    mx = kb < nblk ? mx * cs : -__builtin_inff();
     reinterpret_cast<float*>(lds + L::MAXIMA)[(4 * buf + wave) * 32 + r] = mx;   // (both lanes of a row hold it)
   };
   auto phase_b = [&](int buf) {
@@ -158,7 +154,7 @@ __device__ __forceinline__ void attn_split_body(const AttnArgs& a, const SEQS& s
     const float alpha = __builtin_amdgcn_exp2f(m_old - m_new);
     v8i_t pf;
     int pscale;
-    quantize_probabilities(S, tmx, cs, m_new, h, pf, pscale);
+    quantize_probabilities(S, tile_max, cs, m_new, pf, pscale);
     const int slot = (4 * buf + wave) * 64 + lane;
     reinterpret_cast<v4i_t*>(lds + L::CODES)[slot] = v4i_t{pf[0], pf[1], pf[2], pf[3]};
     reinterpret_cast<uint2*>(lds + L::AUX)[slot] = make_uint2(f2u(alpha), (uint32_t)pscale);
@@ -192,8 +188,8 @@ __device__ __forceinline__ void attn_split_body(const AttnArgs& a, const SEQS& s
 #pragma unroll
       for (int i = 0; i < 4; ++i)
         if (!TAIL || first + i < nblk) {
-          acc_l[0] *= u2f(aux[i].x);   // all 16 registers hold the row sum; only [0] is read
-          acc_l = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(ones, v8i_t{codes[i][0], codes[i][1], codes[i][2], codes[i][3], 0, 0, 0, 0}, acc_l, 4, 4, 0, 127, 0, (int)aux[i].y);
+          acc_l[0] *= u2f(aux[i].x);   // all registers hold the row sum; only [0] is read
+          acc_l = add_row_sums(selector, v8i_t{codes[i][0], codes[i][1], codes[i][2], codes[i][3], 0, 0, 0, 0}, (int)aux[i].y, acc_l);
         }
     }
   };

@@ -82,8 +82,8 @@ __device__ __forceinline__ uint32_t e8m0_from_bf16_bits(uint32_t absbits16) {
   return e > 3u ? e - 2u : 1u;
 }
 __device__ __forceinline__ uint32_t e8m0_from_f32_bits(uint32_t absbits32) {
-  uint32_t e = ((absbits32 + 0x200000u) >> 23) & 0x1FFu;
-  return e > 3u ? e - 2u : 1u;
+  const int e = (int)((absbits32 + 0x200000u) >> 23) - 2;
+  return (uint32_t)(e > 1 ? e : 1);
 }
 // "UOS" rule: ceil(log2(absmax / 7.25)) + 127, all-zero block -> 128, clamped below at 1.
 __device__ __forceinline__ uint32_t e8m0_uos(float absmax) {

@@ -413,3 +413,27 @@ def test_strides_of_dimensions_of_size_one_do_not_matter(m, dtype, slopes):
     assert k1.stride(2) == 1 and k1.is_contiguous() and q1.is_contiguous()
     out, lse, _ = m.triton_attention_mxfp4(q1, k1, v1, al, causal=True, layout="bshd")
     assert torch.equal(out, ref) and torch.equal(lse, ref_lse)
+
+
+@pytest.mark.parametrize("dims", [(64, 64), (64, 128), (128, 64), (128, 128), (192, 128), (256, 128)], ids=lambda d: f"D{d[0]}_Dv{d[1]}")
+def test_rescale_of_single_rows(m, dims):
+    """Blocks in which the running maximum rises in one row, in one group of eight rows, in their corners, in all rows or in none: both
+    kernels against the CPU model (the accumulators are rescaled by groups of rows)."""
+    D, Dv = dims
+    rises = [range(32), [0], [7], [8], [31], range(8, 16), range(24, 32), [], [3, 12, 19, 28], range(0, 32, 2), [], range(32), [16, 17]]
+    Sq, Sk, H = 128, 64 * len(rises), 8
+    g = torch.Generator().manual_seed(D + Dv)
+    q = torch.zeros(1, H, Sq, D)
+    q[:, :, torch.arange(Sq), torch.arange(Sq) % 32] = 4.0      # row i scores element i % 32 of a key
+    k = torch.zeros(1, 1, Sk, D)
+    for b, rows in enumerate(rises):
+        k[:, :, 64 * b + 11 * b % 64, list(rows)] = 1 + b / 2
+    v = torch.randn(1, 1, Sk, Dv, generator=g)
+    q, k, v = (t.to(torch.bfloat16) for t in (q, k, v))
+    ref, ref_lse = attention_fwd_ref(q, k, v, causal=False, sm_scale=0.25)
+    for B in (1, 64):
+        assert attention_rows(B, H, Sq, Sk, D, False) == (32 if B == 1 else 128)
+        out, lse, _ = m.triton_attention_mxfp4(*(t.to(DEV).expand(B, -1, -1, -1).contiguous() for t in (q, k, v)), causal=False, sm_scale=0.25)
+        for i in (0, B - 1):
+            assert _rel(out[i:i + 1].cpu(), ref) <= REL_L2, (B, i)
+            assert float((lse[i:i + 1].cpu() - ref_lse).abs().max()) <= 1e-4, (B, i)
