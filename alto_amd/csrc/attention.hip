@@ -359,17 +359,18 @@ static int launch_attn(const AttnArgs& a, const SEQS& seqs, int B, int row_block
 
 // Rows of one workgroup: 32 where its waves deal out the keys (attention_split.hip), 128 where every wave walks them all.
 //
-// The split kernel takes about 1.5 times the instructions per row and key (1.0 against 0.66 us of a SIMD for 32 rows and 64 keys,
-// head dims of 128) and a quarter of the time for one row's keys, so it pays while the launch is as long as its longest rows,
-// i.e. while its workgroups, each counted as its share of the longest one (6 blocks of keys on top for what does not depend on
-// their number), are about as many as are resident at a time: 4 per compute unit with D = 64, 3 with 128, 2 above, and an
-// eighth more.  Device time, us, 128 rows / 32 rows, share of the slots in brackets:
-//   D = 128, causal: 8 heads x 1024 tokens 22.8 / 13.5 (.22), 8 x 4096 69.3 / 41.5 (.73), 12 x 4096 74.4 / 62.9 (1.1), 24 x 2048
-//   43.5 / 39.5 (1.18), 28 x 2048 44.7 / 44.1 (1.38), 32 x 2048 45.2 / 48.0 (1.58), 4 x 32 heads x 2048 108 / 156;
-//   all keys: 16 x 1024 23.2 / 15.7 (.67), 24 x 1024 25.3 / 21.7 (1.0), 28 x 1024 26.0 / 28.0 (1.17), 8 x 4096 68 / 74 (1.33);
-//   short: 32 x 256 11.8 / 9.2 (.14), 4 x 16 x 512 18.4 / 18.2 (1.0), 4 x 32 x 256 15.0 / 16.5 (1.13);
-//   D = 64: 16 x 2048 causal 36.3 / 23.0 (.59), 28 x 2048 36.8 / 33.0 (1.04), 32 x 2048 37.5 / 35.1 (1.18), 56 x 1024 23.0 / 23.7 (1.15);
-//   D = 192: 16 x 1024 causal 30.3 / 18.1 (.66), D = 256: 16 x 1024 all keys 27.6 / 23.4 (1.0), 32 x 1024 causal 30.5 / 30.6 (1.32).
+// The split kernel takes about 1.6 times the instructions per row and key and a quarter of the time for one row's keys, so it pays while
+// the launch is as long as its longest rows, i.e. while its workgroups, each counted as its share of the longest one (6 blocks of keys
+// on top for what does not depend on their number), are about as many as are resident at a time: 4 per compute unit with D = 64, 3 with
+// 128, 2 above.  How many of these slots may be taken: equal workgroups (all keys) are bound to the round, a causal mask's fill up
+// another's end, more so the more blocks there are; up to 8 blocks the start of a workgroup counts for more; the 128 rows of D = 192 wait
+// for bank conflicts.  Device time, us, 128 rows / 32 rows, share of the slots in brackets:
+//   D = 128, causal: 8 heads x 4096 tokens 60.7 / 34.2 (.73), 14 x 4096 63.9 / 58.1 (1.27), 31 x 2048 36.6 / 38.9 (1.51), 39 x 1024
+//   21.1 / 18.6 (1.05), 56 x 1024 22.3 / 25.1 (1.51), 81 x 256 9.0 / 7.8 (.70), 122 x 256 9.5 / 11.0 (1.05);
+//   all keys: 6 x 4096 60.7 / 45.3 (1.0), 13 x 2048 33.9 / 34.5 (1.08), 30 x 1024 20.5 / 21.8 (1.25), 101 x 256 9.0 / 10.5 (1.05);
+//   D = 192, causal: 8 x 4096 71.7 / 37.5 (1.09), 20 x 2048 42.3 / 32.7 (1.46), 70 x 256 9.8 / 10.3 (.90);
+//   D = 256, all keys: 4 x 4096 69.5 / 54.0 (1.0), 10 x 2048 39.3 / 44.6 (1.25), 67 x 256 9.9 / 12.4 (1.05).
+// Over 238 shapes at .7 to 1.9 of the slots, the mean loss against the better kernel of each is 1.3 % (D = 192: 4 %).
 // Packed sequences are weighed all together, also where there are more than one launch holds (64): such a call keeps to 128 rows
 // sooner than each of its launches by itself would have to.
 static int rows_per_workgroup(const AttnArgs& a, int64_t B, int64_t D, int n_seqs, const int32_t* cu_q, const int32_t* cu_k) {
@@ -382,7 +383,8 @@ static int rows_per_workgroup(const AttnArgs& a, int64_t B, int64_t D, int n_seq
     longest = n > longest ? n : longest;
   }
   const int per_cu = D == 64 ? 4 : (D == 128 ? 3 : 2);
-  return (double)B * a.Hq * work <= 288.0 * per_cu * (double)(longest + 6) ? 32 : 128;
+  const double share = longest <= 8 ? 0.95 : (D == 192 ? 1.4 : (a.causal ? (longest >= 24 ? 1.3 : 1.125) : (D == 64 ? 1.125 : 1.02)));
+  return (double)B * a.Hq * work <= 256.0 * share * per_cu * (double)(longest + 6) ? 32 : 128;
 }
 
 template <typename SEQS>
