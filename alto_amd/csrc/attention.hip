@@ -383,7 +383,7 @@ static int rows_per_workgroup(const AttnArgs& a, int64_t B, int64_t D, int n_seq
     longest = n > longest ? n : longest;
   }
   const int per_cu = D == 64 ? 4 : (D == 128 ? 3 : 2);
-  const double share = longest <= 8 ? 0.95 : (D == 192 ? 1.4 : (a.causal ? (longest >= 24 ? 1.3 : 1.125) : (D == 64 ? 1.125 : 1.02)));
+  const double share = longest <= 8 ? 0.95 : (D == 192 ? 1.4 : (a.causal ? (longest >= 48 ? 1.3 : 1.125) : (D == 64 ? 1.125 : 1.02)));
   return (double)B * a.Hq * work <= 256.0 * share * per_cu * (double)(longest + 6) ? 32 : 128;
 }
 
