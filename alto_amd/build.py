@@ -96,6 +96,11 @@ def _hipcc() -> str:
     return exe
 
 
+def _rocm_include() -> str:
+    """Where the HIP runtime's headers are (torch's stream header names its types)."""
+    return os.path.join(os.path.dirname(os.path.dirname(os.path.realpath(_hipcc()))), "include")
+
+
 def _compile(src: str) -> str:
     obj = os.path.join(OBJDIR, os.path.splitext(src)[0] + ".o")
     cmd = [_hipcc(), *HIPCC_FLAGS, "-c", os.path.join(CSRC, src), "-o", obj]
@@ -116,8 +121,8 @@ def build_host() -> str:
     out = host_path()
     tmp = f"{out}.{os.getpid()}.tmp"
     cmd = [shutil.which("g++") or "g++", *HOST_FLAGS, f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", f"-I{tdir}/include",
-           f"-I{tdir}/include/torch/csrc/api/include", f"-I{sysconfig.get_paths()['include']}", HOSTSRC, "-o", tmp, f"-L{tdir}/lib", "-lc10", "-ltorch_cpu",
-           "-ltorch_python"]
+           f"-I{tdir}/include/torch/csrc/api/include", f"-I{sysconfig.get_paths()['include']}", f"-I{_rocm_include()}", HOSTSRC, "-o", tmp, f"-L{tdir}/lib",
+           "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_python"]
     res = subprocess.run(cmd, capture_output=True, text=True)
     if res.returncode != 0:
         raise RuntimeError(f"g++ failed for host.cpp:\n{res.stdout}\n{res.stderr}")

@@ -13,9 +13,14 @@
 
 #include <ATen/ATen.h>
 #include <c10/core/impl/LocalDispatchKeySet.h>
+#include <c10/hip/HIPStream.h>
+#include <torch/csrc/Exceptions.h>
+#include <torch/csrc/autograd/custom_function.h>
 
 #include <algorithm>
+#include <cstring>
 #include <optional>
+#include <string>
 #include <vector>
 
 #include "../../include/alto_mxfp4.h"
@@ -286,10 +291,12 @@ bool attend(const Tensor& q_in, const Tensor& k_in, const Tensor& v_in, double s
 }
 
 // ------------------------------------------------------------------------------------------------- whole training directions
-// One call per direction of a layer's step: outputs, quantizers and products, with the interpreter lock given up once.  What a
-// direction needs only itself shares one buffer, what the backward needs of either operand has one of its own.  Under the
-// engine's own thread every piece of interpreter work costs twice what it does in a loop (the two threads take turns on two cores):
-// linear step of 512 x 1024 x 1024 forward 71 -> 39 us, backward 53 -> 23, the whole step 188 -> 115 (54 of them a function that does nothing).
+// A layer's step as an autograd node of its own, one native call per direction: outputs, quantizers and products, the interpreter
+// lock given up.  What a direction needs only itself shares one buffer, what the backward needs of either operand has one of its own.
+// The backward runs on the engine's device thread while the caller waits, and every handover of the interpreter lock between the two
+// is a wake-up more: as a Python function whose two directions were native calls, a linear step of 512 x 1024 x 1024 took 119 us, as a
+// node that the engine calls without the interpreter 92 (about 40 of them the engine's own two wake-ups, 17 this backward; where a
+// waiting thread wakes in 3 us instead of 15, 108 -> 50); 2048 x 4096 x 4096 119 -> 97, expert layer of 2560 x 1024 x 1440 139 -> 110.
 struct Failure {
   int rc = 0;
   const char* name = "";
@@ -332,15 +339,29 @@ bool rows_readable(const Tensor& t) {
   return true;
 }
 
+// The options of a step, by value: what its node keeps for the backward besides the saved buffers
+struct StepOptions {
+  bool hadamard = false, permuted = false, uos = false, sr = false, dge = false, trans_weights = false;
+  int clip = 0, packed = 0;
+  int64_t E = 0, N = 0, K = 0;
+  double out_scale = 1.0;   // of the weight gradient
+  at::ScalarType dtype = at::kFloat;
+  int8_t signs[32];
+  uint8_t perm[32];
+  StepOptions() = default;
+  // signs int8[32] and perm uint8[32] on the host, as HadamardTransform keeps them
+  StepOptions(const OptTensor& s, const OptTensor& p, int clip_, bool uos_, bool sr_, bool dge_, double out_scale_) : uos(uos_), sr(sr_), dge(dge_), clip(clip_), out_scale(out_scale_) {
+    hadamard = s.has_value();
+    permuted = p.has_value();
+    if (hadamard) std::memcpy(signs, s->data_ptr(), 32);
+    if (permuted) std::memcpy(perm, p->data_ptr(), 32);
+  }
+};
 struct Hadamard {
   int on = 0;
   const int8_t* signs = nullptr;
   const uint8_t* perm = nullptr;
-  Hadamard(const OptTensor& s, const OptTensor& p) {
-    on = s.has_value();
-    if (s.has_value()) signs = static_cast<const int8_t*>(s->data_ptr());
-    if (p.has_value()) perm = static_cast<const uint8_t*>(p->data_ptr());
-  }
+  explicit Hadamard(const StepOptions& o) : on(o.hadamard), signs(o.hadamard ? o.signs : nullptr), perm(o.permuted ? o.perm : nullptr) {}
 };
 
 // both copies of a gradient [row.rows, col.rows], 1D blocks; sr_mode 0 (nearest) or 3 (the hardware's stochastic converts)
@@ -401,75 +422,163 @@ struct LinearCopies {
   }
 };
 
-// linear.py:MXFP4LinearStep.forward -> (y, buffer of x's column copy, buffer of W's column copy, packed bits)
-py::object linear_forward(const Tensor& x_in, const Tensor& w, const OptTensor& signs, const OptTensor& perm, int clip, bool uos, bool allow_packed, uintptr_t stream) {
-  if (!on_gpu(x_in) || x_in.dim() < 2 || w.dim() != 2 || !rows_readable(w) || being_traced()) return py::none();
-  const int64_t N = w.size(0), K = w.size(1);
-  if (x_in.size(-1) != K || x_in.numel() == 0 || N == 0 || N % 32 != 0 || K % 32 != 0) return py::none();
-  const Tensor x = x_in.dim() == 2 ? x_in : x_in.reshape({-1, K});
-  const int64_t M = x.size(0);
-  if (M % 32 != 0 || !rows_readable(x)) return py::none();
-  int packed = 0;
-  if (allow_packed && x.scalar_type() == at::kBFloat16 && M * std::max(N, K) < (1ll << 36) && N * K < (1ll << 36))
-    packed = (int)packed_gemm_supported(M, N, K) | (int)packed_gemm_supported(M, K, N) << 1 | (int)packed_gemm_supported(N, K, M) << 2;
-  const LinearCopies c(M, N, K, packed);
-  const Hadamard h(signs, perm);
-  Tensor xs, ws, y;
-  Failure f;
-  {
-    py::gil_scoped_release nogil;
-    const Alloc a(x);
-    const Tensor tmp = a.dense({c.w_row.end()});
-    xs = a.dense({c.x_col.end()});
-    ws = a.dense({c.w_col.end()});
-    y = at::empty({M, N}, x.options());
-    void* s = reinterpret_cast<void*>(stream);
-    quantize_operands(f, x, c.x_row, tmp, c.x_col, xs, h, clip, w, c.w_row, tmp, c.w_col, ws, uos, s) && product(f, c.x_row, tmp, c.w_row, tmp, y, 1.0, s);
-    // a view for two dimensions as well, as the general function returns it: autograd refuses to change either in place
-    auto shape = x_in.sizes().vec();
-    shape.back() = N;
-    y = y.view(shape);
+// A call that a node may serve: not under torch.jit.trace, a functorch transform or forward-mode differentiation, which the general
+// functions refuse
+bool node_serves(const Tensor& x, const Tensor& weight) {
+  return !being_traced() && !c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::FuncTorchDynamicLayerFrontMode) && !x._fw_grad(0).defined() &&
+         !weight._fw_grad(0).defined();
+}
+void* current_stream(const Tensor& t) { return c10::hip::getCurrentHIPStream(t.device().index()).stream(); }
+
+// A refused launch on its way out of a node
+struct Refused {
+  Failure failure;
+};
+
+// Inside the engine an error of the interpreter travels as torch's own exception
+template <typename F>
+auto with_interpreter(F&& f) {
+  const py::gil_scoped_acquire gil;
+  try {
+    return f();
+  } catch (py::error_already_set& e) {
+    e.restore();
+    python_error error;
+    error.persist();
+    throw error;
   }
-  f.raise();
-  return py::make_tuple(y, xs, ws, packed);
+}
+void raise_in_engine(const Failure& f) {
+  if (f.rc != 0) with_interpreter([&] { f.raise(); });
+}
+// (a module that is loaded: a lookup)
+py::object python_function(const char* module, const char* name) { return py::module_::import(module).attr(name); }
+bool host_keyed_hardware_rounding() {
+  return with_interpreter([] { return python_function("alto_amd.mxfp4._runtime", "host_keyed_hardware_rounding")().cast<bool>(); });
 }
 
+using torch::autograd::AutogradContext;
+using torch::autograd::variable_list;
+
+std::string to_text(const StepOptions& o) { return std::string(reinterpret_cast<const char*>(&o), sizeof o); }
+StepOptions options_of(AutogradContext* ctx) {
+  StepOptions o;
+  const std::string& text = ctx->saved_data["options"].toStringRef();
+  std::memcpy(&o, text.data(), sizeof o);
+  return o;
+}
+static_assert(std::is_trivially_copyable<StepOptions>::value, "kept as bytes");
+py::object signs_of(const StepOptions& o) { return o.hadamard ? py::cast(at::from_blob(const_cast<int8_t*>(o.signs), {32}, at::kChar).clone()) : py::none(); }
+py::object perm_of(const StepOptions& o) { return o.permuted ? py::cast(at::from_blob(const_cast<uint8_t*>(o.perm), {32}, at::kByte).clone()) : py::none(); }
+
+struct StepOperands {   // what a node's forward works on, beside the tensors that its gradients belong to
+  Tensor x, w, offs;    // x [M, K]; the plain weight behind a wrapper; groups (offsets or ends)
+  bool ends = false;
+  StepOptions o;
+};
 bool whole_buffer(const Tensor& t, int64_t n) { return on_gpu(t) && t.scalar_type() == at::kByte && t.dim() == 1 && t.numel() == n && t.is_contiguous() && aligned16(t); }
 
 // philox_seed_offset(None, None)[0] of _runtime.py: the same draw
 uint64_t draw_seed() { return (uint64_t)at::randint(0, INT64_MAX, {1}, at::TensorOptions().dtype(at::kLong).device(at::kCPU)).item<int64_t>(); }
 
-// linear.py:MXFP4LinearStep.backward -> (dx, dw); sr: the hardware's stochastic converts, keyed with a draw from torch's CPU generator
-py::object linear_backward(const Tensor& go_in, const Tensor& xs, const Tensor& ws, int64_t N, int64_t K, int packed, bool sr, const OptTensor& signs, const OptTensor& perm,
-                           int clip, bool uos, double out_scale, uintptr_t stream) {
-  if (!on_gpu(go_in) || go_in.dim() < 2 || go_in.size(-1) != N) return py::none();
+// -> (dx, dw), or false; sr: the hardware's stochastic converts, keyed with a draw from torch's CPU generator
+bool linear_gradients(const Tensor& go_in, const Tensor& xs, const Tensor& ws, const StepOptions& o, Tensor& dx, Tensor& dw) {
+  const int64_t N = o.N, K = o.K;
+  if (!on_gpu(go_in) || go_in.scalar_type() != o.dtype || go_in.dim() < 2 || go_in.size(-1) != N) return false;
   const Tensor go = go_in.dim() == 2 ? go_in : go_in.reshape({-1, N});
   const int64_t M = go.size(0);
-  const LinearCopies c(M, N, K, packed);
-  if (!rows_readable(go) || !whole_buffer(xs, c.x_col.end()) || !whole_buffer(ws, c.w_col.end())) return py::none();
-  if (packed != 0 && go.scalar_type() != at::kBFloat16) return py::none();
-  const Hadamard h(signs, perm);
-  Tensor dx, dw;
+  const LinearCopies c(M, N, K, o.packed);
+  if (!rows_readable(go) || !whole_buffer(xs, c.x_col.end()) || !whole_buffer(ws, c.w_col.end())) return false;
+  if (o.packed != 0 && go.scalar_type() != at::kBFloat16) return false;
+  if (o.sr && !host_keyed_hardware_rounding()) return false;
+  const Hadamard h(o);
+  Failure f;
+  const uint64_t seed = o.sr ? draw_seed() : 0;
+  const Tensor tmp = Alloc(go).dense({c.go_col.end()});
+  dx = at::empty({M, K}, go.options());
+  dw = at::empty({N, K}, go.options());
+  void* s = current_stream(go);
+  quantize_gradient(f, go, c.go_row, tmp, c.go_col, tmp, o.sr ? 3 : 0, seed, h, o.clip, o.uos, s) && [&] {
+    const alto_mxfp4_product x = product_of(c.go_row, tmp, c.w_col, ws, dx, 1.0), w = product_of(c.go_col, tmp, c.x_col, xs, dw, o.out_scale);
+    return f.ok("alto_mxfp4_gemm_two", api.gemm_two(&x, &w, s));
+  }();
+  raise_in_engine(f);
+  if (go_in.dim() != 2) {
+    auto shape = go_in.sizes().vec();
+    shape.back() = K;
+    dx = dx.view(shape);
+  }
+  return true;
+}
+
+struct LinearNode : torch::autograd::Function<LinearNode> {
+  static Tensor forward(AutogradContext* ctx, const Tensor& x_in, const Tensor&, const StepOperands& op) {
+    const StepOptions& o = op.o;
+    const int64_t M = op.x.size(0);
+    const LinearCopies c(M, o.N, o.K, o.packed);
+    const Hadamard h(o);
+    Failure f;
+    const Alloc a(op.x);
+    const Tensor tmp = a.dense({c.w_row.end()}), xs = a.dense({c.x_col.end()}), ws = a.dense({c.w_col.end()});
+    const Tensor y = at::empty({M, o.N}, op.x.options());
+    void* s = current_stream(op.x);
+    quantize_operands(f, op.x, c.x_row, tmp, c.x_col, xs, h, o.clip, op.w, c.w_row, tmp, c.w_col, ws, o.uos, s) && product(f, c.x_row, tmp, c.w_row, tmp, y, 1.0, s);
+    if (f.rc != 0) throw Refused{f};
+    ctx->save_for_backward({xs, ws});
+    ctx->saved_data["options"] = to_text(o);
+    // a view for two dimensions as well, as the general function returns it: autograd refuses to change either in place
+    auto shape = x_in.sizes().vec();
+    shape.back() = o.N;
+    return y.view(shape);
+  }
+  static variable_list backward(AutogradContext* ctx, variable_list grads) {
+    const StepOptions o = options_of(ctx);
+    const variable_list saved = ctx->get_saved_variables();
+    variable_list out(3);   // x, the weight, the operands
+    if (!linear_gradients(grads[0], saved[0], saved[1], o, out[0], out[1]))
+      with_interpreter([&] {
+        const py::tuple g = python_function("alto_amd.mxfp4.linear", "_declined_backward")(grads[0], saved[0], saved[1], o.N, o.K, o.packed, o.dtype == at::kBFloat16, o.sr,
+                                                                                          signs_of(o), perm_of(o), o.clip, o.uos, o.dge);
+        out[0] = g[0].cast<Tensor>();
+        out[1] = g[1].cast<Tensor>();
+      });
+    return out;
+  }
+};
+
+template <typename Node>
+py::object apply_node(const Tensor& x, const Tensor& weight, const StepOperands& op) {
+  Tensor y;
   Failure f;
   {
     py::gil_scoped_release nogil;
-    const uint64_t seed = sr ? draw_seed() : 0;
-    const Tensor tmp = Alloc(go).dense({c.go_col.end()});
-    dx = at::empty({M, K}, go.options());
-    dw = at::empty({N, K}, go.options());
-    void* s = reinterpret_cast<void*>(stream);
-    quantize_gradient(f, go, c.go_row, tmp, c.go_col, tmp, sr ? 3 : 0, seed, h, clip, uos, s) && [&] {
-      const alto_mxfp4_product x = product_of(c.go_row, tmp, c.w_col, ws, dx, 1.0), w = product_of(c.go_col, tmp, c.x_col, xs, dw, out_scale);
-      return f.ok("alto_mxfp4_gemm_two", api.gemm_two(&x, &w, s));
-    }();
-    if (go_in.dim() != 2) {
-      auto shape = go_in.sizes().vec();
-      shape.back() = K;
-      dx = dx.view(shape);
+    try {
+      y = Node::apply(x, weight, op);
+    } catch (const Refused& r) {
+      f = r.failure;
     }
   }
   f.raise();
-  return py::make_tuple(dx, dw);
+  return py::cast(y);
+}
+
+// linear.py:MXFP4LinearStep -> y, or None.  `weight`: what the gradient belongs to (a wrapper, perhaps), `w`: its values
+py::object linear_step(const Tensor& x, const Tensor& weight, const Tensor& w, const OptTensor& signs, const OptTensor& perm, int clip, bool uos, bool sr, bool dge,
+                       double out_scale, bool allow_packed) {
+  if (!on_gpu(x) || x.dim() < 2 || w.dim() != 2 || !rows_readable(w) || !node_serves(x, weight)) return py::none();
+  StepOperands op{x, w, Tensor(), false, StepOptions(signs, perm, clip, uos, sr, dge, out_scale)};
+  const int64_t N = op.o.N = w.size(0), K = op.o.K = w.size(1);
+  if (x.size(-1) != K || x.numel() == 0 || N == 0 || N % 32 != 0 || K % 32 != 0) return py::none();
+  if (x.dim() != 2) {
+    const at::NoGradGuard guard;
+    op.x = x.reshape({-1, K});
+  }
+  const int64_t M = op.x.size(0);
+  if (M % 32 != 0 || !rows_readable(op.x)) return py::none();
+  op.o.dtype = x.scalar_type();
+  if (allow_packed && op.o.dtype == at::kBFloat16 && M * std::max(N, K) < (1ll << 36) && N * K < (1ll << 36))
+    op.o.packed = (int)packed_gemm_supported(M, N, K) | (int)packed_gemm_supported(M, K, N) << 1 | (int)packed_gemm_supported(N, K, M) << 2;
+  return apply_node<LinearNode>(x, weight, op);
 }
 
 // (a saved-tensor hook may hand a buffer back at any address)
@@ -522,70 +631,87 @@ bool grouped_product(Failure& f, const Copy& a, const Tensor& a_buf, const Copy&
                                   plan.data_ptr(), plan.numel(), (int)planned, s));
 }
 
-// grouped_gemm.py:MXFP4GroupedStep.forward: x [M, K] bf16, w [E, N, K] (trans) or [E, K, N], groups as offsets [E + 1] or, with `ends`, as
-// cumulative group ends [E] -> (out, buffer of x's column copy, buffer of the experts' copy along N, offsets, pass list)
-py::object grouped_forward(const Tensor& x, const Tensor& w, const Tensor& offs_in, bool ends, bool trans_weights, const OptTensor& signs, const OptTensor& perm, int clip,
-                           bool uos, uintptr_t stream) {
+// -> (dx, dw), or false
+bool grouped_gradients(const Tensor& go, const Tensor& xs, const Tensor& ws, const Tensor& offs, const Tensor& plan, const StepOptions& o, Tensor& dx, Tensor& dw) {
+  const int64_t E = o.E, N = o.N, K = o.K;
+  if (go.dim() != 2 || go.size(1) != N || !rows_readable(go) || go.scalar_type() != at::kBFloat16 || !go.is_contiguous()) return false;
+  const int64_t M = go.size(0);
+  const GroupedCopies c(M, E, N, K);
+  if (!whole_buffer(xs, c.x_col.end()) || !whole_buffer(ws, c.wd.end()) || !whole_buffer(plan, api.grouped_gemm_workspace_bytes(M, (int)E))) return false;
+  if (!on_gpu(offs) || offs.scalar_type() != at::kInt || offs.numel() != E + 1 || !offs.is_contiguous()) return false;
+  if (o.sr && !host_keyed_hardware_rounding()) return false;
+  const Hadamard h(o);
+  Failure f;
+  const uint64_t seed = o.sr ? draw_seed() : 0;
+  void* s = current_stream(go);
+  const Tensor tmp = Alloc(go).dense({c.go_col.end()});
+  dx = at::empty({M, K}, go.options());
+  dw = o.trans_weights ? at::empty({E, N, K}, go.options()) : at::empty({E, K, N}, go.options());
+  quantize_gradient(f, go, c.go_row, tmp, c.go_col, tmp, o.sr ? 3 : 0, seed, h, o.clip, o.uos, s) && grouped_product(f, c.go_row, tmp, c.wd, ws, offs, plan, true, dx, s) &&
+      f.ok("alto_mxfp4_grouped_gemm_dw_ps",
+           api.grouped_gemm_dw_ps(c.go_col.codes(tmp), c.go_col.ld(), c.go_col.scales(tmp), c.x_col.codes(xs), c.x_col.ld(), c.x_col.scales(xs),
+                                  static_cast<const int32_t*>(offs.data_ptr()), nullptr, (int)E, (int)E, M, N, K, dw.data_ptr(), dw.stride(0),
+                                  o.trans_weights ? dw.stride(1) : dw.stride(2), o.trans_weights ? dw.stride(2) : dw.stride(1), (float)o.out_scale, s));
+  raise_in_engine(f);
+  return true;
+}
+
+struct GroupedNode : torch::autograd::Function<GroupedNode> {
+  static Tensor forward(AutogradContext* ctx, const Tensor& x, const Tensor&, const StepOperands& op) {
+    const StepOptions& o = op.o;
+    const int64_t M = x.size(0), E = o.E;
+    const GroupedCopies c(M, E, o.N, o.K);
+    const Hadamard h(o);
+    Failure f;
+    const Alloc a(op.x);
+    void* s = current_stream(op.x);
+    const Tensor tmp = a.dense({c.wf.end()}), xs = a.dense({c.x_col.end()}), ws = a.dense({c.wd.end()});
+    const Tensor out = at::empty({M, o.N}, op.x.options()), plan = a.dense({api.grouped_gemm_workspace_bytes(M, (int)E)});
+    Tensor offs = op.offs;
+    bool ok = true;
+    if (op.ends) {
+      offs = at::empty({E + 1}, op.offs.options());
+      ok = f.ok("alto_mxfp4_grouped_gemm_offsets", api.grouped_gemm_offsets(static_cast<const int32_t*>(op.offs.data_ptr()), (int)E, static_cast<int32_t*>(offs.data_ptr()), s));
+    }
+    ok = ok && (o.trans_weights ? quantize_operands(f, op.x, c.x_row, tmp, c.x_col, xs, h, o.clip, op.w, c.wf, tmp, c.wd, ws, o.uos, s)
+                                : quantize_operands(f, op.x, c.x_row, tmp, c.x_col, xs, h, o.clip, op.w, c.wd, ws, c.wf, tmp, o.uos, s));
+    ok = ok && grouped_product(f, c.x_row, tmp, c.wf, tmp, offs, plan, false, out, s);
+    if (!ok) throw Refused{f};
+    ctx->save_for_backward({xs, ws, offs, plan});
+    ctx->saved_data["options"] = to_text(o);
+    return out;
+  }
+  static variable_list backward(AutogradContext* ctx, variable_list grads) {
+    const StepOptions o = options_of(ctx);
+    const variable_list saved = ctx->get_saved_variables();
+    variable_list out(3);   // x, the weights, the operands
+    if (!grouped_gradients(grads[0], saved[0], saved[1], saved[2], saved[3], o, out[0], out[1]))
+      with_interpreter([&] {
+        const py::tuple g = python_function("alto_amd.mxfp4.grouped_gemm", "_declined_backward")(grads[0], saved[0], saved[1], saved[2], saved[3], o.E, o.N, o.K, o.trans_weights,
+                                                                                                o.sr, signs_of(o), perm_of(o), o.clip, o.uos, o.dge);
+        out[0] = g[0].cast<Tensor>();
+        out[1] = g[1].cast<Tensor>();
+      });
+    return out;
+  }
+};
+
+// grouped_gemm.py:MXFP4GroupedStep: x [M, K] bf16, w [E, N, K] (trans) or [E, K, N], groups as offsets [E + 1] or, with `ends`, as
+// cumulative group ends [E] -> out, or None
+py::object grouped_step(const Tensor& x, const Tensor& weight, const Tensor& w, const Tensor& offs, bool ends, bool trans_weights, const OptTensor& signs, const OptTensor& perm,
+                        int clip, bool uos, bool sr, bool dge, double out_scale) {
   if (x.dim() != 2 || w.dim() != 3 || !rows_readable(x) || !rows_readable(w) || x.scalar_type() != at::kBFloat16 || !x.is_contiguous() || !w.is_contiguous()) return py::none();
-  if (being_traced() || !on_gpu(offs_in) || offs_in.dim() != 1 || offs_in.scalar_type() != at::kInt || !offs_in.is_contiguous()) return py::none();
+  if (!node_serves(x, weight) || !on_gpu(offs) || offs.dim() != 1 || offs.scalar_type() != at::kInt || !offs.is_contiguous()) return py::none();
   const int64_t M = x.size(0), E = w.size(0), N = w.size(trans_weights ? 1 : 2), K = w.size(trans_weights ? 2 : 1);
-  if (x.size(1) != K || offs_in.numel() != E + !ends || M == 0 || E == 0 || N % 32 != 0 || K % 32 != 0) return py::none();
+  if (x.size(1) != K || offs.numel() != E + !ends || M == 0 || E == 0 || N % 32 != 0 || K % 32 != 0) return py::none();
   if (M * std::max(N, K) >= (1ll << 36) || N * K >= (1ll << 36) || !grouped_packed_supported(M, N, K, E) || !grouped_packed_supported(M, K, N, E) ||
       !grouped_dw_packed_supported(M, N, K, E, E))
     return py::none();
-  const GroupedCopies c(M, E, N, K);
-  const Hadamard h(signs, perm);
-  Tensor xs, ws, out, offs = offs_in, plan;
-  Failure f;
-  {
-    py::gil_scoped_release nogil;
-    const Alloc a(x);
-    void* s = reinterpret_cast<void*>(stream);
-    const Tensor tmp = a.dense({c.wf.end()});
-    xs = a.dense({c.x_col.end()});
-    ws = a.dense({c.wd.end()});
-    out = at::empty({M, N}, x.options());
-    plan = a.dense({api.grouped_gemm_workspace_bytes(M, (int)E)});
-    bool ok = true;
-    if (ends) {
-      offs = at::empty({E + 1}, offs_in.options());
-      ok = f.ok("alto_mxfp4_grouped_gemm_offsets", api.grouped_gemm_offsets(static_cast<const int32_t*>(offs_in.data_ptr()), (int)E, static_cast<int32_t*>(offs.data_ptr()), s));
-    }
-    ok = ok && (trans_weights ? quantize_operands(f, x, c.x_row, tmp, c.x_col, xs, h, clip, w, c.wf, tmp, c.wd, ws, uos, s)
-                              : quantize_operands(f, x, c.x_row, tmp, c.x_col, xs, h, clip, w, c.wd, ws, c.wf, tmp, uos, s));
-    ok = ok && grouped_product(f, c.x_row, tmp, c.wf, tmp, offs, plan, false, out, s);
-  }
-  f.raise();
-  return py::make_tuple(out, xs, ws, offs, plan);
-}
-
-// grouped_gemm.py:MXFP4GroupedStep.backward -> (dx, dw)
-py::object grouped_backward(const Tensor& go, const Tensor& xs, const Tensor& ws, const Tensor& offs, const Tensor& plan, int64_t E, int64_t N, int64_t K, bool trans_weights,
-                            bool sr, const OptTensor& signs, const OptTensor& perm, int clip, bool uos, double out_scale, uintptr_t stream) {
-  if (go.dim() != 2 || go.size(1) != N || !rows_readable(go) || go.scalar_type() != at::kBFloat16 || !go.is_contiguous()) return py::none();
-  const int64_t M = go.size(0);
-  const GroupedCopies c(M, E, N, K);
-  if (!whole_buffer(xs, c.x_col.end()) || !whole_buffer(ws, c.wd.end()) || !whole_buffer(plan, api.grouped_gemm_workspace_bytes(M, (int)E))) return py::none();
-  if (!on_gpu(offs) || offs.scalar_type() != at::kInt || offs.numel() != E + 1 || !offs.is_contiguous()) return py::none();
-  const Hadamard h(signs, perm);
-  Tensor dx, dw;
-  Failure f;
-  {
-    py::gil_scoped_release nogil;
-    const uint64_t seed = sr ? draw_seed() : 0;
-    void* s = reinterpret_cast<void*>(stream);
-    const Tensor tmp = Alloc(go).dense({c.go_col.end()});
-    dx = at::empty({M, K}, go.options());
-    dw = trans_weights ? at::empty({E, N, K}, go.options()) : at::empty({E, K, N}, go.options());
-    quantize_gradient(f, go, c.go_row, tmp, c.go_col, tmp, sr ? 3 : 0, seed, h, clip, uos, s) &&
-        grouped_product(f, c.go_row, tmp, c.wd, ws, offs, plan, true, dx, s) &&
-        f.ok("alto_mxfp4_grouped_gemm_dw_ps",
-             api.grouped_gemm_dw_ps(c.go_col.codes(tmp), c.go_col.ld(), c.go_col.scales(tmp), c.x_col.codes(xs), c.x_col.ld(), c.x_col.scales(xs),
-                                    static_cast<const int32_t*>(offs.data_ptr()), nullptr, (int)E, (int)E, M, N, K, dw.data_ptr(), dw.stride(0),
-                                    trans_weights ? dw.stride(1) : dw.stride(2), trans_weights ? dw.stride(2) : dw.stride(1), (float)out_scale, s));
-  }
-  f.raise();
-  return py::make_tuple(dx, dw);
+  StepOperands op{x, w, offs, ends, StepOptions(signs, perm, clip, uos, sr, dge, out_scale)};
+  op.o.E = E; op.o.N = N; op.o.K = K;
+  op.o.trans_weights = trans_weights;
+  op.o.dtype = at::kBFloat16;
+  return apply_node<GroupedNode>(x, weight, op);
 }
 
 // The saved buffers as the four tensors that MXFP4GroupedGEMM saves: token-packed codes and scales of x, codes [E, K, N / 2] and scales of W
@@ -629,11 +755,9 @@ PYBIND11_MODULE(alto_mxfp4_host, m) {
   m.def("grouped_packed", &grouped_packed);
   m.def("grouped_dw_packed", &grouped_dw_packed);
   m.def("attend", &attend);
-  m.def("linear_forward", &linear_forward);
-  m.def("linear_backward", &linear_backward);
+  m.def("linear_step", &linear_step);
   m.def("linear_saved", &linear_saved);
-  m.def("grouped_forward", &grouped_forward);
-  m.def("grouped_backward", &grouped_backward);
+  m.def("grouped_step", &grouped_step);
   m.def("grouped_saved", &grouped_saved);
   m.def("draw_hadamard", &draw_hadamard);
   // (the rules that linear.py and grouped_gemm.py state as well, for a comparison of the two)

@@ -11,6 +11,7 @@ from .. import _lib
 DT_BF16, DT_F32 = 0, 1
 ROUND_RNE, ROUND_SR = 0, 1
 CLIP = {"none": 0, "static": 1, "dynamic": 2}
+CLIP_NAME = {code: name for name, code in CLIP.items()}
 
 
 def dtype_code(dt: torch.dtype) -> int:

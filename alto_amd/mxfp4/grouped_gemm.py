@@ -344,43 +344,27 @@ def _grouped_backward(grad_output, saved, groups, plan, packed, num_experts, tra
     return grad_inputs, grad_weights
 
 
-@torch.compiler.allow_in_graph
-class MXFP4GroupedStep(MXFP4GroupedGEMM):
+class MXFP4GroupedStep:
     """:class:`MXFP4GroupedGEMM` for the everyday call (groups by offsets, or by their ends with ``ends``; 1D activation blocks, 2D weight
-    blocks, bf16, no dynamic clip, no weight cache): the same launches and results with one native call per direction.  What
-    those decline takes the general function's way."""
+    blocks, bf16, no dynamic clip, no weight cache): the same launches and results as one native autograd node.  What that
+    declines takes the general function's way."""
 
     @staticmethod
-    def forward(ctx, inputs, expert_weights, offsets, ends, trans_weights, use_sr_grad, use_dge, clip_mode, hadamard_transform, use_uos):
+    def apply(inputs, expert_weights, offsets, ends, trans_weights, use_sr_grad, use_dge, clip_mode, hadamard_transform, use_uos):
         h = hadamard_transform
-        w = unwrap_weight_wrapper(expert_weights)
-        res = rt.host().grouped_forward(inputs, w, offsets, ends, bool(trans_weights), None if h is None else h.signs, None if h is None else h.perm,
-                                        rt.CLIP[clip_mode], bool(use_uos), rt.stream_ptr(inputs.device)) if inputs.is_cuda and packed_scales_enabled() else None
-        ctx.step = None
-        if res is None:
-            return MXFP4GroupedGEMM.forward(ctx, inputs, expert_weights, None, trans_weights, False, True, use_sr_grad, use_dge, clip_mode, False, h, use_uos,
-                                            offsets_from_ends(offsets) if ends else offsets)
-        out, *saved = res
-        ctx.save_for_backward(*saved)
-        ctx.step = (w.shape[0], out.shape[1], inputs.shape[1])
-        ctx.options = (bool(trans_weights), bool(use_sr_grad), h, clip_mode, bool(use_uos), bool(use_dge))
-        return out
+        if inputs.is_cuda and packed_scales_enabled() and not torch.compiler.is_compiling():
+            out = rt.host().grouped_step(inputs, expert_weights, unwrap_weight_wrapper(expert_weights), offsets, ends, bool(trans_weights), None if h is None else h.signs,
+                                         None if h is None else h.perm, rt.CLIP[clip_mode], bool(use_uos), bool(use_sr_grad), bool(use_dge), _wgrad_scale(clip_mode, use_dge))
+            if out is not None:
+                return out
+        return MXFP4GroupedGEMM.apply(inputs, expert_weights, None, trans_weights, False, True, use_sr_grad, use_dge, clip_mode, False, h, use_uos,
+                                      offsets_from_ends(offsets) if ends else offsets)
 
-    @staticmethod
-    def backward(ctx, grad_output):
-        if ctx.step is None:
-            return MXFP4GroupedGEMM.backward(ctx, grad_output)[:2] + (None,) * 8
-        E, N, K = ctx.step
-        trans_weights, sr, h, clip_mode, uos, dge = ctx.options
-        x_saved, w_saved, offs, plan = ctx.saved_tensors
-        res = None
-        if not sr or rt.host_keyed_hardware_rounding():
-            res = rt.host().grouped_backward(grad_output, x_saved, w_saved, offs, plan, E, N, K, trans_weights, sr, None if h is None else h.signs,
-                                             None if h is None else h.perm, rt.CLIP[clip_mode], uos, _wgrad_scale(clip_mode, dge), rt.stream_ptr(grad_output.device))
-        if res is None:
-            res = _grouped_backward(grad_output, rt.host().grouped_saved(x_saved, w_saved, grad_output.shape[0], E, N, K), Groups(offs, None, E), plan, (True, True), E,
-                                    trans_weights, False, True, torch.bfloat16, sr, h, clip_mode, uos, dge)
-        return (*res, None, None, None, None, None, None, None, None)
+
+def _declined_backward(grad_output, x_saved, w_saved, offs, plan, E, N, K, trans_weights, sr, signs, perm, clip, uos, dge):
+    """(dx, dw) of a step's node for a gradient or a source of rounding words that its native form does not take."""
+    return _grouped_backward(grad_output, rt.host().grouped_saved(x_saved, w_saved, grad_output.shape[0], E, N, K), Groups(offs, None, E), plan, (True, True), E,
+                             trans_weights, False, True, torch.bfloat16, sr, HadamardTransform.of(signs, perm), rt.CLIP_NAME[clip], uos, dge)
 
 
 def _quantize_experts(owner: torch.Tensor, w: torch.Tensor, is_2d: bool, use_uos: bool, pack_rows: bool = False, pack_cols: bool = False):

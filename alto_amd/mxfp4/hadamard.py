@@ -26,6 +26,15 @@ class HadamardTransform:
             assert perm.shape == (BLOCK,) and sorted(perm.tolist()) == list(range(BLOCK))
         self.perm = perm
 
+    @classmethod
+    def of(cls, signs: Optional[torch.Tensor], perm: Optional[torch.Tensor]) -> Optional["HadamardTransform"]:
+        """A transform of signs and positions that another one held (None: no transform)."""
+        if signs is None:
+            return None
+        h = cls.__new__(cls)
+        h.signs, h.perm = signs, perm
+        return h
+
     @property
     def weight(self) -> torch.Tensor:
         """The dense 32x32 fp32 matrix (for inspection/tests; the kernels never materialise it)."""
@@ -72,6 +81,4 @@ class HadamardFactory:
             return HadamardTransform(torch.ones(BLOCK, dtype=torch.int8), None)
         # randint(0, 2, (32,)) in cls.dtype, then randperm(32): valid by construction, so the checks of __init__ are not run
         from .._lib import host
-        h = HadamardTransform.__new__(HadamardTransform)
-        h.signs, h.perm = host().draw_hadamard(cls.generator, cls.dtype)
-        return h
+        return HadamardTransform.of(*host().draw_hadamard(cls.generator, cls.dtype))

@@ -361,41 +361,26 @@ def _linear_backward(grad_output, saved, packed, use_2dblock_x, use_2dblock_w, o
     return grad_inputs.view(*original_shape[:-1], -1), grad_weights, None, None, None, None, None, None, None, None
 
 
-@torch.compiler.allow_in_graph
-class MXFP4LinearStep(MXFP4LinearFunction):
+class MXFP4LinearStep:
     """:class:`MXFP4LinearFunction` for the everyday call (1D activation blocks, 2D weight blocks, no dynamic clip, no weight cache):
-    the same launches and results with one native call per direction.  What those decline takes the general function's way."""
+    the same launches and results as one native autograd node.  What that declines takes the general function's way."""
 
     @staticmethod
-    def forward(ctx, x, weight, use_2dblock_x, use_2dblock_w, use_sr_grad, use_dge, clip_mode, use_macro_block_scaling,
-                hadamard_transform: Optional[HadamardTransform] = None, use_uos: bool = False):
+    def apply(x, weight, use_2dblock_x, use_2dblock_w, use_sr_grad, use_dge, clip_mode, use_macro_block_scaling,
+              hadamard_transform: Optional[HadamardTransform] = None, use_uos: bool = False):
         h = hadamard_transform
-        res = rt.host().linear_forward(x, unwrap_weight_wrapper(weight), None if h is None else h.signs, None if h is None else h.perm, rt.CLIP[clip_mode],
-                                       bool(use_uos), _PACKED_SCALES, rt.stream_ptr(x.device)) if x.is_cuda else None
-        ctx.step = None
-        if res is None:
-            return MXFP4LinearFunction.forward(ctx, x, weight, use_2dblock_x, use_2dblock_w, use_sr_grad, use_dge, clip_mode, use_macro_block_scaling, h, use_uos)
-        y, x_saved, w_saved, packed = res
-        ctx.save_for_backward(x_saved, w_saved)
-        ctx.step = (*weight.shape, packed)
-        ctx.original_dtype = x.dtype
-        ctx.options = (bool(use_sr_grad), h, clip_mode, bool(use_uos), bool(use_dge))
-        return y
+        if x.is_cuda and not torch.compiler.is_compiling():
+            y = rt.host().linear_step(x, weight, unwrap_weight_wrapper(weight), None if h is None else h.signs, None if h is None else h.perm, rt.CLIP[clip_mode],
+                                      bool(use_uos), bool(use_sr_grad), bool(use_dge), _wgrad_scale(clip_mode, use_dge), _PACKED_SCALES)
+            if y is not None:
+                return y
+        return MXFP4LinearFunction.apply(x, weight, use_2dblock_x, use_2dblock_w, use_sr_grad, use_dge, clip_mode, use_macro_block_scaling, h, use_uos)
 
-    @staticmethod
-    def backward(ctx, grad_output):
-        if ctx.step is None:
-            return MXFP4LinearFunction.backward(ctx, grad_output)
-        N, K, packed = ctx.step
-        sr, h, clip_mode, uos, dge = ctx.options
-        x_saved, w_saved = ctx.saved_tensors
-        if grad_output.dtype is ctx.original_dtype and (not sr or rt.host_keyed_hardware_rounding()):
-            res = rt.host().linear_backward(grad_output, x_saved, w_saved, N, K, packed, sr, None if h is None else h.signs, None if h is None else h.perm,
-                                            rt.CLIP[clip_mode], uos, _wgrad_scale(clip_mode, dge), rt.stream_ptr(grad_output.device))
-            if res is not None:
-                return (*res, None, None, None, None, None, None, None, None)
-        return _linear_backward(grad_output, rt.host().linear_saved(x_saved, w_saved, grad_output.numel() // N, N, K, packed), (bool(packed & 2), bool(packed & 4)),
-                                False, True, ctx.original_dtype, sr, h, clip_mode, uos, dge)
+
+def _declined_backward(grad_output, x_saved, w_saved, N, K, packed, bf16, sr, signs, perm, clip, uos, dge):
+    """(dx, dw) of a step's node for a gradient or a source of rounding words that its native form does not take."""
+    return _linear_backward(grad_output, rt.host().linear_saved(x_saved, w_saved, grad_output.numel() // N, N, K, packed), (bool(packed & 2), bool(packed & 4)), False, True,
+                            torch.bfloat16 if bf16 else torch.float32, sr, HadamardTransform.of(signs, perm), rt.CLIP_NAME[clip], uos, dge)[:2]
 
 
 def _to_mxfp4_then_scaled_mm(

@@ -332,3 +332,59 @@ def test_a_step_result_is_changed_in_place_where_the_general_functions_allow_it(
         y = fn(a).mul_(2)
         both.append((y.detach(), torch.autograd.grad(y, a, torch.ones_like(y))[0]))
     assert all(torch.equal(s, t) for s, t in zip(*both))
+
+
+def _public(m, kind):
+    """A wrapped weight and the public call on it."""
+    w = randn_outliers((640, 544) if kind == "linear" else (3, 544, 640), torch.bfloat16, seed=2).to(DEV)
+    p = torch.nn.Parameter(m.MXFP4TrainingWeightWrapperTensor(w, m.TrainingOpConfig()))
+    ends = torch.tensor([96, 320, 512], dtype=torch.int32, device=DEV)
+    return p, (lambda a: torch.nn.functional.linear(a, p)) if kind == "linear" else (lambda a: torch._grouped_mm(a, p, offs=ends))
+
+
+@pytest.mark.parametrize("kind", ["linear", "grouped"])
+def test_step_nodes_in_the_engine(m, kind):
+    """What surrounds a node: forward-mode tangents and a used-up graph are refused, an error of the interpreter in the backward arrives,
+    hooks and checkpoints see it, and a graph may be kept."""
+    import torch.autograd.forward_ad as fwad
+    from torch.utils.checkpoint import checkpoint
+    p, fn = _public(m, kind)
+    x = randn_outliers((512, 544), torch.bfloat16, seed=1).to(DEV)
+    go = (randn_outliers((512, 640), torch.bfloat16, seed=3) / 512).to(DEV)
+
+    def seeded(f):
+        torch.manual_seed(4)
+        m.HadamardFactory.configure(seed=4)
+        a = x.clone().requires_grad_(True)
+        y = f(a)
+        p.grad = None
+        y.backward(go, retain_graph=True)
+        return y, (y.detach(), a.grad, getattr(p.grad, "_data", p.grad))
+
+    y, plain = seeded(fn)
+    again = torch.autograd.grad(y, p, go, retain_graph=True)[0]
+    assert again.shape == plain[2].shape
+    _same(seeded(lambda a: checkpoint(fn, a, use_reentrant=False))[1][:1], plain[:1], "checkpoint")
+    with fwad.dual_level(), pytest.raises(NotImplementedError, match="jvp"):
+        fn(fwad.make_dual(x, x))
+    seen = []
+    y.grad_fn.register_prehook(lambda g: seen.append(g[0].shape))
+    y.backward(go)
+    assert seen == [go.shape]
+    with pytest.raises(RuntimeError, match="second time"):
+        y.backward(go)
+
+    def no_words(shape, device):
+        raise ValueError("no words")
+
+    m.set_rand_bits_source(no_words)
+    try:
+        with pytest.raises(ValueError, match="no words"):
+            seeded(fn)
+    finally:
+        m.set_rand_bits_source(None)
+    with torch.no_grad():
+        assert not fn(x).requires_grad
+    if kind == "linear":
+        with pytest.raises(RuntimeError, match="is a view and is being modified inplace"):
+            fn(x).mul_(2)
