@@ -115,7 +115,7 @@ __device__ __forceinline__ uint32_t e2m1_sr_mag(float q, uint32_t r) {
 __device__ __forceinline__ void philox_round(uint32_t (&c)[4], uint32_t k0, uint32_t k1) {
   const uint64_t p0 = (uint64_t)0xD2511F53u * c[0], p1 = (uint64_t)0xCD9E8D57u * c[2];   // 32 x 32 -> 64 bits each
   const uint32_t lo0 = (uint32_t)p0, hi0 = (uint32_t)(p0 >> 32), lo1 = (uint32_t)p1, hi1 = (uint32_t)(p1 >> 32);
-  const uint32_t n0 = hi1 ^ c[1] ^ k0, n2 = hi0 ^ c[3] ^ k1;
+  const uint32_t n0 = __builtin_amdgcn_bitop3_b32(hi1, c[1], k0, 0x96), n2 = __builtin_amdgcn_bitop3_b32(hi0, c[3], k1, 0x96);   // exclusive or of three
   c[0] = n0; c[1] = lo1; c[2] = n2; c[3] = lo0;
 }
 

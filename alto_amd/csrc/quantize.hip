@@ -77,6 +77,53 @@ __device__ __forceinline__ float div_sqrt32_signed(float z, uint32_t flip) {
   return u2f((q & 0x7FFFFFFFu) | (s & 0x80000000u));
 }
 
+// z / float32(sqrt(32)) for a result that is rounded to bf16 next: z rh + z rl with rh + rl = 1 / float32(sqrt(32)) to 49 bits, in two
+// instructions (`flip` = 0 or 0x80000000 goes onto both constants).  The fp32 result is the correctly rounded quotient for every z
+// from 2^-103 on (all 2^23 significands tried: the sequence knows no exponent until z rl loses bits below 2^-126); below, z is a sum
+// of bf16 values, i.e. a multiple of 2^-133, and every one of those gives the same bf16 value as the exact quotient.  Both
+// constants are positive, so infinities stay what they are, and -0 stays -0.  (fp32 tensors keep the correction step and the division
+// fix-up: four instructions.)  With the converts below and the three-operand exclusive or of Philox, dY 8192 x 14336 95.0 -> 85.5 us,
+// 512 x 1024 5.4 -> 4.9; x, round to nearest, 8192 x 4096 24.9 -> 22.3.
+__device__ __forceinline__ float quotient_for_bf16(float z, uint32_t flip) {
+  const float rh = u2f(f2u(0.17677669f) ^ flip), rl = u2f(0x31CFE77Au ^ flip);
+  return __builtin_fmaf(z, rh, z * rl);
+}
+
+// Four pairs of neighbours, rounded stochastically by the hardware with a random dword each, as the eight codes of a dword.  The
+// instruction replaces one byte of its destination; as a builtin it gets a destination of its own each time, and merging the four takes
+// three instructions more.
+__device__ __forceinline__ uint32_t sr_codes8(const uint32_t (&pair)[4], const uint32_t (&word)[4], float scale) {
+  uint32_t o;
+  asm("v_cvt_scalef32_sr_pk_fp4_bf16 %0, %1, %5, %9\n\t"
+      "v_cvt_scalef32_sr_pk_fp4_bf16 %0, %2, %6, %9 op_sel:[0,0,1,0]\n\t"
+      "v_cvt_scalef32_sr_pk_fp4_bf16 %0, %3, %7, %9 op_sel:[0,0,0,1]\n\t"
+      "v_cvt_scalef32_sr_pk_fp4_bf16 %0, %4, %8, %9 op_sel:[0,0,1,1]\n\t"
+      "s_nop 1"
+      : "=&v"(o)
+      : "v"(pair[0]), "v"(pair[1]), "v"(pair[2]), "v"(pair[3]), "v"(word[0]), "v"(word[1]), "v"(word[2]), "v"(word[3]), "v"(scale));
+  return o;
+}
+__device__ __forceinline__ uint32_t sr_codes8(const f2_t (&pair)[4], const uint32_t (&word)[4], float scale) {
+  uint32_t o;
+  asm("v_cvt_scalef32_sr_pk_fp4_f32 %0, %1, %5, %9\n\t"
+      "v_cvt_scalef32_sr_pk_fp4_f32 %0, %2, %6, %9 op_sel:[0,0,1,0]\n\t"
+      "v_cvt_scalef32_sr_pk_fp4_f32 %0, %3, %7, %9 op_sel:[0,0,0,1]\n\t"
+      "v_cvt_scalef32_sr_pk_fp4_f32 %0, %4, %8, %9 op_sel:[0,0,1,1]\n\t"
+      "s_nop 1"
+      : "=&v"(o)
+      : "v"(pair[0]), "v"(pair[1]), "v"(pair[2]), "v"(pair[3]), "v"(word[0]), "v"(word[1]), "v"(word[2]), "v"(word[3]), "v"(scale));
+  return o;
+}
+// Eight bf16 values in four dwords, rounded to nearest, as codes
+__device__ __forceinline__ uint32_t rne_codes8(const uint32_t* w, float scale) {
+  uint32_t o = w[0];   // (every byte is replaced)
+  o = __builtin_amdgcn_cvt_scalef32_pk_fp4_bf16(o, __builtin_bit_cast(bf16x2_t, w[0]), scale, 0);
+  o = __builtin_amdgcn_cvt_scalef32_pk_fp4_bf16(o, __builtin_bit_cast(bf16x2_t, w[1]), scale, 1);
+  o = __builtin_amdgcn_cvt_scalef32_pk_fp4_bf16(o, __builtin_bit_cast(bf16x2_t, w[2]), scale, 2);
+  o = __builtin_amdgcn_cvt_scalef32_pk_fp4_bf16(o, __builtin_bit_cast(bf16x2_t, w[3]), scale, 3);
+  return o;
+}
+
 template <typename T>
 __device__ __forceinline__ float round_to_T(float v) {
   if constexpr (sizeof(T) == 2) {   // float -> bf16 (round to nearest even, one v_cvt_pk_bf16_f32 per pair) -> float
@@ -355,22 +402,27 @@ __device__ __forceinline__ void quant_tile(const QuantParams& p, unsigned wg, un
         }
         uint32_t out = 0;
         if constexpr (SR == 0) {
-          out = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(out, v[0], v[1], scale_f, 0);
-          out = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(out, v[2], v[3], scale_f, 1);
-          out = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(out, v[4], v[5], scale_f, 2);
-          out = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(out, v[6], v[7], scale_f, 3);
-        } else if constexpr (HW) {
-          uint32_t by[4];   // byte 0 of each result holds the pair's two codes; the other bytes are not defined
-  #pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            if constexpr (BF) {
-              const uint32_t src = (GEN && p.clip_row) ? pack_bf16x2(v[2 * e], v[2 * e + 1]) : w[i][e];
-              by[e] = __builtin_amdgcn_cvt_scalef32_sr_pk_fp4_bf16(0u, __builtin_bit_cast(bf16x2_t, src), hw_row[i][0] << (8 * e), scale_f, 0);
-            } else {
-              by[e] = __builtin_amdgcn_cvt_scalef32_sr_pk_fp4_f32(0u, f2_t{v[2 * e], v[2 * e + 1]}, hw_row[i][e], scale_f, 0);
-            }
+          if (BF && !(GEN && p.clip_row)) {
+            out = rne_codes8(w[i], scale_f);
+          } else {
+            out = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(out, v[0], v[1], scale_f, 0);
+            out = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(out, v[2], v[3], scale_f, 1);
+            out = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(out, v[4], v[5], scale_f, 2);
+            out = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(out, v[6], v[7], scale_f, 3);
           }
-          out = __builtin_amdgcn_perm(by[1], by[0], 0x0C0C0400u) | __builtin_amdgcn_perm(by[3], by[2], 0x04000C0Cu);
+        } else if constexpr (HW) {
+          uint32_t word[4];
+  #pragma unroll
+          for (int e = 0; e < 4; ++e) word[e] = BF ? hw_row[i][0] << (8 * e) : hw_row[i][BF ? 0 : e];
+          if constexpr (BF) {
+            uint32_t pair[4];
+  #pragma unroll
+            for (int e = 0; e < 4; ++e) pair[e] = (GEN && p.clip_row) ? pack_bf16x2(v[2 * e], v[2 * e + 1]) : w[i][e];
+            out = sr_codes8(pair, word, scale_f);
+          } else {
+            const f2_t pair[4] = {{v[0], v[1]}, {v[2], v[3]}, {v[4], v[5]}, {v[6], v[7]}};
+            out = sr_codes8(pair, word, scale_f);
+          }
         } else {
           const float inv = u2f((254u - s) << 23);
           // sign bits of the eight codes from four hardware converts (their magnitudes are not used): 5 instructions
@@ -427,27 +479,37 @@ __device__ __forceinline__ void quant_tile(const QuantParams& p, unsigned wg, un
             }
           }
         }
-        // z * (+-1) / float32(sqrt(32)), correctly rounded: quotient estimate, one FMA correction, special cases and the
-        // sign by the division fix-up instruction.
+        // z * (+-1) / float32(sqrt(32)), correctly rounded.  Q[k] = -1: folded into the (wave-uniform) constants in the hardware mode; the
+        // software rule, which is short of scalar registers (the 64 signed constants made it spill 24 of them into vector lanes), divides
+        // by +sqrt(32) and flips the sign bits of the finished codes instead (DEFER_FLIP below: rounding, absmax and both encodes are
+        // symmetric in the sign).
   #pragma unroll
         for (int k = 0; k < 32; ++k) {
-          // Q[k] = -1: folded into the (wave-uniform) constants in the hardware mode; the software rule, which is short of
-          // scalar registers (the 64 signed constants made it spill 24 of them into vector lanes), divides by +sqrt(32) and
-          // flips the sign bits of the finished codes instead (DEFER_FLIP below: rounding, absmax and both encodes are
-          // symmetric in the sign)
           const uint32_t flip = DEFER_FLIP ? 0u : ((p.sign_mask >> k) & 1u) << 31;
-          const float ck = u2f(f2u(5.656854152679443f) ^ flip);
-          const float rck = u2f(f2u(0.17677669529663689f) ^ flip);
-          const float q = z[k] * rck;
-          // v_div_fixup_f32 gives the quotient its sign (sign(z) ^ sign(ck), so -0 stays -0) and returns +-inf for z = +-inf,
-          // where the correction term is NaN; otherwise it passes the magnitude through (measured against a max + bit-field
-          // insert pair doing the same: 0.6 % faster with the software rule, 1.4 % with the hardware converts)
-          z[k] = __builtin_amdgcn_div_fixupf(__builtin_fmaf(__builtin_fmaf(-q, ck, z[k]), rck, q), ck, z[k]);
+          if constexpr (BF) {
+            z[k] = quotient_for_bf16(z[k], flip);
+          } else {
+            // quotient estimate and one FMA correction.  v_div_fixup_f32 gives the quotient its sign (sign(z) ^ sign(ck), so -0 stays -0)
+            // and returns +-inf for z = +-inf, where the correction term is NaN; otherwise it passes the magnitude through.
+            const float ck = u2f(f2u(5.656854152679443f) ^ flip);
+            const float rck = u2f(f2u(0.17677669529663689f) ^ flip);
+            const float q = z[k] * rck;
+            z[k] = __builtin_amdgcn_div_fixupf(__builtin_fmaf(__builtin_fmaf(-q, ck, z[k]), rck, q), ck, z[k]);
+          }
         }
-        if constexpr (BF) {   // round to bf16 two at a time
+      }
+      float am = 0.0f;   // largest magnitude of the column (of a transformed bf16 column: before its rounding, which keeps the order)
+      if constexpr (!B2D) {
+  #pragma unroll
+        for (int k = 0; k < 32; k += 2) am = __builtin_fmaxf(__builtin_fmaxf(am, __builtin_fabsf(z[k])), __builtin_fabsf(z[k + 1]));
+        if constexpr (BF && RHT) am = u2f(pack_bf16x2(am, am) << 16);
+      }
+      if constexpr (BF && RHT) {   // round to bf16 two at a time: the hardware converts take the packed pairs as they are
+  #pragma unroll
+        for (int k = 0; k < 32; k += 2) zp[k >> 1] = pack_bf16x2(z[k], z[k + 1]);
+        if (!PAIRS || (GEN && p.clip_col)) {
   #pragma unroll
           for (int k = 0; k < 32; k += 2) {
-            zp[k >> 1] = pack_bf16x2(z[k], z[k + 1]);   // the hardware convert takes the packed pairs as they are
             z[k] = u2f(zp[k >> 1] << 16);
             z[k + 1] = u2f(zp[k >> 1] & 0xFFFF0000u);
           }
@@ -459,9 +521,6 @@ __device__ __forceinline__ void quant_tile(const QuantParams& p, unsigned wg, un
         if (GEN && p.uos) s = e8m0_uos(BF ? u2f(a << 16) : u2f(a));
         else s = BF ? e8m0_from_bf16_bits(a) : e8m0_from_f32_bits(a);
       } else {
-        float am = 0.0f;
-  #pragma unroll
-        for (int k = 0; k < 32; k += 2) am = __builtin_fmaxf(__builtin_fmaxf(am, __builtin_fabsf(z[k])), __builtin_fabsf(z[k + 1]));
         if (GEN && p.uos) s = e8m0_uos(am);
         else s = BF ? e8m0_from_bf16_bits(f2u(am) >> 16) : e8m0_from_f32_bits(f2u(am));
       }
@@ -499,7 +558,6 @@ __device__ __forceinline__ void quant_tile(const QuantParams& p, unsigned wg, un
         }
         uint32_t* strip = reinterpret_cast<uint32_t*>(tile) + tid * STRIP;
         const uint64_t nrow = (uint64_t)gridDim.z * nby * (uint64_t)C;   // calls of the row copy: batch * bands * C
-        uint32_t by[16];
         if constexpr (BF) {
           uint32_t pr[16];
   #pragma unroll
@@ -520,18 +578,13 @@ __device__ __forceinline__ void quant_tile(const QuantParams& p, unsigned wg, un
             const uint4 a = philox4x32_10(q, q < ctr0 ? 1ull : 0ull, key);
             const uint32_t wd[4] = {a.x, a.y, a.z, a.w};
   #pragma unroll
-            for (int j = 0; j < 16; ++j)
-              by[j] = __builtin_amdgcn_cvt_scalef32_sr_pk_fp4_bf16(0u, __builtin_bit_cast(bf16x2_t, pr[j]), wd[j >> 2] << (8 * (j & 3)), scale_f, 0);
+            for (int j = 0; j < 4; ++j) {
+              const uint32_t pair[4] = {pr[4 * j], pr[4 * j + 1], pr[4 * j + 2], pr[4 * j + 3]}, word[4] = {wd[j], wd[j] << 8, wd[j] << 16, wd[j] << 24};
+              out[j] = sr_codes8(pair, word, scale_f);
+            }
           } else {
   #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-              uint32_t o = 0;
-              o = __builtin_amdgcn_cvt_scalef32_pk_fp4_bf16(o, __builtin_bit_cast(bf16x2_t, pr[4 * j + 0]), scale_f, 0);
-              o = __builtin_amdgcn_cvt_scalef32_pk_fp4_bf16(o, __builtin_bit_cast(bf16x2_t, pr[4 * j + 1]), scale_f, 1);
-              o = __builtin_amdgcn_cvt_scalef32_pk_fp4_bf16(o, __builtin_bit_cast(bf16x2_t, pr[4 * j + 2]), scale_f, 2);
-              o = __builtin_amdgcn_cvt_scalef32_pk_fp4_bf16(o, __builtin_bit_cast(bf16x2_t, pr[4 * j + 3]), scale_f, 3);
-              out[j] = o;
-            }
+            for (int j = 0; j < 4; ++j) out[j] = rne_codes8(pr + 4 * j, scale_f);
           }
         } else {
           if (RHT) {
@@ -547,10 +600,9 @@ __device__ __forceinline__ void quant_tile(const QuantParams& p, unsigned wg, un
             for (int g = 0; g < 4; ++g) {
               const uint64_t q = ctr0 + 4 * nrow + (band * (uint64_t)C + (uint64_t)cc) * 4 + (uint64_t)g;
               const uint4 a = philox4x32_10(q, q < ctr0 ? 1ull : 0ull, key);
-              const uint32_t wd[4] = {a.x, a.y, a.z, a.w};
-  #pragma unroll
-              for (int e = 0; e < 4; ++e)
-                by[4 * g + e] = __builtin_amdgcn_cvt_scalef32_sr_pk_fp4_f32(0u, f2_t{z[8 * g + 2 * e], z[8 * g + 2 * e + 1]}, wd[e], scale_f, 0);
+              const uint32_t word[4] = {a.x, a.y, a.z, a.w};
+              const f2_t pair[4] = {{z[8 * g], z[8 * g + 1]}, {z[8 * g + 2], z[8 * g + 3]}, {z[8 * g + 4], z[8 * g + 5]}, {z[8 * g + 6], z[8 * g + 7]}};
+              out[g] = sr_codes8(pair, word, scale_f);
             }
           } else {
   #pragma unroll
@@ -563,11 +615,6 @@ __device__ __forceinline__ void quant_tile(const QuantParams& p, unsigned wg, un
               out[j] = o;
             }
           }
-        }
-        if constexpr (HW) {
-  #pragma unroll
-          for (int j = 0; j < 4; ++j)
-            out[j] = __builtin_amdgcn_perm(by[4 * j + 1], by[4 * j], 0x0C0C0400u) | __builtin_amdgcn_perm(by[4 * j + 3], by[4 * j + 2], 0x04000C0Cu);
         }
       }
       if constexpr (!HW && !PAIRS) {

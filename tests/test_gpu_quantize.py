@@ -378,3 +378,21 @@ def test_in_kernel_philox_equals_supplied_words(m, dtype, shape, software_sr):
             cq, cs = m.convert_to_mxfp4(x, axis=0, use_sr=True, philox_seed=seed, philox_offset=offset, hadamard=h)
             assert_bytes_equal(cq, eq, "Hadamard column codes (in-kernel Philox)")
             assert_bytes_equal(cs, es, "Hadamard column scales (in-kernel Philox)")
+
+
+@pytest.mark.parametrize("exponent", [-133, -126, -124, -118, -104, -96, 0, 100, 121])
+def test_hadamard_quotient_over_the_range(m, exponent):
+    """The transform's division by sqrt(32) in front of the rounding to bf16, from sums of the smallest bf16 values to overflow, infinities
+    and zeros of either sign among them: codes and scales of the column copy against the CPU model."""
+    g = torch.Generator().manual_seed(exponent + 200)
+    x = (torch.randn(96, 256, generator=g) * torch.randint(0, 3, (96, 256), generator=g)).double() * 2.0 ** exponent
+    x[::7, ::5] = -0.0
+    if exponent == 0:
+        x[3, 17], x[40, 200] = float("inf"), float("-inf")
+    x = x.to(torch.bfloat16)
+    signs, perm = hadamard_from_seed(abs(exponent))
+    h = m.HadamardTransform(signs, perm)
+    _, _, codes, scales = m.quantize_rowcol(x.to(DEV), False, hadamard=h)
+    ref, ref_scales = O.quantize(O.rht_left(x, signs, perm), axis=0)
+    finite = ~torch.isinf(x.float()).any(0)   # (columns with an infinity hold NaN codes of no particular sign)
+    assert torch.equal(codes.cpu()[:, finite], ref[:, finite]) and torch.equal(scales.cpu()[:, finite], ref_scales[:, finite])
