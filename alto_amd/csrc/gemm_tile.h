@@ -34,6 +34,19 @@ constexpr int GT_SCALE_PITCH = 5;                                // dwords per r
 constexpr int GT_SCALE_BUF_DW = (GT_TM + GT_TN) * GT_SCALE_PITCH;  // one buffer, in dwords
 constexpr int GT_LDS_BYTES = GT_NSTAGE * GT_STAGE_BYTES + 2 * GT_SCALE_BUF_DW * 4;  // 131072 + 20480 = 151552
 
+// The tile routines for WN waves along N: 4, the 256x256 tile; 2, a tile of 256x128 with four waves, for results that have too few
+// 256x256 tiles to keep the chip busy (packed scales and bf16 results only).  A wave's part, 128x64, and its loop are the same.  With one
+// such workgroup on every compute unit the loop runs at 4.6 PFLOP/s (2048 x 4096: 0.93 us per 256 of K), near what the power limit allows
+// (4.9), against 1.16 us with 256x256 tiles on half of the units; a third ring slot (156 KB of LDS) would have nothing left to hide.
+template <int WN>
+struct TileOf {
+  static constexpr int TN = 64 * WN, WAVES = 2 * WN, THREADS = 64 * WAVES;
+  static constexpr int STAGE = (GT_TM + TN) * (GT_TK / 2);
+  static constexpr int LOADS = (GT_TM + TN) / 8 / WAVES, LOADS_A = GT_TM / 8 / WAVES;   // load instructions of a wave and stage, of A among them
+  static constexpr int LDS = WN == 4 ? GT_LDS_BYTES : GT_NSTAGE * STAGE + 2 * (GT_TM + TN) * 16;
+  static_assert(WN == 4 ? TN == GT_TN && THREADS == GT_THREADS && STAGE == GT_STAGE_BYTES : WN == 2, "");
+};
+
 // Workgroups are dealt round-robin to the 8 XCDs (each with its own L2).  Every XCD gets a contiguous range of the
 // tile sequence, and the sequence walks 8 N-tiles per M-tile before moving on, so the ~32 tiles an XCD has in flight
 // share A rows and B rows through its L2.
@@ -122,7 +135,9 @@ __device__ __forceinline__ void gemm_tile_zero(TileAcc& acc) {
 //   rides in the scalar offset, and a piece beyond the end of K gets an out-of-range offset, for which the hardware
 //   returns zeros.  (Per-load offsets are recomputed at every stage rather than kept in 8 registers.)
 //   Scales: thread t owns tile row t of A (t < 256) or tile row t - 256 of B (unit stride along K, any alignment).
+template <int WN>
 struct TileLoader {
+  using W = TileOf<WN>;
   __amdgpu_buffer_rsrc_t rsrc_a, rsrc_b, rsrc_s;
   int wave, gpiece, arow0, brow0, a_last, a_first, b_last, kbytes, G, s_k0, s_row, k_lead;
   uint32_t ld_a, ld_b, soff;
@@ -146,6 +161,7 @@ struct TileLoader {
     s_k0 = ta.s_k0;
     s_row = ta.s_row;
     k_lead = ta.k_lead;
+    if constexpr (WN != 4) return;   // (packed scales)
     const bool s_is_a = wave < GT_TM / 64;   // scalar: the descriptor choice below must be provably wave-uniform
     rsrc_s = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(s_is_a ? ta.A.scales : ta.B.scales), 0,
                                                (int)(s_is_a ? ta.as_bytes : ta.bs_bytes), 0x00020000);
@@ -174,19 +190,20 @@ struct TileLoader {
     for (int i = i0; i < i1; ++i) {
       int row;
       uint32_t off;
-      if (i < 4) {
-        row = arow0 + 64 * i;
+      if (i < W::LOADS_A) {
+        row = arow0 + 8 * W::WAVES * i;
         row = row < a_last ? row : a_last;
         row = row > a_first ? row : a_first;
         off = (uint32_t)row * ld_a;
       } else {
-        row = brow0 + 64 * (i - 4);
+        row = brow0 + 8 * W::WAVES * (i - W::LOADS_A);
         row = row < b_last ? row : b_last;
         off = (uint32_t)row * ld_b;
       }
       off = (off + gpiece * 16) | oob;
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(i < 4 ? rsrc_a : rsrc_b,
-                                               (__attribute__((address_space(3))) void*)(lds + slot * GT_STAGE_BYTES + (8 * i + wave) * 1024),
+      const int at = slot * W::STAGE + (W::WAVES * i + wave) * 1024;
+      const bool of_a = i < W::LOADS_A;
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(of_a ? rsrc_a : rsrc_b, (__attribute__((address_space(3))) void*)(lds + at),
                                                16, (int)off, koff, 0, 0);
     }
   }
@@ -275,19 +292,21 @@ struct TileLoader {
 // 1 KB, which the eight waves move straight into LDS with one load each (no registers, no fix-up, no ds_write; 8 cache
 // lines per load instead of the 64 of per-row scale rows).  Needs the end of K at compile time (LMS >= 0, or no K tail) or
 // LMS = -2.
-template <bool KTAIL, int LMS = -1, int NST = 4, int PS = 0>
+template <bool KTAIL, int LMS = -1, int NST = 4, int PS = 0, int WN = 4>
 __device__ __forceinline__ void gemm_tile_mainloop(const TileArgs& ta, TileAcc& acc, uint8_t* smem) {
+  using W = TileOf<WN>;
+  static_assert(WN == 4 || PS == 1, "the narrow tile reads packed scales");
   static_assert(PS != 1 || !KTAIL || LMS >= 0 || LMS == -2, "packed scales: the end of K is known at compile time, or whole stages run (-2)");
   static_assert(PS != 2 || (KTAIL && LMS < 0), "packed scales of a sub-range of K: the generic endings only");
   constexpr int SP = PS ? 4 : GT_SCALE_PITCH;   // dwords per row of a scale buffer in LDS
-  TileLoader ld;
+  TileLoader<WN> ld;
   v4i_t sraw;   // scale bytes of a later block, as loaded
   __syncthreads();   // the LDS ring may still be read by a previous call
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;   // the wave index lives in a scalar register
-  const int wm = wave >> 2, wn = wave & 3;
+  const int wm = wave / WN, wn = wave % WN;
   const int r = lane & 31, h = lane >> 5;
-  uint32_t* sscale = reinterpret_cast<uint32_t*>(smem + GT_NSTAGE * GT_STAGE_BYTES);
+  uint32_t* sscale = reinterpret_cast<uint32_t*>(smem + GT_NSTAGE * W::STAGE);
   const int KB = (ta.G + 15) / 16;       // loop iterations: blocks of 512 K = 2 macro stages
 
   // ---- fragment read offsets (bytes inside a stage): row * 128 + ((2 j + h) ^ ((row / 2) % 8)) * 16; the j-dependent
@@ -319,7 +338,7 @@ __device__ __forceinline__ void gemm_tile_mainloop(const TileArgs& ta, TileAcc& 
   v8i_t fa0[4], fb0[2], fa1[4], fb1[2];
   int sa[4][2], sb[2][2], sa_next[4][2], sb_next[2][2];
   auto read_frags = [&](int slot, int j, v8i_t (&fa)[4], v8i_t (&fb)[2]) {
-    const uint8_t* base = smem + slot * GT_STAGE_BYTES;
+    const uint8_t* base = smem + slot * W::STAGE;
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
       uint4 a4 = *reinterpret_cast<const uint4*>(base + ((a_off ^ (j * 32)) + t * 4096));
@@ -336,8 +355,8 @@ __device__ __forceinline__ void gemm_tile_mainloop(const TileArgs& ta, TileAcc& 
   // (packed block q sits in scale buffer q & 1).
   const int sh = PS == 2 ? ta.ps_sh : 0;
   auto read_scales2 = [&](int kn, int (&xa)[4][2], int (&xb)[2][2]) {
-    const uint32_t o0 = (uint32_t)((kn & 1) * (GT_TM + GT_TN) * SP * 4 + 4 * sh);
-    const uint32_t o1 = (uint32_t)(((kn + sh) & 1) * (GT_TM + GT_TN) * SP * 4 + 4 - 4 * sh);
+    const uint32_t o0 = (uint32_t)((kn & 1) * (GT_TM + W::TN) * SP * 4 + 4 * sh);
+    const uint32_t o1 = (uint32_t)(((kn + sh) & 1) * (GT_TM + W::TN) * SP * 4 + 4 - 4 * sh);
     const uint8_t* sb8 = reinterpret_cast<const uint8_t*>(sscale);
     const uint8_t *a0 = sb8 + (sa_off + o0), *a1 = sb8 + (sa_off + o1), *b0 = sb8 + (sb_off + o0), *b1 = sb8 + (sb_off + o1);
 #pragma unroll
@@ -377,8 +396,15 @@ __device__ __forceinline__ void gemm_tile_mainloop(const TileArgs& ta, TileAcc& 
     const int buf = kb & 1;
     if constexpr (PS == 1 && KTAIL && LMS == -2) kb = kb < KB ? kb : KB - 1;   // (a block beyond K is loaded but not used; the end of the buffer is never passed)
     const int so = __builtin_amdgcn_readfirstlane((kb + ps_q0) * ps_blk + ps_row0);
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_ps, (__attribute__((address_space(3))) void*)((lds_u8s*)sscale + buf * (GT_TM + GT_TN) * SP * 4 + wave * 1024), 16,
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_ps, (__attribute__((address_space(3))) void*)((lds_u8s*)sscale + buf * (GT_TM + W::TN) * SP * 4 + wave * 1024), 16,
                                              lane * 16, so, 0, 0);
+    if constexpr (WN == 2) {   // (all four waves have 64 rows of A each, and the first two 64 rows of B as well)
+      const __amdgpu_buffer_rsrc_t rsrc_b = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(ta.B.scales), 0, (int)ta.bs_bytes, 0x00020000);
+      const int so_b = __builtin_amdgcn_readfirstlane(kb * (int)ta.B.ss_k + ((int)ta.n0 + 64 * wave) * 16);
+      if (wave < 2)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_b, (__attribute__((address_space(3))) void*)((lds_u8s*)sscale + buf * (GT_TM + W::TN) * SP * 4 + (4 + wave) * 1024), 16,
+                                                 lane * 16, so_b, 0, 0);
+    }
   };
   // 8 MFMAs of K step J (0..3) of macro stage MS (0..1 inside its 512-K block): scale byte J of dword MS
   auto mfma8 = [&](auto msc, auto jc, const v8i_t (&fa)[4], const v8i_t (&fb)[2]) {
@@ -397,7 +423,17 @@ __device__ __forceinline__ void gemm_tile_mainloop(const TileArgs& ta, TileAcc& 
     }
     __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
   };
-  auto interleave_loads = [&]() {   // the same with one global->LDS load after every second MFMA
+  auto interleave_loads = [&]() {   // the same with one global->LDS load after every second MFMA (narrow tile: 6 loads to 8 MFMAs)
+    if constexpr (WN == 2) {
+#pragma unroll
+      for (int q = 0; q < 6; ++q) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+      }
+      __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
+      return;
+    }
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
       __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
@@ -419,7 +455,7 @@ __device__ __forceinline__ void gemm_tile_mainloop(const TileArgs& ta, TileAcc& 
     constexpr int MS = decltype(msc)::value;
     constexpr bool PEN = decltype(penc)::value;
     __builtin_amdgcn_s_setprio(2);
-    ld.gload(smem, s + 1, MS ^ 1, 4, 8);
+    ld.gload(smem, s + 1, MS ^ 1, W::LOADS / 2, W::LOADS);
     mfma8(msc, std::integral_constant<int, 0>{}, fa0, fb0);
     read_frags(MS, 1, fa1, fb1);
     interleave_loads();
@@ -448,10 +484,10 @@ __device__ __forceinline__ void gemm_tile_mainloop(const TileArgs& ta, TileAcc& 
       }
       __builtin_amdgcn_sched_barrier(0);
     }
-    if constexpr (!PEN) ld.gload(smem, s + 2, MS, 0, 4);
+    if constexpr (!PEN) ld.gload(smem, s + 2, MS, 0, W::LOADS / 2);
     if constexpr (MS == 1) {   // the next block's scales (in LDS since this stage's barrier) ride along with the last step
       if constexpr (PS == 2) read_scales2(kb + 1, sa_next, sb_next);
-      else read_scales(reinterpret_cast<const uint8_t*>(sscale + ((kb + 1) & 1) * (GT_TM + GT_TN) * SP), sa_next, sb_next);
+      else read_scales(reinterpret_cast<const uint8_t*>(sscale + ((kb + 1) & 1) * (GT_TM + W::TN) * SP), sa_next, sb_next);
     }
     mfma8(msc, std::integral_constant<int, 3>{}, fa1, fb1);
     read_frags(MS ^ 1, 0, fa0, fb0);
@@ -467,16 +503,18 @@ __device__ __forceinline__ void gemm_tile_mainloop(const TileArgs& ta, TileAcc& 
   if constexpr (PS) {
     sdma(0);
     if constexpr (PS == 2) sdma(sh);   // with the shift, block 0 also needs packed block 1 (without: block 0 once more)
-    ld.gload(smem, 0, 0, 0, 8);
+    ld.gload(smem, 0, 0, 0, W::LOADS);
     (void)sraw;
   } else {
     ld.template sload<KTAIL>(0, sraw);
-    ld.gload(smem, 0, 0, 0, 8);
+    ld.gload(smem, 0, 0, 0, W::LOADS);
     swrite(0, std::false_type{});
     ld.template sload<KTAIL>(1, sraw);
   }
-  ld.gload(smem, 1, 1, 0, 4);   // the other half goes out in the first step of the loop
-  asm volatile("s_waitcnt vmcnt(4) lgkmcnt(0)\n\ts_barrier" ::: "memory");   // all but stage 1's four loads
+  ld.gload(smem, 1, 1, 0, W::LOADS / 2);   // the other half goes out in the first step of the loop
+  static_assert(W::LOADS / 2 == (WN == 4 ? 4 : 6), "the waits below");
+  if constexpr (WN == 4) asm volatile("s_waitcnt vmcnt(4) lgkmcnt(0)\n\ts_barrier" ::: "memory");   // all but stage 1's loads
+  else asm volatile("s_waitcnt vmcnt(6) lgkmcnt(0)\n\ts_barrier" ::: "memory");
   read_frags(0, 0, fa0, fb0);
   if constexpr (PS == 2) read_scales2(0, sa, sb);
   else read_scales(reinterpret_cast<const uint8_t*>(sscale), sa, sb);
@@ -539,14 +577,17 @@ __device__ __forceinline__ void gemm_tile_mainloop(const TileArgs& ta, TileAcc& 
 //   m = m0 + 128 wm + 32 t + r,  n = n0 + 64 wn + 32 u + 8 (v / 4) + 4 h + v % 4.
 // Rows outside [m_lo, m_hi) and columns at or beyond n_hi are not written.  Host-checked: N % 8 == 0, ldc % 8 == 0,
 // 16-byte aligned c.
-template <typename OutT>
+template <typename OutT, int WN = 4>
 __device__ __forceinline__ void gemm_tile_store(const TileArgs& ta, TileAcc& acc, OutT* __restrict__ c, int64_t ldc, uint8_t* smem) {
+  using W = TileOf<WN>;
+  constexpr int ROW = W::TN * 2, CHUNKS = ROW / 16;   // a bf16 row of the tile: bytes, 16-byte chunks
+  static_assert(WN == 4 || sizeof(OutT) == 2, "");
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
-  const int wm = wave >> 2, wn = wave & 3;
+  const int wm = wave / WN, wn = wave % WN;
   const int r = lane & 31, h = lane >> 5;
   if constexpr (sizeof(OutT) == 2) {
-    // bf16: the 256x256 tile (128 KB) is assembled in LDS as rows of 32 16-byte chunks, chunk index XORed with row % 32
+    // bf16: the 256x256 tile (128 KB) is assembled in LDS as rows of 32 (narrow: 16) 16-byte chunks, chunk index XORed with row % 32
     // (conflict-free for the 8-byte writes of 32 different rows and for the row-wise 16-byte reads), then stored as
     // whole rows: 32 lanes x 16 bytes = one 512-byte row segment per half-wave.
     __syncthreads();   // every wave is done reading operand pieces
@@ -556,7 +597,7 @@ __device__ __forceinline__ void gemm_tile_store(const TileArgs& ta, TileAcc& acc
       for (int u = 0; u < 2; ++u)
 #pragma unroll
         for (int vq = 0; vq < 4; ++vq) {
-          const uint32_t off = (uint32_t)(128 * wm + r) * 512 + (((8 * wn + 4 * u + vq) ^ r) << 4) + 8 * h;
+          const uint32_t off = (uint32_t)(128 * wm + r) * ROW + (((8 * wn + 4 * u + vq) ^ (r & (CHUNKS - 1))) << 4) + 8 * h;
 #pragma unroll
           for (int t = 0; t < 4; ++t) {
             float f0 = acc[t][u][4 * vq + 0], f1 = acc[t][u][4 * vq + 1], f2 = acc[t][u][4 * vq + 2], f3 = acc[t][u][4 * vq + 3];
@@ -566,25 +607,26 @@ __device__ __forceinline__ void gemm_tile_store(const TileArgs& ta, TileAcc& acc
             uint2 o;
             o.x = pack_bf16x2(f0, f1);
             o.y = pack_bf16x2(f2, f3);
-            *reinterpret_cast<uint2*>(smem + off + t * (32 * 512)) = o;
+            *reinterpret_cast<uint2*>(smem + off + t * (32 * ROW)) = o;
           }
         }
     };
     if (ta.out_scale == 1.0f) stage_out(std::false_type{});
     else stage_out(std::true_type{});
     __syncthreads();
-    // thread -> chunk ch of rows row0 + 16 it: the XOR term alternates between two values
-    const int row0 = tid >> 5, ch = tid & 31;
-    const uint32_t rd_even = (uint32_t)row0 * 512 + ((ch ^ row0) << 4), rd_odd = (uint32_t)(row0 + 16) * 512 + ((ch ^ (row0 + 16)) << 4);
-    const bool full = ta.m0 >= ta.m_lo && ta.m0 + GT_TM <= ta.m_hi && ta.n0 + GT_TN <= ta.n_hi && ldc < (1 << 22);
+    // thread -> chunk ch of rows row0 + 16 it: the XOR term alternates between two values (narrow: one)
+    static_assert(W::THREADS / CHUNKS == 16, "16 rows a pass");
+    const int row0 = tid / CHUNKS, ch = tid % CHUNKS;
+    const uint32_t rd_even = (uint32_t)row0 * ROW + ((ch ^ row0) << 4), rd_odd = (uint32_t)(row0 + 16) * ROW + ((ch ^ ((row0 + 16) & (CHUNKS - 1))) << 4);
+    const bool full = ta.m0 >= ta.m_lo && ta.m0 + GT_TM <= ta.m_hi && ta.n0 + W::TN <= ta.n_hi && ldc < (1 << 22);
     if (full) {   // no bounds to check; one 64-bit tile origin plus 32-bit offsets
       OutT* origin = c + ta.m0 * ldc + ta.n0;
       const uint32_t step = (uint32_t)ldc * 16;
       uint32_t eoff = (uint32_t)row0 * (uint32_t)ldc + 8 * ch;
 #pragma unroll
       for (int it = 0; it < 16; it += 2) {
-        const uint4 v0 = *reinterpret_cast<const uint4*>(smem + rd_even + (it / 2) * (32 * 512));
-        const uint4 v1 = *reinterpret_cast<const uint4*>(smem + rd_odd + (it / 2) * (32 * 512));
+        const uint4 v0 = *reinterpret_cast<const uint4*>(smem + rd_even + (it / 2) * (32 * ROW));
+        const uint4 v1 = *reinterpret_cast<const uint4*>(smem + rd_odd + (it / 2) * (32 * ROW));
         __builtin_nontemporal_store(*reinterpret_cast<const v4i_t*>(&v0), reinterpret_cast<v4i_t*>(origin + eoff));
         __builtin_nontemporal_store(*reinterpret_cast<const v4i_t*>(&v1), reinterpret_cast<v4i_t*>(origin + (eoff + step)));
         eoff += 2 * step;
@@ -593,7 +635,7 @@ __device__ __forceinline__ void gemm_tile_store(const TileArgs& ta, TileAcc& acc
 #pragma unroll
       for (int it = 0; it < 16; ++it) {
         const int row = row0 + 16 * it;
-        const uint4 v = *reinterpret_cast<const uint4*>(smem + ((it & 1) ? rd_odd : rd_even) + (it / 2) * (32 * 512));
+        const uint4 v = *reinterpret_cast<const uint4*>(smem + ((it & 1) ? rd_odd : rd_even) + (it / 2) * (32 * ROW));
         const int64_t m = ta.m0 + row, n = ta.n0 + 8 * ch;
         if (m >= ta.m_lo && m < ta.m_hi && n + 8 <= ta.n_hi) __builtin_nontemporal_store(*reinterpret_cast<const v4i_t*>(&v), reinterpret_cast<v4i_t*>(c + m * ldc + n));
       }
@@ -618,13 +660,13 @@ __device__ __forceinline__ void gemm_tile_store(const TileArgs& ta, TileAcc& acc
 }
 
 // LMS / NST: how the reduction ends, as in gemm_tile_mainloop.
-template <typename OutT, bool KTAIL, int LMS = -1, int NST = 4, int PS = 0>
+template <typename OutT, bool KTAIL, int LMS = -1, int NST = 4, int PS = 0, int WN = 4>
 __device__ __forceinline__ void gemm_tile_256x256(const TileArgs& ta, OutT* __restrict__ c, int64_t ldc, uint8_t* smem) {
   TileAcc acc;
   gemm_tile_zero(acc);
   // (with fp32 output and no K tail the specialised ending pushes the register allocation into spilling: plain loop there)
-  gemm_tile_mainloop<KTAIL, (!KTAIL && sizeof(OutT) == 4) ? -3 : LMS, NST, PS>(ta, acc, smem);
-  gemm_tile_store<OutT>(ta, acc, c, ldc, smem);
+  gemm_tile_mainloop<KTAIL, (!KTAIL && sizeof(OutT) == 4) ? -3 : LMS, NST, PS, WN>(ta, acc, smem);
+  gemm_tile_store<OutT, WN>(ta, acc, c, ldc, smem);
 }
 
 // The (LMS, NST) pair of a reduction over G groups of 32 whose length is known at launch (see gemm_tile_mainloop):

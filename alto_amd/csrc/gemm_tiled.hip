@@ -6,17 +6,17 @@
 namespace alto {
 namespace {
 
-template <typename OutT, bool KTAIL, int LMS, int NST, bool PS>
-__global__ __launch_bounds__(GT_THREADS) void gemm_tiled_kernel(OperandView A, OperandView B, int64_t M, int64_t N, int G,
+template <typename OutT, bool KTAIL, int LMS, int NST, bool PS, int WN>
+__global__ __launch_bounds__(TileOf<WN>::THREADS) void gemm_tiled_kernel(OperandView A, OperandView B, int64_t M, int64_t N, int G,
                                                          OutT* c, int64_t ldc, float out_scale, int tiles_m, int tiles_n) {
   extern __shared__ __align__(16) uint8_t smem[];
   int tm, tn;
   if (!tile_coords(blockIdx.x, tiles_m, tiles_n, tm, tn)) return;
   const int KB = (G + 15) / 16;
-  TileArgs ta{A, B, (int64_t)tm * GT_TM, (int64_t)tn * GT_TN, 0, M, N, G, out_scale,
+  TileArgs ta{A, B, (int64_t)tm * GT_TM, (int64_t)tn * TileOf<WN>::TN, 0, M, N, G, out_scale,
               (M - 1) * A.ld + G * 16, (N - 1) * B.ld + G * 16,
               PS ? KB * A.ss_k : ((A.is_2d ? M / 32 : M) - 1) * A.ss_r + G, PS ? KB * B.ss_k : ((B.is_2d ? N / 32 : N) - 1) * B.ss_r + G, 0, G};
-  gemm_tile_256x256<OutT, KTAIL, LMS, NST, PS>(ta, c, ldc, smem);
+  gemm_tile_256x256<OutT, KTAIL, LMS, NST, PS, WN>(ta, c, ldc, smem);
 }
 
 // Two products on packed scales, bf16 results (no KTAIL: K a multiple of 512 in both).  The tiles of the second fill the units that
@@ -58,15 +58,16 @@ __global__ __launch_bounds__(256) void pack_scales_kernel(const uint8_t* __restr
   *reinterpret_cast<uint4*>(dst + ((int64_t)kb * rows + row) * 16) = make_uint4(w[0], w[1], w[2], w[3]);
 }
 
-template <typename OutT, bool KTAIL, int LMS = -1, int NST = 4, bool PS = false>
+template <typename OutT, bool KTAIL, int LMS = -1, int NST = 4, bool PS = false, int WN = 4>
 int launch_tiled(const OperandView& A, const OperandView& B, int64_t M, int64_t N, int64_t K, void* c, int64_t ldc, float out_scale, hipStream_t st) {
-  auto kern = gemm_tiled_kernel<OutT, KTAIL, LMS, NST, PS>;
+  using W = TileOf<WN>;
+  auto kern = gemm_tiled_kernel<OutT, KTAIL, LMS, NST, PS, WN>;
   static LdsLimit lds;
-  if (const int rc = lds.raise(reinterpret_cast<const void*>(kern), GT_LDS_BYTES, "gemm")) return rc;
-  const int tiles_m = (int)((M + GT_TM - 1) / GT_TM), tiles_n = (int)((N + GT_TN - 1) / GT_TN);
+  if (const int rc = lds.raise(reinterpret_cast<const void*>(kern), W::LDS, "gemm")) return rc;
+  const int tiles_m = (int)((M + GT_TM - 1) / GT_TM), tiles_n = (int)((N + W::TN - 1) / W::TN);
   const int T = tiles_m * tiles_n;
   const int per_xcd = (T + 7) / 8;
-  hipLaunchKernelGGL(kern, dim3((unsigned)(per_xcd * 8)), dim3(GT_THREADS), GT_LDS_BYTES, st, A, B, M, N, (int)(K / 32), (OutT*)c, ldc, out_scale, tiles_m, tiles_n);
+  hipLaunchKernelGGL(kern, dim3((unsigned)(per_xcd * 8)), dim3(W::THREADS), W::LDS, st, A, B, M, N, (int)(K / 32), (OutT*)c, ldc, out_scale, tiles_m, tiles_n);
   return check_launch("gemm");
 }
 
@@ -113,10 +114,10 @@ int gemm_tiled_launch(const OperandView& A, const OperandView& B, int64_t M, int
 }
 
 // Both operands with packed scales (A.scales / B.scales = packed base, ss_k = bytes per block), bf16 output.
-int gemm_tiled_launch_ps(const OperandView& A, const OperandView& B, int64_t M, int64_t N, int64_t K, void* c, int64_t ldc, float out_scale,
-                         hipStream_t st) {
+template <int WN>   // (see TileOf)
+static int launch_ps(const OperandView& A, const OperandView& B, int64_t M, int64_t N, int64_t K, void* c, int64_t ldc, float out_scale, hipStream_t st) {
   const bool tail = (K / 32) % 16 != 0;
-#define ALTO_TILED_LAUNCH(...) launch_tiled<__bf16, __VA_ARGS__, true>(A, B, M, N, K, c, ldc, out_scale, st)
+#define ALTO_TILED_LAUNCH(...) launch_tiled<__bf16, __VA_ARGS__, true, WN>(A, B, M, N, K, c, ldc, out_scale, st)
   if (!tail) {
     return ALTO_TILED_LAUNCH(false, -1, 4);
   } else {
@@ -134,6 +135,21 @@ int gemm_tiled_launch_ps(const OperandView& A, const OperandView& B, int64_t M, 
     }
   }
 #undef ALTO_TILED_LAUNCH
+}
+
+// Up to 256 tiles of 256x128, one per compute unit, that tile: each 256x256 tile's work is then done by two units at once, where the
+// 256x256 tile leaves half of them idle or more.  us at 256x256 / 256x128 (same bits):
+//   M x N x K             tiles of 256x128                   M x N x K             tiles of 256x128
+//   1100 x 4096 x 512           160   7.9 /  6.4             1536 x 4096 x 14336         192  64.6 / 51.5
+//   1376 x 4096 x 2880          192  18.3 / 15.1             2560 x 3072 x 14336         240  72.7 / 59.0
+//   512 x 14336 x 4096          224  25.1 / 20.6             2048 x 4224 x 4096          264  26.6 / 36.3
+//   2048 x 4096 x 1024          256  11.3 / 11.2             3000 x 3072 x 1536          288  14.4 / 19.0
+//   2048 x 4096 x 4096          256  25.1 / 21.7             4096 x 4096 x 4096          512  35.9 / 41.1
+// (From 257 tiles on a second round begins, and a narrow tile reads 1.5 times the bytes per product.)
+int gemm_tiled_launch_ps(const OperandView& A, const OperandView& B, int64_t M, int64_t N, int64_t K, void* c, int64_t ldc, float out_scale,
+                         hipStream_t st) {
+  const int64_t narrow = ((M + GT_TM - 1) / GT_TM) * ((N + TileOf<2>::TN - 1) / TileOf<2>::TN);
+  return narrow <= 256 ? launch_ps<2>(A, B, M, N, K, c, ldc, out_scale, st) : launch_ps<4>(A, B, M, N, K, c, ldc, out_scale, st);
 }
 
 template <bool KTAIL>

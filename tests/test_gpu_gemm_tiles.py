@@ -68,6 +68,26 @@ def test_gemm_tiles_of_every_size_give_the_same_bits(m, K, packed):
     assert torch.equal(product(500), whole[:500])
 
 
+# Every ending of the reduction that the 256x128 tile has a kernel for, ragged rows and columns
+@pytest.mark.parametrize("K", [512, 544, 640, 704, 768, 832, 864, 960, 1024, 1184])
+def test_gemm_narrow_tile(m, K):
+    """Packed scales: 2304 x 4104 takes the 256x256 tile (297 tiles of 256x128), its first 1791 rows the 256x128 tile (231)."""
+    from alto_amd.mxfp4.linear import gemm_packed, pack_scales
+    M, N, rows = 2304, 4104, 1791
+    a, b = randn_outliers((M, K), torch.bfloat16, seed=K), randn_outliers((N, K), torch.bfloat16, seed=K + 1)
+    aq, as_ = m.convert_to_mxfp4(a.to(DEV))
+    bq, bs = m.convert_to_mxfp4(b.to(DEV))
+    def product(r, out_scale=1.0):
+        return gemm_packed(aq[:r], pack_scales(as_[:r], r, K), bq, pack_scales(bs, N, K), out_scale)
+    print(f"narrow {rows}x{N}x{K}", flush=True)
+    got = product(rows)
+    assert torch.equal(got, product(M)[:rows])
+    for i0 in (0, rows - 96):   # (the oracle takes a while for all of it)
+        ref = O.gemm_ref(aq[i0:i0 + 96].cpu(), as_[i0:i0 + 96].cpu(), bq.cpu(), bs.cpu(), trans_b=True)
+        assert O.rel_frobenius(got[i0:i0 + 96].cpu(), ref) < TOL[torch.bfloat16]
+        assert O.rel_frobenius(product(rows, 0.75)[i0:i0 + 96].cpu(), ref * 0.75) < TOL[torch.bfloat16]
+
+
 # Both sides of the lines where a short reduction goes to the direct kernel, to the kernel for few rows (16, 32 or 64 columns per
 # workgroup) or to the small tiles
 @pytest.mark.parametrize("M,N,K", [(16, 6144, 288), (16, 6144, 320), (17, 6144, 384), (17, 6144, 416), (1, 6160, 480), (1, 6160, 512), (32, 6160, 544),
