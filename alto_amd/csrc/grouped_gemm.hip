@@ -157,12 +157,12 @@ __device__ __forceinline__ bool grouped_tile_coords(int wg, int n_pass, int tile
 // workgroups to launch for that order: 8 x the tile count of the XCD with the most bands
 __host__ __device__ inline int64_t grouped_grid_size(int64_t tiles_m, int64_t tiles_n) { return 8 * ((tiles_m + 7) / 8) * tiles_n; }
 
-template <typename OutT>
+template <typename OutT, int THREADS>
 __device__ __forceinline__ void zero_rows(OutT* out, int64_t ldo, int64_t r0, int64_t r1, int64_t n0, int64_t n1) {
   constexpr int PER = 16 / sizeof(OutT);
-  const int chunks = (int)((n1 - n0) / PER);   // N % 8 == 0 and n0 % 256 == 0: whole 16-byte chunks
+  const int chunks = (int)((n1 - n0) / PER);   // N % 8 == 0 and n0 % 128 == 0: whole 16-byte chunks
   const int64_t total = (r1 - r0) * chunks;
-  for (int64_t i = threadIdx.x; i < total; i += GT_THREADS) {
+  for (int64_t i = threadIdx.x; i < total; i += THREADS) {
     const int64_t row = r0 + i / chunks;
     const int ch = (int)(i % chunks);
     *reinterpret_cast<uint4*>(out + row * ldo + n0 + (int64_t)ch * PER) = make_uint4(0, 0, 0, 0);
@@ -303,21 +303,25 @@ __global__ __launch_bounds__(PLAN_THREADS) void grouped_plan_kernel(PassWalk wk,
   if (t == PLAN_THREADS - 1) ws[0] = upto < max_pass ? upto : max_pass;
 }
 
-template <typename OutT, bool KTAIL, int LMS, int NST, bool PS>
-__global__ __launch_bounds__(GT_THREADS) void grouped_tiled_kernel(OperandView A, const uint8_t* w, int64_t w_stride_e, int64_t ldw,
+template <typename OutT, bool KTAIL, int LMS, int NST, bool PS, int WN>
+__global__ __launch_bounds__(TileOf<WN>::THREADS) void grouped_tiled_kernel(OperandView A, const uint8_t* w, int64_t w_stride_e, int64_t ldw,
                                                                    const uint8_t* w_scales, int64_t ws_stride_e, int64_t ws_r, int w_is_2d,
                                                                    const int32_t* plan, int64_t M_total, int64_t N, int G, OutT* out, int64_t ldo, int tiles_n, int run_log2) {
   extern __shared__ __align__(16) uint8_t smem[];
   const int n_pass = __builtin_amdgcn_readfirstlane(plan[0]);
   int pi, tn;
-  if (!grouped_tile_coords(blockIdx.x, n_pass, tiles_n, run_log2, pi, tn)) return;
+  if constexpr (WN == 2) {   // one round: what counts is that no XCD gets more tiles than the others
+    if (!tile_coords((int)blockIdx.x, n_pass, tiles_n, pi, tn)) return;
+  } else {
+    if (!grouped_tile_coords(blockIdx.x, n_pass, tiles_n, run_log2, pi, tn)) return;
+  }
   const int4 d = reinterpret_cast<const int4*>(plan + 4)[pi];
   const int row0 = __builtin_amdgcn_readfirstlane(d.x), m_lo = __builtin_amdgcn_readfirstlane(d.y), m_hi = __builtin_amdgcn_readfirstlane(d.z);
   const int e = __builtin_amdgcn_readfirstlane(d.w);
-  const int n0 = tn * GT_TN;
+  const int n0 = tn * TileOf<WN>::TN;
   if (e < 0) {
-    const int n1 = n0 + GT_TN < (int)N ? n0 + GT_TN : (int)N;
-    zero_rows<OutT>(out, ldo, m_lo, m_hi, n0, n1);
+    const int n1 = n0 + TileOf<WN>::TN < (int)N ? n0 + TileOf<WN>::TN : (int)N;
+    zero_rows<OutT, TileOf<WN>::THREADS>(out, ldo, m_lo, m_hi, n0, n1);
     return;
   }
   // (packed scales: A.scales / w_scales + e * ws_stride_e are the packed bases, ss_k the bytes from block to block)
@@ -326,7 +330,7 @@ __global__ __launch_bounds__(GT_THREADS) void grouped_tiled_kernel(OperandView A
   TileArgs ta{A, B, row0, n0, m_lo, m_hi, N, G, 1.0f,
               (M_total - 1) * A.ld + G * 16, (N - 1) * ldw + G * 16,
               PS ? KB * A.ss_k : ((A.is_2d ? M_total / 32 : M_total) - 1) * A.ss_r + G, PS ? KB * N * 16 : ((w_is_2d ? N / 32 : N) - 1) * ws_r + G, 0, G};
-  gemm_tile_256x256<OutT, KTAIL, LMS, NST, PS>(ta, out, ldo, smem);
+  gemm_tile_256x256<OutT, KTAIL, LMS, NST, PS, WN>(ta, out, ldo, smem);
 }
 
 // dW[e] tile: rows [256 tm, +256) of the first operand (P) x rows [256 tn, +256) of the second (Q), reduced over the
@@ -470,18 +474,33 @@ __global__ __launch_bounds__(GT_THREADS) void grouped_dw_tiled_kernel(OperandVie
 inline int64_t grouped_max_passes(int64_t M_total, int64_t num_groups) { return (M_total + GT_TM - 1) / GT_TM + num_groups + 2; }
 inline int64_t grouped_workspace_bytes(int64_t M_total, int64_t num_groups) { return 16 + 16 * grouped_max_passes(M_total, num_groups); }
 
-template <typename OutT, bool KTAIL, int LMS = -1, int NST = 4, bool PS = false>
+// Packed scales, bf16 result: the 256x128 tile where one round of the 256 compute units takes all tiles, as in the dense product
+// (gemm_tiled_launch_ps).  Only the device knows how many passes there are; expected are the whole bands of 256 rows and half a
+// pass more per group (a partial tile each, half of them filling up a band), at least one per group.  A wrong guess costs either way
+// what the wrong side of the line below does.  us at 256x256 / 256x128, even routing:
+//   rows  groups    N     K   tiles of 256x128              rows  groups    N     K   tiles of 256x128
+//   2560    8    1440  1024      168  10.6 /  9.1           2048    4    2880  1440      230  13.3 / 11.4
+//   4096    8    1440  2880      240  19.8 / 17.1           8192   64     512  2048      288  16.1 / 21.7
+//   2048   16    1024  4096      136  22.1 / 18.2           8192    8    1024  2880      304  21.1 / 28.3
+//   4096   32     768  2048      210  15.0 / 12.9           8192    8    2048  2880      608  43.0 / 43.4
+inline bool grouped_narrow_pays(int64_t M_total, int64_t num_groups, int64_t N) {
+  const int64_t bands = M_total / GT_TM + 1, half = (num_groups + 1) / 2;
+  return ((bands > half ? bands : half) + half) * ((N + TileOf<2>::TN - 1) / TileOf<2>::TN) <= 256;
+}
+
+template <typename OutT, bool KTAIL, int LMS = -1, int NST = 4, bool PS = false, int WN = 4>
 int launch_grouped_tiled(const OperandView& A, const uint8_t* w, int64_t w_stride_e, int64_t ldw, const uint8_t* w_scales, int64_t ws_stride_e,
                          int64_t ws_r, int w_is_2d, const int32_t* offs, const int32_t* group_expert, int num_groups, int num_experts,
                          int64_t M_total, int64_t N, int64_t K, void* out, int64_t ldo, int32_t* plan, bool build_plan, hipStream_t st) {
-  auto kern = grouped_tiled_kernel<OutT, KTAIL, LMS, NST, PS>;
+  using W = TileOf<WN>;
+  auto kern = grouped_tiled_kernel<OutT, KTAIL, LMS, NST, PS, WN>;
   static LdsLimit lds;
-  if (const int rc = lds.raise(reinterpret_cast<const void*>(kern), GT_LDS_BYTES, "grouped_gemm")) return rc;
-  const int tiles_m = (int)((M_total + GT_TM - 1) / GT_TM), tiles_n = (int)((N + GT_TN - 1) / GT_TN);
+  if (const int rc = lds.raise(reinterpret_cast<const void*>(kern), W::LDS, "grouped_gemm")) return rc;
+  const int tiles_m = (int)((M_total + GT_TM - 1) / GT_TM), tiles_n = (int)((N + W::TN - 1) / W::TN);
   const int max_pass = (int)grouped_max_passes(M_total, num_groups);
   PassWalk wk{offs, group_expert, num_groups, num_experts, M_total};
   if (build_plan) hipLaunchKernelGGL(grouped_plan_kernel, dim3(1), dim3(PLAN_THREADS), 0, st, wk, tiles_m, plan, max_pass);
-  hipLaunchKernelGGL(kern, dim3((unsigned)grouped_grid_size(max_pass, tiles_n)), dim3(GT_THREADS), GT_LDS_BYTES, st, A, w, w_stride_e, ldw, w_scales, ws_stride_e, ws_r,
+  hipLaunchKernelGGL(kern, dim3((unsigned)grouped_grid_size(max_pass, tiles_n)), dim3(W::THREADS), W::LDS, st, A, w, w_stride_e, ldw, w_scales, ws_stride_e, ws_r,
                      w_is_2d, plan, M_total, N, (int)(K / 32), (OutT*)out, ldo, tiles_n, M_total >= 4ll * GT_TM * num_experts ? 2 : 0);
   return check_launch("grouped_gemm");
 }
@@ -564,17 +583,20 @@ int grouped_gemm_impl(const uint8_t* a, int64_t lda, const uint8_t* a_scales, in
     if (ps) {
       int lms = -1, nst = 4;
       if (tail) gemm_tile_last_stage(K / 32, lms, nst);
+      const bool narrow = grouped_narrow_pays(M_total, num_groups, N);
+#define ALTO_GROUPED_LAUNCH_PS(...) (narrow ? ALTO_GROUPED_LAUNCH(__bf16, __VA_ARGS__, true, 2) : ALTO_GROUPED_LAUNCH(__bf16, __VA_ARGS__, true, 4))
       switch (tail ? lms * 4 + nst - 1 : -1) {
-        case -1: rc = ALTO_GROUPED_LAUNCH(__bf16, false, -1, 4, true); break;
-        case 0: rc = ALTO_GROUPED_LAUNCH(__bf16, true, 0, 1, true); break;
-        case 1: rc = ALTO_GROUPED_LAUNCH(__bf16, true, 0, 2, true); break;
-        case 2: rc = ALTO_GROUPED_LAUNCH(__bf16, true, 0, 3, true); break;
-        case 3: rc = ALTO_GROUPED_LAUNCH(__bf16, true, 0, 4, true); break;
-        case 4: rc = ALTO_GROUPED_LAUNCH(__bf16, true, 1, 1, true); break;
-        case 5: rc = ALTO_GROUPED_LAUNCH(__bf16, true, 1, 2, true); break;
-        case 6: rc = ALTO_GROUPED_LAUNCH(__bf16, true, 1, 3, true); break;
-        default: rc = ALTO_GROUPED_LAUNCH(__bf16, true, 1, 4, true); break;
+        case -1: rc = ALTO_GROUPED_LAUNCH_PS(false, -1, 4); break;
+        case 0: rc = ALTO_GROUPED_LAUNCH_PS(true, 0, 1); break;
+        case 1: rc = ALTO_GROUPED_LAUNCH_PS(true, 0, 2); break;
+        case 2: rc = ALTO_GROUPED_LAUNCH_PS(true, 0, 3); break;
+        case 3: rc = ALTO_GROUPED_LAUNCH_PS(true, 0, 4); break;
+        case 4: rc = ALTO_GROUPED_LAUNCH_PS(true, 1, 1); break;
+        case 5: rc = ALTO_GROUPED_LAUNCH_PS(true, 1, 2); break;
+        case 6: rc = ALTO_GROUPED_LAUNCH_PS(true, 1, 3); break;
+        default: rc = ALTO_GROUPED_LAUNCH_PS(true, 1, 4); break;
       }
+#undef ALTO_GROUPED_LAUNCH_PS
     } else if (!tail) {
       rc = out_dtype == ALTO_DT_BF16 ? ALTO_GROUPED_LAUNCH(__bf16, false) : ALTO_GROUPED_LAUNCH(float, false);
     } else if (out_dtype != ALTO_DT_BF16) {

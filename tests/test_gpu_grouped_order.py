@@ -39,3 +39,24 @@ def test_every_pass_and_column_tile(m, sizes, tail, N, packed):
             assert torch.equal(out[lo:lo + n], ref), f"expert {e} of {sizes}"
         lo += n
     assert not out[lo:].any()
+
+
+# Packed scales and few tiles: 256x128 ones.  Every ending of the reduction, ragged rows and columns, an empty expert, rows of nobody
+# at the end; 8 experts of 257 rows have more tiles (304) than the 256 that the host expects to fit one round.
+@pytest.mark.parametrize("sizes,tail,N,K", [([300, 0, 32, 517], 64, 1160, K) for K in (512, 544, 640, 704, 768, 832, 896, 960, 1024)] + [([257] * 8, 0, 2432, 512), ([128], 0, 128, 512)])
+def test_narrow_tiles(m, sizes, tail, N, K):
+    from alto_amd.mxfp4 import grouped_gemm as G
+    from alto_amd.mxfp4.linear import pack_scales
+    E, M = len(sizes), sum(sizes) + tail
+    aq, as_ = m.convert_to_mxfp4(randn_outliers((M, K), torch.bfloat16, seed=M + K).to(DEV))
+    wq, ws = m.convert_to_mxfp4((randn_outliers((E, N, K), torch.bfloat16, seed=N) * 0.02).to(DEV))
+    groups = G.groups_from_offsets(torch.tensor([0] + sizes).cumsum(0).to(torch.int32).to(DEV))
+    print(f"narrow {sizes} {N}x{K}", flush=True)
+    out = G.grouped_forward_packed(aq, pack_scales(as_, M, K), wq, G.pack_expert_scales(ws, N, K, False), groups)
+    lo = 0
+    for e, n in enumerate(sizes):   # (the dense product of plain scales: 64x64 tiles or the direct kernel)
+        if n:
+            ref = m.blockwise_mxfp4_gemm(aq[lo:lo + n], as_[lo:lo + n], wq[e], ws[e], trans_b=True, output_dtype=torch.bfloat16)
+            assert torch.equal(out[lo:lo + n], ref), f"expert {e}"
+        lo += n
+    assert not out[lo:].any()
