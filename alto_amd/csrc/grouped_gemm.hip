@@ -303,34 +303,56 @@ __global__ __launch_bounds__(PLAN_THREADS) void grouped_plan_kernel(PassWalk wk,
   if (t == PLAN_THREADS - 1) ws[0] = upto < max_pass ? upto : max_pass;
 }
 
+// Arguments of the product of the rows with their expert's weights (forward / dX) on large tiles.
+struct GroupedRows {
+  OperandView A;
+  const uint8_t* w;
+  int64_t w_stride_e, ldw;
+  const uint8_t* w_scales;
+  int64_t ws_stride_e, ws_r;
+  int w_is_2d;
+  const int32_t* plan;
+  int64_t M_total, N;
+  int G;
+  void* out;
+  int64_t ldo;
+  int tiles_n, run_log2;
+};
+
 template <typename OutT, bool KTAIL, int LMS, int NST, bool PS, int WN>
-__global__ __launch_bounds__(TileOf<WN>::THREADS) void grouped_tiled_kernel(OperandView A, const uint8_t* w, int64_t w_stride_e, int64_t ldw,
-                                                                   const uint8_t* w_scales, int64_t ws_stride_e, int64_t ws_r, int w_is_2d,
-                                                                   const int32_t* plan, int64_t M_total, int64_t N, int G, OutT* out, int64_t ldo, int tiles_n, int run_log2) {
-  extern __shared__ __align__(16) uint8_t smem[];
-  const int n_pass = __builtin_amdgcn_readfirstlane(plan[0]);
+__device__ __forceinline__ void grouped_rows_tile(const GroupedRows& q, int wg, uint8_t* smem) {
+  const int n_pass = __builtin_amdgcn_readfirstlane(q.plan[0]);
   int pi, tn;
   if constexpr (WN == 2) {   // one round: what counts is that no XCD gets more tiles than the others
-    if (!tile_coords((int)blockIdx.x, n_pass, tiles_n, pi, tn)) return;
+    if (!tile_coords(wg, n_pass, q.tiles_n, pi, tn)) return;
   } else {
-    if (!grouped_tile_coords(blockIdx.x, n_pass, tiles_n, run_log2, pi, tn)) return;
+    if (!grouped_tile_coords(wg, n_pass, q.tiles_n, q.run_log2, pi, tn)) return;
   }
-  const int4 d = reinterpret_cast<const int4*>(plan + 4)[pi];
+  const int4 d = reinterpret_cast<const int4*>(q.plan + 4)[pi];
   const int row0 = __builtin_amdgcn_readfirstlane(d.x), m_lo = __builtin_amdgcn_readfirstlane(d.y), m_hi = __builtin_amdgcn_readfirstlane(d.z);
   const int e = __builtin_amdgcn_readfirstlane(d.w);
   const int n0 = tn * TileOf<WN>::TN;
+  OutT* out = static_cast<OutT*>(q.out);
   if (e < 0) {
-    const int n1 = n0 + TileOf<WN>::TN < (int)N ? n0 + TileOf<WN>::TN : (int)N;
-    zero_rows<OutT, TileOf<WN>::THREADS>(out, ldo, m_lo, m_hi, n0, n1);
+    const int n1 = n0 + TileOf<WN>::TN < (int)q.N ? n0 + TileOf<WN>::TN : (int)q.N;
+    zero_rows<OutT, TileOf<WN>::THREADS>(out, q.ldo, m_lo, m_hi, n0, n1);
     return;
   }
   // (packed scales: A.scales / w_scales + e * ws_stride_e are the packed bases, ss_k the bytes from block to block)
-  OperandView B{w + e * w_stride_e, ldw, w_scales + e * ws_stride_e, ws_r, PS ? N * 16 : 1, w_is_2d};
-  const int KB = (G + 15) / 16;
-  TileArgs ta{A, B, row0, n0, m_lo, m_hi, N, G, 1.0f,
-              (M_total - 1) * A.ld + G * 16, (N - 1) * ldw + G * 16,
-              PS ? KB * A.ss_k : ((A.is_2d ? M_total / 32 : M_total) - 1) * A.ss_r + G, PS ? KB * N * 16 : ((w_is_2d ? N / 32 : N) - 1) * ws_r + G, 0, G};
-  gemm_tile_256x256<OutT, KTAIL, LMS, NST, PS, WN>(ta, out, ldo, smem);
+  const int64_t N = q.N;
+  OperandView B{q.w + e * q.w_stride_e, q.ldw, q.w_scales + e * q.ws_stride_e, q.ws_r, PS ? N * 16 : 1, q.w_is_2d};
+  const int KB = (q.G + 15) / 16;
+  TileArgs ta{q.A, B, row0, n0, m_lo, m_hi, N, q.G, 1.0f,
+              (q.M_total - 1) * q.A.ld + q.G * 16, (N - 1) * q.ldw + q.G * 16,
+              PS ? KB * q.A.ss_k : ((q.A.is_2d ? q.M_total / 32 : q.M_total) - 1) * q.A.ss_r + q.G,
+              PS ? KB * N * 16 : ((q.w_is_2d ? N / 32 : N) - 1) * q.ws_r + q.G, 0, q.G};
+  gemm_tile_256x256<OutT, KTAIL, LMS, NST, PS, WN>(ta, out, q.ldo, smem);
+}
+
+template <typename OutT, bool KTAIL, int LMS, int NST, bool PS, int WN>
+__global__ __launch_bounds__(TileOf<WN>::THREADS) void grouped_tiled_kernel(GroupedRows q) {
+  extern __shared__ __align__(16) uint8_t smem[];
+  grouped_rows_tile<OutT, KTAIL, LMS, NST, PS, WN>(q, (int)blockIdx.x, smem);
 }
 
 // dW[e] tile: rows [256 tm, +256) of the first operand (P) x rows [256 tn, +256) of the second (Q), reduced over the
@@ -350,14 +372,13 @@ template <typename OutT, bool PS>
 __device__ __forceinline__ void grouped_dw_tile(const OperandView& P, const OperandView& Q, int64_t NP, int64_t NQ,
                                                 const int32_t* offs, const int32_t* group_expert, int num_groups,
                                                 int64_t M_total, OutT* __restrict__ dw, int64_t s_e, int64_t ld, float out_scale,
-                                                int tiles_p, int tiles_q, int xq_log2, uint8_t* smem) {
-  const int e = blockIdx.y;
+                                                int tiles_p, int tiles_q, int xq_log2, int wg, int e, uint8_t* smem) {
   int tm, tn;
   {
-    // Each XCD (blockIdx.x % 8) owns one rectangular block of every expert's tile grid, the XCDs forming a
+    // Each XCD (wg % 8) owns one rectangular block of every expert's tile grid, the XCDs forming a
     // (8 >> xq_log2) x (1 << xq_log2) arrangement: its ~32 resident workgroups then share the P and Q bands of one
     // expert's token range through its L2, and each band is fetched by few XCDs.
-    const int k = blockIdx.x & 7, j = blockIdx.x >> 3;
+    const int k = wg & 7, j = wg >> 3;
     const int xq = 1 << xq_log2, xp = 8 >> xq_log2;
     const int bp = (tiles_p + xp - 1) / xp, bq = (tiles_q + xq - 1) / xq;
     const int p0 = (k >> xq_log2) * bp, q0 = (k & (xq - 1)) * bq;
@@ -461,13 +482,60 @@ __device__ __forceinline__ void grouped_dw_tile(const OperandView& P, const Oper
   gemm_tile_store<OutT>(ta, acc, dw + e * s_e, ld, smem);
 }
 
+// Arguments of the weight gradient on large tiles.
+struct GroupedDw {
+  OperandView P, Q;
+  int64_t NP, NQ;
+  const int32_t* offs;
+  const int32_t* group_expert;
+  int num_groups;
+  int64_t M_total;
+  void* dw;
+  int64_t s_e, ld;
+  float out_scale;
+  int tiles_p, tiles_q, xq_log2, per_expert;   // workgroups per expert: 8 times the largest block that an XCD owns
+};
+
 template <typename OutT, bool PS = false>
-__global__ __launch_bounds__(GT_THREADS) void grouped_dw_tiled_kernel(OperandView P, OperandView Q, int64_t NP, int64_t NQ,
-                                                                      const int32_t* offs, const int32_t* group_expert, int num_groups,
-                                                                      int64_t M_total, OutT* dw, int64_t s_e, int64_t ld, float out_scale,
-                                                                      int tiles_p, int tiles_q, int xq_log2) {
+__global__ __launch_bounds__(GT_THREADS) void grouped_dw_tiled_kernel(GroupedDw q) {
   extern __shared__ __align__(16) uint8_t smem[];
-  grouped_dw_tile<OutT, PS>(P, Q, NP, NQ, offs, group_expert, num_groups, M_total, dw, s_e, ld, out_scale, tiles_p, tiles_q, xq_log2, smem);
+  grouped_dw_tile<OutT, PS>(q.P, q.Q, q.NP, q.NQ, q.offs, q.group_expert, q.num_groups, q.M_total, static_cast<OutT*>(q.dw), q.s_e, q.ld, q.out_scale, q.tiles_p,
+                            q.tiles_q, q.xq_log2, (int)blockIdx.x, (int)blockIdx.y, smem);
+}
+
+// Input and weight gradient of the same groups (in expert order, packed scales) in one launch.  They are independent, and in a
+// launch each both end with units idle while their last tiles run; a weight gradient of short experts is bound by the write of
+// its result and an input gradient by its products, which side by side cost less than in turn.  The tiles with the longer
+// reduction go first (the input gradient's is N, the weight gradient's on average M_total / num_experts), so that short ones fill
+// the end.  Backward pass with the gradient's quantizer, us: a launch each / dX first / dW first
+//   rows  experts  K     N    skew    each    dX     dW            rows  experts  K     N    skew    each    dX     dW
+//   2560     8   1024  1440   0.5     47.0   43.0   46.0          65536     4   2880   512   0.2     274    268    218
+//   1024    16   2048  4096   0.2      121     92    103          32768     4   4096   512   1.0     194    192    150
+//   4096     8   5760  5760   0.3      328    304    319          16384     4    512  4096   1.0     123    106    101
+//  16384     8   2048  5760   0.3      337    317    328          65536     4   1440  2880   1.0     513    497    448
+//  16384    32   5760  5760   0.8     1195   1184   1148          32768     8   2880  1440   1.2     238    232    227
+//  65536    32   2880  5760   1.1     1636   1624   1612          65536    32   5760  2880   1.1    1556   1555   1573
+// Fifty layers of 1024 to 65536 rows and 4 to 32 experts: 1 to 27 % less, none more than 2 % more.  Dealt out alternately the two
+// share no L2 lines: 65536 x 2880 x 2880 with 8 equal experts 768 -> 877, so they stay one after the other.
+struct GroupedPair {
+  GroupedRows dx;
+  GroupedDw dw;
+  int before, dw_first;   // workgroups of the part that goes first
+};
+
+template <bool KTAIL>
+__global__ __launch_bounds__(GT_THREADS) void grouped_gradients_kernel(GroupedPair p) {
+  extern __shared__ __align__(16) uint8_t smem[];
+  const bool second = (int)blockIdx.x >= p.before;
+  const int wg = (int)blockIdx.x - (second ? p.before : 0);   // (both parts are multiples of 8 workgroups: wg % 8 is the XCD)
+  if (second == (p.dw_first != 0)) {
+    grouped_rows_tile<__bf16, KTAIL, -2, 4, true, 4>(p.dx, wg, smem);
+  } else {
+    const GroupedDw& q = p.dw;
+    const int e = wg / q.per_expert;
+    grouped_dw_tile<__bf16, true>(q.P, q.Q, q.NP, q.NQ, q.offs, nullptr, q.num_groups, q.M_total, static_cast<__bf16*>(q.dw), q.s_e, q.ld, q.out_scale, q.tiles_p,
+                                  q.tiles_q, q.xq_log2, wg - e * q.per_expert, e, smem);
+  }
 }
 
 // upper bound on the number of passes: every band is one, every group start inside a band adds one, plus the unrouted head and tail
@@ -488,6 +556,8 @@ inline bool grouped_narrow_pays(int64_t M_total, int64_t num_groups, int64_t N) 
   return ((bands > half ? bands : half) + half) * ((N + TileOf<2>::TN - 1) / TileOf<2>::TN) <= 256;
 }
 
+inline int grouped_run_log2(int64_t M_total, int64_t num_experts) { return M_total >= 4ll * GT_TM * num_experts ? 2 : 0; }   // see grouped_tile_coords
+
 template <typename OutT, bool KTAIL, int LMS = -1, int NST = 4, bool PS = false, int WN = 4>
 int launch_grouped_tiled(const OperandView& A, const uint8_t* w, int64_t w_stride_e, int64_t ldw, const uint8_t* w_scales, int64_t ws_stride_e,
                          int64_t ws_r, int w_is_2d, const int32_t* offs, const int32_t* group_expert, int num_groups, int num_experts,
@@ -500,17 +570,13 @@ int launch_grouped_tiled(const OperandView& A, const uint8_t* w, int64_t w_strid
   const int max_pass = (int)grouped_max_passes(M_total, num_groups);
   PassWalk wk{offs, group_expert, num_groups, num_experts, M_total};
   if (build_plan) hipLaunchKernelGGL(grouped_plan_kernel, dim3(1), dim3(PLAN_THREADS), 0, st, wk, tiles_m, plan, max_pass);
-  hipLaunchKernelGGL(kern, dim3((unsigned)grouped_grid_size(max_pass, tiles_n)), dim3(W::THREADS), W::LDS, st, A, w, w_stride_e, ldw, w_scales, ws_stride_e, ws_r,
-                     w_is_2d, plan, M_total, N, (int)(K / 32), (OutT*)out, ldo, tiles_n, M_total >= 4ll * GT_TM * num_experts ? 2 : 0);
+  const GroupedRows q{A, w, w_stride_e, ldw, w_scales, ws_stride_e, ws_r, w_is_2d, plan, M_total, N, (int)(K / 32), out, ldo, tiles_n, grouped_run_log2(M_total, num_experts)};
+  hipLaunchKernelGGL(kern, dim3((unsigned)grouped_grid_size(max_pass, tiles_n)), dim3(W::THREADS), W::LDS, st, q);
   return check_launch("grouped_gemm");
 }
 
-template <typename OutT, bool PS = false>
-int launch_dw_tiled(const OperandView& P, const OperandView& Q, int64_t NP, int64_t NQ, const int32_t* offs, const int32_t* group_expert,
-                    int num_groups, int num_experts, int64_t M_total, void* dw, int64_t s_e, int64_t ld, float out_scale, hipStream_t st) {
-  auto kern = grouped_dw_tiled_kernel<OutT, PS>;
-  static LdsLimit lds;
-  if (const int rc = lds.raise(reinterpret_cast<const void*>(kern), GT_DW_LDS_BYTES, "grouped_gemm_dw")) return rc;
+GroupedDw dw_args(const OperandView& P, const OperandView& Q, int64_t NP, int64_t NQ, const int32_t* offs, const int32_t* group_expert, int num_groups,
+                  int64_t M_total, void* dw, int64_t s_e, int64_t ld, float out_scale) {
   const int tiles_p = (int)((NP + GT_TM - 1) / GT_TM), tiles_q = (int)((NQ + GT_TN - 1) / GT_TN);
   // split of the 8 XCDs over the tile grid: the smallest blocks (least idle workgroups), then the smallest perimeter
   int xq_log2 = 0;
@@ -524,9 +590,25 @@ int launch_dw_tiled(const OperandView& P, const OperandView& Q, int64_t NP, int6
       xq_log2 = l;
     }
   }
-  hipLaunchKernelGGL(kern, dim3((unsigned)(8 * best_area), (unsigned)num_experts), dim3(GT_THREADS), GT_DW_LDS_BYTES, st, P, Q, NP, NQ, offs,
-                     group_expert, num_groups, M_total, (OutT*)dw, s_e, ld, out_scale, tiles_p, tiles_q, xq_log2);
+  return {P, Q, NP, NQ, offs, group_expert, num_groups, M_total, dw, s_e, ld, out_scale, tiles_p, tiles_q, xq_log2, (int)(8 * best_area)};
+}
+
+template <typename OutT, bool PS = false>
+int launch_dw_tiled(const GroupedDw& q, int num_experts, hipStream_t st) {
+  auto kern = grouped_dw_tiled_kernel<OutT, PS>;
+  static LdsLimit lds;
+  if (const int rc = lds.raise(reinterpret_cast<const void*>(kern), GT_DW_LDS_BYTES, "grouped_gemm_dw")) return rc;
+  hipLaunchKernelGGL(kern, dim3((unsigned)q.per_expert, (unsigned)num_experts), dim3(GT_THREADS), GT_DW_LDS_BYTES, st, q);
   return check_launch("grouped_gemm_dw");
+}
+
+template <bool KTAIL>
+int launch_gradients(const GroupedPair& p, int64_t workgroups, hipStream_t st) {
+  auto kern = grouped_gradients_kernel<KTAIL>;
+  static LdsLimit lds;
+  if (const int rc = lds.raise(reinterpret_cast<const void*>(kern), GT_LDS_BYTES, "grouped_gradients_ps")) return rc;   // (no group ids: no masks behind the tile)
+  hipLaunchKernelGGL(kern, dim3((unsigned)workgroups), dim3(GT_THREADS), GT_LDS_BYTES, st, p);
+  return check_launch("grouped_gradients_ps");
 }
 
 }  // namespace
@@ -535,13 +617,14 @@ int launch_dw_tiled(const OperandView& P, const OperandView& Q, int64_t NP, int6
 namespace alto {
 namespace {
 
-// `plan` = device memory for the pass list (plan_bytes of it), needed by the tiled path only
+// `plan` = device memory for the pass list (plan_bytes of it), needed by the tiled path only; with `hand_out` (packed scales, pass
+// list built) the arguments of a launch on 256x256 tiles go there instead
 int grouped_gemm_impl(const uint8_t* a, int64_t lda, const uint8_t* a_scales, int64_t a_ss_r, int64_t a_ss_k, int a_is_2d,
                       const uint8_t* w, int64_t w_stride_e, int64_t ldw,
                       const uint8_t* w_scales, int64_t ws_stride_e, int64_t ws_r, int64_t ws_k, int w_is_2d,
                       const int32_t* offs, const int32_t* group_expert, int num_groups, int num_experts,
                       int64_t M_total, int64_t N, int64_t K, void* out, int out_dtype, int64_t ldo,
-                      void* plan, int64_t plan_bytes, const char* plan_name, bool build_plan, void* stream, bool ps = false) {
+                      void* plan, int64_t plan_bytes, const char* plan_name, bool build_plan, void* stream, bool ps = false, GroupedRows* hand_out = nullptr) {
   ALTO_REQUIRE(a && a_scales && w && w_scales && offs && out, "grouped_gemm: NULL pointer");
   ALTO_REQUIRE(((reinterpret_cast<uintptr_t>(offs) | reinterpret_cast<uintptr_t>(group_expert)) & 3) == 0, "grouped_gemm: offs and group_expert must be 4-byte aligned");
   ALTO_REQUIRE(num_groups > 0 && num_groups <= 65536, "grouped_gemm: num_groups (%d) out of range", num_groups);
@@ -580,7 +663,11 @@ int grouped_gemm_impl(const uint8_t* a, int64_t lda, const uint8_t* a_scales, in
     int32_t* pl = reinterpret_cast<int32_t*>(plan);
     int rc = ALTO_MXFP4_EINVAL;
 #define ALTO_GROUPED_LAUNCH(T, ...) launch_grouped_tiled<T, __VA_ARGS__>(A, w, w_stride_e, ldw, w_scales, ws_stride_e, ws_r, w_is_2d, offs, group_expert, num_groups, num_experts, M_total, N, K, out, ldo, pl, build_plan, st)
-    if (ps) {
+    if (hand_out) {
+      *hand_out = {A, w, w_stride_e, ldw, w_scales, ws_stride_e, ws_r, 0, pl, M_total, N, (int)(K / 32), out, ldo, (int)((N + GT_TN - 1) / GT_TN),
+                   grouped_run_log2(M_total, num_experts)};
+      rc = ALTO_MXFP4_OK;
+    } else if (ps) {
       int lms = -1, nst = 4;
       if (tail) gemm_tile_last_stage(K / 32, lms, nst);
       const bool narrow = grouped_narrow_pays(M_total, num_groups, N);
@@ -768,12 +855,13 @@ extern "C" int alto_mxfp4_grouped_gemm_noalloc(const uint8_t* a, int64_t lda, co
 
 namespace alto {
 namespace {
+// hand_out: the launch's arguments go there instead, once every check has passed (as in grouped_gemm_impl)
 // ps: go_scales / x_scales are packed along the tokens ([ceil(M_total / 512)][N or K][16]); tile kernel and bf16 only
 int grouped_dw_impl(const uint8_t* go, int64_t ld_go, const uint8_t* go_scales, int64_t gs_r, int64_t gs_k, int go_is_2d,
                     const uint8_t* x, int64_t ld_xq, const uint8_t* x_scales, int64_t xs_r, int64_t xs_k, int x_is_2d,
                     const int32_t* offs, const int32_t* group_expert, int num_groups, int num_experts,
                     int64_t M_total, int64_t N, int64_t K, void* dw, int dw_dtype, int64_t dw_stride_e, int64_t dw_stride_n, int64_t dw_stride_k,
-                    float out_scale, void* stream, bool ps) {
+                    float out_scale, void* stream, bool ps, GroupedDw* hand_out = nullptr) {
   ALTO_REQUIRE(go && go_scales && x && x_scales && offs && dw, "grouped_gemm_dw: NULL pointer");
   ALTO_REQUIRE(((reinterpret_cast<uintptr_t>(offs) | reinterpret_cast<uintptr_t>(group_expert)) & 3) == 0, "grouped_gemm_dw: offs and group_expert must be 4-byte aligned");
   ALTO_REQUIRE((reinterpret_cast<uintptr_t>(dw) & (dw_dtype == ALTO_DT_F32 ? 3 : 1)) == 0, "grouped_gemm_dw: dw must be aligned to its element size");
@@ -809,11 +897,13 @@ int grouped_dw_impl(const uint8_t* go, int64_t ld_go, const uint8_t* go_scales, 
       return ALTO_MXFP4_ENOTIMPL;
     }
     if (tiled) {
-      const int rc = ps ? launch_dw_tiled<__bf16, true>(P, Q, NP, NQ, offs, group_expert, num_groups, num_experts, M_total, dw, dw_stride_e, ld, out_scale, st)
-                     : dw_dtype == ALTO_DT_BF16
-                         ? launch_dw_tiled<__bf16>(P, Q, NP, NQ, offs, group_expert, num_groups, num_experts, M_total, dw, dw_stride_e, ld, out_scale, st)
-                         : launch_dw_tiled<float>(P, Q, NP, NQ, offs, group_expert, num_groups, num_experts, M_total, dw, dw_stride_e, ld, out_scale, st);
-      return rc;
+      const GroupedDw q = dw_args(P, Q, NP, NQ, offs, group_expert, num_groups, M_total, dw, dw_stride_e, ld, out_scale);
+      if (hand_out) {
+        *hand_out = q;
+        return ALTO_MXFP4_OK;
+      }
+      return ps ? launch_dw_tiled<__bf16, true>(q, num_experts, st)
+                : dw_dtype == ALTO_DT_BF16 ? launch_dw_tiled<__bf16>(q, num_experts, st) : launch_dw_tiled<float>(q, num_experts, st);
     }
   }
   dim3 grid((unsigned)((K + 63) / 64), (unsigned)((N + 63) / 64), (unsigned)num_experts);
@@ -847,4 +937,39 @@ extern "C" int alto_mxfp4_grouped_gemm_dw_ps(const uint8_t* go, int64_t ld_go, c
   // go: [blocks][N][16], x: [blocks][K][16]; ss_k carries the bytes from block to block
   return grouped_dw_impl(go, ld_go, go_packed, 16, N * 16, 0, x, ld_xq, x_packed, 16, K * 16, 0, offs, group_expert, num_groups, num_experts,
                          M_total, N, K, dw, ALTO_DT_BF16, dw_stride_e, dw_stride_n, dw_stride_k, out_scale, stream, true);
+}
+
+extern "C" int alto_mxfp4_grouped_gradients_ps(const uint8_t* go, int64_t ld_go, const uint8_t* go_packed, const uint8_t* w, int64_t w_stride_e, int64_t ldw,
+                                               const uint8_t* w_packed, int64_t wp_stride_e, const uint8_t* got, int64_t ld_got, const uint8_t* got_packed,
+                                               const uint8_t* xt, int64_t ld_xt, const uint8_t* xt_packed, const int32_t* offs, int num_experts,
+                                               int64_t M_total, int64_t N, int64_t K, void* dx, int64_t ld_dx, void* dw, int64_t dw_stride_e,
+                                               int64_t dw_stride_n, int64_t dw_stride_k, float out_scale, const void* workspace, int64_t workspace_bytes, void* stream) {
+  using namespace alto;
+  ALTO_REQUIRE(((reinterpret_cast<uintptr_t>(go_packed) | reinterpret_cast<uintptr_t>(w_packed) | (uintptr_t)wp_stride_e | reinterpret_cast<uintptr_t>(got_packed) |
+                 reinterpret_cast<uintptr_t>(xt_packed)) & 15) == 0, "grouped_gradients_ps: packed scales (and the stride between experts) must be 16-byte aligned");
+  ALTO_REQUIRE(M_total >= 0 && M_total < (1ll << 31) && N >= 0 && N < (1ll << 31) && K >= 0 && K < (1ll << 31) &&
+               product_below(1ll << 31, (N / 32 + 15) / 16, M_total > K ? M_total : K, 16) && product_below(1ll << 31, (M_total + 511) / 512, N > K ? N : K, 16),
+               "grouped_gradients_ps: size out of range, or packed scales beyond 2 GiB");
+  auto rows = [&](GroupedRows* hand_out) {
+    return grouped_gemm_impl(go, ld_go, go_packed, 16, 1, 0, w, w_stride_e, ldw, w_packed, wp_stride_e, 16, 1, 0, offs, nullptr, num_experts, num_experts,
+                             M_total, K, N, dx, ALTO_DT_BF16, ld_dx, const_cast<void*>(workspace), workspace_bytes, "the workspace", false, stream, true, hand_out);
+  };
+  auto weights = [&](GroupedDw* hand_out) {
+    return grouped_dw_impl(got, ld_got, got_packed, 16, N * 16, 0, xt, ld_xt, xt_packed, 16, K * 16, 0, offs, nullptr, num_experts, num_experts,
+                           M_total, N, K, dw, ALTO_DT_BF16, dw_stride_e, dw_stride_n, dw_stride_k, out_scale, stream, true, hand_out);
+  };
+  GroupedPair p{};
+  if (M_total > 0 && N > 0 && K > 0) {
+    if (const int rc = rows(&p.dx)) return rc;
+    if (const int rc = weights(&p.dw)) return rc;
+    const int64_t dx_wgs = grouped_grid_size(grouped_max_passes(M_total, num_experts), p.dx.tiles_n), dw_wgs = (int64_t)p.dw.per_expert * num_experts;
+    if (dx_wgs + dw_wgs < (1ll << 32) / GT_THREADS) {   // (threads of a launch)
+      p.dw_first = M_total >= N * num_experts;
+      p.before = (int)(p.dw_first ? dw_wgs : dx_wgs);
+      hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+      return (N / 32) % 16 ? launch_gradients<true>(p, dx_wgs + dw_wgs, st) : launch_gradients<false>(p, dx_wgs + dw_wgs, st);
+    }
+  }
+  if (const int rc = rows(nullptr)) return rc;
+  return weights(nullptr);
 }

@@ -43,6 +43,7 @@ struct Api {
   ALTO_FN(grouped_gemm_ps);
   ALTO_FN(grouped_gemm_workspace_bytes);
   ALTO_FN(grouped_gemm_dw_ps);
+  ALTO_FN(grouped_gradients_ps);
   ALTO_FN(attention_quantize);
   ALTO_FN(attention_fwd_strided);
   ALTO_FN(attention_quantize_kv);
@@ -66,6 +67,7 @@ void bind(const py::dict& address, py::object check) {
   ALTO_FN(grouped_gemm_ps);
   ALTO_FN(grouped_gemm_workspace_bytes);
   ALTO_FN(grouped_gemm_dw_ps);
+  ALTO_FN(grouped_gradients_ps);
   ALTO_FN(attention_quantize);
   ALTO_FN(attention_fwd_strided);
   ALTO_FN(attention_quantize_kv);
@@ -647,11 +649,13 @@ bool grouped_gradients(const Tensor& go, const Tensor& xs, const Tensor& ws, con
   const Tensor tmp = Alloc(go).dense({c.go_col.end()});
   dx = at::empty({M, K}, go.options());
   dw = o.trans_weights ? at::empty({E, N, K}, go.options()) : at::empty({E, K, N}, go.options());
-  quantize_gradient(f, go, c.go_row, tmp, c.go_col, tmp, o.sr ? 3 : 0, seed, h, o.clip, o.uos, s) && grouped_product(f, c.go_row, tmp, c.wd, ws, offs, plan, true, dx, s) &&
-      f.ok("alto_mxfp4_grouped_gemm_dw_ps",
-           api.grouped_gemm_dw_ps(c.go_col.codes(tmp), c.go_col.ld(), c.go_col.scales(tmp), c.x_col.codes(xs), c.x_col.ld(), c.x_col.scales(xs),
-                                  static_cast<const int32_t*>(offs.data_ptr()), nullptr, (int)E, (int)E, M, N, K, dw.data_ptr(), dw.stride(0),
-                                  o.trans_weights ? dw.stride(1) : dw.stride(2), o.trans_weights ? dw.stride(2) : dw.stride(1), (float)o.out_scale, s));
+  const Copy &g = c.go_row, &w = c.wd, &gt = c.go_col, &xt = c.x_col;
+  quantize_gradient(f, go, g, tmp, gt, tmp, o.sr ? 3 : 0, seed, h, o.clip, o.uos, s) &&
+      f.ok("alto_mxfp4_grouped_gradients_ps",
+           api.grouped_gradients_ps(g.codes(tmp), g.ld(), g.scales(tmp), w.codes(ws), w.rows * w.ld(), w.ld(), w.scales(ws), w.scale_bytes(), gt.codes(tmp), gt.ld(),
+                                    gt.scales(tmp), xt.codes(xs), xt.ld(), xt.scales(xs), static_cast<const int32_t*>(offs.data_ptr()), (int)E, M, N, K, dx.data_ptr(), K,
+                                    dw.data_ptr(), dw.stride(0), o.trans_weights ? dw.stride(1) : dw.stride(2), o.trans_weights ? dw.stride(2) : dw.stride(1),
+                                    (float)o.out_scale, plan.data_ptr(), plan.numel(), s));
   raise_in_engine(f);
   return true;
 }

@@ -421,6 +421,15 @@ int alto_mxfp4_grouped_gemm_dw_ps(const uint8_t* go, int64_t ld_go, const uint8_
                                   int64_t M_total, int64_t N, int64_t K, void* dw, int64_t dw_stride_e, int64_t dw_stride_n, int64_t dw_stride_k,
                                   float out_scale, void* stream);
 
+/* Input and weight gradient of the same groups, in expert order, in one launch: dX [M_total][K] = dY . W (go, w: as
+ * alto_mxfp4_grouped_gemm_ps with the pass list already in the workspace) and dW (got, xt: as alto_mxfp4_grouped_gemm_dw_ps).
+ * Same results bit for bit as the two calls. */
+int alto_mxfp4_grouped_gradients_ps(const uint8_t* go, int64_t ld_go, const uint8_t* go_packed, const uint8_t* w, int64_t w_stride_e, int64_t ldw,
+                                    const uint8_t* w_packed, int64_t wp_stride_e, const uint8_t* got, int64_t ld_got, const uint8_t* got_packed,
+                                    const uint8_t* xt, int64_t ld_xt, const uint8_t* xt_packed, const int32_t* offs, int num_experts,
+                                    int64_t M_total, int64_t N, int64_t K, void* dx, int64_t ld_dx, void* dw, int64_t dw_stride_e,
+                                    int64_t dw_stride_n, int64_t dw_stride_k, float out_scale, const void* workspace, int64_t workspace_bytes, void* stream);
+
 /*
  * Fused quantize -> dequantize: y = convert_from_mxfp4(convert_to_mxfp4(x, axis=-1, is_2d_block), output_dtype = dtype
  * of x), round to nearest even, no clipping, in one pass (no codes or scales are written).  Replaces the pair of

@@ -174,6 +174,22 @@ def test_grouped_step_equals_the_general_function(m, N, K, trans, kw):
         assert torch.equal(got[3], ref[3])
 
 
+# The two gradients share a launch, the input gradient's tiles first below as many rows as N x experts and the weight gradient's from there
+# on: every ending of the reduction over N, an empty expert, rows of nobody, experts that start anywhere in a 512-token block.
+@pytest.mark.parametrize("sizes,tail,trans", [([320, 0, 32, 544], 64, True), ([1280], 0, False), ([2400, 1696], 32, True)])
+@pytest.mark.parametrize("N,K", [(N, 544 if N % 128 else 1024) for N in (512, 544, 640, 704, 768, 832, 896, 960, 1024)] + [(512, 2336), (2304, 512)])
+def test_gradients_of_a_grouped_step_share_a_launch(m, sizes, tail, trans, N, K):
+    E, M = len(sizes), sum(sizes) + tail
+    print(f"gradients {sizes} {N}x{K}", flush=True)
+    offs = torch.tensor([0] + sizes).cumsum(0).to(torch.int32).to(DEV)
+    x = randn_outliers((M, K), torch.bfloat16, seed=M).to(DEV)
+    w = randn_outliers((E, N, K) if trans else (E, K, N), torch.bfloat16, seed=N).to(DEV)
+    go = (randn_outliers((M, N), torch.bfloat16, seed=K) / (M * N)).to(DEV)
+    got = _grouped(m, "step", x, w, go, offs, trans, native=(True, True))
+    _same(got[:3], _grouped(m, "general", x, w, go, offs, trans)[:3])   # (a launch each)
+    assert not got[1][M - tail:].any()
+
+
 def test_grouped_step_forms_and_hooks_of_native_calls(m):
     """Shapes that the native calls serve: what else makes them decline, in the forward or in the backward alone."""
     N, K = 544, 800
