@@ -69,6 +69,7 @@ SIGNATURES = {
                                                 c_vp, c_i64, c_i64, c_vp, c_i64, c_i64, c_i64, c_int,
                                                 c_vp, c_vp, c_int, c_int, c_i64, c_i64, c_i64, c_vp, c_int, c_i64, c_vp]),
     "alto_mxfp4_grouped_gemm_workspace_bytes": (c_i64, [c_i64, c_int]),
+    "alto_mxfp4_grouped_gemm_plan_ends": (c_int, [c_vp, c_int, c_vp, c_i64, c_vp, c_i64, c_vp]),
     "alto_mxfp4_grouped_gemm_offsets": (c_int, [c_vp, c_int, c_vp, c_vp]),
     "alto_mxfp4_grouped_gemm_dw": (c_int, [c_vp, c_i64, c_vp, c_i64, c_i64, c_int,
                                            c_vp, c_i64, c_vp, c_i64, c_i64, c_int,

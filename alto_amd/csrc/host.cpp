@@ -48,7 +48,7 @@ struct Api {
   ALTO_FN(attention_fwd_strided);
   ALTO_FN(attention_quantize_kv);
   ALTO_FN(attention_fwd_bf16q);
-  ALTO_FN(grouped_gemm_offsets);
+  ALTO_FN(grouped_gemm_plan_ends);
   ALTO_FN(quantize_operands);
   ALTO_FN(gemm_two);
 #undef ALTO_FN
@@ -72,7 +72,7 @@ void bind(const py::dict& address, py::object check) {
   ALTO_FN(attention_fwd_strided);
   ALTO_FN(attention_quantize_kv);
   ALTO_FN(attention_fwd_bf16q);
-  ALTO_FN(grouped_gemm_offsets);
+  ALTO_FN(grouped_gemm_plan_ends);
   ALTO_FN(quantize_operands);
   ALTO_FN(gemm_two);
 #undef ALTO_FN
@@ -675,11 +675,12 @@ struct GroupedNode : torch::autograd::Function<GroupedNode> {
     bool ok = true;
     if (op.ends) {
       offs = at::empty({E + 1}, op.offs.options());
-      ok = f.ok("alto_mxfp4_grouped_gemm_offsets", api.grouped_gemm_offsets(static_cast<const int32_t*>(op.offs.data_ptr()), (int)E, static_cast<int32_t*>(offs.data_ptr()), s));
+      ok = f.ok("alto_mxfp4_grouped_gemm_plan_ends", api.grouped_gemm_plan_ends(static_cast<const int32_t*>(op.offs.data_ptr()), (int)E, static_cast<int32_t*>(offs.data_ptr()), M,
+                                                                                plan.data_ptr(), plan.numel(), s));
     }
     ok = ok && (o.trans_weights ? quantize_operands(f, op.x, c.x_row, tmp, c.x_col, xs, h, o.clip, op.w, c.wf, tmp, c.wd, ws, o.uos, s)
                                 : quantize_operands(f, op.x, c.x_row, tmp, c.x_col, xs, h, o.clip, op.w, c.wd, ws, c.wf, tmp, o.uos, s));
-    ok = ok && grouped_product(f, c.x_row, tmp, c.wf, tmp, offs, plan, false, out, s);
+    ok = ok && grouped_product(f, c.x_row, tmp, c.wf, tmp, offs, plan, op.ends, out, s);
     if (!ok) throw Refused{f};
     ctx->save_for_backward({xs, ws, offs, plan});
     ctx->saved_data["options"] = to_text(o);

@@ -332,6 +332,9 @@ int alto_mxfp4_grouped_gemm(const uint8_t* a, int64_t lda, const uint8_t* a_scal
  */
 int alto_mxfp4_grouped_gemm_plan(const int32_t* offs, const int32_t* group_expert, int num_groups, int num_experts, int64_t M_total,
                                  void* workspace, int64_t workspace_bytes, void* stream);
+/* The same for groups in expert order that come as their ends [num_groups]; the offsets [num_groups + 1] go to offs. */
+int alto_mxfp4_grouped_gemm_plan_ends(const int32_t* ends, int num_groups, int32_t* offs, int64_t M_total, void* workspace, int64_t workspace_bytes,
+                                      void* stream);
 int alto_mxfp4_grouped_gemm_planned(const uint8_t* a, int64_t lda, const uint8_t* a_scales, int64_t a_ss_r, int64_t a_ss_k, int a_is_2d,
                                     const uint8_t* w, int64_t w_stride_e, int64_t ldw,
                                     const uint8_t* w_scales, int64_t ws_stride_e, int64_t ws_r, int64_t ws_k, int w_is_2d,

@@ -60,3 +60,48 @@ def test_narrow_tiles(m, sizes, tail, N, K):
             assert torch.equal(out[lo:lo + n], ref), f"expert {e}"
         lo += n
     assert not out[lo:].any()
+
+
+# The pass list itself, against the rule in Python: groups from their own first row in steps of 256, each starting where the furthest
+# earlier one ended, rows of nobody as passes of expert -1.  254 groups are the most whose passes the threads share out; then they walk.
+@pytest.mark.parametrize("groups", [1, 2, 31, 253, 254, 255, 600])
+@pytest.mark.parametrize("form", ["even", "one", "wild", "none"])
+def test_pass_list(m, groups, form):
+    from alto_amd import _lib
+    lib = _lib.load()
+    g = torch.Generator().manual_seed(groups)
+    M = 32 * groups + 5000
+    if form == "even":
+        offs = torch.arange(groups + 1) * 32 + 96
+    elif form == "one":   # all rows but the first and last few are one group's
+        offs = torch.where(torch.arange(groups + 1) <= groups // 2, 7, M - 3)
+    elif form == "wild":
+        offs = torch.randint(-500, M + 500, (groups + 1,), generator=g)
+    else:
+        offs = torch.zeros(groups + 1, dtype=torch.int64)
+
+    def expected(offs):
+        out, at = [], 0
+        for i, end in enumerate(offs.tolist() + [M]):
+            end = max(at, min(max(end, 0), M))
+            out += [(r, r, min(r + 256, end), i - 1 if 1 <= i <= groups else -1) for r in range(at, end, 256)]
+            at = end
+        return out
+
+    size = lib.alto_mxfp4_grouped_gemm_workspace_bytes(M, groups)
+    ws = torch.full((size // 4,), -7, dtype=torch.int32, device=DEV)
+    dev = offs.to(torch.int32).to(DEV)
+    stream = torch.cuda.current_stream().cuda_stream
+    assert lib.alto_mxfp4_grouped_gemm_plan(dev.data_ptr(), None, groups, groups, M, ws.data_ptr(), size, stream) == 0
+    want = expected(offs)
+    got = ws.cpu()
+    assert got[0] == len(want) and got[4:4 + 4 * len(want)].view(-1, 4).tolist() == [list(w) for w in want]
+    ws.fill_(-7)
+    back = torch.empty(groups + 1, dtype=torch.int32, device=DEV)
+    ends = dev[1:].clone()
+    assert lib.alto_mxfp4_grouped_gemm_plan_ends(ends.data_ptr(), groups, back.data_ptr(), M, ws.data_ptr(), size, stream) == 0
+    offs[0] = 0
+    want = expected(offs)
+    got = ws.cpu()
+    assert torch.equal(back.cpu(), offs.to(torch.int32))
+    assert got[0] == len(want) and got[4:4 + 4 * len(want)].view(-1, 4).tolist() == [list(w) for w in want]
