@@ -46,6 +46,7 @@ struct GemmCall {
   int c_dtype;
   bool packed;
   Route route;
+  bool narrow = false;   // MID128, but 256x128 tiles where the product has a launch to itself
 };
 
 int plan_gemm(const alto_mxfp4_product& p, GemmCall& g) {
@@ -74,6 +75,8 @@ int plan_gemm(const alto_mxfp4_product& p, GemmCall& g) {
     if (tile == 256 && !tiled) tile = 128;   // (a long, narrow result or a short reduction)
     if (tile != 256 && gemm_mid_supported(A, B, p.M, p.N, p.K, p.c, p.ldc)) g.route = tile == 64 ? Route::MID64 : Route::MID128;
     else if (tiled) g.route = Route::TILED;
+    // (fp32: the 128x128 tile's range reaches into that of the 256x128 tile; two products that share a launch stay on 128x128)
+    g.narrow = g.route == Route::MID128 && tiled && ((p.M + 127) / 128) * ((p.N + 127) / 128) > 256 && gemm_narrow_pays(p.M, p.N);
     if (g.route != Route::NONE) return ALTO_MXFP4_OK;
   }
   ALTO_REQUIRE((p.M + 63) / 64 <= 65535, "gemm: M too large for the fallback kernel");
@@ -154,7 +157,10 @@ int launch_gemm(const GemmCall& g, hipStream_t st) {
   switch (g.route) {
     case Route::NONE: return ALTO_MXFP4_OK;
     case Route::SKINNY: gemm_skinny_launch(q.A, q.B, q.M, q.N, g.K, q.c, g.c_dtype, q.ldc, q.out_scale, st); break;
-    case Route::MID64: case Route::MID128: gemm_mid_launch(g.route == Route::MID64 ? 64 : 128, q, nullptr, g.c_dtype, g.packed, st); break;
+    case Route::MID64: case Route::MID128:
+      if (g.narrow) return gemm_tiled_launch(q.A, q.B, q.M, q.N, g.K, q.c, g.c_dtype, q.ldc, q.out_scale, st);
+      gemm_mid_launch(g.route == Route::MID64 ? 64 : 128, q, nullptr, g.c_dtype, g.packed, st);
+      break;
     case Route::TILED:
       if (g.packed) return gemm_tiled_launch_ps(q.A, q.B, q.M, q.N, g.K, q.c, q.ldc, q.out_scale, st);
       return gemm_tiled_launch(q.A, q.B, q.M, q.N, g.K, q.c, g.c_dtype, q.ldc, q.out_scale, st);

@@ -68,8 +68,8 @@ bool gemm_mid_supported(const OperandView& A, const OperandView& B, int64_t M, i
 //   3000 x 3072 x 1536        2256      576     13.8    17.2    19.6
 // A smaller tile reads its operands from L2 more often and does less with each byte, so it pays while it is what lets
 // (nearly) every compute unit work: two 64x64 tiles per compute unit, then one 128x128 tile.  Beyond that the 256x256
-// kernel is as fast with half of the units idle (and with packed scales up to 256 tiles of 256x128 run there, see
-// gemm_tiled_launch_ps: 512 x 14336 x 4096 in 20.6, 2048 x 4096 x 4096 in 21.7).  With fp32 results its stores are slower and the 128x128 tile holds on
+// kernel is as fast with half of the units idle (and up to 256 tiles of 256x128 run there, see gemm_narrow_pays:
+// 512 x 14336 x 4096 in 20.6, 2048 x 4096 x 4096 in 21.7).  With fp32 results its stores are slower and the 128x128 tile holds on
 // for twice as long (2048 x 4096 x 4096: 33.3 / 30.6; 4096 x 4096 x 2048, 1024 tiles: 31.2 / 35.8).
 int gemm_mid_tile_size(int64_t M, int64_t N, int c_dtype) {
   const int64_t t64 = ((M + 63) / 64) * ((N + 63) / 64), t128 = ((M + 127) / 128) * ((N + 127) / 128);

@@ -31,11 +31,10 @@ constexpr int GT_THREADS = 512;
 constexpr int GT_STAGE_BYTES = (GT_TM + GT_TN) * (GT_TK / 2);   // 65536
 constexpr int GT_NSTAGE = 2;
 constexpr int GT_SCALE_PITCH = 5;                                // dwords per row (16 B + 4 B pad)
-constexpr int GT_SCALE_BUF_DW = (GT_TM + GT_TN) * GT_SCALE_PITCH;  // one buffer, in dwords
-constexpr int GT_LDS_BYTES = GT_NSTAGE * GT_STAGE_BYTES + 2 * GT_SCALE_BUF_DW * 4;  // 131072 + 20480 = 151552
+constexpr int GT_LDS_BYTES = GT_NSTAGE * GT_STAGE_BYTES + 2 * (GT_TM + GT_TN) * GT_SCALE_PITCH * 4;  // 131072 + 20480 = 151552
 
 // The tile routines for WN waves along N: 4, the 256x256 tile; 2, a tile of 256x128 with four waves, for results that have too few
-// 256x256 tiles to keep the chip busy (packed scales and bf16 results only).  A wave's part, 128x64, and its loop are the same.  With one
+// 256x256 tiles to keep the chip busy.  A wave's part, 128x64, and its loop are the same.  With one
 // such workgroup on every compute unit the loop runs at 4.6 PFLOP/s (2048 x 4096: 0.93 us per 256 of K), near what the power limit allows
 // (4.9), against 1.16 us with 256x256 tiles on half of the units; a third ring slot (156 KB of LDS) would have nothing left to hide.
 template <int WN>
@@ -43,8 +42,8 @@ struct TileOf {
   static constexpr int TN = 64 * WN, WAVES = 2 * WN, THREADS = 64 * WAVES;
   static constexpr int STAGE = (GT_TM + TN) * (GT_TK / 2);
   static constexpr int LOADS = (GT_TM + TN) / 8 / WAVES, LOADS_A = GT_TM / 8 / WAVES;   // load instructions of a wave and stage, of A among them
-  static constexpr int LDS = WN == 4 ? GT_LDS_BYTES : GT_NSTAGE * STAGE + 2 * (GT_TM + TN) * 16;
-  static_assert(WN == 4 ? TN == GT_TN && THREADS == GT_THREADS && STAGE == GT_STAGE_BYTES : WN == 2, "");
+  static constexpr int LDS = GT_NSTAGE * STAGE + 2 * (GT_TM + TN) * GT_SCALE_PITCH * 4;
+  static_assert(WN == 4 ? TN == GT_TN && THREADS == GT_THREADS && STAGE == GT_STAGE_BYTES && LDS == GT_LDS_BYTES : WN == 2, "");
 };
 
 // Workgroups are dealt round-robin to the 8 XCDs (each with its own L2).  Every XCD gets a contiguous range of the
@@ -134,13 +133,14 @@ __device__ __forceinline__ void gemm_tile_zero(TileAcc& acc) {
 //   (l % 8) ^ ((row / 2) % 8) of that row.  Raw buffer loads: 32-bit per-lane byte offsets, the K offset of the stage
 //   rides in the scalar offset, and a piece beyond the end of K gets an out-of-range offset, for which the hardware
 //   returns zeros.  (Per-load offsets are recomputed at every stage rather than kept in 8 registers.)
-//   Scales: thread t owns tile row t of A (t < 256) or tile row t - 256 of B (unit stride along K, any alignment).
+//   Scales: thread t owns tile row t of A (t < 256) or tile row t - 256 of B (unit stride along K, any alignment); with four waves row t of
+//   A and row t % 128 of B (two threads then write the same bytes: no branch around the loads and the writes).
 template <int WN>
 struct TileLoader {
   using W = TileOf<WN>;
-  __amdgpu_buffer_rsrc_t rsrc_a, rsrc_b, rsrc_s;
+  __amdgpu_buffer_rsrc_t rsrc_a, rsrc_b, rsrc_s, rsrc_sb;
   int wave, gpiece, arow0, brow0, a_last, a_first, b_last, kbytes, G, s_k0, s_row, k_lead;
-  uint32_t ld_a, ld_b, soff;
+  uint32_t ld_a, ld_b, soff, soff_b;
 
   __device__ __forceinline__ void init(const TileArgs& ta) {
     const int tid = threadIdx.x;
@@ -161,8 +161,7 @@ struct TileLoader {
     s_k0 = ta.s_k0;
     s_row = ta.s_row;
     k_lead = ta.k_lead;
-    if constexpr (WN != 4) return;   // (packed scales)
-    const bool s_is_a = wave < GT_TM / 64;   // scalar: the descriptor choice below must be provably wave-uniform
+    const bool s_is_a = WN == 2 || wave < GT_TM / 64;   // scalar: the descriptor choice below must be provably wave-uniform
     rsrc_s = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(s_is_a ? ta.A.scales : ta.B.scales), 0,
                                                (int)(s_is_a ? ta.as_bytes : ta.bs_bytes), 0x00020000);
     int64_t row;
@@ -175,6 +174,12 @@ struct TileLoader {
       row = ta.n0 + (tid - GT_TM);
       row = row < ta.n_hi ? row : ta.n_hi - 1;
       soff = (uint32_t)((ta.B.is_2d ? (row >> 5) : row) * ta.B.ss_r);
+    }
+    if constexpr (WN == 2) {
+      rsrc_sb = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(ta.B.scales), 0, (int)ta.bs_bytes, 0x00020000);
+      row = ta.n0 + (tid & (W::TN - 1));
+      row = row < ta.n_hi ? row : ta.n_hi - 1;
+      soff_b = (uint32_t)((ta.B.is_2d ? (row >> 5) : row) * ta.B.ss_r);
     }
   }
 
@@ -208,15 +213,16 @@ struct TileLoader {
     }
   }
 
-  // 16 scale bytes of K block kb for this thread's row, in two parts so that nothing touches the loaded registers until
+  // 16 scale bytes of K block kb for this thread's row (raw_b: narrow tile, its row of B), in two parts so that nothing touches the loaded registers until
   // they are used (the wave would otherwise sit out the load's latency right here, two blocks before the bytes are needed):
   // sload sends the load, sfix -- called when the bytes go to LDS -- makes groups at or beyond G read as 127 (scale 1.0),
   // so that the zero codes of a K tail never meet a NaN scale byte.
   template <bool KTAIL>
-  __device__ __forceinline__ void sload(int kb, v4i_t& raw) const {
+  __device__ __forceinline__ void sload(int kb, v4i_t& raw, v4i_t& raw_b) const {
     const int kb16 = __builtin_amdgcn_readfirstlane(kb * 16);
     if constexpr (!KTAIL) {   // G % 4 == 0 and the whole K range: every dword is all inside or all beyond K, one 16-byte load
       raw = __builtin_amdgcn_raw_buffer_load_b128(rsrc_s, (int)soff, kb16, 0);
+      if constexpr (WN == 2) raw_b = __builtin_amdgcn_raw_buffer_load_b128(rsrc_sb, (int)soff_b, kb16, 0);
       return;
     }
     // General case (any G, any sub-range of K): still one 16-byte load per row.  A block that would reach past the end
@@ -226,6 +232,7 @@ struct TileLoader {
     const int last = s_row - 16;
     const int off = __builtin_amdgcn_readfirstlane(want < last ? want : last);
     raw = __builtin_amdgcn_raw_buffer_load_b128(rsrc_s, (int)soff, off, 0);
+    if constexpr (WN == 2) raw_b = __builtin_amdgcn_raw_buffer_load_b128(rsrc_sb, (int)soff_b, off, 0);
   }
   // FAST: the caller knows that the block lies inside its scale row and inside K (every block but the last of a
   // reduction): the bytes are used as loaded
@@ -295,12 +302,12 @@ struct TileLoader {
 template <bool KTAIL, int LMS = -1, int NST = 4, int PS = 0, int WN = 4>
 __device__ __forceinline__ void gemm_tile_mainloop(const TileArgs& ta, TileAcc& acc, uint8_t* smem) {
   using W = TileOf<WN>;
-  static_assert(WN == 4 || PS == 1, "the narrow tile reads packed scales");
+  static_assert(WN == 4 || PS != 2, "sub-ranges of K: the wide tile");
   static_assert(PS != 1 || !KTAIL || LMS >= 0 || LMS == -2, "packed scales: the end of K is known at compile time, or whole stages run (-2)");
   static_assert(PS != 2 || (KTAIL && LMS < 0), "packed scales of a sub-range of K: the generic endings only");
   constexpr int SP = PS ? 4 : GT_SCALE_PITCH;   // dwords per row of a scale buffer in LDS
   TileLoader<WN> ld;
-  v4i_t sraw;   // scale bytes of a later block, as loaded
+  v4i_t sraw, sraw_b;   // scale bytes of a later block, as loaded
   __syncthreads();   // the LDS ring may still be read by a previous call
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;   // the wave index lives in a scalar register
@@ -323,14 +330,18 @@ __device__ __forceinline__ void gemm_tile_mainloop(const TileArgs& ta, TileAcc& 
 
   // LDS row layout (4 dwords): [h=0: K 0..255 | h=0: K 256..511 | h=1: K 0..255 | h=1: K 256..511], where the half-wave h
   // of the MFMA uses group 8 ms + 2 j + h at K step j of macro stage ms: byte j of dword 2 h + ms.
-  auto swrite = [&](int kb, auto fastc) {
+  auto swrite_row = [&](int kb, auto fastc, const v4i_t& raw, int at) {
     uint32_t sreg[4];
-    ld.template sfix<KTAIL, decltype(fastc)::value>(kb, sraw, sreg);
-    uint32_t* row = sscale + (kb & 1) * GT_SCALE_BUF_DW + tid * GT_SCALE_PITCH;
+    ld.template sfix<KTAIL, decltype(fastc)::value>(kb, raw, sreg);
+    uint32_t* row = sscale + (kb & 1) * (GT_TM + W::TN) * SP + at * SP;
     row[0] = __builtin_amdgcn_perm(sreg[1], sreg[0], 0x06040200u);   // groups 0, 2, 4, 6
     row[1] = __builtin_amdgcn_perm(sreg[3], sreg[2], 0x06040200u);   // groups 8, 10, 12, 14
     row[2] = __builtin_amdgcn_perm(sreg[1], sreg[0], 0x07050301u);   // groups 1, 3, 5, 7
     row[3] = __builtin_amdgcn_perm(sreg[3], sreg[2], 0x07050301u);   // groups 9, 11, 13, 15
+  };
+  auto swrite = [&](int kb, auto fastc) {
+    swrite_row(kb, fastc, sraw, tid);
+    if constexpr (WN == 2) swrite_row(kb, fastc, sraw_b, GT_TM + (tid & (W::TN - 1)));
   };
 
   // Fragment / scale registers: F0 = pieces of K step j = 0 of the current stage (read during the previous stage),
@@ -480,7 +491,7 @@ __device__ __forceinline__ void gemm_tile_mainloop(const TileArgs& ta, TileAcc& 
         sdma(kb + 1 + sh);       // block kb+1 (+1 with a half-block shift) -> the buffer whose bytes are all in registers; this block's second stage waits for it
       } else {
         swrite(kb + 1, fastc);   // block kb+1 -> the other scale buffer (last read at the end of block kb-1)
-        ld.template sload<KTAIL>(kb + 2, sraw);
+        ld.template sload<KTAIL>(kb + 2, sraw, sraw_b);
       }
       __builtin_amdgcn_sched_barrier(0);
     }
@@ -505,11 +516,12 @@ __device__ __forceinline__ void gemm_tile_mainloop(const TileArgs& ta, TileAcc& 
     if constexpr (PS == 2) sdma(sh);   // with the shift, block 0 also needs packed block 1 (without: block 0 once more)
     ld.gload(smem, 0, 0, 0, W::LOADS);
     (void)sraw;
+    (void)sraw_b;
   } else {
-    ld.template sload<KTAIL>(0, sraw);
+    ld.template sload<KTAIL>(0, sraw, sraw_b);
     ld.gload(smem, 0, 0, 0, W::LOADS);
     swrite(0, std::false_type{});
-    ld.template sload<KTAIL>(1, sraw);
+    ld.template sload<KTAIL>(1, sraw, sraw_b);
   }
   ld.gload(smem, 1, 1, 0, W::LOADS / 2);   // the other half goes out in the first step of the loop
   static_assert(W::LOADS / 2 == (WN == 4 ? 4 : 6), "the waits below");
@@ -581,7 +593,6 @@ template <typename OutT, int WN = 4>
 __device__ __forceinline__ void gemm_tile_store(const TileArgs& ta, TileAcc& acc, OutT* __restrict__ c, int64_t ldc, uint8_t* smem) {
   using W = TileOf<WN>;
   constexpr int ROW = W::TN * 2, CHUNKS = ROW / 16;   // a bf16 row of the tile: bytes, 16-byte chunks
-  static_assert(WN == 4 || sizeof(OutT) == 2, "");
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int wm = wave / WN, wn = wave % WN;

@@ -33,7 +33,8 @@ inline GemmPair pair_of(const GemmProblem& first, const GemmProblem& second, int
 }
 
 bool gemm_tiled_supported(const OperandView& A, const OperandView& B, int64_t M, int64_t N, int64_t K, const void* c, int c_dtype, int64_t ldc);
-// (the tiled launches return the status of the call)
+// (the tiled launches return the status of the call; they choose between 256x256 and 256x128 tiles by the second rule)
+bool gemm_narrow_pays(int64_t M, int64_t N);
 int gemm_tiled_launch(const OperandView& A, const OperandView& B, int64_t M, int64_t N, int64_t K, void* c, int c_dtype, int64_t ldc,
                       float out_scale, hipStream_t st);
 // Packed scales (see pack_scales_kernel): the converter, and the tiled GEMM on operands that bring them (bf16 output).

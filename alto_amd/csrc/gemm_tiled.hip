@@ -86,15 +86,16 @@ bool gemm_tiled_supported(const OperandView& A, const OperandView& B, int64_t M,
   return tiles < (1ll << 28);
 }
 
-int gemm_tiled_launch(const OperandView& A, const OperandView& B, int64_t M, int64_t N, int64_t K, void* c, int c_dtype, int64_t ldc,
-                      float out_scale, hipStream_t st) {
+template <int WN>   // (see TileOf)
+static int launch_plain(const OperandView& A, const OperandView& B, int64_t M, int64_t N, int64_t K, void* c, int c_dtype, int64_t ldc, float out_scale,
+                        hipStream_t st) {
   const bool tail = (K / 32) % 16 != 0;   // K not a multiple of 512: the last scale block of a row is partial
-#define ALTO_TILED_LAUNCH(T, ...) launch_tiled<T, __VA_ARGS__>(A, B, M, N, K, c, ldc, out_scale, st)
+#define ALTO_TILED_LAUNCH(T, ...) launch_tiled<T, __VA_ARGS__, false, WN>(A, B, M, N, K, c, ldc, out_scale, st)
   if (!tail) {
-    if (c_dtype == ALTO_DT_BF16) return ALTO_TILED_LAUNCH(__bf16, false);
-    else return ALTO_TILED_LAUNCH(float, false);
+    if (c_dtype == ALTO_DT_BF16) return ALTO_TILED_LAUNCH(__bf16, false, -1, 4);
+    else return ALTO_TILED_LAUNCH(float, false, -1, 4);
   } else if (c_dtype != ALTO_DT_BF16) {
-    return ALTO_TILED_LAUNCH(float, true);   // (fp32 output: the general ending)
+    return ALTO_TILED_LAUNCH(float, true, -1, 4);   // (fp32 output: the general ending)
   } else {
     // K is known here: the kernel that ends the reduction exactly where K ends
     int lms, nst;
@@ -114,7 +115,7 @@ int gemm_tiled_launch(const OperandView& A, const OperandView& B, int64_t M, int
 }
 
 // Both operands with packed scales (A.scales / B.scales = packed base, ss_k = bytes per block), bf16 output.
-template <int WN>   // (see TileOf)
+template <int WN>
 static int launch_ps(const OperandView& A, const OperandView& B, int64_t M, int64_t N, int64_t K, void* c, int64_t ldc, float out_scale, hipStream_t st) {
   const bool tail = (K / 32) % 16 != 0;
 #define ALTO_TILED_LAUNCH(...) launch_tiled<__bf16, __VA_ARGS__, true, WN>(A, B, M, N, K, c, ldc, out_scale, st)
@@ -145,11 +146,21 @@ static int launch_ps(const OperandView& A, const OperandView& B, int64_t M, int6
 //   512 x 14336 x 4096          224  25.1 / 20.6             2048 x 4224 x 4096          264  26.6 / 36.3
 //   2048 x 4096 x 1024          256  11.3 / 11.2             3000 x 3072 x 1536          288  14.4 / 19.0
 //   2048 x 4096 x 4096          256  25.1 / 21.7             4096 x 4096 x 4096          512  35.9 / 41.1
-// (From 257 tiles on a second round begins, and a narrow tile reads 1.5 times the bytes per product.)
+// (From 257 tiles on a second round begins, and a narrow tile reads 1.5 times the bytes per product.)  Plain scales, as the inference and
+// the fp32 entry points bring them: bf16 results at 256x256 / 256x128, fp32 results at 128x128 / 256x128, which is what they had:
+//   M x N x K             tiles     bf16          fp32                  M x N x K             tiles     bf16          fp32
+//   2048 x 4096 x 4096     256   28.3 / 23.9   30.9 / 26.8              1000 x 6144 x 1440     192   13.4 / 11.0   18.3 / 16.3
+//   1376 x 4096 x 2880     192   22.1 / 17.3   26.1 / 22.2              333 x 14336 x 7200     224   54.1 / 39.2   60.7 / 45.1
+//   1536 x 4096 x 14336    192   72.4 / 59.6   71.9 / 62.2              1100 x 4096 x 512      160    8.4 /  6.8   10.8 / 10.3
+bool gemm_narrow_pays(int64_t M, int64_t N) { return ((M + GT_TM - 1) / GT_TM) * ((N + TileOf<2>::TN - 1) / TileOf<2>::TN) <= 256; }
+
 int gemm_tiled_launch_ps(const OperandView& A, const OperandView& B, int64_t M, int64_t N, int64_t K, void* c, int64_t ldc, float out_scale,
                          hipStream_t st) {
-  const int64_t narrow = ((M + GT_TM - 1) / GT_TM) * ((N + TileOf<2>::TN - 1) / TileOf<2>::TN);
-  return narrow <= 256 ? launch_ps<2>(A, B, M, N, K, c, ldc, out_scale, st) : launch_ps<4>(A, B, M, N, K, c, ldc, out_scale, st);
+  return gemm_narrow_pays(M, N) ? launch_ps<2>(A, B, M, N, K, c, ldc, out_scale, st) : launch_ps<4>(A, B, M, N, K, c, ldc, out_scale, st);
+}
+
+int gemm_tiled_launch(const OperandView& A, const OperandView& B, int64_t M, int64_t N, int64_t K, void* c, int c_dtype, int64_t ldc, float out_scale, hipStream_t st) {
+  return gemm_narrow_pays(M, N) ? launch_plain<2>(A, B, M, N, K, c, c_dtype, ldc, out_scale, st) : launch_plain<4>(A, B, M, N, K, c, c_dtype, ldc, out_scale, st);
 }
 
 template <bool KTAIL>

@@ -88,6 +88,25 @@ def test_gemm_narrow_tile(m, K):
         assert O.rel_frobenius(product(rows, 0.75)[i0:i0 + 96].cpu(), ref * 0.75) < TOL[torch.bfloat16]
 
 
+@pytest.mark.parametrize("K", [512, 544, 640, 704, 768, 832, 864, 960, 1024, 1184])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("N,b_2d", [(4104, False), (4128, True)])
+def test_gemm_narrow_tile_plain_scales(m, K, dtype, N, b_2d):
+    """1791 rows take the 256x128 tile, 100 of them at a time the 64x64 tile."""
+    rows = 1791
+    a, b = randn_outliers((rows, K), torch.bfloat16, seed=K), randn_outliers((N, K), torch.bfloat16, seed=K + 1)
+    aq, as_ = m.convert_to_mxfp4(a.to(DEV))
+    bq, bs = m.convert_to_mxfp4(b.to(DEV), is_2d_block=b_2d)
+    def product(i, j):
+        return m.blockwise_mxfp4_gemm(aq[i:j], as_[i:j], bq, bs, use_2dblock_b=b_2d, trans_b=True, output_dtype=dtype)
+    print(f"narrow {rows}x{N}x{K}", flush=True)
+    got = product(0, rows)
+    for i0 in range(0, rows, 100):
+        assert torch.equal(got[i0:i0 + 100], product(i0, i0 + 100)), i0
+    ref = O.gemm_ref(aq[-96:].cpu(), as_[-96:].cpu(), bq.cpu(), bs.cpu(), use_2dblock_b=b_2d, trans_b=True)   # (the oracle takes a while for all of it)
+    assert O.rel_frobenius(got[-96:].cpu(), ref) < TOL[dtype]
+
+
 # Both sides of the lines where a short reduction goes to the direct kernel, to the kernel for few rows (16, 32 or 64 columns per
 # workgroup) or to the small tiles
 @pytest.mark.parametrize("M,N,K", [(16, 6144, 288), (16, 6144, 320), (17, 6144, 384), (17, 6144, 416), (1, 6160, 480), (1, 6160, 512), (32, 6160, 544),
