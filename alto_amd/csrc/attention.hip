@@ -371,6 +371,10 @@ static int launch_attn(const AttnArgs& a, const SEQS& seqs, int B, int row_block
 //   D = 192, causal: 8 x 4096 71.7 / 37.5 (1.09), 20 x 2048 42.3 / 32.7 (1.46), 70 x 256 9.8 / 10.3 (.90);
 //   D = 256, all keys: 4 x 4096 69.5 / 54.0 (1.0), 10 x 2048 39.3 / 44.6 (1.25), 67 x 256 9.9 / 12.4 (1.05).
 // Over 238 shapes at .7 to 1.9 of the slots, the mean loss against the better kernel of each is 1.3 % (D = 192: 4 %).
+// Sequences of different lengths, all keys: the workgroups of the short ones fill the ends of the others' as a causal mask's do, from 16
+// blocks on (2016 tokens in two sequences, 16 heads of 128: 33.5 / 25.2 (1.14), 36.0 / 32.6 (1.19), 39.9 / 35.5 (1.30); 3360 in seven, 16 of 64:
+// 30.5 / 28.3 (1.17), 27.6 / 26.7 (1.19), with 14 blocks 22.2 / 23.6 (1.31); 4096 in three, 8 of 128: 37.3 / 37.9 (1.23); 2976 in six, 20 of 64:
+// 27.9 / 27.5 (1.32), 30.5 / 29.6 (1.37), with 11 blocks 21.1 / 23.9 (1.58)).
 // Packed sequences are weighed all together, also where there are more than one launch holds (64): such a call keeps to 128 rows
 // sooner than each of its launches by itself would have to.
 static int rows_per_workgroup(const AttnArgs& a, int64_t B, int64_t D, int n_seqs, const int32_t* cu_q, const int32_t* cu_k) {
@@ -383,7 +387,8 @@ static int rows_per_workgroup(const AttnArgs& a, int64_t B, int64_t D, int n_seq
     longest = n > longest ? n : longest;
   }
   const int per_cu = D == 64 ? 4 : (D == 128 ? 3 : 2);
-  const double share = longest <= 8 ? 0.95 : (D == 192 ? 1.4 : (a.causal ? (longest >= 48 ? 1.3 : 1.125) : (D == 64 ? 1.125 : 1.02)));
+  const bool unequal = n_seqs > 1 && !a.causal && longest >= 16 && D <= 128;
+  const double share = longest <= 8 ? 0.95 : (D == 192 || unequal ? 1.4 : (a.causal ? (longest >= 48 ? 1.3 : 1.125) : (D == 64 ? 1.125 : 1.02)));
   return (double)B * a.Hq * work <= 256.0 * share * per_cu * (double)(longest + 6) ? 32 : 128;
 }
 

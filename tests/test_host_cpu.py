@@ -401,3 +401,20 @@ def test_native_and_python_rules_for_packed_scales_agree():
             seen["grouped"].add(a)
             seen["dw"].add(b)
     assert all(s == {True, False} for s in seen.values())
+
+
+def test_packed_sequences_of_different_lengths_share_the_chip_by_a_wider_line():
+    """All keys, 16 blocks of 64 and more in the longest sequence: 1.4 of the slots (sizes from the table at the rule); shorter ones, one sequence and
+    a causal mask keep their lines."""
+    from alto_amd import _lib
+    lib = _lib.load()
+
+    def rows(H, D, causal, cu):
+        c = (ctypes.c_int32 * len(cu))(*cu)
+        return lib.alto_mxfp4_attention_rows_per_workgroup(1, H, cu[-1], cu[-1], D, len(cu) - 1, c, c, int(causal))
+
+    assert rows(16, 128, False, [0, 288, 2016]) == 32 and rows(16, 128, False, [0, 2048]) == 128
+    seven = [0, 288, 576, 1056, 2336, 3136, 3296, 3360]
+    assert rows(16, 64, False, seven) == 32 and rows(19, 64, False, seven) == 128
+    assert rows(16, 64, False, list(range(0, 3361, 480))) == 128   # seven of 8 blocks
+    assert rows(16, 256, False, [0, 288, 2016]) == 128
