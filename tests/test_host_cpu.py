@@ -418,3 +418,22 @@ def test_packed_sequences_of_different_lengths_share_the_chip_by_a_wider_line():
     assert rows(16, 64, False, seven) == 32 and rows(19, 64, False, seven) == 128
     assert rows(16, 64, False, list(range(0, 3361, 480))) == 128   # seven of 8 blocks
     assert rows(16, 256, False, [0, 288, 2016]) == 128
+
+
+def test_converts_in_assembly_keep_their_distance():
+    """A scaled convert writes part of its destination and does not forward it: in assembly, where the compiler puts in no wait states, the next
+    instruction names another register, and a block ends with a wait (the rule that the compiler follows for its own converts)."""
+    csrc = os.path.join(ROOT, "alto_amd", "csrc")
+    blocks = 0
+    for f in sorted(os.listdir(csrc)):
+        for block in re.findall(r'\basm\s*(?:volatile\s*)?\(\s*((?:"[^"]*"\s*)+)', open(os.path.join(csrc, f)).read()):
+            lines = "".join(re.findall(r'"([^"]*)"', block)).replace(r"\t", "").split(r"\n")
+            if not any("cvt_scalef32" in t for t in lines):
+                continue
+            blocks += 1
+            assert lines[-1].startswith("s_nop"), (f, lines[-1])
+            for now, after in zip(lines, lines[1:]):
+                if "cvt_scalef32" in now:
+                    destination = re.search(r"%\w+", now).group()
+                    assert not re.search(destination + r"\b", after), (f, now, after)
+    assert blocks
