@@ -437,3 +437,31 @@ def test_converts_in_assembly_keep_their_distance():
                     destination = re.search(r"%\w+", now).group()
                     assert not re.search(destination + r"\b", after), (f, now, after)
     assert blocks
+
+
+def _kernel_metadata(path):
+    """What the compiler recorded about each kernel of a library built here: mangled name -> registers and memory (the note of the code
+    objects in its offload bundles)."""
+    import struct
+    msgpack = pytest.importorskip("msgpack")
+    data, kernels = open(path, "rb").read(), {}
+    for bundle in (m.start() for m in re.finditer(b"__CLANG_OFFLOAD_BUNDLE__", data)):
+        at = bundle + 32
+        for _ in range(struct.unpack_from("<Q", data, bundle + 24)[0]):
+            offset, size, name = struct.unpack_from("<QQQ", data, at)
+            if b"gfx950" in data[at + 24:at + 24 + name]:
+                image = data[bundle + offset:bundle + offset + size]
+                note = image.index(b"AMDGPU\0\0")   # (its sizes stand in front of the name)
+                for k in msgpack.unpackb(image[note + 8:note + 8 + struct.unpack_from("<I", image, note - 8)[0]])["amdhsa.kernels"]:
+                    kernels[k[".name"]] = k
+            at += 24 + name
+    return kernels
+
+
+def test_registers_of_the_quantizers_with_clip_or_uos():
+    """bf16, transform, 1D blocks: 64 registers allow the eight waves a SIMD that these kernels hide their memory time with."""
+    from alto_amd import build
+    # quant_kernel<bf16, row, col = 1, rounding 0 or 3, transform, 1D, clip or UOS>, quant_operands_kernel<bf16, transform, clip or UOS>
+    wanted = {n: k[".vgpr_count"] for n, k in _kernel_metadata(build.lib_path()).items()
+              if re.search(r"12quant_kernelIDF16bLb[01]ELb1ELi[03]ELb1ELb0ELb1E|quant_operands_kernelIDF16bLb1ELb1E", n)}
+    assert len(wanted) == 5 and max(wanted.values()) <= 64, wanted
