@@ -375,20 +375,27 @@ static int launch_attn(const AttnArgs& a, const SEQS& seqs, int B, int row_block
 // blocks on (2016 tokens in two sequences, 16 heads of 128: 33.5 / 25.2 (1.14), 36.0 / 32.6 (1.19), 39.9 / 35.5 (1.30); 3360 in seven, 16 of 64:
 // 30.5 / 28.3 (1.17), 27.6 / 26.7 (1.19), with 14 blocks 22.2 / 23.6 (1.31); 4096 in three, 8 of 128: 37.3 / 37.9 (1.23); 2976 in six, 20 of 64:
 // 27.9 / 27.5 (1.32), 30.5 / 29.6 (1.37), with 11 blocks 21.1 / 23.9 (1.58)).
+// Packed sequences of one length are equal workgroups like a batch's: D = 128 keeps to the batch's line while the 128 rows have a compute unit
+// for each workgroup (two of 1024: 13 heads 26.5 / 28.0 (1.08), 16 heads 28.2 / 29.9 (1.33); three of 1536, 7 heads 35.3 / 37.1 (1.31)) and goes on
+// once they do not (two of 1280, 13 heads 36.2 / 33.9 (1.35); three of 1344, 8 heads 38.5 / 34.7 (1.31)); D = 64 goes on from 20 blocks
+// (three of 1024, 14 heads 27.4 / 28.1 (1.31); two of 1536, 14 heads 35.8 / 35.0 (1.31); two of 2048, 11 heads 43.4 / 42.7 (1.38)).
 // Packed sequences are weighed all together, also where there are more than one launch holds (64): such a call keeps to 128 rows
 // sooner than each of its launches by itself would have to.
 static int rows_per_workgroup(const AttnArgs& a, int64_t B, int64_t D, int n_seqs, const int32_t* cu_q, const int32_t* cu_k) {
   if (a.bias || a.alibi || a.Sq / 32 > 65535) return 128;
   double work = 0.0;
-  int64_t longest = 0;
+  int64_t longest = 0, rows_128 = 0;   // rows_128: workgroups of 128 rows
+  bool equal = true;
   for (int i = 0; i < (n_seqs ? n_seqs : 1); ++i) {
     const int64_t bands = (n_seqs ? cu_q[i + 1] - cu_q[i] : a.Sq) / 32, n = ((n_seqs ? cu_k[i + 1] - cu_k[i] : a.Sk_used) + 63) / 64;
     work += (double)bands * (double)(n + 6) - (a.causal ? 0.25 * (double)bands * (double)(bands - 1) : 0.0);   // (a causal band ends half a block before the next)
     longest = n > longest ? n : longest;
+    rows_128 += (bands + 3) / 4;
+    if (n_seqs) equal = equal && cu_q[i + 1] - cu_q[i] == cu_q[1] - cu_q[0] && cu_k[i + 1] - cu_k[i] == cu_k[1] - cu_k[0];
   }
   const int per_cu = D == 64 ? 4 : (D == 128 ? 3 : 2);
-  const bool unequal = n_seqs > 1 && !a.causal && longest >= 16 && D <= 128;
-  const double share = longest <= 8 ? 0.95 : (D == 192 || unequal ? 1.4 : (a.causal ? (longest >= 48 ? 1.3 : 1.125) : (D == 64 ? 1.125 : 1.02)));
+  const bool wide = n_seqs > 1 && !a.causal && longest >= 16 && D <= 128 && (!equal || (D == 64 ? longest >= 20 : B * a.Hq * rows_128 > 256));
+  const double share = longest <= 8 ? 0.95 : (D == 192 || wide ? 1.4 : (a.causal ? (longest >= 48 ? 1.3 : 1.125) : (D == 64 ? 1.125 : 1.02)));
   return (double)B * a.Hq * work <= 256.0 * share * per_cu * (double)(longest + 6) ? 32 : 128;
 }
 

@@ -465,3 +465,29 @@ def test_registers_of_the_quantizers_with_clip_or_uos():
     wanted = {n: k[".vgpr_count"] for n, k in _kernel_metadata(build.lib_path()).items()
               if re.search(r"12quant_kernelIDF16bLb[01]ELb1ELi[03]ELb1ELb0ELb1E|quant_operands_kernelIDF16bLb1ELb1E", n)}
     assert len(wanted) == 5 and max(wanted.values()) <= 64, wanted
+
+
+def test_packed_sequences_of_one_length_share_the_chip_as_a_batch_does():
+    """All keys, the same work packed and as a batch: the same kernel while the 128 rows have a compute unit for each workgroup (heads of 128) or below
+    20 blocks (heads of 64); the line of different lengths beyond."""
+    from alto_amd import _lib
+    lib = _lib.load()
+
+    def rows(H, D, length, n, packed):
+        c = (ctypes.c_int32 * (n + 1))(*range(0, length * n + 1, length)) if packed else None
+        if packed:
+            return lib.alto_mxfp4_attention_rows_per_workgroup(1, H, length * n, length * n, D, n, c, c, 0)
+        return lib.alto_mxfp4_attention_rows_per_workgroup(n, H, length, length, D, 0, None, None, 0)
+
+    seen = set()
+    for D, lengths in ((128, (1024, 1120, 1536, 2048)), (64, (1024, 1184))):
+        for length in lengths:
+            for n in (2, 3, 8):
+                for H in range(1, 41):
+                    if D == 64 or H * n * -(-length // 128) <= 256:
+                        assert rows(H, D, length, n, True) == rows(H, D, length, n, False), (D, length, n, H)
+                        seen.add((D, rows(H, D, length, n, True)))
+    assert seen == {(128, 32), (128, 128), (64, 32), (64, 128)}
+    # 260 workgroups of 128 rows; 22 blocks of keys: beyond the batch's line
+    assert rows(13, 128, 1280, 2, True) == 32 and rows(13, 128, 1280, 2, False) == 128
+    assert rows(14, 64, 1408, 2, True) == 32 and rows(14, 64, 1408, 2, False) == 128
