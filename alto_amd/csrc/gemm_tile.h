@@ -1,5 +1,5 @@
 // LDS-tiled MXFP4 GEMM tile for gfx950: one workgroup of 512 threads (8 waves, 2 x 4) computes a 256x256 tile of
-// C = A . B^T with v_mfma_scale_f32_32x32x64_f8f6f4; each wave owns 128 (M) x 64 (N) = 4 x 2 MFMA tiles (128 accumulator
+// C = A . B^T (or one of 256 threads a tile of 256x128, see TileOf) with v_mfma_scale_f32_32x32x64_f8f6f4; each wave owns 128 (M) x 64 (N) = 4 x 2 MFMA tiles (128 accumulator
 // registers), so two waves share every SIMD and cover each other's waits.
 //
 // Data path per macro stage of 256 K elements (128 B = one cache line per operand row):
@@ -279,7 +279,7 @@ struct TileLoader {
   }
 };
 
-// K loop of one 256x256 tile: acc += A[m0.., :] . B[n0.., :]^T over G groups of 32.  KTAIL = false requires G % 16 == 0
+// K loop of one 256x256 tile (WN = 2: 256x128): acc += A[m0.., :] . B[n0.., :]^T over G groups of 32.  KTAIL = false requires G % 16 == 0
 // (K a multiple of 512) and s_k0 == 0: then every 16-byte scale block of a row lies inside the row.  KTAIL = true
 // handles any G and any start inside the scale rows (a reduction over a sub-range of K).  Requirements
 // checked by the host: unit-stride scale rows, operand extents below 2^31 bytes.  Every thread of the workgroup must
@@ -672,7 +672,7 @@ __device__ __forceinline__ void gemm_tile_store(const TileArgs& ta, TileAcc& acc
 
 // LMS / NST: how the reduction ends, as in gemm_tile_mainloop.
 template <typename OutT, bool KTAIL, int LMS = -1, int NST = 4, int PS = 0, int WN = 4>
-__device__ __forceinline__ void gemm_tile_256x256(const TileArgs& ta, OutT* __restrict__ c, int64_t ldc, uint8_t* smem) {
+__device__ __forceinline__ void gemm_tile_product(const TileArgs& ta, OutT* __restrict__ c, int64_t ldc, uint8_t* smem) {
   TileAcc acc;
   gemm_tile_zero(acc);
   // (with fp32 output and no K tail the specialised ending pushes the register allocation into spilling: plain loop there)

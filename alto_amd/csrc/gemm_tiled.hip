@@ -1,4 +1,4 @@
-// Tuned LDS-tiled MXFP4 GEMM for gfx950: dense entry (one 256x256 tile per 512-thread workgroup, XCD-aware tile order).
+// Tuned LDS-tiled MXFP4 GEMM for gfx950: dense entry (one 256x256 tile per 512-thread workgroup or 256x128 per 256-thread one, XCD-aware tile order).
 
 #include "gemm_tiled.h"
 #include "gemm_tile.h"
@@ -16,7 +16,7 @@ __global__ __launch_bounds__(TileOf<WN>::THREADS) void gemm_tiled_kernel(Operand
   TileArgs ta{A, B, (int64_t)tm * GT_TM, (int64_t)tn * TileOf<WN>::TN, 0, M, N, G, out_scale,
               (M - 1) * A.ld + G * 16, (N - 1) * B.ld + G * 16,
               PS ? KB * A.ss_k : ((A.is_2d ? M / 32 : M) - 1) * A.ss_r + G, PS ? KB * B.ss_k : ((B.is_2d ? N / 32 : N) - 1) * B.ss_r + G, 0, G};
-  gemm_tile_256x256<OutT, KTAIL, LMS, NST, PS, WN>(ta, c, ldc, smem);
+  gemm_tile_product<OutT, KTAIL, LMS, NST, PS, WN>(ta, c, ldc, smem);
 }
 
 // Two products on packed scales, bf16 results (no KTAIL: K a multiple of 512 in both).  The tiles of the second fill the units that
@@ -32,7 +32,7 @@ __global__ __launch_bounds__(GT_THREADS) void gemm_tiled_two_kernel(GemmPair p) 
   const int KB = (q.G + 15) / 16;
   TileArgs ta{q.A, q.B, (int64_t)tm * GT_TM, (int64_t)tn * GT_TN, 0, q.M, q.N, q.G, q.out_scale, (q.M - 1) * q.A.ld + q.G * 16, (q.N - 1) * q.B.ld + q.G * 16,
               KB * q.A.ss_k, KB * q.B.ss_k, 0, q.G};
-  gemm_tile_256x256<__bf16, KTAIL, -2, 4, 1>(ta, static_cast<__bf16*>(q.c), q.ldc, smem);
+  gemm_tile_product<__bf16, KTAIL, -2, 4, 1>(ta, static_cast<__bf16*>(q.c), q.ldc, smem);
 }
 
 // Plain scales of one operand -> the packed form the PS kernels read: dst[(kb * rows + row) * 16 + 4 (2 h + ms) + j] =

@@ -127,7 +127,7 @@ __global__ __launch_bounds__(256) void grouped_dw_simple_kernel(OperandView GO, 
   }
 }
 
-// ----------------------------------------------------------------------------- 256x256 tiles (large problems)
+// ----------------------------------------------------------------------------- 256x256 and 256x128 tiles (large problems)
 
 // Tile order of the grouped kernels.  As in the dense kernel an XCD (wg % 8) works on 8 neighbouring N-tiles of a few passes
 // at a time, so its L2 shares the A rows and the expert's weight rows.  The passes are dealt to the XCDs in runs of
@@ -374,7 +374,7 @@ __device__ __forceinline__ void grouped_rows_tile(const GroupedRows& q, int wg, 
               (q.M_total - 1) * q.A.ld + q.G * 16, (N - 1) * q.ldw + q.G * 16,
               PS ? KB * q.A.ss_k : ((q.A.is_2d ? q.M_total / 32 : q.M_total) - 1) * q.A.ss_r + q.G,
               PS ? KB * N * 16 : ((q.w_is_2d ? N / 32 : N) - 1) * q.ws_r + q.G, 0, q.G};
-  gemm_tile_256x256<OutT, KTAIL, LMS, NST, PS, WN>(ta, out, q.ldo, smem);
+  gemm_tile_product<OutT, KTAIL, LMS, NST, PS, WN>(ta, out, q.ldo, smem);
 }
 
 template <typename OutT, bool KTAIL, int LMS, int NST, bool PS, int WN>

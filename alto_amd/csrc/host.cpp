@@ -296,9 +296,11 @@ bool attend(const Tensor& q_in, const Tensor& k_in, const Tensor& v_in, double s
 // A layer's step as an autograd node of its own, one native call per direction: outputs, quantizers and products, the interpreter
 // lock given up.  What a direction needs only itself shares one buffer, what the backward needs of either operand has one of its own.
 // The backward runs on the engine's device thread while the caller waits, and every handover of the interpreter lock between the two
-// is a wake-up more: as a Python function whose two directions were native calls, a linear step of 512 x 1024 x 1024 took 119 us, as a
-// node that the engine calls without the interpreter 92 (about 40 of them the engine's own two wake-ups, 17 this backward; where a
-// waiting thread wakes in 3 us instead of 15, 108 -> 50); 2048 x 4096 x 4096 119 -> 97, expert layer of 2560 x 1024 x 1440 139 -> 110.
+// is a wake-up more.  A node of its own needs the interpreter only where the gradient is rounded stochastically, to ask which source of
+// random words is installed; a Python function whose two directions were native calls needed it for each.  Whole steps, five processes
+// of either in turn: 512 x 1024 x 1024 110 to 114 us as that function (one process 68: how fast a waiting thread wakes differs from
+// process to process), 90 to 94 as a node; 2048 x 4096 x 4096 102 to 111, 96; fp32 1376 x 2880 x 2144 94 to 97 (one 69), 78 to 83; expert
+// layer of 2560 x 1024 x 1440 120 to 123, 94 to 98.  (About 40 us of a small step are the engine's own two wake-ups.)
 struct Failure {
   int rc = 0;
   const char* name = "";

@@ -79,8 +79,9 @@ __device__ __forceinline__ float div_sqrt32_signed(float z, uint32_t flip) {
 
 // z / float32(sqrt(32)) for a result that is rounded to bf16 next: z rh + z rl with rh + rl = 1 / float32(sqrt(32)) to 49 bits, in two
 // instructions (`flip` = 0 or 0x80000000 goes onto both constants).  The fp32 result is the correctly rounded quotient for every z
-// from 2^-103 on (all 2^23 significands tried: the sequence knows no exponent until z rl loses bits below 2^-126); below, z is a sum
-// of bf16 values, i.e. a multiple of 2^-133, and every one of those gives the same bf16 value as the exact quotient.  Both
+// from 2^-100 on (all 2^23 significands tried: the sequence knows no exponent until z rl loses bits below 2^-126).  Below that it may be
+// the neighbour, but rounds to the same bf16 value as the exact quotient: from 2^-111 on for every z, and further down for the multiples of
+// 2^-133 (all tried), which is what sums of bf16 values are.  Both
 // constants are positive, so infinities stay what they are, and -0 stays -0.  (fp32 tensors keep the correction step and the division
 // fix-up: four instructions.)  With the converts below and the three-operand exclusive or of Philox, dY 8192 x 14336 95.0 -> 85.5 us,
 // 512 x 1024 5.4 -> 4.9; x, round to nearest, 8192 x 4096 24.9 -> 22.3.
