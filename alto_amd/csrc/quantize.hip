@@ -134,6 +134,16 @@ __device__ __forceinline__ uint32_t rne_codes8(const uint32_t* w, float scale) {
   return o;
 }
 
+// The dwords of a lane's four rows of eight fp32 elements, one for each pair: Philox calls 4 `call` .. + 4 of the stream
+__device__ __forceinline__ void row_words_f32(uint32_t (&word)[4][4], uint64_t call, uint64_t ctr0, uint64_t key) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const uint64_t q = ctr0 + call * 4 + (uint64_t)i;
+    const uint4 a = philox4x32_10(q, q < ctr0 ? 1ull : 0ull, key);
+    word[i][0] = a.x; word[i][1] = a.y; word[i][2] = a.z; word[i][3] = a.w;
+  }
+}
+
 template <typename T>
 __device__ __forceinline__ float round_to_T(float v) {
   if constexpr (sizeof(T) == 2) {   // float -> bf16 (round to nearest even, one v_cvt_pk_bf16_f32 per pair) -> float
@@ -277,19 +287,18 @@ __device__ __forceinline__ void quant_tile(const QuantParams& p, unsigned wg, un
     uint32_t rr[4][((SR == 1 || SR == 2) && (DO_ROW || STASH)) ? 8 : 1];
     constexpr bool ROW_CODES = DO_ROW || XCODES;   // the row phase encodes (and stores, when DO_ROW)
     uint32_t hw_row[4][(HW && ROW_CODES) ? (BF ? 1 : 4) : 1];
-    if constexpr (HW && ROW_CODES) {
+    // fp32, column copy without the transform: the four calls behind the loads, or the compiler sends those after the third (8192 x 4096, static
+    // clip 39.6 -> 36.1 us, UOS 40.0 -> 36.1, neither 37.4 -> 35.7; before the three-operand exclusive or it moved the calls to their uses: 38.0,
+    // 39.7, 37.4).  With the transform they are better ahead (40.6 / 41.2), and in the row copy alone, 1024 x 2048, 3.36 / 3.42.
+    constexpr bool WORDS_BEHIND_LOADS = HW && ROW_CODES && !BF && !RHT && DO_COL;
+    if constexpr (HW && ROW_CODES && !WORDS_BEHIND_LOADS) {
       const uint64_t call = (band * (uint64_t)(C >> 3) + (uint64_t)((col0 >> 3) + (tid & 31))) * 8 + (uint64_t)(tid >> 5);
       if constexpr (BF) {
         const uint64_t q = ctr0 + call;
         const uint4 a = philox4x32_10(q, q < ctr0 ? 1ull : 0ull, key);
         hw_row[0][0] = a.x; hw_row[1][0] = a.y; hw_row[2][0] = a.z; hw_row[3][0] = a.w;
       } else {
-  #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const uint64_t q = ctr0 + call * 4 + (uint64_t)i;
-          const uint4 a = philox4x32_10(q, q < ctr0 ? 1ull : 0ull, key);
-          hw_row[i][0] = a.x; hw_row[i][1] = a.y; hw_row[i][2] = a.z; hw_row[i][3] = a.w;
-        }
+        row_words_f32(hw_row, call, ctr0, key);
       }
     }
     uint32_t amax_i[4];
@@ -314,6 +323,8 @@ __device__ __forceinline__ void quant_tile(const QuantParams& p, unsigned wg, un
         rr[i][4] = r1[0]; rr[i][5] = r1[1]; rr[i][6] = r1[2]; rr[i][7] = r1[3];
       }
     }
+    if constexpr (WORDS_BEHIND_LOADS)
+      row_words_f32(hw_row, (band * (uint64_t)(C >> 3) + (uint64_t)((col0 >> 3) + (tid & 31))) * 8 + (uint64_t)(tid >> 5), ctr0, key);
     uint32_t rc[EARLY ? 32 : 1];
     if constexpr (EARLY) {
       const int cvoff = (col0 + tid < C) ? tid * 4 + col0 * 4 : OOB;

@@ -439,23 +439,53 @@ def test_converts_in_assembly_keep_their_distance():
     assert blocks
 
 
-def _kernel_metadata(path):
-    """What the compiler recorded about each kernel of a library built here: mangled name -> registers and memory (the note of the code
-    objects in its offload bundles)."""
+def _code_objects(path):
+    """The gfx950 code objects in the offload bundles of a library built here."""
     import struct
-    msgpack = pytest.importorskip("msgpack")
-    data, kernels = open(path, "rb").read(), {}
+    data = open(path, "rb").read()
     for bundle in (m.start() for m in re.finditer(b"__CLANG_OFFLOAD_BUNDLE__", data)):
         at = bundle + 32
         for _ in range(struct.unpack_from("<Q", data, bundle + 24)[0]):
             offset, size, name = struct.unpack_from("<QQQ", data, at)
             if b"gfx950" in data[at + 24:at + 24 + name]:
-                image = data[bundle + offset:bundle + offset + size]
-                note = image.index(b"AMDGPU\0\0")   # (its sizes stand in front of the name)
-                for k in msgpack.unpackb(image[note + 8:note + 8 + struct.unpack_from("<I", image, note - 8)[0]])["amdhsa.kernels"]:
-                    kernels[k[".name"]] = k
+                yield data[bundle + offset:bundle + offset + size]
             at += 24 + name
+
+
+def _kernel_metadata(path):
+    """What the compiler recorded about each kernel of a library built here: mangled name -> registers and memory (the note of its code
+    objects)."""
+    import struct
+    msgpack = pytest.importorskip("msgpack")
+    kernels = {}
+    for image in _code_objects(path):
+        note = image.index(b"AMDGPU\0\0")   # (its sizes stand in front of the name)
+        for k in msgpack.unpackb(image[note + 8:note + 8 + struct.unpack_from("<I", image, note - 8)[0]])["amdhsa.kernels"]:
+            kernels[k[".name"]] = k
     return kernels
+
+
+def _kernel_instructions(path, wanted, directory):
+    """The instructions of the kernels of a library built here whose mangled names match `wanted`: name -> list of mnemonics."""
+    import shutil
+    import subprocess
+    objdump = shutil.which("llvm-objdump") or "/opt/rocm/llvm/bin/llvm-objdump"
+    if not os.path.exists(objdump):
+        pytest.skip("no llvm-objdump")
+    found = {}
+    for image in _code_objects(path):
+        names = {n for n in re.findall(rb"_ZN\w+", image) if re.search(wanted, n.decode())}
+        if names:
+            obj = os.path.join(str(directory), "object.o")
+            with open(obj, "wb") as fh:
+                fh.write(image)
+            symbols = ",".join(sorted(n.decode() for n in names))
+            text = subprocess.run([objdump, "-d", "--no-show-raw-insn", f"--disassemble-symbols={symbols}", obj], capture_output=True, text=True, check=True).stdout
+            for part in text.split("\n\n"):
+                m = re.search(r"<(_ZN\w+)>:", part)
+                if m:
+                    found[m.group(1)] = [t.split()[0] for t in part[m.end():].split("\n") if t.strip() and not t.strip().startswith("<")]
+    return found
 
 
 def test_registers_of_the_quantizers_with_clip_or_uos():
@@ -491,3 +521,17 @@ def test_packed_sequences_of_one_length_share_the_chip_as_a_batch_does():
     # 260 workgroups of 128 rows; 22 blocks of keys: beyond the batch's line
     assert rows(13, 128, 1280, 2, True) == 32 and rows(13, 128, 1280, 2, False) == 128
     assert rows(14, 64, 1408, 2, True) == 32 and rows(14, 64, 1408, 2, False) == 128
+
+
+def test_words_of_fp32_rows_stand_behind_the_loads(tmp_path):
+    """fp32, both copies without the transform, rounded stochastically: the tile's eight loads leave before the work on the random words (four
+    Philox calls of 20 products) begins."""
+    from alto_amd import build
+    # quant_kernel<float, row, column, hardware rounding, no transform, 1D>, with and without clip or UOS
+    kernels = _kernel_instructions(build.lib_path(), r"12quant_kernelIfLb1ELb1ELi3ELb0ELb0ELb[01]ELi1ELb0E\w*QuantParamsE$", tmp_path)
+    assert len(kernels) == 2
+    for name, ops in kernels.items():
+        loads = [i for i, op in enumerate(ops) if op.startswith("buffer_load_dwordx4")]
+        products = [i for i, op in enumerate(ops) if op.startswith("v_mad_u64")]
+        assert len(loads) == 8 and len(products) > 80, (name, len(loads), len(products))
+        assert sum(i < loads[-1] for i in products) <= 8, name   # (those before are addresses)
