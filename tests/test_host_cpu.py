@@ -535,3 +535,13 @@ def test_words_of_fp32_rows_stand_behind_the_loads(tmp_path):
         products = [i for i, op in enumerate(ops) if op.startswith("v_mad_u64")]
         assert len(loads) == 8 and len(products) > 80, (name, len(loads), len(products))
         assert sum(i < loads[-1] for i in products) <= 8, name   # (those before are addresses)
+
+
+def test_clipped_bf16_rows_are_converted_in_pairs(tmp_path):
+    """Row copies of bf16 rounded to nearest with static clip or UOS: the one convert is the one of bf16 pairs, four a dword, and no branch chooses
+    between two forms."""
+    from alto_amd import build
+    kernels = _kernel_instructions(build.lib_path(), r"12quant_kernelIDF16bLb1ELb0ELi0ELb0ELb[01]ELb1ELi1ELb0E\w*QuantParamsE$", tmp_path)
+    assert len(kernels) == 2
+    for name, ops in kernels.items():
+        assert not any(op.startswith("v_cvt_scalef32_pk_fp4_f32") for op in ops) and sum(op.startswith("v_cvt_scalef32_pk_fp4_bf16") for op in ops) == 16, name
