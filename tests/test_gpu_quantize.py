@@ -383,12 +383,28 @@ def test_in_kernel_philox_equals_supplied_words(m, dtype, shape, software_sr):
 @pytest.mark.parametrize("exponent", [-133, -126, -124, -118, -104, -96, 0, 100, 121])
 def test_hadamard_quotient_over_the_range(m, exponent):
     """The transform's division by sqrt(32) in front of the rounding to bf16, from sums of the smallest bf16 values to overflow, infinities
-    and zeros of either sign among them: codes and scales of the column copy against the CPU model.  A block with one infinity becomes 32 of
-    definite signs, alone in its block or beside finite values (two in a block would be NaN where they cancel)."""
+    and zeros of either sign among them: codes and scales of the column copy against the CPU model."""
     g = torch.Generator().manual_seed(exponent + 200)
     x = (torch.randn(96, 256, generator=g) * torch.randint(0, 3, (96, 256), generator=g)).double() * 2.0 ** exponent
     x[::7, ::5] = -0.0
-    blocks = ((3, 17), (40, 200), (95, 200), (64, 31)) if exponent in (-133, 0, 100) else ()   # (row, column), each in a block of its own
+    if exponent == 0:
+        x[3, 17], x[40, 200] = float("inf"), float("-inf")
+    x = x.to(torch.bfloat16)
+    signs, perm = hadamard_from_seed(abs(exponent))
+    h = m.HadamardTransform(signs, perm)
+    _, _, codes, scales = m.quantize_rowcol(x.to(DEV), False, hadamard=h)
+    ref, ref_scales = O.quantize(O.rht_left(x, signs, perm), axis=0)
+    finite = ~torch.isinf(x.float()).any(0)   # (columns with an infinity hold NaN codes of no particular sign)
+    assert torch.equal(codes.cpu()[:, finite], ref[:, finite]) and torch.equal(scales.cpu()[:, finite], ref_scales[:, finite])
+
+
+@pytest.mark.parametrize("exponent", [-133, 0, 100])
+def test_hadamard_of_blocks_with_an_infinity(m, exponent):
+    """A block with one infinity becomes 32 of definite signs (two in a block would be NaN where they cancel), scale 253 and the largest codes, beside
+    blocks of sums of the smallest bf16 values, ordinary and large ones; one infinity alone in its block, the others among finite values."""
+    g = torch.Generator().manual_seed(exponent + 500)
+    x = (torch.randn(96, 256, generator=g) * torch.randint(0, 3, (96, 256), generator=g)).double() * 2.0 ** exponent
+    blocks = ((3, 17), (40, 200), (95, 200), (64, 31))   # (row, column), each in a block of its own
     for i, (row, column) in enumerate(blocks):
         x[row, column] = float("inf") if i % 2 == 0 else float("-inf")
     x[64 + 1:96, 31] = 0.0
@@ -397,8 +413,8 @@ def test_hadamard_quotient_over_the_range(m, exponent):
     h = m.HadamardTransform(signs, perm)
     y = O.rht_left(x, signs, perm)
     assert not torch.isnan(y).any() and int(torch.isinf(y).sum()) == 32 * len(blocks)
-    _, _, codes, scales = m.quantize_rowcol(x.to(DEV), False, hadamard=h)
     ref, ref_scales = O.quantize(y, axis=0)
     for row, column in blocks:
         assert set(ref[row // 32 * 16:row // 32 * 16 + 16, column].tolist()) <= {0x77, 0x7F, 0xF7, 0xFF} and ref_scales[row // 32, column] == 253
+    _, _, codes, scales = m.quantize_rowcol(x.to(DEV), False, hadamard=h)
     assert torch.equal(codes.cpu(), ref) and torch.equal(scales.cpu(), ref_scales)
