@@ -195,7 +195,9 @@ __device__ __forceinline__ void mask_scores(v16f_t (&S)[2], int seen) {
 
 // Largest score of row r = lane % 32 in the tile h = lane / 32 (S: two tiles of 32 keys, a row's keys over the lanes r and r + 32), and
 // in both tiles.  One swap hands either lane of a row the other one's part of its tile (a swap for each tile, as before, does the work
-// for both tiles in both lanes).
+// for both tiles in both lanes).  ALONE (one wave a SIMD, nothing to fill a wait): the second swap does not wait for the first, for an
+// instruction more.
+template <bool ALONE>
 __device__ __forceinline__ void row_maxima(const v16f_t (&S)[2], float& tile_max, float& row_max) {
   float x[2];
 #pragma unroll
@@ -205,7 +207,8 @@ __device__ __forceinline__ void row_maxima(const v16f_t (&S)[2], float& tile_max
     for (int v = 0; v < 16; ++v) x[t] = fmaxf(x[t], S[t][v]);
   }
   tile_max = max_of_pair(__builtin_amdgcn_permlane32_swap(f2u(x[0]), f2u(x[1]), false, false));
-  row_max = max_of_pair(__builtin_amdgcn_permlane32_swap(f2u(tile_max), f2u(tile_max), false, false));
+  const float mine = ALONE ? max_one(x[0], x[1]) : tile_max;
+  row_max = max_of_pair(__builtin_amdgcn_permlane32_swap(f2u(mine), f2u(mine), false, false));
 }
 
 // Probabilities of a wave's 32 rows and 64 keys (S: scores of this lane's row, keys as score_key() deals them; tile_max: the row's

@@ -58,7 +58,10 @@ struct AttnTile {
 // wait, the priority lets the arithmetic behind it through), Q read non-temporally 2 less; of use to the kernel on codes as well:
 // the heads dealt to the XCDs in ranges 195 -> 187, the results stored as whole rows 187 -> 181 (then through the LDS).
 // SEQS: AttnSeqs, or AttnNoSeqs for B sequences of one length.
-template <int NK, int ND, bool BIASED, bool QBF, typename SEQS>
+// ALONE: for launches that leave a SIMD about one wave (see launch_plan): what a wave waits for costs its time, and instructions cost none.  The
+// rescale takes all rows without a branch (four branches of which none is taken, in nearly every block of the first thousand keys,
+// cost 90 clocks a block), V's codes are read ahead of it, and the second swap of row_maxima() does not wait for the first.
+template <int NK, int ND, bool BIASED, bool QBF, bool ALONE, typename SEQS>
 __device__ __forceinline__ void attn_fwd_body(const AttnArgs& a, const SEQS& seqs, __bf16* __restrict__ out, float* __restrict__ lse_out, uint8_t* ring) {
   constexpr int D = NK * 64, DV = ND * 32;
   constexpr int K_BYTES = AttnTile<NK, ND>::K_BYTES, V_BYTES = AttnTile<NK, ND>::V_BYTES, SLOT = AttnTile<NK, ND>::SLOT;
@@ -274,7 +277,7 @@ __device__ __forceinline__ void attn_fwd_body(const AttnArgs& a, const SEQS& seq
         mask_scores(S, (a.causal && qrow + shift + 1 < kn ? qrow + shift + 1 : kn) - key0 - 8 * h);
       }
       float tile_max, mx;
-      row_maxima(S, tile_max, mx);
+      row_maxima<ALONE>(S, tile_max, mx);
       float m_new = max_one(m_i, mx * cs);
       // a bias may hide every key a row has seen so far (-inf): such a row keeps m = -inf and takes exp2(-inf - 0) = 0
       // everywhere instead of exp2(-inf + inf)
@@ -288,6 +291,12 @@ __device__ __forceinline__ void attn_fwd_body(const AttnArgs& a, const SEQS& seq
       quantize_probabilities(S, tile_max, cs, m_new, pf, pscale);
 
       // ---- row sums of the quantised probabilities (a column of ones) and O += P V
+      v8i_t vf[ALONE ? ND : 1];
+      auto read_v = [&](int d) { return frag16(tile + K_BYTES + (32 * d + r) * 32 + ((16 * h) ^ v_swz)); };
+      if constexpr (ALONE) {
+#pragma unroll
+        for (int d = 0; d < ND; ++d) vf[d] = read_v(d);
+      }
       const uint32_t changed = (uint32_t)__builtin_amdgcn_ballot_w64(alpha != 1.0f);   // (both lanes of a row have its alpha)
       if (changed != 0) {
         acc_l[0] *= alpha;   // all registers hold the row sum; only [0] is read
@@ -298,8 +307,8 @@ __device__ __forceinline__ void attn_fwd_body(const AttnArgs& a, const SEQS& seq
         for (int g = 0; g < 4; ++g) f[g] = *reinterpret_cast<const v4f_t*>(factors + 8 * g + 4 * h);
         static_for<4>([&](auto gc) {
           constexpr int g = decltype(gc)::value;   // registers 4 g .. + 4 of the two halves: rows 8 g .. + 8
-          if (changed & (0xFFu << (8 * g))) {
-            asm volatile("" ::: "memory");   // keep this a branch
+          if (ALONE || changed & (0xFFu << (8 * g))) {
+            if constexpr (!ALONE) asm volatile("" ::: "memory");   // keep this a branch
 #pragma unroll
             for (int i = 0; i < 4; ++i)
 #pragma unroll
@@ -312,8 +321,7 @@ __device__ __forceinline__ void attn_fwd_body(const AttnArgs& a, const SEQS& seq
       const int vsh = DV == 128 ? (int)((h ? vsw[VS_DW - 1] : vsw[0]) >> (8 * (r >> 3))) : (int)(vsw[0] >> (16 * h + 8 * (r >> 4)));
       static_for<ND>([&](auto dc) {
         constexpr int d = decltype(dc)::value;
-        const v8i_t vf = frag16(tile + K_BYTES + (32 * d + r) * 32 + ((16 * h) ^ v_swz));
-        acc_o[d] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(pf, vf, acc_o[d], 4, 4, 0, pscale, 0, vsh);
+        acc_o[d] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(pf, ALONE ? vf[ALONE ? d : 0] : read_v(d), acc_o[d], 4, 4, 0, pscale, 0, vsh);
       });
     }
     wait_dma(kb + 2 < wg_blk);   // block kb + 1 has landed (this wave's part; the barrier collects the others')
@@ -342,20 +350,36 @@ __device__ __forceinline__ void attn_fwd_body(const AttnArgs& a, const SEQS& seq
   if (h == 0) lse_out[b * a.l_sb + hq * a.l_sh + (q_first + qrow) * a.l_ss] = (m_i + log2f(l)) * ATTN_LN2;
 }
 
-template <int NK, int ND, bool BIASED, bool QBF, typename SEQS>
+template <int NK, int ND, bool BIASED, bool QBF, bool ALONE, typename SEQS>
 __global__ __launch_bounds__(256, BIASED ? 2 : ATTN_WG_PER_CU) void attn_fwd_kernel(AttnArgs a, SEQS seqs) {
   __shared__ __attribute__((aligned(16))) uint8_t ring[AttnTile<NK, ND>::QUERY + (QBF ? 4 * NK * 1024 : 0)];
-  attn_fwd_body<NK, ND, BIASED, QBF>(a, seqs, reinterpret_cast<__bf16*>(a.out), a.lse, ring);
+  attn_fwd_body<NK, ND, BIASED, QBF, ALONE>(a, seqs, reinterpret_cast<__bf16*>(a.out), a.lse, ring);
 }
 
 template <int NK, int ND, typename SEQS>
-static int launch_attn(const AttnArgs& a, const SEQS& seqs, int B, int row_blocks, hipStream_t st) {
+static int launch_attn(const AttnArgs& a, const SEQS& seqs, int B, int row_blocks, bool alone, hipStream_t st) {
   dim3 grid((unsigned)a.Hq, (unsigned)B, (unsigned)row_blocks);
-  if (a.bias || a.alibi) hipLaunchKernelGGL((attn_fwd_kernel<NK, ND, true, false, SEQS>), grid, dim3(256), 0, st, a, seqs);
-  else if (a.qx) hipLaunchKernelGGL((attn_fwd_kernel<NK, ND, false, true, SEQS>), grid, dim3(256), 0, st, a, seqs);
-  else hipLaunchKernelGGL((attn_fwd_kernel<NK, ND, false, false, SEQS>), grid, dim3(256), 0, st, a, seqs);
+  if (a.bias || a.alibi) {
+    hipLaunchKernelGGL((attn_fwd_kernel<NK, ND, true, false, false, SEQS>), grid, dim3(256), 0, st, a, seqs);
+    return check_launch("attention_fwd");
+  }
+  if constexpr (NK <= 2) {
+    if (alone) {
+      if (a.qx) hipLaunchKernelGGL((attn_fwd_kernel<NK, ND, false, true, true, SEQS>), grid, dim3(256), 0, st, a, seqs);
+      else hipLaunchKernelGGL((attn_fwd_kernel<NK, ND, false, false, true, SEQS>), grid, dim3(256), 0, st, a, seqs);
+      return check_launch("attention_fwd");
+    }
+  }
+  if (a.qx) hipLaunchKernelGGL((attn_fwd_kernel<NK, ND, false, true, false, SEQS>), grid, dim3(256), 0, st, a, seqs);
+  else hipLaunchKernelGGL((attn_fwd_kernel<NK, ND, false, false, false, SEQS>), grid, dim3(256), 0, st, a, seqs);
   return check_launch("attention_fwd");
 }
+
+// What a call is launched as: the rows of one workgroup, and for 128 of them whether a SIMD has its waves ALONE.
+struct LaunchPlan {
+  int rows;
+  bool alone;
+};
 
 // Rows of one workgroup: 32 where its waves deal out the keys (attention_split.hip), 128 where every wave walks them all.
 //
@@ -381,8 +405,17 @@ static int launch_attn(const AttnArgs& a, const SEQS& seqs, int B, int row_block
 // (three of 1024, 14 heads 27.4 / 28.1 (1.31); two of 1536, 14 heads 35.8 / 35.0 (1.31); two of 2048, 11 heads 43.4 / 42.7 (1.38)).
 // Packed sequences are weighed all together, also where there are more than one launch holds (64): such a call keeps to 128 rows
 // sooner than each of its launches by itself would have to.
-static int rows_per_workgroup(const AttnArgs& a, int64_t B, int64_t D, int n_seqs, const int32_t* cu_q, const int32_t* cu_k) {
-  if (a.bias || a.alibi || a.Sq / 32 > 65535) return 128;
+//
+// ALONE: all keys, heads of 64 and 128, up to one 128-row workgroup a unit; two with heads of 64, and a few more with sequences of different
+// lengths, whose long ones end alone.  us without / with (and the kernel with O's rows in lanes, which had no groups to branch over):
+//   D = 128: 14 heads x 2048 tokens (224 workgroups) 40.0 / 39.7 (39.4), 16 x 2048 (256) 41.1 / 40.7 (39.7), 4 x 8 x 1024 (256) 27.4 / 26.8 (26.8), two packed
+//   of 1024, 16 heads 27.4 / 26.7 (26.5); beyond: 9 x 4096 (288) .947 / .986 of the old time, 12 x 4096 (384) .939 / .975;
+//   eight of 4064 tokens, 12 heads (408) 35.2 / 34.3 (34.4), 16 heads (544) 35.5 / 34.8 (34.9), 20 heads (680) .934 / .951 of the old time;
+//   D = 64: 40 x 1024 (320) 24.9 / 24.2 (24.6), 64 x 1024 (512) 27.2 / 26.7 (26.9), 16 x 4096 (512) 77.3 / 77.0 (78.3), eight of 4064, 16 heads (544) 28.7 / 28.0
+//   (27.8); beyond: 20 x 4096 (640) .918 / .948, 96 x 1024 (768) .957 / .967 of the old time.
+// A causal mask fills up the units with other workgroups (all at .90 to .98 of the old time without), and D = 192 and 256 gain nothing.
+static LaunchPlan launch_plan(const AttnArgs& a, int64_t B, int64_t D, int n_seqs, const int32_t* cu_q, const int32_t* cu_k) {
+  if (a.bias || a.alibi || a.Sq / 32 > 65535) return {128, false};
   double work = 0.0;
   int64_t longest = 0, rows_128 = 0;   // rows_128: workgroups of 128 rows
   bool equal = true;
@@ -396,21 +429,22 @@ static int rows_per_workgroup(const AttnArgs& a, int64_t B, int64_t D, int n_seq
   const int per_cu = D == 64 ? 4 : (D == 128 ? 3 : 2);
   const bool wide = n_seqs > 1 && !a.causal && longest >= 16 && D <= 128 && (!equal || (D == 64 ? longest >= 20 : B * a.Hq * rows_128 > 256));
   const double share = longest <= 8 ? 0.95 : (D == 192 || wide ? 1.4 : (a.causal ? (longest >= 48 ? 1.3 : 1.125) : (D == 64 ? 1.125 : 1.02)));
-  return (double)B * a.Hq * work <= 256.0 * share * per_cu * (double)(longest + 6) ? 32 : 128;
+  if ((double)B * a.Hq * work <= 256.0 * share * per_cu * (double)(longest + 6)) return {32, false};
+  return {128, !a.causal && D <= 128 && B * a.Hq * rows_128 <= (!equal ? 576 : (D == 64 ? 512 : 256))};
 }
 
 template <typename SEQS>
-static int launch_attn_dims(const AttnArgs& a, const SEQS& seqs, int B, int row_blocks, int rows, int64_t D, int64_t Dv, hipStream_t st) {
-  if (rows == 32) return launch_attn_split(a, seqs, B, row_blocks, D, Dv, st);
+static int launch_attn_dims(const AttnArgs& a, const SEQS& seqs, int B, int row_blocks, const LaunchPlan& plan, int64_t D, int64_t Dv, hipStream_t st) {
+  if (plan.rows == 32) return launch_attn_split(a, seqs, B, row_blocks, D, Dv, st);
   switch (D + (Dv == 128 ? 1 : 0)) {
-    case 64: return launch_attn<1, 2>(a, seqs, B, row_blocks, st);
-    case 65: return launch_attn<1, 4>(a, seqs, B, row_blocks, st);
-    case 128: return launch_attn<2, 2>(a, seqs, B, row_blocks, st);
-    case 129: return launch_attn<2, 4>(a, seqs, B, row_blocks, st);
-    case 192: return launch_attn<3, 2>(a, seqs, B, row_blocks, st);
-    case 193: return launch_attn<3, 4>(a, seqs, B, row_blocks, st);
-    case 256: return launch_attn<4, 2>(a, seqs, B, row_blocks, st);
-    case 257: return launch_attn<4, 4>(a, seqs, B, row_blocks, st);
+    case 64: return launch_attn<1, 2>(a, seqs, B, row_blocks, plan.alone, st);
+    case 65: return launch_attn<1, 4>(a, seqs, B, row_blocks, plan.alone, st);
+    case 128: return launch_attn<2, 2>(a, seqs, B, row_blocks, plan.alone, st);
+    case 129: return launch_attn<2, 4>(a, seqs, B, row_blocks, plan.alone, st);
+    case 192: return launch_attn<3, 2>(a, seqs, B, row_blocks, plan.alone, st);
+    case 193: return launch_attn<3, 4>(a, seqs, B, row_blocks, plan.alone, st);
+    case 256: return launch_attn<4, 2>(a, seqs, B, row_blocks, plan.alone, st);
+    case 257: return launch_attn<4, 4>(a, seqs, B, row_blocks, plan.alone, st);
   }
   return ALTO_MXFP4_EINVAL;
 }
@@ -452,8 +486,8 @@ extern "C" int alto_mxfp4_attention_fwd_ex(const void* q_codes, const void* q_sc
              (const uint8_t*)vt_codes, (const uint8_t*)v_scales, out, lse, Hq * Sq * Dv, Sq * Dv, Dv, Hq * Sq, Sq, 1, (int)Hq, (int)Hk, (int)Sq, (int)Sk,
              (int)Sk_used, B * Hk * Sk * (D / 2), B * Hk * Dv * (Sk / 2), sm_scale, causal ? 1 : 0,
              bias, bias_sb, bias_sh, bias_sm, bias_bytes, alibi_slopes, alibi_sb, alibi_sh};
-  const int rows = rows_per_workgroup(a, B, D, 0, nullptr, nullptr);
-  return launch_attn_dims(a, AttnNoSeqs{}, (int)B, (int)((Sq + rows - 1) / rows), rows, D, Dv, (hipStream_t)stream);
+  const LaunchPlan plan = launch_plan(a, B, D, 0, nullptr, nullptr);
+  return launch_attn_dims(a, AttnNoSeqs{}, (int)B, (int)((Sq + plan.rows - 1) / plan.rows), plan, D, Dv, (hipStream_t)stream);
 }
 
 namespace alto {
@@ -501,8 +535,8 @@ static int attention_fwd_strided(const QueryOperand& q, const void* k_codes, con
   if (n_seqs == 0) {
     ALTO_REQUIRE(!causal || Sq <= Sk, "attention_fwd: causal attention needs Sq <= Sk (got %lld > %lld)", (long long)Sq, (long long)Sk);
     ALTO_REQUIRE((Sq + 127) / 128 <= 65535, "attention_fwd: Sq / 128 must fit a grid dimension");
-    const int rows = rows_per_workgroup(a, B, D, 0, nullptr, nullptr);
-    return launch_attn_dims(a, AttnNoSeqs{}, (int)B, (int)((Sq + rows - 1) / rows), rows, D, Dv, st);
+    const LaunchPlan plan = launch_plan(a, B, D, 0, nullptr, nullptr);
+    return launch_attn_dims(a, AttnNoSeqs{}, (int)B, (int)((Sq + plan.rows - 1) / plan.rows), plan, D, Dv, st);
   }
   if (const int rc = check_boundaries(B, Sq, Sk, n_seqs, cu_q, cu_k, causal)) return rc;
   // longest sequences first, up to ATTN_MAX_SEQS of them and 65535 row blocks per launch
@@ -516,7 +550,8 @@ static int attention_fwd_strided(const QueryOperand& q, const void* k_codes, con
     const int kx = cu_k[x + 1] - cu_k[x], ky = cu_k[y + 1] - cu_k[y];
     return kx != ky ? kx > ky : x < y;
   });
-  const int rows = rows_per_workgroup(a, 1, D, n_seqs, cu_q, cu_k);
+  const LaunchPlan plan = launch_plan(a, 1, D, n_seqs, cu_q, cu_k);
+  const int rows = plan.rows;
   for (int at = 0; at < n_seqs;) {
     AttnSeqs t;
     t.n = 0;
@@ -529,7 +564,7 @@ static int attention_fwd_strided(const QueryOperand& q, const void* k_codes, con
       t.z0[t.n + 1] = t.z0[t.n] + blocks;
       ++t.n;
     }
-    const int rc = launch_attn_dims(a, t, 1, t.z0[t.n], rows, D, Dv, st);
+    const int rc = launch_attn_dims(a, t, 1, t.z0[t.n], plan, D, Dv, st);
     if (rc != ALTO_MXFP4_OK) return rc;
   }
   return ALTO_MXFP4_OK;
@@ -568,7 +603,7 @@ extern "C" int alto_mxfp4_attention_rows_per_workgroup(int64_t B, int64_t Hq, in
     if (const int rc = check_boundaries(B, Sq, Sk, n_seqs, cu_q, cu_k, causal)) return rc;
   AttnArgs a{};
   a.Hq = (int)Hq; a.Sq = (int)Sq; a.Sk_used = (int)Sk; a.causal = causal ? 1 : 0;
-  return rows_per_workgroup(a, B, D, n_seqs, cu_q, cu_k);
+  return launch_plan(a, B, D, n_seqs, cu_q, cu_k).rows;
 }
 
 extern "C" int alto_mxfp4_attention_fwd(const void* q_codes, const void* q_scales, const void* k_codes, const void* k_scales,

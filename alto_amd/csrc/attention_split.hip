@@ -138,7 +138,7 @@ __device__ __forceinline__ void attn_split_body(const AttnArgs& a, const SEQS& s
       mask_scores(S, (a.causal && qrow + shift + 1 < kn ? qrow + shift + 1 : kn) - key0 - 8 * h);
     }
     float mx;
-    row_maxima(S, tile_max, mx);
+    row_maxima<false>(S, tile_max, mx);
     mx = kb < nblk ? mx * cs : -__builtin_inff();
     reinterpret_cast<float*>(lds + L::MAXIMA)[(4 * buf + wave) * 32 + r] = mx;   // (both lanes of a row hold it)
   };

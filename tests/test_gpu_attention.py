@@ -437,3 +437,36 @@ def test_rescale_of_single_rows(m, dims):
         for i in (0, B - 1):
             assert _rel(out[i:i + 1].cpu(), ref) <= REL_L2, (B, i)
             assert float((lse[i:i + 1].cpu() - ref_lse).abs().max()) <= 1e-4, (B, i)
+
+
+# (head dim, query length, key length or sequence boundaries, heads of a launch with the waves alone, heads of one without)
+ALONE = [(64, 288, 288, 110, 176), (64, 96, 544, 400, 520), (64, 1024, 1024, 40, 72), (128, 288, 288, 84, 96), (128, 1056, 1056, 26, 32),
+         (64, [0, 288, 2016], None, 28, 36), (128, [0, 288, 2016], None, 20, 36)]
+
+
+@pytest.mark.parametrize("Dv", [64, 128])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("case", ALONE, ids=lambda c: f"D{c[0]}_{c[1] if isinstance(c[1], int) else 'packed'}")
+def test_launches_with_the_waves_alone_keep_their_bits(m, case, dtype, Dv):
+    """All keys: up to one workgroup of 128 rows a unit (two with heads of 64, 576 with sequences of different lengths) the kernel that rescales all rows at once,
+    beyond it the one that takes them in groups.  The same heads in a launch on either side of the line."""
+    D, Sq, Sk, few, many = case
+    g = torch.Generator(device=DEV).manual_seed(D + few)
+    packed = not isinstance(Sq, int)
+    tokens = (Sq[-1], Sq[-1]) if packed else (Sq, Sk)
+    bands = sum((b - a + 127) // 128 for a, b in zip(Sq, Sq[1:])) if packed else (Sq + 127) // 128
+    limit = 576 if packed else 512 if D == 64 else 256
+    assert few * bands <= limit < many * bands
+    cu = (Sq, Sq) if packed else (None, None)
+    assert {attention_rows(1, H, *tokens, D, False, *cu) for H in (few, many)} == {128}
+    q, k, v = (torch.randn(n, many, d, device=DEV, generator=g).to(dtype) for n, d in ((tokens[0], D), (tokens[1], D), (tokens[1], Dv)))
+    q[: tokens[0] // 2] *= 4   # maxima that rise late in some rows and early in others
+
+    def run(H):
+        if packed:
+            return m.triton_attention_mxfp4(q[:, :H], k[:, :H], v[:, :H], cu_seqlens_q=Sq, cu_seqlens_k=Sq, causal=False, layout="thd")[:2]
+        out, lse, _ = m.triton_attention_mxfp4(*(t[:, :H].transpose(0, 1).unsqueeze(0) for t in (q, k, v)), causal=False)
+        return out[0].transpose(0, 1), lse[0].transpose(0, 1)
+
+    (out, lse), (ref, ref_lse) = run(few), run(many)
+    assert torch.equal(out, ref[:, :few]) and torch.equal(lse, ref_lse[:, :few])

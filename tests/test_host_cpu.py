@@ -545,3 +545,14 @@ def test_clipped_bf16_rows_are_converted_in_pairs(tmp_path):
     assert len(kernels) == 2
     for name, ops in kernels.items():
         assert not any(op.startswith("v_cvt_scalef32_pk_fp4_f32") for op in ops) and sum(op.startswith("v_cvt_scalef32_pk_fp4_bf16") for op in ops) == 16, name
+
+
+def test_attention_of_waves_alone_rescales_without_branches(tmp_path):
+    """The kernel for launches of about one wave a SIMD has one branch where the other chooses between four groups of rows, and no spills."""
+    from alto_amd import build
+    kernels = _kernel_instructions(build.lib_path(), r"15attn_fwd_kernelILi[12]ELi[24]ELb0ELb[01]ELb[01]E\w*$", tmp_path)
+    alone = [n for n in kernels if re.search(r"ELb1ENS_", n)]
+    assert len(alone) == 16 and len(kernels) == 32
+    for name in alone:
+        branches, grouped = (sum(op.startswith("s_cbranch") for op in kernels[n]) for n in (name, name.replace("ELb1ENS_", "ELb0ENS_")))
+        assert branches <= grouped - 4 and not any(op.startswith("scratch_") for op in kernels[name]), name
