@@ -16,6 +16,7 @@
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/custom_function.h>
+#include <torch/csrc/autograd/python_cpp_function.h>
 
 #include <algorithm>
 #include <cstring>
@@ -751,9 +752,38 @@ py::tuple draw_hadamard(const std::optional<at::Generator>& gen, at::ScalarType 
   return py::make_tuple(signs, perm);
 }
 
+// A node as the interpreter sees it (y.grad_fn): torch's own attributes, with the name and the saved tensors that a Python function's node has.
+template <typename Step>
+PyObject* node_saved_tensors(PyObject* self, void*) {
+  HANDLE_TH_ERRORS
+  const auto& node = reinterpret_cast<torch::autograd::THPCppFunction*>(self)->cdata;
+  const variable_list saved = static_cast<torch::autograd::CppNode<Step>&>(*node).ctx_.get_saved_variables();
+  py::tuple out(saved.size());
+  for (size_t i = 0; i < saved.size(); ++i) out[i] = py::cast(saved[i]);
+  return out.release().ptr();
+  END_HANDLE_TH_ERRORS
+}
+PyObject* node_name(PyObject* self, PyObject*) { return PyUnicode_FromString(Py_TYPE(self)->tp_name); }
+
+template <typename Step>
+void introduce_node(const char* name) {
+  static PyTypeObject type;
+  static PyGetSetDef saved_tensors = {"saved_tensors", node_saved_tensors<Step>, nullptr, nullptr, nullptr};
+  static PyMethodDef name_method = {"name", node_name, METH_NOARGS, nullptr};
+  torch::autograd::_initFunctionPyTypeObject(type, name, nullptr, nullptr);
+  const py::object getter = py::reinterpret_steal<py::object>(PyDescr_NewGetSet(&type, &saved_tensors));
+  const py::object method = py::reinterpret_steal<py::object>(PyDescr_NewMethod(&type, &name_method));
+  if (!getter || !method || PyDict_SetItemString(type.tp_dict, "saved_tensors", getter.ptr()) != 0 || PyDict_SetItemString(type.tp_dict, "name", method.ptr()) != 0)
+    throw py::error_already_set();
+  PyType_Modified(&type);
+  torch::autograd::registerCppFunction(typeid(torch::autograd::CppNode<Step>), &type);
+}
+
 }  // namespace
 
 PYBIND11_MODULE(alto_mxfp4_host, m) {
+  introduce_node<LinearNode>("MXFP4LinearStepBackward");
+  introduce_node<GroupedNode>("MXFP4GroupedStepBackward");
   m.def("bind", &bind);
   m.def("quantize", &quantize);
   m.def("dequantize", &dequantize);

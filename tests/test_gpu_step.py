@@ -404,3 +404,33 @@ def test_step_nodes_in_the_engine(m, kind):
     if kind == "linear":
         with pytest.raises(RuntimeError, match="is a view and is being modified inplace"):
             fn(x).mul_(2)
+
+
+@pytest.mark.parametrize("kind", ["linear", "grouped"])
+def test_a_steps_node_shows_its_name_and_saved_tensors(m, kind):
+    """y.grad_fn of a native node: the name and the saved tensors that a Python function's node has, released by the backward like those, and the
+    attributes of any node."""
+    from alto_amd.mxfp4 import grouped_gemm as G
+    from alto_amd.mxfp4.linear import MXFP4LinearStep
+    x = randn_outliers((512, 544), torch.bfloat16, seed=1).to(DEV).requires_grad_(True)
+    if kind == "linear":
+        w = randn_outliers((160, 544), torch.bfloat16, seed=2).to(DEV).requires_grad_(True)
+        apply = lambda: MXFP4LinearStep.apply(x, w, False, True, False, False, "none", False, None, False)
+    else:
+        w = randn_outliers((4, 512, 544), torch.bfloat16, seed=2).to(DEV).requires_grad_(True)
+        offs = torch.tensor([0, 96, 320, 320, 512], dtype=torch.int32, device=DEV)
+        apply = lambda: G.MXFP4GroupedStep.apply(x, w, offs, False, True, False, False, "none", None, False)
+    with _routes() as declined:
+        y = apply()
+    assert declined["forward"] == 0
+    node = y.grad_fn
+    name = {"linear": "MXFP4LinearStepBackward", "grouped": "MXFP4GroupedStepBackward"}[kind]
+    assert type(node).__name__ == name and node.name() == name and name in repr(node)
+    saved = node.saved_tensors
+    assert isinstance(saved, tuple) and all(t.is_cuda for t in saved) and len(saved) == {"linear": 2, "grouped": 4}[kind]
+    assert [f.variable is v for (f, _), v in zip(node.next_functions, (x, w))] == [True, True]
+    y.backward(torch.ones_like(y), retain_graph=True)
+    assert all(torch.equal(a, b) for a, b in zip(node.saved_tensors, saved))
+    y.backward(torch.ones_like(y))
+    with pytest.raises(RuntimeError, match="second time"):
+        node.saved_tensors
