@@ -94,23 +94,33 @@ static int launch_plain(const OperandView& A, const OperandView& B, int64_t M, i
   if (!tail) {
     if (c_dtype == ALTO_DT_BF16) return ALTO_TILED_LAUNCH(__bf16, false, -1, 4);
     else return ALTO_TILED_LAUNCH(float, false, -1, 4);
-  } else if (c_dtype != ALTO_DT_BF16) {
-    return ALTO_TILED_LAUNCH(float, true, -1, 4);   // (fp32 output: the general ending)
-  } else {
-    // K is known here: the kernel that ends the reduction exactly where K ends
-    int lms, nst;
-    gemm_tile_last_stage(K / 32, lms, nst);
-    switch (lms * 4 + nst - 1) {
-      case 0: return ALTO_TILED_LAUNCH(__bf16, true, 0, 1);
-      case 1: return ALTO_TILED_LAUNCH(__bf16, true, 0, 2);
-      case 2: return ALTO_TILED_LAUNCH(__bf16, true, 0, 3);
-      case 3: return ALTO_TILED_LAUNCH(__bf16, true, 0, 4);
-      case 4: return ALTO_TILED_LAUNCH(__bf16, true, 1, 1);
-      case 5: return ALTO_TILED_LAUNCH(__bf16, true, 1, 2);
-      case 6: return ALTO_TILED_LAUNCH(__bf16, true, 1, 3);
-      default: return ALTO_TILED_LAUNCH(__bf16, true, 1, 4);
-    }
   }
+  // K is known here: the kernel that ends the reduction exactly where K ends
+  int lms, nst;
+  gemm_tile_last_stage(K / 32, lms, nst);
+#define ALTO_TILED_ENDINGS(T)                             \
+  switch (lms * 4 + nst - 1) {                            \
+    case 0: return ALTO_TILED_LAUNCH(T, true, 0, 1);      \
+    case 1: return ALTO_TILED_LAUNCH(T, true, 0, 2);      \
+    case 2: return ALTO_TILED_LAUNCH(T, true, 0, 3);      \
+    case 3: return ALTO_TILED_LAUNCH(T, true, 0, 4);      \
+    case 4: return ALTO_TILED_LAUNCH(T, true, 1, 1);      \
+    case 5: return ALTO_TILED_LAUNCH(T, true, 1, 2);      \
+    case 6: return ALTO_TILED_LAUNCH(T, true, 1, 3);      \
+    default: return ALTO_TILED_LAUNCH(T, true, 1, 4);     \
+  }
+  if (c_dtype == ALTO_DT_BF16) {
+    ALTO_TILED_ENDINGS(__bf16)
+  }
+  // fp32: the 256x256 tile has no registers for these; the 256x128 tile needs them: with whole blocks of 512 the products beyond K (1280 x 512 of
+  // 1536) made short reductions slower than the 128x128 tile they had before, 1408 x 5160 x 1280 15.4 -> 16.1 us (now 14.5), 3585 x 2048 x 1664
+  // 18.5 -> 19.4; over 187 shapes 0.92 of the time of whole blocks.
+  if constexpr (WN == 2) {
+    ALTO_TILED_ENDINGS(float)
+  } else {
+    return ALTO_TILED_LAUNCH(float, true, -1, 4);
+  }
+#undef ALTO_TILED_ENDINGS
 #undef ALTO_TILED_LAUNCH
 }
 
@@ -149,8 +159,8 @@ static int launch_ps(const OperandView& A, const OperandView& B, int64_t M, int6
 // (From 257 tiles on a second round begins, and a narrow tile reads 1.5 times the bytes per product.)  Plain scales, as the inference and
 // the fp32 entry points bring them: bf16 results at 256x256 / 256x128, fp32 results at 128x128 / 256x128, which is what they had:
 //   M x N x K             tiles     bf16          fp32                  M x N x K             tiles     bf16          fp32
-//   2048 x 4096 x 4096     256   28.3 / 23.9   30.9 / 26.8              1000 x 6144 x 1440     192   13.4 / 11.0   18.3 / 16.3
-//   1376 x 4096 x 2880     192   22.1 / 17.3   26.1 / 22.2              333 x 14336 x 7200     224   54.1 / 39.2   60.7 / 45.1
+//   2048 x 4096 x 4096     256   28.3 / 23.9   30.9 / 26.8              1000 x 6144 x 1440     192   13.4 / 11.0   18.7 / 15.7
+//   1376 x 4096 x 2880     192   22.1 / 17.3   25.1 / 20.9              333 x 14336 x 7200     224   54.1 / 39.2   52.7 / 40.4
 //   1536 x 4096 x 14336    192   72.4 / 59.6   71.9 / 62.2              1100 x 4096 x 512      160    8.4 /  6.8   10.8 / 10.3
 bool gemm_narrow_pays(int64_t M, int64_t N) { return ((M + GT_TM - 1) / GT_TM) * ((N + TileOf<2>::TN - 1) / TileOf<2>::TN) <= 256; }
 

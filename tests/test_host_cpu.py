@@ -556,3 +556,12 @@ def test_attention_of_waves_alone_rescales_without_branches(tmp_path):
     for name in alone:
         branches, grouped = (sum(op.startswith("s_cbranch") for op in kernels[n]) for n in (name, name.replace("ELb1ENS_", "ELb0ENS_")))
         assert branches <= grouped - 4 and not any(op.startswith("scratch_") for op in kernels[name]), name
+
+
+def test_fp32_products_on_narrow_tiles_end_where_k_ends():
+    """A 256x128 tile with fp32 results has a kernel for each place where a reduction can end inside its blocks of 512, as with bf16 results."""
+    from alto_amd import build
+    names = "\n".join(_kernel_metadata(build.lib_path()))
+    for result in ("IDF16b", "If"):
+        ends = set(re.findall(r"17gemm_tiled_kernel" + result + r"Lb1ELi([01])ELi([1-4])ELb0ELi2E", names))
+        assert ends == {(a, b) for a in "01" for b in "1234"}, result
