@@ -1,4 +1,5 @@
 // Ragged grouped MXFP4 GEMMs for MoE experts (gfx950): forward / dX (rows grouped by expert) and dW (reduction grouped by expert).
+#include <cmath>
 #include <mutex>
 
 #include "common.h"
@@ -571,17 +572,25 @@ inline int64_t grouped_max_passes(int64_t M_total, int64_t num_groups) { return 
 inline int64_t grouped_workspace_bytes(int64_t M_total, int64_t num_groups) { return 16 + 16 * grouped_max_passes(M_total, num_groups); }
 
 // Packed scales, bf16 result: the 256x128 tile where one round of the 256 compute units takes all tiles, as in the dense product
-// (gemm_tiled_launch_ps).  Only the device knows how many passes there are; expected are the whole bands of 256 rows and half a
-// pass more per group (a partial tile each, half of them filling up a band), at least one per group.  A wrong guess costs either way
-// what the wrong side of the line below does.  us at 256x256 / 256x128, even routing:
+// (gemm_tiled_launch_ps).  Only the device knows how many passes there are; expected are one per 256 rows and half a pass more per group (a
+// partial tile each, half of them filling up a band), at least one per group, with a deviation of sqrt(groups / 12).  A wrong guess costs what the wrong
+// side of the line below does, more on the narrow side: what has to fit is the expectation and 1.5 deviations (no more than there can be), and the
+// passes of groups of equal size.  Of 110 forwards with 190 to 256 tiles by the expectation (even, random and 1 / rank routing) the 88 that this lets
+// through take 0.94 of the 256x256 tile's time, none more than 0.99; of the others some 9 to 11 % more, where a few passes came on top (768 x 3648 x 512,
+// 8 groups of 1 / rank, 261 tiles: 26.4 / 28.7; 2240 x 2912 x 1760, 4 equal groups, 276: 38.1 / 41.6).  (A kernel that holds both tiles and chooses by the
+// passes spills 30 to 60 registers.)  us at 256x256 / 256x128, even routing:
 //   rows  groups    N     K   tiles of 256x128              rows  groups    N     K   tiles of 256x128
 //   2560    8    1440  1024      168  10.6 /  9.1           2048    4    2880  1440      230  13.3 / 11.4
 //   4096    8    1440  2880      240  19.8 / 17.1           8192   64     512  2048      288  16.1 / 21.7
 //   2048   16    1024  4096      136  22.1 / 18.2           8192    8    1024  2880      304  21.1 / 28.3
 //   4096   32     768  2048      210  15.0 / 12.9           8192    8    2048  2880      608  43.0 / 43.4
 inline bool grouped_narrow_pays(int64_t M_total, int64_t num_groups, int64_t N) {
-  const int64_t bands = M_total / GT_TM + 1, half = (num_groups + 1) / 2;
-  return ((bands > half ? bands : half) + half) * ((N + TileOf<2>::TN - 1) / TileOf<2>::TN) <= 256;
+  const double rows = (double)M_total / GT_TM, half = 0.5 * (double)num_groups;
+  const int64_t likely = (int64_t)((rows > half ? rows : half) + half + 1.5 * std::sqrt((double)num_groups / 12.0));
+  const int64_t most = M_total > num_groups ? (M_total - num_groups) / GT_TM + num_groups : M_total;
+  const int64_t even = num_groups * ((M_total + num_groups * GT_TM - 1) / (num_groups * GT_TM));
+  const int64_t passes = likely < most ? likely : most;
+  return (passes > even ? passes : even) * ((N + TileOf<2>::TN - 1) / TileOf<2>::TN) <= 256;
 }
 
 inline int grouped_run_log2(int64_t M_total, int64_t num_experts) { return M_total >= 4ll * GT_TM * num_experts ? 2 : 0; }   // see grouped_tile_coords

@@ -105,3 +105,21 @@ def test_pass_list(m, groups, form):
     got = ws.cpu()
     assert torch.equal(back.cpu(), offs.to(torch.int32))
     assert got[0] == len(want) and got[4:4 + 4 * len(want)].view(-1, 4).tolist() == [list(w) for w in want]
+
+
+# Seven experts of 257 rows and one of one: 15 passes where 11 to 12 are expected, 285 narrow tiles in two rounds
+@pytest.mark.parametrize("K", [512, 544, 1024])
+def test_narrow_tiles_in_two_rounds(m, K):
+    from alto_amd.mxfp4 import grouped_gemm as G
+    from alto_amd.mxfp4.linear import pack_scales
+    sizes, N = [257] * 7 + [1], 2432
+    E, M = len(sizes), sum(sizes)
+    aq, as_ = m.convert_to_mxfp4(randn_outliers((M, K), torch.bfloat16, seed=M + K).to(DEV))
+    wq, ws = m.convert_to_mxfp4((randn_outliers((E, N, K), torch.bfloat16, seed=N) * 0.02).to(DEV))
+    groups = G.groups_from_offsets(torch.tensor([0] + sizes).cumsum(0).to(torch.int32).to(DEV))
+    out = G.grouped_forward_packed(aq, pack_scales(as_, M, K), wq, G.pack_expert_scales(ws, N, K, False), groups)
+    lo = 0
+    for e, n in enumerate(sizes):
+        ref = m.blockwise_mxfp4_gemm(aq[lo:lo + n], as_[lo:lo + n], wq[e], ws[e], trans_b=True, output_dtype=torch.bfloat16)
+        assert torch.equal(out[lo:lo + n], ref), f"expert {e}"
+        lo += n

@@ -67,3 +67,50 @@ def test_a_failed_kernel_set_up_is_reported_by_every_call(tmp_path):
             assert code == -2 and "LDS" in message, (name, calls)
         assert launched == 0, (name, launched)   # no kernel ran on operands that only it would have completed
         assert pending == 0, name                # and the next call of anything does not report this one's error
+
+
+TILE_STAND_INS = r"""
+typedef struct { unsigned x, y, z; } dim3;
+static unsigned threads = 0;
+int hipFuncSetAttribute(const void* f, int what, int value) { return 0; }
+int hipGetLastError(void) { return 0; }
+int __hipPushCallConfiguration(dim3 grid, dim3 block, unsigned long lds, void* stream) { threads = block.x; return 1; }   /* (no launch follows) */
+unsigned last_threads(void) { return threads; }
+"""
+
+TILE_CHILD = r"""
+import ctypes, json, sys
+runtime = ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)
+lib = ctypes.CDLL(sys.argv[2])
+args, res, shapes = json.loads(sys.argv[3])
+fn = lib.alto_mxfp4_grouped_gemm_ps
+fn.argtypes, fn.restype = [getattr(ctypes, t) for t in args], getattr(ctypes, res)
+lib.alto_mxfp4_last_error.restype = ctypes.c_char_p
+memory = ctypes.create_string_buffer(1 << 16)
+p = (ctypes.addressof(memory) + 255) // 256 * 256
+out = []
+for rows, groups, N, K in shapes:
+    rc = fn(p, K // 2, p, p, N * K // 2, K // 2, p, N * 16 * ((K + 511) // 512), p, None, groups, groups, rows, N, K, p, N, p, 1 << 20, 1, None)
+    out.append([rc, runtime.last_threads(), lib.alto_mxfp4_last_error().decode()])
+print(json.dumps(out))
+"""
+
+
+def test_narrow_grouped_tiles_leave_room_for_more_passes_than_expected(tmp_path):
+    """Which tile a grouped product takes (threads of its launch: 256 for 256x128, 512 for 256x256): one round of 256 narrow tiles has to hold with some more
+    passes than expected, and with the passes of equal groups."""
+    (tmp_path / "stand_ins.c").write_text(TILE_STAND_INS)
+    stand_ins = str(tmp_path / "stand_ins.so")
+    subprocess.run(["gcc", "-shared", "-fPIC", "-w", str(tmp_path / "stand_ins.c"), "-o", stand_ins], check=True)
+    _lib.load()
+    narrow = [(2560, 8, 1440, 1024), (2048, 4, 2560, 1440), (2048, 16, 1024, 4096), (4096, 32, 768, 2048), (4096, 8, 1440, 2880), (2048, 4, 2880, 1440), (256, 1, 4096, 512), (1800, 8, 2432, 512)]
+    wide = [(2240, 4, 2912, 1760), (768, 8, 3648, 512), (2432, 16, 1728, 512), (3168, 32, 960, 2048),   # (no room)
+            (4160, 16, 1152, 1024),                                                                      # (equal groups of 260 rows: 32 passes, 25 expected)
+            (8192, 64, 512, 2048), (8192, 8, 2048, 2880)]
+    sig = _lib.SIGNATURES["alto_mxfp4_grouped_gemm_ps"]
+    r = subprocess.run([sys.executable, "-c", TILE_CHILD, stand_ins, os.path.join(B.LIBDIR, B.LIBNAME), json.dumps([[t.__name__ for t in sig[1]], sig[0].__name__, narrow + wide])],
+                       capture_output=True, text=True, timeout=120)
+    assert r.returncode == 0, r.stderr[-2000:]
+    got = json.loads(r.stdout.splitlines()[-1])
+    assert [g[0] for g in got] == [0] * len(got), got
+    assert [g[1] for g in got] == [256] * len(narrow) + [512] * len(wide), list(zip(narrow + wide, got))
