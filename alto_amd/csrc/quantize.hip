@@ -580,7 +580,8 @@ __device__ __forceinline__ void quant_tile(const QuantParams& p, unsigned wg, un
         // convert per pair of rows
         if (GEN && p.clip_col) {
           // Transformed bf16: in the pairs, so that z ends above.  Unpacked under this condition it stayed beside the pairs in 81 to 104 registers
-          // instead of 42 to 64 (8 waves a SIMD): static clip, 8192 x 4096, dY 35.9 -> 30.2 us, x 27.5 -> 24.6; with UOS 34.5 -> 31.1, 27.2 -> 25.9.
+          // instead of 42 to 64 (8 waves a SIMD): static clip, 8192 x 4096, both copies, plain scales, dY 39.4 -> 34.3 us, x 31.0 -> 29.5; with UOS 38.5 -> 35.3, 31.1
+          // -> 30.2 (and with the rows as they are above 31.5, 29.3; 32.3, 30.0).
           if constexpr (BF && RHT) {
   #pragma unroll
             for (int j = 0; j < 16; ++j) zp[j] = pack_bf16x2(bf16_lo(zp[j]) * 0.75f, bf16_hi(zp[j]) * 0.75f);
